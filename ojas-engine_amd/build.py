@@ -34,6 +34,7 @@ FAMILIES = {
     "glue": ("glue.hip", []),
     "gemm": ("gemm.hip", ["-ffp-contract=off"]),
     "gemm_xl": ("gemm_xl.hip", ["-ffp-contract=off"]),
+    "gemm_f16": ("gemm_f16.hip", []),
     "gemm_q8k": ("gemm_q8k.hip", []),
     "moe": ("moe.hip", ["-DOJK_ASM_FIRST_DOT"]),
     "moe_iq": ("moe_iq.hip", []),

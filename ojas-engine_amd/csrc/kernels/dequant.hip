@@ -10,6 +10,7 @@
 // Signature convention: pointers first, then u32 scalars.
 //   dequant_<fmt>_f16(const uchar* w, ushort* out, uint nblocks)
 #include "ojk_common.h"
+#include "ojk_map.h"
 
 // The f32 value is pinned in a register before the conversion: left to itself the compiler folds
 // "multiply, then convert" into one mixed-precision FMA, which rounds once instead of twice and
@@ -38,10 +39,8 @@ __device__ __forceinline__ void store8_f16(ushort* o, const ushort (&h)[8]) {
 }
 __device__ __forceinline__ uint byte_of(uint lo, uint hi, int i) { return ((i < 4 ? lo : hi) >> (8 * (i & 3))) & 0xFFu; }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q80_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q80(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // four threads per block, eight consecutive weights each
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 2;
     if (b >= nblocks) return;
     const uint j = (uint)tid & 3u;
@@ -81,11 +80,9 @@ embed_q80_g(const uchar* __restrict__ table, float* __restrict__ out, const uint
     embed_q80_row(table, out, ctl[0], d, ROWS);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q4k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q4k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // 32 threads per super-block; thread t owns eight consecutive weights: chunk c = t / 8 (64 weights, the low
     // nibbles of its 32 bytes then the high ones), half hi = (t / 4) % 2, bytes 8 (t % 4) .. + 7 of the chunk.
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, c = t >> 3, hi = (t >> 2) & 1u, part = t & 3u;
@@ -104,10 +101,8 @@ dequant_q4k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblo
     store8_f16(out + b * 256u + c * 64u + hi * 32u + part * 8u, h);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q5k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q5k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // As Q4_K, plus the fifth bit: bit 2 c + hi of qh[l], l the byte's place among the chunk's 32.
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, c = t >> 3, hi = (t >> 2) & 1u, part = t & 3u;
@@ -130,13 +125,11 @@ dequant_q5k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblo
     store8_f16(out + b * 256u + c * 64u + hi * 32u + part * 8u, h);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q6k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q6k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // 32 threads per super-block; thread t owns eight consecutive weights: half hf = t / 16, quarter j = (t / 4) % 4 of
     // its 128 (weights 32 j ..: the low nibbles of ql[0..31], of ql[32..63], then the high nibbles of each), places
     // l = 8 (t % 4) .. + 7; bits 2 j, 2 j + 1 of qh[l] on top, scale l / 16 + 2 j.
     // The value is (d * sc) * q, left to right, as the reference writes it.
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, hf = t >> 4, j = (t >> 2) & 3u, l0 = (t & 3u) * 8u;
@@ -189,11 +182,9 @@ relayout_q4k_q4l(const uchar* __restrict__ w, uchar* __restrict__ nib, ushort* _
     *(uint4*)(nib + tid * 16u) = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_iq4nl_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_iq4nl(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // four threads per block, eight consecutive weights each: weights 0..15 are the low nibbles of qs[0..15], 16..31
     // the high nibbles
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 2;
     if (b >= nblocks) return;
     const uint j = (uint)tid & 3u, hi = j >> 1, part = j & 1u;
@@ -207,11 +198,9 @@ dequant_iq4nl_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nb
     store8_f16(out + b * 32u + 16u * hi + 8u * part, h);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_iq4xs_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_iq4xs(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // 32 threads per super-block; thread t owns eight consecutive weights of sub-block ib = t / 4: the low (hi = 0) or
     // high nibbles of its bytes 8 (t % 2) .. + 7, which are weights 16 hi + 8 (t % 2) .. of the sub-block.
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, ib = t >> 2, hi = (t >> 1) & 1u, part = t & 1u;
@@ -234,11 +223,9 @@ dequant_iq4xs_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nb
 // bytes holds weights l, l + 32, l + 64, l + 96 at bits 0, 2, 4, 6, and scale 8 half + 2 j + l / 16 covers the
 // 16 weights (plane j, l / 16).  32 threads per super-block; thread t decodes the eight consecutive weights
 // 128 half + 32 j + 8 (t % 4) .. + 7 with half = t / 16, j = (t / 4) % 4.
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q2k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q2k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // block { u8 scales[16]; u8 qs[64]; half d; half dmin; }: w = (d * sc) * q - dmin * m, every step rounded
     // (crates/ojas-formats/src/gguf.rs:730-754)
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, half = t >> 4, j = (t >> 2) & 3u, l0 = (t & 3u) * 8u;
@@ -255,12 +242,10 @@ dequant_q2k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblo
     store8_f16(out + b * 256u + half * 128u + j * 32u + l0, h);
 }
 
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q3k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_q3k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // block { u8 hmask[32]; u8 qs[64]; u8 scales[12]; half d; }: w = (d * (sc - 32)) * (q - (mask bit ? 0 : 4)),
     // bit 4 half + j of hmask[l] belonging to weight (half, j, l) (crates/ojas-formats/src/gguf.rs:755-795).
     // Blocks are 110 bytes: two-byte alignment is all a block has.
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 5;
     if (b >= nblocks) return;
     const uint t = (uint)tid & 31u, half = t >> 4, j = (t >> 2) & 3u, l0 = (t & 3u) * 8u;
@@ -288,9 +273,8 @@ dequant_q3k_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblo
 // of qs[j], else the high nibble of qs[j - 16]).  AFFINE: {d, m} header and w = d * q + m (a product and a sum, each
 // rounded), else w = d * (q - 8 | 16); FIVE: a 4-byte field of fifth bits ahead of the nibbles.
 template <bool FIVE, bool AFFINE>
-__device__ __forceinline__ void dequant_legacy(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_legacy(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     const uint BYTES = 18u + (AFFINE ? 2u : 0u) + (FIVE ? 4u : 0u), HDR = AFFINE ? 4u : 2u;
-    size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     size_t b = tid >> 2;
     if (b >= nblocks) return;
     const uint j4 = (uint)tid & 3u, hi = j4 >> 1, part = j4 & 1u;
@@ -313,21 +297,10 @@ __device__ __forceinline__ void dequant_legacy(const uchar* __restrict__ w, usho
     }
     store8_f16(out + b * 32u + 16u * hi + 8u * part, h);
 }
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q40_f16(const uchar* w, ushort* out, uint nblocks) { dequant_legacy<false, false>(w, out, nblocks); }
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q41_f16(const uchar* w, ushort* out, uint nblocks) { dequant_legacy<false, true>(w, out, nblocks); }
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q50_f16(const uchar* w, ushort* out, uint nblocks) { dequant_legacy<true, false>(w, out, nblocks); }
-extern "C" __global__ void __launch_bounds__(256)
-dequant_q51_f16(const uchar* w, ushort* out, uint nblocks) { dequant_legacy<true, true>(w, out, nblocks); }
-
 // MXFP4 (crates/ojas-formats/src/mxfp4.rs:40-58): { u8 e; u8 qs[16] }, w = 2^(e - 127) * E2M1[code], weight 2j the low
 // and 2j + 1 the high nibble of qs[j].  The product of a power of two and a 2-bit significand is exact; one rounding to f16.
-extern "C" __global__ void __launch_bounds__(256)
-dequant_mxfp4_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks) {
+__device__ __forceinline__ void decode_mxfp4(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // four threads per block, eight consecutive weights each: the nibbles of four consecutive bytes of codes
-    const size_t tid = (size_t)blockIdx.x * 256u + threadIdx.x;
     const size_t b = tid >> 2;
     if (b >= nblocks) return;
     const uint p = (uint)tid & 3u;
@@ -346,3 +319,42 @@ dequant_mxfp4_f16(const uchar* __restrict__ w, ushort* __restrict__ out, uint nb
     }
     store8_f16(out + b * 32u + 8u * p, h);
 }
+
+// dequant_<fmt>_f16(w, out, nblocks): the rows as f16.
+// dequant_<fmt>_f16_x(w, out, x, xh, z, nblocks, n, nz, CB, BF16): everything a batch needs ahead of its f16 product in one
+// launch — the first CB workgroups convert n activations (f32, or bf16 where BF16 is set) to f16 and clear nz dwords of z
+// (an output that K slices add into), the others decode.  Bound by memory; as launches of
+// their own the parts would each add a few us of an idle chip (6914 x 2816 Q6_K rows beside 333 tokens: 12 us, 60 MB).
+template <class F>
+__device__ __forceinline__ void decode_beside(F decode, const void* __restrict__ x, ushort* __restrict__ xh, uint* __restrict__ z,
+                                              uint n, uint nz, uint CB, uint BF16) {
+    if (blockIdx.x >= CB) {
+        decode((size_t)(blockIdx.x - CB) * 256u + threadIdx.x);
+        return;
+    }
+    const uint t = blockIdx.x * 256u + threadIdx.x, stride = CB * 256u;
+    if (BF16) map8_at((const ushort*)x, xh, n, [](ushort v) { return __half_as_ushort(__float2half_rn(bf16_bits_to_f32(v))); }, t, stride);
+    else map8_at((const float*)x, xh, n, [](float v) { return __half_as_ushort(__float2half_rn(v)); }, t, stride);
+    if (nz) fill_zero_at(z, nz, t, stride);
+}
+#define DEQUANT_ENTRIES(FMT, DECODE)                                                                              \
+    extern "C" __global__ void __launch_bounds__(256) dequant_##FMT##_f16(const uchar* w, ushort* out, uint nblocks) { \
+        DECODE(w, out, nblocks, (size_t)blockIdx.x * 256u + threadIdx.x);                                         \
+    }                                                                                                             \
+    extern "C" __global__ void __launch_bounds__(256) dequant_##FMT##_f16_x(                                      \
+        const uchar* w, ushort* out, const void* x, ushort* xh, uint* z, uint nblocks, uint n, uint nz, uint CB, uint BF16) { \
+        decode_beside([&](size_t tid) { DECODE(w, out, nblocks, tid); }, x, xh, z, n, nz, CB, BF16);              \
+    }
+DEQUANT_ENTRIES(q80, decode_q80)
+DEQUANT_ENTRIES(q4k, decode_q4k)
+DEQUANT_ENTRIES(q5k, decode_q5k)
+DEQUANT_ENTRIES(q6k, decode_q6k)
+DEQUANT_ENTRIES(iq4nl, decode_iq4nl)
+DEQUANT_ENTRIES(iq4xs, decode_iq4xs)
+DEQUANT_ENTRIES(q2k, decode_q2k)
+DEQUANT_ENTRIES(q3k, decode_q3k)
+DEQUANT_ENTRIES(mxfp4, decode_mxfp4)
+DEQUANT_ENTRIES(q40, (decode_legacy<false, false>))
+DEQUANT_ENTRIES(q41, (decode_legacy<false, true>))
+DEQUANT_ENTRIES(q50, (decode_legacy<true, false>))
+DEQUANT_ENTRIES(q51, (decode_legacy<true, true>))

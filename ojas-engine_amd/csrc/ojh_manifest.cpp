@@ -1168,6 +1168,31 @@ static int check_dequant(const ojh_kernel_spec *s, const uint32_t *c, const uint
     return OJH_OK;
 }
 
+// dequant_<fmt>_f16_x(w, out, x, xh, z, nblocks, n, nz, CB, BF16): the decoder with n activations converted to f16 and nz
+// dwords cleared beside it by the first CB workgroups
+static int check_dequant_x(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3],
+                           const uint32_t block[3], size_t need[16], size_t align[16]) {
+    const ojh_block_format *f = ojh_format(s->type);
+    const uint32_t nb = c[0], cb = c[3];
+    if (!f || nb == 0 || cb == 0 || c[1] == 0) return ojh_fail(OJH_ERR_ARG, "%s: nblocks, n and CB must be positive", s->name);
+    int rc = check_block(block, 256);
+    if (rc) return rc;
+    const uint64_t tpb = dequant_threads_per_block(s->type);
+    if (grid[1] != 1 || grid[2] != 1 || (uint64_t)grid[0] < cb + (nb * tpb + 255) / 256)
+        return ojh_fail(OJH_ERR_ARG, "%s: grid does not cover %u blocks beside %u workgroups", s->name, nb, cb);
+    need[0] = (size_t)nb * f->bytes;
+    need[1] = (size_t)nb * f->weights * 2;
+    need[2] = (size_t)c[1] * (c[4] ? 2 : 4);
+    need[3] = (size_t)c[1] * 2;
+    need[4] = (size_t)c[2] * 4;
+    align[0] = ojh_block_align(f);
+    align[1] = 8;
+    align[2] = c[4] ? 2 : 4;
+    align[3] = 2;
+    align[4] = 4;
+    return OJH_OK;
+}
+
 // embed_q80(table, out, token, d) / embed_q80_g(table, out, ctl, d): a thread per weight, grid-stride
 static int check_embed(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3],
                        const uint32_t block[3], size_t need[16], size_t align[16]) {
@@ -1329,6 +1354,49 @@ static int shape_gemm(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t 
         if (s->rows_per_wave == 13 && z > steps / 16) z = steps / 16;   // K over the waves: a super-block per wave and slice at least
         if (z > 16) z = 16;
         grid[2] = z ? z : 1;
+    }
+    block[0] = 256;
+    block[1] = block[2] = 1;
+    return OJH_OK;
+}
+
+// gemm_f16d_{128,256x128,256}(xh, w, y, K, N, accum, M), gemm_f16d_128_sk(xh, w, y, K, N, M, nsplit): plain f16 rows, both
+// operands copied into LDS by the memory system; grid [8 ceil(row tiles / 8) x token tiles, 1 | nsplit, 1].
+// `rows_per_wave`: 16 x (tokens / 128) + rows / 128, + 1024 for the split form
+static int check_gemm_f16d(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3],
+                           const uint32_t block[3], size_t need[16], size_t align[16]) {
+    const bool sk = s->rows_per_wave & 1024;
+    const uint32_t bm = 128u * ((uint32_t)s->rows_per_wave >> 4 & 15u), bn = 128u * ((uint32_t)s->rows_per_wave & 15u);
+    const uint32_t K = c[0], N = c[1], M = sk ? c[2] : c[3], nsplit = sk ? c[3] : 1;
+    if (!K || !N || K % 64) return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u (K a positive multiple of 64)", s->name, K, N);
+    if (!M || !nsplit) return ojh_fail(OJH_ERR_ARG, "%s: M and nsplit must be positive", s->name);
+    int rc = check_block(block, 256);
+    if (rc) return rc;
+    const uint64_t nt = ((uint64_t)N + bn - 1) / bn, mt = ((uint64_t)M + bm - 1) / bm, want = (nt + 7) / 8 * 8 * mt;
+    if (grid[0] != want || grid[1] != nsplit || grid[2] != 1)
+        return ojh_fail(OJH_ERR_ARG, "%s: grid must be [%llu,%u,1]", s->name, (unsigned long long)want, nsplit);
+    // 32-bit byte offsets into both operands
+    if ((uint64_t)M * K * 2 > 0xFFFFFFFFull || (uint64_t)N * K * 2 > 0xFFFFFFFFull)
+        return ojh_fail(OJH_ERR_ARG, "%s: an operand exceeds 4 GiB", s->name);
+    need[0] = (size_t)M * K * 2;
+    need[1] = (size_t)N * K * 2;
+    need[2] = (size_t)M * N * 4;
+    align[0] = align[1] = 16;
+    align[2] = 4;
+    return OJH_OK;
+}
+static int shape_gemm_f16d(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M,
+                           uint32_t grid[3], uint32_t block[3]) {
+    const uint32_t bm = 128u * ((uint32_t)s->rows_per_wave >> 4 & 15u), bn = 128u * ((uint32_t)s->rows_per_wave & 15u);
+    const uint32_t nt = (N + bn - 1) / bn, mt = (M + bm - 1) / bm;
+    grid[0] = (nt + 7) / 8 * 8 * mt;
+    grid[1] = grid[2] = 1;
+    if (s->rows_per_wave & 1024) {   // slices of eight K steps at least, until every CU has one
+        const uint32_t cus = dev ? (uint32_t)dev->prop.multiProcessorCount : 256u, tiles = nt * mt;
+        uint32_t z = tiles ? cus / tiles : 1;
+        if (z > K / 512) z = K / 512;
+        if (z > 16) z = 16;
+        grid[1] = z ? z : 1;
     }
     block[0] = 256;
     block[1] = block[2] = 1;
@@ -1913,6 +1981,14 @@ static int shape_dequant(const ojh_kernel_spec *s, const ojh_device *, uint32_t,
     return OJH_OK;
 }
 
+// ... with activations converted beside it: K = those workgroups
+static int shape_dequant_x(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M,
+                           uint32_t grid[3], uint32_t block[3]) {
+    int rc = shape_dequant(s, dev, 0, N, M, grid, block);
+    grid[0] += K;
+    return rc;
+}
+
 static std::vector<ojh_kernel_spec> build_manifest() {
     std::vector<ojh_kernel_spec> m;
     // `names` must outlive the table: keep them in a static pool.
@@ -1928,6 +2004,7 @@ static std::vector<ojh_kernel_spec> build_manifest() {
         const bool grid_fmt = ojh_grid_type(f.type);
         const char *fam_nat = grid_fmt ? "iq_grid" : "gemv", *fam_q8k = grid_fmt ? "iq_grid" : "gemv_q8k";
         add("dequant_" + t + "_f16", grid_fmt ? "iq_grid" : "dequant", 2, 1, f.type, 0, check_dequant, shape_dequant);
+        if (!grid_fmt) add("dequant_" + t + "_f16_x", "dequant", 5, 5, f.type, 0, check_dequant_x, shape_dequant_x);
         if (f.type == OJH_Q5_K) {   // Q5_K: the decoder, the CPU path's int8-activation matvec
             std::string q5 = "gemv_q8k_" + t;
             add(q5, "gemv_q8k", 4, 2, f.type, 4, check_gemv_q8k, shape_rows);
@@ -2074,6 +2151,10 @@ static std::vector<ojh_kernel_spec> build_manifest() {
     add("gemm_mm_f16_sk", "gemm", 3, 4, OJH_F16, 1, check_gemm, shape_gemm);
     add("gemm_mm_f16_m128", "gemm", 3, 4, OJH_F16, 14, check_gemm, shape_gemm);
     add("gemm_mm_f16_m128_sk", "gemm", 3, 4, OJH_F16, 15, check_gemm, shape_gemm);
+    add("gemm_f16d_128", "gemm_f16", 3, 4, OJH_F16, 16 + 1, check_gemm_f16d, shape_gemm_f16d);
+    add("gemm_f16d_256x128", "gemm_f16", 3, 4, OJH_F16, 32 + 1, check_gemm_f16d, shape_gemm_f16d);
+    add("gemm_f16d_256", "gemm_f16", 3, 4, OJH_F16, 32 + 2, check_gemm_f16d, shape_gemm_f16d);
+    add("gemm_f16d_128_sk", "gemm_f16", 3, 4, OJH_F16, 1024 + 16 + 1, check_gemm_f16d, shape_gemm_f16d);
     // Q4L (relaid Q4_K + side arrays) under the reference's names and argument lists
     add("gemm_mm_q4l", "gemm", 5, 4, 0, 8, check_gemm_q4l, shape_gemm);
     add("gemm_mm_q4l_sk", "gemm", 5, 4, 0, 9, check_gemm_q4l, shape_gemm);

@@ -542,6 +542,72 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
                       {K, ends[0], ends[1], ends[2], ends[3], nrb, (uint32_t)(accum != 0)}, grid, block);
 }
 
+// A batch on plain f16 rows: the format's rows decoded into scratch and the activations converted in one launch, then the
+// tile whose operands the memory system copies (`gemm_f16d_*`) — the same weights (dequant_to_f16's bits) and f16 activations
+// as the tile that decodes on the way into LDS, sums in another order.  That tile's loaders fetch a row's block piecemeal,
+// 64 weights a step (a 210-byte Q6_K block is touched in four cache lines four times over), and decode every weight once per
+// 128 or 256 tokens; the pass reads and writes everything once (0.5 us per 2^20 weights), so it pays from some batch on.
+// Measured, decoding tile -> pass + copying tile, us:
+//   Q6_K   6914 x 2816 at 333 tokens 60 -> 35, 14336 x 4096 at 130 79 -> 71, at 700 200 -> 129, 4096^2 at 700 83 -> 45,
+//          4096 x 14336 at 700 267 -> 145; but 30000 x 2048 at 130 .. 256 tokens 58 .. 61 against 72 .. 75, at 400 114 -> 98
+//   Q5_K   6914 x 2816 at 400 46 -> 38, 4096 x 14336 at 400 108 -> 105, at 700 196 -> 146; 14336 x 4096 at 400 87 against 98,
+//          at 700 170 -> 130, 30000 x 2048 at 400 96 against 99, at 700 144 -> 143 (Q8_0 and IQ4_XS within 6 % of these)
+//   formats decoded ahead of a batch in any case (grid codebooks, Q3_K beyond its cap), against `gemm_mm_f16*`: from 129
+//   tokens 73 -> 65 (Q3_K 14336 x 4096 at 160), 229 -> 171 (30000 x 2048 at 1024); level below.
+static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
+    const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
+    if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || q4kl || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
+    if (dev->deq_big_m > 1) return m >= dev->deq_big_m;
+    if (decoded) return m >= 129u;
+    if (w->type == OJH_Q6_K) return m >= (w->n > 16384u ? 257u : 129u);
+    return m >= (w->n > 8192u ? 513u : 257u);
+}
+static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, uint32_t m,
+                       int accum) {
+    const uint32_t K = w->k, N = w->n, cus = (uint32_t)dev->prop.multiProcessorCount;
+    const bool grid_fmt = ojh_grid_type(w->type);
+    int rc;
+    if ((rc = ensure(dev, grid_fmt ? "iq_grid" : "dequant")) || (rc = ensure(dev, "gemm_f16")) || (rc = ensure(dev, "glue"))) return rc;
+    ojh_buf *xh, *wdeq;
+    if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
+    if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;
+    auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm); };
+    auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + cus - 1) / cus; };
+    // rounds of workgroups over the chip times a tile's measured time per K step (0.34 / 0.55 / 0.98 us at 128 x 128, 256 x
+    // 128, 256 x 256): 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 /
+    // 279 / 388; 6914 x 2816 at 333 35 / 51 / 76
+    const char *name = "gemm_f16d_128";
+    const uint64_t c1 = 8 * rounds(128, 128), c2 = 13 * rounds(256, 128), c3 = 23 * rounds(256, 256);
+    if (dev->f16d_tile == 3 || (!dev->f16d_tile && c3 <= c1 && c3 <= c2)) name = "gemm_f16d_256";
+    else if (dev->f16d_tile == 2 || (!dev->f16d_tile && c2 < c1)) name = "gemm_f16d_256x128";
+    uint32_t sg[3], sb[3];
+    bool sk = false;
+    if (!strcmp(name, "gemm_f16d_128")) {
+        if ((rc = ojh_launch_shape(dev, "gemm_f16d_128_sk", K, N, m, sg, sb))) return rc;
+        sk = sg[1] > 1 && !dev->gemm_sr;
+        if (sk) name = "gemm_f16d_128_sk";
+    }
+    if (!sk && (rc = ojh_launch_shape(dev, name, K, N, m, sg, sb))) return rc;
+    const uint32_t n_el = m * K, nz = sk && !accum ? m * N : 0, nb = (uint32_t)((uint64_t)N * K / f->weights);
+    const uint32_t cb = (uint32_t)(((uint64_t)n_el / 8 + nz / 4 + 255) / 256 + 1);
+    uint32_t dg[3], db[3];
+    const std::string dq = std::string("dequant_") + f->tag + "_f16";
+    if (!grid_fmt) {
+        if ((rc = ojh_launch_shape(dev, (dq + "_x").c_str(), cb, nb, 0, dg, db))) return rc;
+        if ((rc = ojh_launch(dev, (dq + "_x").c_str(), {at(w->raw, w->off), wdeq->ptr, xp, xh->ptr, yp},
+                             {nb, n_el, nz, cb, (uint32_t)(x_dtype == OJH_X_BF16)}, dg, db)))
+            return rc;
+    } else {
+        uint32_t block[3] = {256, 1, 1}, cg[3] = {cb, 1, 1};
+        if ((rc = ojh_launch_shape(dev, dq.c_str(), 0, nb, 0, dg, db))) return rc;
+        if ((rc = ojh_launch(dev, dq.c_str(), {at(w->raw, w->off), wdeq->ptr}, {nb}, dg, db))) return rc;
+        if ((rc = ojh_launch(dev, x_dtype == OJH_X_BF16 ? "copy_bf16_half" : "copy_f32_half", {xp, xh->ptr}, {n_el}, cg, block))) return rc;
+        if (nz && (rc = ojh_launch(dev, "fill_zero_u32", {yp}, {nz}, cg, block))) return rc;
+    }
+    if (sk) return ojh_launch(dev, name, {xh->ptr, wdeq->ptr, yp}, {K, N, m, sg[1]}, sg, sb);
+    return ojh_launch(dev, name, {xh->ptr, wdeq->ptr, yp}, {K, N, (uint32_t)(accum != 0), m}, sg, sb);
+}
+
 extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dtype, const ojh_lin *w, ojh_buf *y,
                       size_t y_off, const ojh_buf *bias, uint32_t m, int accum, int act_mode) {
     if (!dev) return ojh_fail(OJH_ERR_ARG, "ojh_mm: NULL device");
@@ -630,13 +696,6 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
     // the decoders at 22 - 31 us for 14336 x 4096, pass + tile 50 - 56 us flat against 37 - 41 / 66 / 98 us at 4 / 8 / 12
     // tokens; on 4096 x 4096 28 against 13 / 22 / 31 / 39 at 4 / 8 / 12 / 16)
     const uint32_t deq_min = dev->deq_min_m != 1 ? dev->deq_min_m : (uint64_t)N * K >= (32ull << 20) ? 5u : 9u;
-    // Q6_K rows against a long prefill batch likewise: the tile that dequantizes them on the way into LDS spends a fifth
-    // of its time on that (14336 x 4096 at 2048 tokens 399 us against 288 for plain f16 rows), and the decode pass costs
-    // 29 us — the same weights, dequant_to_f16's bits, either way (OJAS_HIP_DEQ_BIG_M: tokens from which, 0 = never).
-    // (Q5_K and Q8_0 rows, whose loaders are lighter, from twice as many tokens: 14336 x 4096 at 2048 tokens 368 / 352 us
-    // against 327)
-    const uint32_t big_from = w->type == OJH_Q6_K ? dev->deq_big_m : w->type == OJH_Q5_K || w->type == OJH_Q8_0 ? 2 * dev->deq_big_m : 0u;
-    const bool deq_big = big_from && m >= big_from && m >= tile_min && act_mode != OJH_ACT_Q8K && (uint64_t)N * K >= (32ull << 20);
     // IQ4_NL / IQ4_XS rows have loaders in the tile: short of the long batches they skip the decode pass (14336 x 4096:
     // 53 - 62 -> 32 - 42 us up to 128 tokens, 114 -> 93 at 512; 4096 x 4096 at 16 tokens 29 -> 14; from 1024 tokens
     // the pass pays for itself as it does for Q6_K) and take the tile from 5 tokens on every shape (the matvec that
@@ -646,11 +705,14 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
                             w->type == OJH_Q4_1 || w->type == OJH_Q5_0 || w->type == OJH_Q5_1 || w->type == OJH_MXFP4 ||
                             ((w->type == OJH_Q2_K || w->type == OJH_Q3_K) && K % 256 == 0);
     const bool iq4_own = dev->iq4_tile && own_loader &&
-                         act_asked != OJH_ACT_Q8K && m >= dev->iq4_tile && (!dev->deq_big_m || m < dev->deq_big_m) &&
+                         act_asked != OJH_ACT_Q8K && m >= dev->iq4_tile &&
                          (w->type != OJH_Q3_K || m <= dev->iq4_tile_cap) &&   // (Q3_K: eight loads at 2-byte alignment per thread and step, 55 against 68 us at 128 tokens, 86 against 82 at 256)
                          K % 64 == 0;
-    const bool deq_tile = ((iq4 || grid_fmt) && !iq4_own && !q5_float && act_asked != OJH_ACT_Q8K && deq_min && m >= deq_min || deq_big) &&
+    const bool deq_tile = ((iq4 || grid_fmt) && !iq4_own && !q5_float && act_asked != OJH_ACT_Q8K && deq_min && m >= deq_min) &&
                           !dev->no_scratch && K % 64 == 0 && (uint64_t)N * K / f->weights <= 0x7FFFFFFFu / 64;
+    const bool tile_fits = K % 64 == 0 && (uint64_t)m * K < 0x7FFFFFFFull && (uint64_t)m * N < 0x7FFFFFFFull;
+    const bool tile_taken = (deq_tile || iq4_own || (m >= tile_min && act_mode != OJH_ACT_Q8K && !iq4 && !grid_fmt)) && tile_fits;
+    if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum);
     void *tile_w = wp;
     if (deq_tile) {
         ojh_buf *wdeq;
@@ -663,8 +725,7 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         if ((rc = ojh_launch(dev, dq.c_str(), {wp, wdeq->ptr}, {nb}, dg, db))) return rc;
         tile_w = wdeq->ptr;
     }
-    if ((deq_tile || iq4_own || (m >= tile_min && act_mode != OJH_ACT_Q8K && !iq4 && !grid_fmt)) && K % 64 == 0 &&
-        (uint64_t)m * K < 0x7FFFFFFFull && (uint64_t)m * N < 0x7FFFFFFFull) {
+    if (tile_taken) {
         // Q4_K takes the 256-wide tile with the reference GPU kernel's arithmetic (f16 qa*q + qb)
         // unless the tile that reproduces dequant_to_f16 bit for bit is asked for.
         const bool xl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT &&

@@ -428,3 +428,53 @@ def test_few_token_kernel_by_name(gpu, orc, pkg, ty, tag, m, k, n, accum, thread
         with pytest.raises(pkg.OjasHipError, match="tokens"):
             gpu.dispatch(gpu.begin(), "gemm_few_%s_t%d" % (tag, tg), [(xd, 0), (wd, 0), (yd, 0)], [k, n, 0, 16 * tg + 1], [(n + 15) // 16, 1, 1],
                          [256, 1, 1])
+
+
+@pytest.mark.parametrize("kernel,bm,bn", [("gemm_f16d_128", 128, 128), ("gemm_f16d_256x128", 256, 128), ("gemm_f16d_256", 256, 256),
+                                          ("gemm_f16d_128_sk", 128, 128)])
+@pytest.mark.parametrize("m,k,n,accum", [(1, 64, 1, False), (129, 128, 127, True), (257, 192, 1100, False), (300, 1088, 385, True)])
+def test_copied_f16_tile_by_name(gpu, pkg, kernel, bm, bn, m, k, n, accum):
+    """`gemm_f16d_*`: plain f16 rows, both operands copied into LDS a ring of K steps ahead — fewer steps than the ring is
+    deep, one row and token past a tile, row tiles past the XCDs' share, K slices (some of them empty); f64 product of the
+    same f16 values, f32 sums of up to 1088 products: 1e-5 of the peak; nothing written outside y."""
+    gpu.ensure_family("gemm_f16")
+    sk = kernel.endswith("_sk")
+    x = pkg.synth.normal_f32(m * k, "f16d", "x", m, k).astype(np.float16)
+    w = pkg.synth.normal_f32(n * k, "f16d", "w", n, k).astype(np.float16)
+    want = x.astype(np.float64).reshape(m, k) @ w.astype(np.float64).reshape(n, k).T
+    y0 = pkg.synth.normal_f32(m * n, "f16d", "y0").reshape(m, n) if accum or sk else np.zeros((m, n), np.float32)
+    xd, wd = gpu.upload_bytes(x.view(np.uint8)), gpu.upload_bytes(w.view(np.uint8))
+    tiles = ((n + bn - 1) // bn + 7) // 8 * 8 * ((m + bm - 1) // bm)
+    for z in (1, 3, 20) if sk else (1,):
+        yd = gpu.upload(np.concatenate([y0.ravel(), np.full(256, 777.25, np.float32)]))
+        gpu.dispatch(gpu.begin(), kernel, [(xd, 0), (wd, 0), (yd, 0)], [k, n, m, z] if sk else [k, n, int(accum), m], [tiles, z, 1], [256, 1, 1])
+        got = gpu.read(yd, m * n + 256)
+        assert np.all(got[m * n:] == np.float32(777.25))
+        assert peak_err(got[:m * n].reshape(m, n), want + y0) <= 1e-5, z
+    with pytest.raises(pkg.OjasHipError, match="grid must be"):
+        gpu.dispatch(gpu.begin(), kernel, [(xd, 0), (wd, 0), (yd, 0)], [k, n, m, 1] if sk else [k, n, 0, m], [tiles + 8, 1, 1], [256, 1, 1])
+
+
+@pytest.mark.parametrize("ty,tag", [(8, "q80"), (14, "q6k"), (2, "q40"), (11, "q3k")])
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_decoder_with_activations_converted_beside_it(gpu, orc, pkg, ty, tag, bf16):
+    """`dequant_<fmt>_f16_x`: the decoder's bits, the activations' f16 bits and the cleared dwords, nothing past any of them."""
+    gpu.ensure_family("dequant")
+    n, k, m, nz = 37, 512, 11, 1001
+    raw = pkg.synth.weights(ty, n, k, "beside", tag)
+    x = pkg.synth.normal_f32(m * k + 5, "beside", "x")
+    xb = pkg.synth.to_bf16_bits(x) if bf16 else x
+    if bf16:
+        x = pkg.synth.bf16_bits_to_f32(xb)
+    ne = x.size
+    nb = n * k // pkg.synth.BLOCK_SHAPE[ty][1]
+    out, xh = gpu.upload(np.full(n * k // 2 + 8, 7.5, np.float32)), gpu.upload(np.full(ne // 2 + 9, 7.5, np.float32))
+    z = gpu.upload(np.full(nz + 8, 7.5, np.float32))
+    grid, block = gpu.launch_shape("dequant_%s_f16_x" % tag, 3, nb, 0)
+    gpu.dispatch(gpu.begin(), "dequant_%s_f16_x" % tag, [(gpu.upload_bytes(raw), 0), (out, 0), (gpu.upload_bytes(xb.view(np.uint8)), 0), (xh, 0), (z, 0)],
+                 [nb, ne, nz, 3, bf16], grid, block)
+    assert np.array_equal(gpu.read(out, n * k, np.uint16), orc.dequant_to_f16(raw, ty, n * k))
+    assert np.array_equal(gpu.read(xh, ne, np.uint16), x.astype(np.float16).view(np.uint16))
+    got = gpu.read(z, nz + 8)
+    assert np.all(got[:nz] == 0) and np.all(got[nz:] == 7.5)
+    assert np.all(gpu.read(out, n * k // 2 + 8)[-8:] == 7.5)
