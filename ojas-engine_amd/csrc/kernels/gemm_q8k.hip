@@ -594,28 +594,16 @@ __device__ __forceinline__ void gxt_copy16(const void* base, uint voff, uint lds
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds_addr) : "memory");
 }
 
-// the two planes of one 16-row tile's super-block: BA = (sc & 7) * code, BB = (sc >> 3) * code, a chunk per register quad;
-// and the row's side of the min term for the f32 matrix unit: n0 = -dmin * m[kg], n1 = -dmin * m[kg + 4] (sh = 8 kg)
+// one 16-row tile's super-block: its two planes, and the row's side of the min term for the f32 matrix unit:
+// n0 = -dmin * m[kg], n1 = -dmin * m[kg + 4] (sh = 8 kg)
 __device__ __forceinline__ void gxt_planes(const GqW& w, gq_i4 (&BA)[4], gq_i4 (&BB)[4], float& n0, float& n1, float& d, uint sh) {
     d = f16_bits_to_f32(w.hdr.x & 0xFFFFu);
     const float ndmin = -f16_bits_to_f32(w.hdr.x >> 16);
-    const uint sc_lo = w.hdr.y & 0x3F3F3F3Fu, mn_lo = w.hdr.z & 0x3F3F3F3Fu;
-    const uint sc_hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
+    const uint mn_lo = w.hdr.z & 0x3F3F3F3Fu;
     const uint mn_hi = ((w.hdr.w >> 4) & 0x0F0F0F0Fu) | ((w.hdr.z >> 2) & 0x30303030u);
     n0 = __fmul_rn(ndmin, (float)((mn_lo >> sh) & 0xFFu));
     n1 = __fmul_rn(ndmin, (float)((mn_hi >> sh) & 0xFFu));
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const uint se = 2 * c < 4 ? (sc_lo >> (16 * c)) & 0xFFu : (sc_hi >> (16 * (c - 2))) & 0xFFu;
-        const uint so = 2 * c < 4 ? (sc_lo >> (16 * c + 8)) & 0xFFu : (sc_hi >> (16 * (c - 2) + 8)) & 0xFFu;
-        const gq_u16x2 el = {(ushort)(se & 7u), (ushort)(se & 7u)}, eh = {(ushort)(se >> 3), (ushort)(se >> 3)};
-        const gq_u16x2 ol = {(ushort)(so & 7u), (ushort)(so & 7u)}, oh = {(ushort)(so >> 3), (ushort)(so >> 3)};
-        const uint2 qq = w.q[c];
-        const uint lx = qq.x & 0x0F0F0F0Fu, ly = qq.y & 0x0F0F0F0Fu;
-        const uint hx = (qq.x >> 4) & 0x0F0F0F0Fu, hy = (qq.y >> 4) & 0x0F0F0F0Fu;
-        BA[c] = (gq_i4){(int)gq_mul4(lx, el), (int)gq_mul4(ly, el), (int)gq_mul4(hx, ol), (int)gq_mul4(hy, ol)};
-        BB[c] = (gq_i4){(int)gq_mul4(lx, eh), (int)gq_mul4(ly, eh), (int)gq_mul4(hx, oh), (int)gq_mul4(hy, oh)};
-    }
+    gq_planes(w, BA, BB);
 }
 
 // TH = 1: eight row tiles (128 rows) per workgroup, a wave takes one of them against all eight passes of 16 tokens;

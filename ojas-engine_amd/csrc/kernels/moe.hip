@@ -1007,18 +1007,27 @@ moe_down_q4k_mm(const signed char* __restrict__ aq, const float* __restrict__ as
 }
 
 // ------------------------------------------------------------------ grouped products, a wave per row tile
-//   moe_gu_q4k_mt / moe_down_q4k_mt (the arguments of the _m entries)   grid [RG, E, 1], block 512,
+//   moe_gu_q4k_mt / moe_down_q4k_mt (the arguments of the _m entries)   grid [RG, E, 1], block 512 or 1024,
 //                                                                       16 (K + 32) + 5 K / 4 + 320 <= 81920
 // With many small experts (128 x 768 x 2048) the _mm form spends its time around the products: a
 // workgroup per 16-row tile and expert (16384 of them for the down matrices, three super-blocks
 // each), activations fetched from global memory per super-block, partial sums of four waves
-// through LDS.  Here RG workgroups share an expert: each stages the expert's next 16 assignments
+// through LDS.  Here RG workgroups share an expert: each stages the expert's next assignments
 // once (token rows gathered through the list into LDS, scales, sums split into int8 parts; rows
-// past the count are one block of zeros), then every wave walks whole row tiles, all of K, with
-// the dense entries' super-block routine (10 MFMAs instead of 24 per super-block and tensor
-// pair) and writes its own outputs; no partial sums meet.  Tile i of the expert belongs to
-// workgroup i % RG, wave (i / RG) % 8.  Super-blocks are added in order.
+// past the count are one block of zeros), then every wave walks whole row tiles, all of K, and no partial sums meet.
+// A gate and an up wave share a tile: the up wave's sums pass through LDS to the gate wave, which writes silu(g) u.
+// What bounds it is the stream of weights: copied alone the gate/up launch (128 experts of 768 x 2048, 2048 assignments,
+// 226 MB) takes 48 us and 9 of them are the launch and the staging.  So the rows travel global -> LDS by
+// global_load_lds_dwordx4 (nine lanes per row, two units of 16 rows x one super-block in flight per wave, sixteen waves:
+// 74 KB per CU) instead of by loads into registers, whose 8-byte pieces of sixteen far-apart rows kept the address unit
+// busy; and a super-block's scales are folded into two int8 planes once for all its passes (gq_planes) instead of
+// multiplied onto every result.  Eight waves with one tile of both tensors each 68 us, twelve 58, sixteen with a tile of
+// both 55 - 59 by how evenly the tiles divide.  Before (loads into registers, gq_superblock): gate/up 81 us, down 46;
+// now 58 and 33.  Super-blocks are added in order.
 #define MT_LDS 81920u
+#define MT_UNIT 2304u
+#define MT_DEPTH 2
+#define MT_RING (16u * MT_DEPTH * MT_UNIT)
 // A pass stages 16 P assignments; P = 2 where 32 token rows fit (32 (K + 32) + 5 K / 2 + 384 <= 81920): an expert with
 // 17 .. 32 assignments then has its rows read and unpacked once instead of twice (at 256 tokens over 128 experts with
 // 8 slots each, 16 per expert on average, that is every other expert).
@@ -1028,13 +1037,13 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
                                             const uint* __restrict__ offsets, const uint* __restrict__ list,
                                             uint K, uint N, uint KSEL, uint NA, uchar* lds) {
     constexpr uint TP = 16u * P;
-    constexpr int NT = GU ? 2 : 1;
+    constexpr int D = MT_DEPTH;
     const uint e = blockIdx.y;
     const uint a0 = min(offsets[e], NA), a1 = min(offsets[e + 1], NA);
     if (a0 >= a1) return;
     const uint tid = threadIdx.x, lane = tid & 63u, nt = blockDim.x;
     const uint wave = (uint)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), nw = nt >> 6;
-    const uint nsb = K >> 8, S = K + 32u, per_row = K >> 4;
+    const uint nsb = K >> 8, S = K + 16u, per_row = K >> 4;     // (rows 16 bytes past a bank period: 16 lanes' reads of 16 bytes cover every bank once)
     const uint o_lsx = TP * S, o_lbq = o_lsx + nsb * TP * 4u, o_zero = o_lbq + nsb * TP * 16u, o_av = o_zero + 256u;
     float* lsx = (float*)(lds + o_lsx);            // [sb][TP] token scales
     uchar* lbq = lds + o_lbq;                      // [sb][TP][16]: lo_0..7, hi_0..7 of the bsums
@@ -1043,48 +1052,77 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
     const uint n = lane & 15u, kg = lane >> 4;
     const size_t rb = (size_t)nsb * Q4K_BYTES;
     const uint tiles = (N + 15u) >> 4;
+    // copies of a unit: nine lanes per row, seven rows per copy (rows 14 and 15 in the third)
+    const uint cq = lane / 9u, cpc16 = (lane - cq * 9u) * 16u, c_off = cq * (uint)rb + cpc16;
+    // tile r of wave group g: (r groups + g) gridDim.x + blockIdx.x; a group is a wave, or a pair (even: gate, odd: up)
+    const uint groups = GU ? nw >> 1 : nw, group = GU ? wave >> 1 : wave, stride = groups * gridDim.x;
+    const uint first = group * gridDim.x + blockIdx.x, rounds = (tiles + stride - 1u) / stride;
+    const uint my_tiles = first < tiles ? (tiles - first + stride - 1u) / stride : 0u;
+    const uchar* const w = GU && (wave & 1u) ? w1 : w0;
+    const uint ring = (uint)(size_t)(__attribute__((address_space(3))) uchar*)lds + MT_LDS + wave * ((uint)D * MT_UNIT);
+    const uchar* const rd = lds + MT_LDS + wave * ((uint)D * MT_UNIT) + n * Q4K_BYTES;
     for (uint tt = a0; tt < a1; tt += TP) {
         const uint cnt = min(TP, a1 - tt);
+        // This wave's tiles as one stream of units (16 rows at one super-block), copied by the memory system into the wave's
+        // ring of D and asked for D units ahead across tile borders; the first D are on their way while the tokens are staged.
+        const uint units = my_tiles * nsb;
+        uint i_u = 0u, i_sb = 0u, i_tile = first, i_slot = 0u;
+        auto issue_next = [&]() {
+            const size_t at = (size_t)w + ((size_t)e * N + i_tile * 16u) * rb + (size_t)i_sb * Q4K_BYTES;
+            const uchar* base = (const uchar*)(((size_t)(uint)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
+                                               (uint)__builtin_amdgcn_readfirstlane((int)(uint)at));   // (the copy wants it in scalar registers)
+            const uint dst = ring + i_slot * MT_UNIT;
+            uint o0 = c_off, o1 = c_off + 7u * (uint)rb, o2 = c_off + 14u * (uint)rb;
+            if (N - i_tile * 16u < 16u) {                          // the last tile of a ragged matrix: no row past N
+                const uint top = N - i_tile * 16u - 1u;
+                o0 = min(cq, top) * (uint)rb + cpc16;
+                o1 = min(7u + cq, top) * (uint)rb + cpc16;
+                o2 = min(14u + cq, top) * (uint)rb + cpc16;
+            }
+            if (lane < 63u) {
+                lds_dma16(base, o0, dst);
+                lds_dma16(base, o1, dst + 1008u);
+            }
+            if (lane < 18u) lds_dma16(base, o2, dst + 2016u);
+            i_u++;
+            i_slot = i_slot + 1u == (uint)D ? 0u : i_slot + 1u;
+            if (++i_sb == nsb) {
+                i_sb = 0u;
+                i_tile += stride;
+            }
+        };
+        for (uint k = 0; k < (uint)D; k++)
+            if (i_u < units) issue_next();
         __syncthreads();                           // the previous pass is done with the staged tokens
         if (tid < TP) lav[tid] = min(list[min(tt + tid, a1 - 1u)], NA - 1u);
-        __syncthreads();
-        // token rows 0 .. cnt - 1, eight loads in flight per thread
+        auto source = [&](uint t) { const uint av = min(list[min(tt + t, a1 - 1u)], NA - 1u); return GU ? av / KSEL : av; };
+        // token rows 0 .. cnt - 1, four loads of 16 bytes in flight per thread; two neighbours hold one run of 32 positions
+        // and leave its sum (the even one the low part, the odd one the high part)
         const uint total = cnt * per_row;
-        for (uint i0 = tid; i0 < total; i0 += 8u * nt) {
-            uint4 v[8];
-            uint dst[8];
+        for (uint i0 = tid; i0 < total; i0 += 4u * nt) {
+            uint4 v[4];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const uint i = i0 + (uint)u * nt, t = min(i / per_row, TP - 1u), o = (i - (i / per_row) * per_row) << 4;
-                const uint src = GU ? lav[t] / KSEL : lav[t];
-                v[u] = make_uint4(0u, 0u, 0u, 0u);
-                dst[u] = t * S + o;
-                if (i < total) v[u] = *(const uint4*)(xq + (size_t)src * K + o);
+            for (int q = 0; q < 4; q++) {
+                const uint i = min(i0 + (uint)q * nt, total - 2u + (tid & 1u)), t = i / per_row;
+                v[q] = *(const uint4*)(xq + (size_t)source(t) * K + ((i - t * per_row) << 4));
             }
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (i0 + (uint)u * nt < total) *(uint4*)(lds + dst[u]) = v[u];
+            for (int q = 0; q < 4; q++) {
+                const uint i = i0 + (uint)q * nt, t = i / per_row, o = (i - t * per_row) << 4;
+                int bs = dot4_i8(v[q].x, 0x01010101u, 0);
+                bs = dot4_i8(v[q].y, 0x01010101u, bs); bs = dot4_i8(v[q].z, 0x01010101u, bs); bs = dot4_i8(v[q].w, 0x01010101u, bs);
+                bs += dpp_i32<OJK_DPP_QUAD_XOR1>(bs);
+                if (i < total) {
+                    uchar* const x = lds + (size_t)t * S + (o & ~63u) + ((o & 16u) << 1) + ((o & 32u) >> 2);
+                    *(uint2*)x = make_uint2(v[q].x, v[q].y);
+                    *(uint2*)(x + 16u) = make_uint2(v[q].z, v[q].w);
+                    lbq[((o >> 8) * TP + t) * 16u + 8u * (tid & 1u) + ((o >> 5) & 7u)] = (uchar)((tid & 1u) ? bs >> 6 : bs & 63);
+                }
+            }
         }
         for (uint i = tid; i < nsb * TP; i += nt) {
-            const uint sb = i / TP, t = i - sb * TP;
-            const uint src = GU ? lav[t] / KSEL : lav[t];
-            lsx[i] = t < cnt ? xs[(size_t)src * nsb + sb] : 0.0f;
-        }
-        __syncthreads();
-        for (uint i = tid; i < nsb * TP * 8u; i += nt) {
-            const uint jj = i & 7u, t = (i >> 3) % TP, sb = (i >> 3) / TP;
-            int bs = 0;
-            if (t < cnt) {
-                const uint4* px = (const uint4*)(lds + (size_t)t * S + sb * 256u + jj * 32u);
-                const uint4 a = px[0], b = px[1];
-                bs = dot4_i8(a.x, 0x01010101u, 0);
-                bs = dot4_i8(a.y, 0x01010101u, bs); bs = dot4_i8(a.z, 0x01010101u, bs); bs = dot4_i8(a.w, 0x01010101u, bs);
-                bs = dot4_i8(b.x, 0x01010101u, bs); bs = dot4_i8(b.y, 0x01010101u, bs);
-                bs = dot4_i8(b.z, 0x01010101u, bs); bs = dot4_i8(b.w, 0x01010101u, bs);
-            }
-            uchar* o = lbq + ((size_t)sb * TP + t) * 16u;
-            o[jj] = (uchar)(bs & 63);
-            o[8u + jj] = (uchar)(bs >> 6);
+            const uint t = i / nsb, sb = i - t * nsb;
+            lsx[sb * TP + t] = t < cnt ? xs[(size_t)source(t) * nsb + sb] : 0.0f;
         }
         __syncthreads();
         const uint np = (cnt + 15u) >> 4;          // token tiles of 16 this pass holds
@@ -1093,106 +1131,97 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
 #pragma unroll
         for (int p = 0; p < P; p++) {
             const bool on = n + 16u * p < cnt;
-            xa[p] = on ? lds + (size_t)(n + 16u * p) * S + 8u * kg : lds + o_zero + 8u * kg;
+            xa[p] = on ? lds + (size_t)(n + 16u * p) * S + 16u * kg : lds + o_zero + 16u * kg;
             xstep[p] = on ? 256u : 0u;
         }
-        // This wave's tiles as one stream of (tile, super-block) steps, the blocks of three steps on their
-        // way: a wave that loads a step only when it starts the one before it walks a chain of memory
-        // latencies (32 of them per pass at 768 x 2048) and the launch is bound by that chain.
-        const uint first = wave * gridDim.x + blockIdx.x, stride = nw * gridDim.x;
-        const uint my_tiles = first < tiles ? (tiles - first + stride - 1u) / stride : 0u;
-        const uint steps = my_tiles * nsb;
-        uint i_u = 0u, i_sb = 0u, i_tile = first;
-        auto next_step = [&](GqW (&blk)[NT]) {   // loads past the last step repeat it
-            const size_t off = ((size_t)e * N + min(i_tile * 16u + n, N - 1u)) * rb + (size_t)i_sb * Q4K_BYTES;
-            blk[0] = gq_load(w0 + off, kg);
-            if (GU) blk[NT - 1] = gq_load(w1 + off, kg);
-            if (i_u + 1u < steps) {
-                i_u++;
-                if (++i_sb == nsb) {
-                    i_sb = 0u;
-                    i_tile += stride;
-                }
-            }
-        };
-        if (steps == 0u) continue;
-        GqW c0[NT], c1[NT], c2[NT];
-        next_step(c0);
-        next_step(c1);
-        next_step(c2);
-        float acc[NT][P][4];
-#pragma unroll
-        for (int w = 0; w < NT; w++)
+        uint c_tile = first, c_slot = 0u, u = 0u;
+        for (uint r = 0; r < rounds; r++, c_tile += stride) {
+            float acc[P][4];
 #pragma unroll
             for (int p = 0; p < P; p++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) acc[w][p][v] = 0.0f;
-        uint c_sb = 0u, c_tile = first;
-        for (uint u = 0; u < steps; u++) {
-            GqW c3[NT];
-            next_step(c3);
+                for (int v = 0; v < 4; v++) acc[p][v] = 0.0f;
+            const bool has = c_tile < tiles;
+            if (has)
+                for (uint sb = 0; sb < nsb; sb++, u++) {
+                    if (units - u >= (uint)D) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(3 * (D - 1)) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+                    const uchar* blk = rd + c_slot * MT_UNIT;
+                    c_slot = c_slot + 1u == (uint)D ? 0u : c_slot + 1u;
+                    GqW c;
+                    c.hdr = *(const uint4*)blk;
 #pragma unroll
-            for (int w = 0; w < NT; w++)
-#pragma unroll
-                for (int p = 0; p < P; p++)
-                    if ((uint)p < np)
-                        gq_superblock(c0[w], xa[p] + c_sb * xstep[p], lbq + ((size_t)c_sb * TP + 16u * p + n) * 16u,
-                                      lsx + c_sb * TP + 16u * p, kg, acc[w][p]);
-#pragma unroll
-            for (int w = 0; w < NT; w++) {
-                c0[w] = c1[w];
-                c1[w] = c2[w];
-                c2[w] = c3[w];
-            }
-            if (++c_sb == nsb) {
-                // D register v of lane (n, kg): assignment 16 p + 4 kg + v of the pass, row n of the tile
-                if (c_tile * 16u + n < N) {
+                    for (int q = 0; q < 4; q++) c.q[q] = *(const uint2*)(blk + 16u + 32u * q + 8u * kg);
+                    gq_i4 BA[4], BB[4];
+                    const float d = f16_bits_to_f32(c.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(c.hdr.x >> 16);
+                    const uint mn_lo = c.hdr.z & 0x3F3F3F3Fu;
+                    const uint mn_hi = ((c.hdr.w >> 4) & 0x0F0F0F0Fu) | ((c.hdr.z >> 2) & 0x30303030u);
+                    const long Bm = kg == 0u ? gq_pack(mn_lo, mn_hi) : 0;
+                    gq_planes(c, BA, BB);
+                    // the unit is in registers: its slot takes the unit D ahead
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    if (i_u < units) issue_next();
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int p = 0; p < P; p++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            const uint t = 16u * p + 4u * kg + (uint)v;
-                            if (t < cnt) {
-                                float* o = out + (size_t)lav[t] * N + c_tile * 16u + n;
-                                if (GU) {
-                                    const float g = acc[0][p][v];
-                                    *o = (g / (1.0f + expf(-g))) * acc[NT - 1][p][v];
-                                } else {
-                                    *o = acc[0][p][v];
-                                }
-                            }
-                        }
+                        if ((uint)p < np)
+                            gq_planes_pass(BA, BB, Bm, d, dmin, xa[p] + sb * xstep[p], lbq + ((size_t)sb * TP + 16u * p + n) * 16u,
+                                           lsx + sb * TP + 16u * p, kg, acc[p]);
                 }
+            // D register v of lane (n, kg): assignment 16 p + 4 kg + v of the pass, row n of the tile
+            const bool mine = has && c_tile * 16u + n < N;
 #pragma unroll
-                for (int w = 0; w < NT; w++)
+            for (int p = 0; p < P; p++) {
+                if ((uint)p >= np) break;
+                float* const ex = (float*)(lds + MT_LDS + MT_RING) + ((wave >> 1) * 64u + lane) * 4u;
+                float up[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (GU) {
+                    if (wave & 1u) *(float4*)ex = make_float4(acc[p][0], acc[p][1], acc[p][2], acc[p][3]);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_s_barrier();
+                    if ((wave & 1u) == 0u) {
+                        const float4 t = *(const float4*)ex;
+                        up[0] = t.x, up[1] = t.y, up[2] = t.z, up[3] = t.w;
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_s_barrier();
+                }
+                if (mine && (!GU || (wave & 1u) == 0u)) {
 #pragma unroll
-                    for (int p = 0; p < P; p++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) acc[w][p][v] = 0.0f;
-                c_sb = 0u;
-                c_tile += stride;
+                    for (int v = 0; v < 4; v++) {
+                        const uint t = 16u * p + 4u * kg + (uint)v;
+                        if (t < cnt) {
+                            const float g = acc[p][v];
+                            out[(size_t)lav[t] * N + c_tile * 16u + n] = GU ? (g / (1.0f + expf(-g))) * up[v] : g;
+                        }
+                    }
+                }
             }
         }
     }
 }
 
-extern "C" __global__ void __launch_bounds__(512)
+#define MT_RUN(GU, X, S, W0, W1, OUT, KS)                                                                              \
+    do {                                                                                                              \
+        if (32u * (K + 32u) + 5u * (K >> 1) + 384u <= MT_LDS) moe_mt_body<GU, 2>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt); \
+        else moe_mt_body<GU, 1>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt);                              \
+    } while (0)
+extern "C" __global__ void __launch_bounds__(1024)
 moe_gu_q4k_mt(const signed char* __restrict__ xq, const float* __restrict__ xs, const uchar* __restrict__ wg,
               const uchar* __restrict__ wu, float* __restrict__ act, const uint* __restrict__ offsets,
               const uint* __restrict__ list, uint K, uint N, uint KSEL, uint NA) {
-    __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS];
-    if (32u * (K + 32u) + 5u * (K >> 1) + 384u <= MT_LDS) moe_mt_body<true, 2>(xq, xs, wg, wu, act, offsets, list, K, N, KSEL, NA, lds_mt);
-    else moe_mt_body<true, 1>(xq, xs, wg, wu, act, offsets, list, K, N, KSEL, NA, lds_mt);
+    __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS + MT_RING + 8192u];
+    MT_RUN(true, xq, xs, wg, wu, act, KSEL);
 }
 
-extern "C" __global__ void __launch_bounds__(512)
+extern "C" __global__ void __launch_bounds__(1024)
 moe_down_q4k_mt(const signed char* __restrict__ aq, const float* __restrict__ as_, const uchar* __restrict__ wd,
                 float* __restrict__ dv, const uint* __restrict__ offsets, const uint* __restrict__ list,
                 uint K, uint N, uint NA) {
-    __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS];
-    if (32u * (K + 32u) + 5u * (K >> 1) + 384u <= MT_LDS) moe_mt_body<false, 2>(aq, as_, wd, wd, dv, offsets, list, K, N, 1u, NA, lds_mt);
-    else moe_mt_body<false, 1>(aq, as_, wd, wd, dv, offsets, list, K, N, 1u, NA, lds_mt);
+    __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS + MT_RING];
+    MT_RUN(false, aq, as_, wd, wd, dv, 1u);
 }
+#undef MT_RUN
 
 // ------------------------------------------------------------------ combine
 // y[t][i] (=, +=) sum_j wgt[t][j] * dv[t*KSEL + j][i], slots in order.

@@ -71,3 +71,44 @@ __device__ __forceinline__ void gq_superblock(const GqW& cur, const uchar* xp, c
     acc[3] += sx.w * (d * (float)isum[3] - dmin * (float)(64 * Dhi[3] + Dlo[3]));
 }
 
+// The two planes of one 16-row tile's super-block, for operands that span two sub-blocks (v_mfma_i32_16x16x64_i8): a
+// 6-bit scale is 8 sh + sl with both parts <= 7, so BA = sl * code and BB = sh * code fit int8 and
+// sum_j sc_j idot_j = 8 D_B + D_A exactly.  A chunk of 64 weights per register quad: the lane's eight low-nibble codes in
+// positions 0 .. 7 of its sixteen, its eight high-nibble codes in 8 .. 15.
+__device__ __forceinline__ void gq_planes(const GqW& w, gq_i4 (&BA)[4], gq_i4 (&BB)[4]) {
+    const uint sc_lo = w.hdr.y & 0x3F3F3F3Fu;
+    const uint sc_hi = (w.hdr.w & 0x0F0F0F0Fu) | ((w.hdr.y >> 2) & 0x30303030u);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const uint se = 2 * c < 4 ? (sc_lo >> (16 * c)) & 0xFFu : (sc_hi >> (16 * (c - 2))) & 0xFFu;
+        const uint so = 2 * c < 4 ? (sc_lo >> (16 * c + 8)) & 0xFFu : (sc_hi >> (16 * (c - 2) + 8)) & 0xFFu;
+        const gq_u16x2 el = {(ushort)(se & 7u), (ushort)(se & 7u)}, eh = {(ushort)(se >> 3), (ushort)(se >> 3)};
+        const gq_u16x2 ol = {(ushort)(so & 7u), (ushort)(so & 7u)}, oh = {(ushort)(so >> 3), (ushort)(so >> 3)};
+        const uint2 qq = w.q[c];
+        const uint lx = qq.x & 0x0F0F0F0Fu, ly = qq.y & 0x0F0F0F0Fu;
+        const uint hx = (qq.x >> 4) & 0x0F0F0F0Fu, hy = (qq.y >> 4) & 0x0F0F0F0Fu;
+        BA[c] = (gq_i4){(int)gq_mul4(lx, el), (int)gq_mul4(ly, el), (int)gq_mul4(hx, ol), (int)gq_mul4(hy, ol)};
+        BB[c] = (gq_i4){(int)gq_mul4(lx, eh), (int)gq_mul4(ly, eh), (int)gq_mul4(hx, oh), (int)gq_mul4(hy, oh)};
+    }
+}
+// One pass of 16 tokens against those planes: gq_superblock's sums and its last line, bit for bit.
+// xp: 16 bytes of token n per chunk, 64 bytes apart, in the planes' order (low-nibble sub-block's eight, then the
+// high-nibble one's); pq: token n's split sums; Bm: the eight mins in positions 0 .. 7 of lanes kg = 0, zeros elsewhere.
+__device__ __forceinline__ void gq_planes_pass(const gq_i4 (&BA)[4], const gq_i4 (&BB)[4], long Bm, float d, float dmin,
+                                               const uchar* xp, const uchar* pq, const float* sx16, uint kg, float (&acc)[4]) {
+    const gq_i4 zero = {0, 0, 0, 0};
+    const gq_i4 lh = *(const gq_i4*)pq;
+    gq_i4 DA = zero, DB = zero;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const gq_i4 A = *(const gq_i4*)(xp + 64 * c);
+        DA = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, BA[c], DA, 0, 0, 0);
+        DB = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, BB[c], DB, 0, 0, 0);
+    }
+    const gq_i4 Dlo = __builtin_amdgcn_mfma_i32_16x16x32_i8(gq_pack((uint)lh[0], (uint)lh[1]), Bm, zero, 0, 0, 0);
+    const gq_i4 Dhi = __builtin_amdgcn_mfma_i32_16x16x32_i8(gq_pack((uint)lh[2], (uint)lh[3]), Bm, zero, 0, 0, 0);
+    const float4 sx = *(const float4*)(sx16 + 4u * kg);
+    const float sxv[4] = {sx.x, sx.y, sx.z, sx.w};
+#pragma unroll
+    for (int v = 0; v < 4; v++) acc[v] += sxv[v] * (d * (float)(8 * DB[v] + DA[v]) - dmin * (float)(64 * Dhi[v] + Dlo[v]));
+}

@@ -1452,7 +1452,7 @@ uint64_t ojh_moe_mt_lds(uint32_t K) { return 16 * ((uint64_t)K + 32) + K / 4 + K
 //   4 moe_down_q4k_m(aq, as, wd, dv, offsets, list, K, N, NA)                     grid [ceil(N/16), E, 1]; ceil(N/32) for K <= 1024
 //   5 moe_combine(dv, wgt, y, T, KSEL, D, ACC)                                    grid [ceil(T*D/256),1,1]
 //   6 moe_gu_q4k_mm, 7 moe_down_q4k_mm: the arguments of 3 and 4, grid [ceil(N/16), E, 1]
-//  12 moe_gu_q4k_mt, 13 moe_down_q4k_mt: the arguments of 3 and 4, grid [1 .. ceil(N/16), E, 1] x 512
+//  12 moe_gu_q4k_mt, 13 moe_down_q4k_mt: the arguments of 3 and 4, grid [1 .. ceil(N/16), E, 1] x 512 | 1024
 //   8 moe_gu_q4k_dec(x, wg, wu, act, idx, K, N, KSEL, NA, E)                      grid [ceil(N/8), NA, 1]
 //   9 moe_down_q4k_dec(act, wd, idx, wgt, y, K, N, KSEL, E, ACC)                  grid [ceil(N/8), T, 1]
 //  14 moe_gu_q80(x, wg, wu, act, idx, K, N)                                     grid [ceil(N/8), KSEL, tokens]
@@ -1518,7 +1518,7 @@ static int check_moe(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t
         uint32_t K = c[0], N = c[1], KS = c[2], NA = c[3], E = grid[1];
         const uint32_t per = s->rows_per_wave == 3 ? 8 : 16;   // rows per workgroup
         const bool mt = s->rows_per_wave == 12;
-        if ((rc = check_block(block, mt ? 512 : 256))) return rc;
+        if ((rc = check_block(block, !mt ? 256 : block[0] == 512 ? 512 : 1024))) return rc;
         if (!K || K % 256 || !N || !KS || !NA || NA % KS) return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u KSEL=%u NA=%u", s->name, K, N, KS, NA);
         if (mt) {
             if (ojh_moe_mt_lds(K) > 81920) return ojh_fail(OJH_ERR_ARG, "%s: 16 tokens of K=%u do not fit its 80 KB of LDS", s->name, K);
@@ -1540,7 +1540,7 @@ static int check_moe(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t
         uint32_t K = c[0], N = c[1], NA = c[2], E = grid[1];
         const uint32_t per = s->rows_per_wave == 4 && K <= 1024 ? 32 : 16;   // short rows: two row sets per wave
         const bool mt = s->rows_per_wave == 13;
-        if ((rc = check_block(block, mt ? 512 : 256))) return rc;
+        if ((rc = check_block(block, !mt ? 256 : block[0] == 512 ? 512 : 1024))) return rc;
         if (!K || K % 256 || !N || !NA) return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u NA=%u", s->name, K, N, NA);
         if (mt) {
             if (ojh_moe_mt_lds(K) > 81920) return ojh_fail(OJH_ERR_ARG, "%s: 16 tokens of K=%u do not fit its 80 KB of LDS", s->name, K);
@@ -1720,17 +1720,18 @@ static int check_moe(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t
 }
 
 // K, N as named by the kernel; M = tokens (topk, combine) or assignments (group)
-// Workgroups per expert for the moe_*_mt entries: about `per_cu` workgroups per CU over all experts (what
-// is resident at once: one for the gate/up entry, which holds two tensors' blocks of four steps in
-// registers, two for the down entry), fewer until the expert's tiles divide evenly over the workgroups'
-// eight waves (or one workgroup is left).
-uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t N, uint32_t E, uint32_t per_cu) {
+// Workgroups per expert for the moe_*_mt entries, whose sixteen waves walk `side` row tiles side by side (a gate and an up
+// wave per tile: 8; down: 16) and whose LDS leaves room for one per CU: the count with the fewest rounds of tiles over the
+// whole launch, the smallest of those (every workgroup stages its expert's tokens once).
+uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t N, uint32_t E, uint32_t side) {
     const uint32_t cus = dev ? (uint32_t)dev->prop.multiProcessorCount : 256u, tiles = (N + 15) / 16;
-    uint32_t rg = per_cu * cus / (E ? E : 1), cap = (tiles + 7) / 8;
-    if (rg > cap) rg = cap;
-    if (rg < 1) rg = 1;
-    while (rg > 1 && tiles % (8 * rg)) rg--;
-    return rg;
+    uint32_t best = 1;
+    uint64_t least = ~0ull;
+    for (uint32_t rg = 1; rg <= (tiles + side - 1) / side && rg <= cus; rg++) {
+        const uint64_t cost = (uint64_t)((tiles + side * rg - 1) / (side * rg)) * (((uint64_t)(E ? E : 1) * rg + cus - 1) / cus);
+        if (cost < least) best = rg, least = cost;
+    }
+    return best;
 }
 static int shape_moe(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M,
                      uint32_t grid[3], uint32_t block[3]) {
@@ -1749,7 +1750,7 @@ static int shape_moe(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K
     case 6: case 7: grid[0] = (N + 15) / 16; grid[1] = M ? M : 1; break;
     case 14: case 16: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = slots, one token
     case 15: case 17: grid[0] = (N + 3) / 4; break;                           // one token
-    case 12: case 13: grid[0] = ojh_moe_mt_groups(dev, N, M ? M : 1, s->rows_per_wave == 12 ? 1 : 2); grid[1] = M ? M : 1; block[0] = 512; break;  // M = experts
+    case 12: case 13: grid[0] = ojh_moe_mt_groups(dev, N, M ? M : 1, s->rows_per_wave == 12 ? 8 : 16); grid[1] = M ? M : 1; block[0] = 1024; break;  // M = experts
     case 8: case 10: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = assignments
     case 9: case 11: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = tokens
     default: grid[0] = (uint32_t)(((uint64_t)M * N + 255) / 256); break;  // N = D, M = tokens

@@ -217,6 +217,42 @@ def test_q5k_q6k_down_tensors_on_the_int8_matrix_tile(gpu, orc, pkg, T, E, ksel,
     assert peak_err(outs["1"], outs["0"]) <= TOL
 
 
+@pytest.mark.parametrize("k,n", [(256, 8), (768, 328), (2048, 200), (2304, 40), (2560, 72)])
+def test_grouped_wave_tiles_by_name(gpu, orc, pkg, k, n):
+    """`moe_{gu,down}_q4k_mt` where their tiles end: rows that do not fill the last 16, experts with 0, 1, 16, 17, 32 and 33
+    assignments, K on both sides of the two-tile pass, one or three workgroups per expert, eight or sixteen waves; every
+    assignment against matvec_kq (2e-5 of peak, the bar of the int8 forms), the launches bit for bit alike."""
+    counts = [0, 1, 16, 17, 32, 33]
+    E, na, nsb = len(counts), sum(counts), k // 256
+    w = [pkg.synth.q4k_weights(E * n, k, "moemt", t, k, n) for t in ("g", "u")]
+    act = pkg.synth.normal_f32(na * k, "moemt", "act", k).reshape(na, k)
+    perm = pkg.synth.rng("moemt", "perm").permutation(na).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    gpu.ensure_family("moe")
+    gpu.ensure_family("gemv_q8k")
+    aq, as_ = gpu.alloc_bytes(na * k), gpu.alloc(na * nsb)
+    gpu.quant_q8k(gpu.upload(act), na, k, aq, as_)
+    wg, wu, od, ld = gpu.upload_bytes(w[0]), gpu.upload_bytes(w[1]), gpu.upload_bytes(offsets), gpu.upload_bytes(perm)
+    rb = len(w[0]) // (E * n)
+    ref = [np.stack([orc.matvec_kq(t[e * n * rb:(e + 1) * n * rb], Q4_K, n, k, act[perm[i]]) for e in range(E)
+                     for i in range(offsets[e], offsets[e + 1])]) for t in w]
+    with np.errstate(over="ignore"):
+        wants = {"moe_down_q4k_mt": ref[0], "moe_gu_q4k_mt": ref[0] / (1 + np.exp(-ref[0].astype(np.float64))) * ref[1]}
+    for name, want in wants.items():
+        seen = []
+        for rg, block in ((1, 1024), (min(3, (n + 15) // 16), 1024), (1, 512)):
+            dv = gpu.upload(np.full(na * n + n, 777.25, np.float32))
+            bufs = [(aq, 0), (as_, 0), (wg, 0)] + ([(wu, 0)] if "gu" in name else []) + [(dv, 0), (od, 0), (ld, 0)]
+            gpu.dispatch(gpu.begin(), name, bufs, [k, n] + ([1] if "gu" in name else []) + [na], [rg, E, 1], [block, 1, 1])
+            got = gpu.read(dv, na * n + n)
+            assert np.all(got[na * n:] == np.float32(777.25))
+            seen.append(got[:na * n].view(np.uint32).copy())
+        assert np.array_equal(seen[0], seen[1]) and np.array_equal(seen[0], seen[2])
+        got = seen[0].view(np.float32).reshape(na, n)[perm]
+        for i in range(na):
+            assert peak_err(got[i], want[i]) <= 2e-5, (name, i)
+
+
 @pytest.mark.parametrize("dty", [13, 14])
 def test_grouped_int8_tile_by_name(gpu, orc, pkg, dty):
     """`moe_down_{q5k,q6k}_gs(aq, as, wd, dv, offsets, list, K, N, NA)`: every assignment's row against matvec_kq of its
