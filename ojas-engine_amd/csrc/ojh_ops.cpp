@@ -557,6 +557,13 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
     const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
     if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || q4kl || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
+    // while a graph is recorded nothing can be loaded or grown: what is not there yet leaves the call on the tile it has
+    if (dev->capturing) {
+        const auto slot = dev->scratch.find("wdeq");
+        if (!dev->modules.count("gemm_f16") || !dev->modules.count(ojh_grid_type(w->type) ? "iq_grid" : "dequant") ||
+            slot == dev->scratch.end() || !slot->second || slot->second->bytes < (size_t)w->n * w->k * 2)
+            return false;
+    }
     if (dev->deq_big_m > 1) return m >= dev->deq_big_m;
     if (decoded) return m >= 129u;
     if (w->type == OJH_Q6_K) return m >= (w->n > 16384u ? 257u : 129u);
@@ -712,7 +719,13 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
                           !dev->no_scratch && K % 64 == 0 && (uint64_t)N * K / f->weights <= 0x7FFFFFFFu / 64;
     const bool tile_fits = K % 64 == 0 && (uint64_t)m * K < 0x7FFFFFFFull && (uint64_t)m * N < 0x7FFFFFFFull;
     const bool tile_taken = (deq_tile || iq4_own || (m >= tile_min && act_mode != OJH_ACT_Q8K && !iq4 && !grid_fmt)) && tile_fits;
-    if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum);
+    if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) {
+        // (a format with a loader needs no room for the decoded rows: without that room it keeps the loader)
+        ojh_buf *room;
+        rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &room);
+        if (!rc) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum);
+        if (deq_tile) return rc;
+    }
     void *tile_w = wp;
     if (deq_tile) {
         ojh_buf *wdeq;

@@ -96,3 +96,30 @@ def test_a_failed_call_while_recording_leaves_the_device_usable(gpu, pkg, replay
     gpu.memset0(yd)
     gpu.mm(xd, lin, yd, 1, act_mode=pkg.ACT_Q8K)
     assert np.array_equal(gpu.read(yd, n), want)
+
+
+def test_recorded_batch_needs_no_more_scratch_than_the_calls_before_it(gpu, orc, pkg):
+    """A batch of Q6_K rows is decoded into scratch from some token count on.  Recorded after eager calls that left
+    everything but that scratch in place, it runs on the tile that decodes on the way into LDS instead of being refused."""
+    n, k, few, m = 16448, 256, 256, 300           # (257 tokens is where rows of this many start to be decoded first)
+    w = pkg.synth.q6k_weights(n, k, "graph", "w6")
+    x = pkg.synth.normal_f32(m * k, "graph", "x6").reshape(m, k)
+    g = pkg.HipGpu(0)
+    try:
+        lin, xd, yd = g.lin(14, n, k, w), g.upload(x), g.alloc(m * n)
+        g.mm(xd, lin, yd, few, act_mode=pkg.ACT_FLOAT)
+        g.capture_begin()
+        g.mm(xd, lin, yd, m, act_mode=pkg.ACT_FLOAT)
+        graph = g.capture_end()
+        rows = np.r_[0:16, n - 16:n]
+        rb = len(w) // n
+        want = orc.matmul_ref(np.concatenate([w[r * rb:(r + 1) * rb] for r in rows]), 14, len(rows), k, x, wmode=1, xmode=1)
+        for _ in range(3):
+            g.memset0(yd)
+            graph.launch()
+            # f16 operands: exact products, K of them added in f32 — about sqrt(K) 2^-24 of sum |products|, itself some
+            # 0.15 sqrt(K) peaks for such inputs: 2.3e-6; K 2^-24 = 1.5e-5 leaves a factor of six
+            assert peak_err(g.read(yd, m * n).reshape(m, n)[:, rows], want) <= k * 2.0 ** -24
+        graph.free()
+    finally:
+        g.close()
