@@ -852,8 +852,13 @@ GEMM_ENTRIES(q3k, LoaderQ3K)
 // operands agree, so lane (n, g) decodes the whole 32-weight block g of the chunk for row n (the per-thread loaders of the
 // tile: one or two wide loads) and feeds it to four instructions, 8 weights each; lane (m, g) reads the matching 64 bytes
 // of token m.  Up to 16 TG tokens per launch (TG accumulators); partial sums of the waves meet in LDS in wave order.
-//   gemm_few_<fmt>{,_r4}_t{1,2,4}(xh, w, y, K, N, accum, M)     grid [ceil(N / 16 RG),1,1] x 256 (or 512 where RG TG <= 4),
+//   gemm_few_<fmt>{,_r4}_t{1,2,4}(xh, w, y, K, N, accum, M)     grid [ceil(N / 16 RG),1,1] x 256 (or 512 where RG TG <= 8),
 //   K a multiple of 128, M <= 16 TG; `_r4`: RG = 4 groups of 16 rows per workgroup
+// Bound by latency: a wave waits a trip to memory per chunk for its tokens and the next block, and with 64 rows a workgroup
+// there is less than one workgroup per CU on most matrices.  So `_r4_t2` runs eight waves where there are fewer than two
+// workgroups per CU, each with half the chunks; the kernel alone, four -> eight waves, us: IQ4_XS 14336 x 4096 at 17 / 32 tokens
+// 20.0 -> 16.0 / 22.1 -> 18.9, x 14336 69.9 -> 48.7 / 76.6 -> 56.0, 28672 x 4096 31.2 -> 30.0 / 36.0 -> 35.6; Q8_0, whose
+// bytes bound it sooner, 0 - 2 % (30.4 -> 29.6 at 14336 x 4096), never slower up to 32640 rows.
 typedef float float4v __attribute__((ext_vector_type(4)));
 template <int J, class L>
 __device__ __forceinline__ half8 gm_frag(const L& ld) {
@@ -867,7 +872,8 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
                                               uint K, uint N, uint accum, uint M, const TM tm) {
     // RG groups of 16 rows per workgroup share every token fragment a lane reads (the tokens' bytes, re-read by every
     // workgroup, are most of the traffic of the 16-row form: 14336 rows x 16 tokens of K = 4096 read them 896 times)
-    __shared__ float red[RG * TG > 4 ? 4 : 8][RG * TG][256];     // (eight waves only where that stays within 32 KB)
+    constexpr uint S = RG * TG > 4 ? 4 : 8;                      // waves whose sums meet in LDS at once: 32 KB (64 KB for RG TG = 16)
+    __shared__ float red[S][RG * TG][256];
     const uint tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, nw = blockDim.x >> 6;
     const uint i16 = lane & 15u, g = lane >> 4;
     const uint n0 = blockIdx.x * (16u * RG);
@@ -928,17 +934,22 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
     }
 #undef GF_GROUP
     // D: lane (n = lane % 16, g) holds tokens 4 g + v of its group against row n
-#pragma unroll
-    for (int r = 0; r < RG; r++)
-#pragma unroll
-        for (int tg = 0; tg < TG; tg++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) red[wave][r * TG + tg][(g * 4u + v) * 16u + i16] = acc[r][tg][v];
+#define GF_SLOT(W) red[W][r * TG + tg][(g * 4u + v) * 16u + i16]
+#define GF_EACH _Pragma("unroll") for (int r = 0; r < RG; r++) _Pragma("unroll") for (int tg = 0; tg < TG; tg++) _Pragma("unroll") for (int v = 0; v < 4; v++)
+    if (nw > S) {                                                // eight waves on four slots: waves 4 .. 7 hand theirs to waves 0 .. 3
+        if (wave >= S) GF_EACH GF_SLOT(wave - S) = acc[r][tg][v];
+        __syncthreads();
+        if (wave < S) GF_EACH acc[r][tg][v] += GF_SLOT(wave);
+        __syncthreads();
+    }
+    if (wave < S) GF_EACH GF_SLOT(wave) = acc[r][tg][v];
     __syncthreads();
+#undef GF_SLOT
+#undef GF_EACH
     for (uint e = tid; e < (uint)(RG * TG) * 256u; e += blockDim.x) {
         const uint rt = e >> 8, r = rt / TG, tg = rt % TG, idx = e & 255u, tok = 16u * tg + (idx >> 4), row = n0 + 16u * r + (idx & 15u);
         float sum = red[0][rt][idx];
-        for (uint k = 1; k < nw; k++) sum += red[k][rt][idx];
+        for (uint k = 1; k < min(nw, S); k++) sum += red[k][rt][idx];
         if (tok < M && row < N) {
             float* o = y + (size_t)tm.out_row(tok) * N + row;
             *o = accum ? *o + sum : sum;

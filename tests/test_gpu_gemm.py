@@ -430,6 +430,25 @@ def test_few_token_kernel_by_name(gpu, orc, pkg, ty, tag, m, k, n, accum, thread
                          [256, 1, 1])
 
 
+@pytest.mark.parametrize("ty,tag", [(8, "q8_0"), (20, "iq4nl")])
+@pytest.mark.parametrize("m,k,n,accum", [(17, 128, 64, False), (24, 640, 65, True), (32, 1152, 127, False), (1, 2048, 1, False)])
+def test_few_token_kernel_with_eight_waves_on_four_slots(gpu, orc, pkg, ty, tag, m, k, n, accum):
+    """`gemm_few_<fmt>_r4_t2` on 512 threads: waves 4 .. 7 hand their sums to waves 0 .. 3 before those meet; chunk counts below,
+    at no multiple of and at twice the eight waves.  The bound of the 256-thread form."""
+    raw = pkg.synth.weights(ty, n, k, "few8", tag, n, k)
+    wf = orc.dequant_to_f16(raw, ty, n * k).view(np.float16).astype(np.float64).reshape(n, k)
+    x = pkg.synth.normal_f32(m * k, "few8", "x", m, k).astype(np.float16)
+    y0 = pkg.synth.normal_f32(m * n, "few8", "y0", m, n) if accum else np.full(m * n, 777.25, np.float32)
+    gpu.ensure_family("gemm")
+    yd = gpu.upload(np.concatenate([y0, np.full(n, 4242.5, np.float32)]))
+    gpu.dispatch(gpu.begin(), "gemm_few_%s_r4_t2" % tag, [(gpu.upload_bytes(x.view(np.uint8)), 0), (gpu.upload_bytes(raw), 0), (yd, 0)],
+                 [k, n, int(accum), m], [(n + 63) // 64, 1, 1], [512, 1, 1])
+    got = gpu.read(yd, m * n + n)
+    assert np.all(got[m * n:] == np.float32(4242.5)), "wrote past the last token"
+    got = got[:m * n].reshape(m, n) - (y0.reshape(m, n) if accum else 0.0)
+    assert peak_err(got, x.astype(np.float64).reshape(m, k) @ wf.T) <= (2e-5 if accum else 2e-6)
+
+
 @pytest.mark.parametrize("kernel,bm,bn", [("gemm_f16d_128", 128, 128), ("gemm_f16d_256x128", 256, 128), ("gemm_f16d_256", 256, 256),
                                           ("gemm_f16d_128_sk", 128, 128)])
 @pytest.mark.parametrize("m,k,n,accum", [(1, 64, 1, False), (129, 128, 127, True), (257, 192, 1100, False), (300, 1088, 385, True)])
