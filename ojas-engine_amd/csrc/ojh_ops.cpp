@@ -575,6 +575,8 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     const bool grid_fmt = ojh_grid_type(w->type);
     int rc;
     if ((rc = ensure(dev, grid_fmt ? "iq_grid" : "dequant")) || (rc = ensure(dev, "gemm_f16")) || (rc = ensure(dev, "glue"))) return rc;
+    // (the tiles a recorded call of fewer tokens would take: nothing can be loaded then)
+    if (!dev->capturing && (rc = ensure(dev, "gemm"))) return rc;
     ojh_buf *xh, *wdeq;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
     if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;

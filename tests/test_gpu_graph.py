@@ -123,3 +123,28 @@ def test_recorded_batch_needs_no_more_scratch_than_the_calls_before_it(gpu, orc,
         graph.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("ty", [14, 18])
+def test_a_smaller_batch_is_recorded_after_eager_long_ones(orc, pkg, ty):
+    """Eager calls long enough for the decode pass and the copied tile leave behind what a recorded call of fewer tokens
+    needs: the tile that decodes Q6_K rows on the way into LDS, the plain f16 tile behind the decoded rows of IQ3_XXS."""
+    n, k, many, few = 256, 512, 300, 100
+    w = pkg.synth.weights(ty, n, k, "graph", "w7")
+    x = pkg.synth.normal_f32(many * k, "graph", "x7").reshape(many, k)
+    g = pkg.HipGpu(0)
+    try:
+        lin, xd, yd = g.lin(ty, n, k, w), g.upload(x), g.alloc(many * n)
+        g.mm(xd, lin, yd, many, act_mode=pkg.ACT_FLOAT)
+        g.capture_begin()
+        g.mm(xd, lin, yd, few, act_mode=pkg.ACT_FLOAT)
+        graph = g.capture_end()
+        want = orc.matmul_ref(w, ty, n, k, x[:few], wmode=1, xmode=1)
+        for _ in range(3):
+            g.memset0(yd)
+            graph.launch()
+            # f16 operands, K products added in f32: K 2^-24 of the peak (the magnitudes sum to some 0.15 sqrt(K) peaks)
+            assert peak_err(g.read(yd, few * n).reshape(few, n), want) <= k * 2.0 ** -24
+        graph.free()
+    finally:
+        g.close()
