@@ -84,6 +84,7 @@ struct ojh_device {
     bool q8row_dec = true;       // OJAS_HIP_Q8ROW_DEC=0: 1 to 8 tokens on the per-row kernel instead of the one that stages the tokens in LDS
     uint32_t q8row_t128_min_m = 1; // OJAS_HIP_Q8ROW_T128_MIN_M: tokens from which that tile covers 128 tokens (0: never, 1: measured default, n: n)
     uint32_t q8row_split = 1;    // OJAS_HIP_Q8ROW_SPLIT: K slices of that tile (0: never, 1: by shape, n: n)
+    uint64_t scratch_max = 0;    // OJAS_HIP_SCRATCH_MAX: bytes of device memory the library's scratch may take (0: no limit of its own)
     int f16d_tile = 0;           // OJAS_HIP_F16D_TILE: that tile's size (0: by shape, 1: 128 x 128, 2: 256 x 128, 3: 256 x 256 tokens x rows)
     uint32_t deq_big_m = 1;      // OJAS_HIP_DEQ_BIG_M: tokens from which a format with a loader in the f16 tile is decoded into scratch all the same, ahead of the tile that copies both operands (0: never, 1: by shape, n: from n)
     uint32_t deq_min_m = 1;      // OJAS_HIP_DEQ_MIN_M: tokens from which a format without a tile of its own is decoded into scratch and multiplied on the f16 tile (0: never, 1: by matrix size, n: n)

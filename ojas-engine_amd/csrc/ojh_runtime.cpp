@@ -102,6 +102,7 @@ extern "C" int ojh_open(int ordinal, ojh_device **out) {
     if (const char *r = getenv("OJAS_HIP_MOE_DOWN_GS")) d->moe_down_gs = (uint32_t)atoi(r);
     if (const char *r = getenv("OJAS_HIP_Q8ROW_DEC")) d->q8row_dec = atoi(r) != 0;
     if (const char *r = getenv("OJAS_HIP_Q8ROW_SPLIT")) d->q8row_split = (uint32_t)atoi(r);
+    if (const char *r = getenv("OJAS_HIP_SCRATCH_MAX")) d->scratch_max = strtoull(r, nullptr, 10);
     if (const char *r = getenv("OJAS_HIP_F16D_TILE")) d->f16d_tile = atoi(r);
     if (const char *r = getenv("OJAS_HIP_DEQ_BIG_M")) d->deq_big_m = (uint32_t)atoi(r);
     if (const char *r = getenv("OJAS_HIP_DEQ_MIN_M")) d->deq_min_m = (uint32_t)atoi(r);
@@ -254,6 +255,13 @@ extern "C" int ojh_memset0(ojh_device *dev, ojh_buf *dst, size_t off, size_t byt
     return OJH_OK;
 }
 
+static size_t scratch_held(const ojh_device *dev) {
+    size_t held = 0;
+    for (const auto &slot : dev->scratch) held += slot.second ? slot.second->bytes : 0;
+    for (const ojh_buf *b : dev->parked) held += b->bytes;
+    return held;
+}
+
 // `fresh` (optional) tells whether the slot was (re)allocated by this call: its contents are then undefined.
 static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool *fresh) {
     ojh_buf *&slot = dev->scratch[name];
@@ -271,6 +279,12 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
             if (rc) return rc;
         }
         size_t cap = bytes < 4096 ? 4096 : bytes + bytes / 4;
+        if (dev->scratch_max) {
+            const size_t held = scratch_held(dev);
+            if (held + cap > dev->scratch_max) cap = bytes;
+            if (held + cap > dev->scratch_max)
+                return ojh_fail(OJH_ERR_HIP, "scratch '%s' of %zu bytes beside %zu exceeds OJAS_HIP_SCRATCH_MAX", name, bytes, held);
+        }
         int rc = ojh_alloc(dev, cap, &slot);
         if (rc) return rc;
         if (fresh) *fresh = true;
