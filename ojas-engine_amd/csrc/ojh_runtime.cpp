@@ -263,30 +263,41 @@ static size_t scratch_held(const ojh_device *dev) {
 }
 
 // `fresh` (optional) tells whether the slot was (re)allocated by this call: its contents are then undefined.
-static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool *fresh) {
+// `spare`: a buffer the caller can do without.  It is not allocated ahead of its size, nor where it would leave less memory
+// free than it takes, and a smaller one in the slot is given up only once the larger is there.
+static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool *fresh, bool spare = false) {
     ojh_buf *&slot = dev->scratch[name];
     if (fresh) *fresh = false;
     if (!slot || slot->bytes < bytes) {
         if (dev->capturing)
             return ojh_fail(OJH_ERR_ARG, "scratch '%s' would have to grow while recording a graph: run the call once "
                                           "eagerly first", name);
-        if (slot && dev->live_graphs > 0) {   // a recorded chain may still replay into it
-            dev->parked.push_back(slot);
-            slot = nullptr;
-        } else if (slot) {
-            int rc = ojh_free(dev, slot);
-            slot = nullptr;
-            if (rc) return rc;
-        }
-        size_t cap = bytes < 4096 ? 4096 : bytes + bytes / 4;
+        const bool park = slot && dev->live_graphs > 0;   // a recorded chain may still replay into it
+        size_t cap = bytes < 4096 ? 4096 : spare ? bytes : bytes + bytes / 4;
         if (dev->scratch_max) {
-            const size_t held = scratch_held(dev);
+            const size_t held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
             if (held + cap > dev->scratch_max) cap = bytes;
             if (held + cap > dev->scratch_max)
                 return ojh_fail(OJH_ERR_HIP, "scratch '%s' of %zu bytes beside %zu exceeds OJAS_HIP_SCRATCH_MAX", name, bytes, held);
         }
-        int rc = ojh_alloc(dev, cap, &slot);
-        if (rc) return rc;
+        ojh_buf *grown = nullptr;
+        int rc;
+        if (spare) {
+            size_t left = 0, total = 0;
+            OJH_HIP(hipSetDevice(dev->ordinal));
+            OJH_HIP(hipMemGetInfo(&left, &total));
+            if (left / 2 < cap) return ojh_fail(OJH_ERR_HIP, "scratch '%s' of %zu bytes: %zu left on the device", name, bytes, left);
+            if ((rc = ojh_alloc(dev, cap, &grown))) return rc;
+        }
+        if (park) {
+            dev->parked.push_back(slot);
+        } else if (slot && (rc = ojh_free(dev, slot))) {
+            slot = nullptr;
+            ojh_free(dev, grown);
+            return rc;
+        }
+        slot = grown;
+        if (!slot && (rc = ojh_alloc(dev, cap, &slot))) return rc;
         if (fresh) *fresh = true;
     }
     *out = slot;
@@ -295,6 +306,9 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
 
 int ojh_scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out) {
     return scratch_get(dev, name, bytes, out, nullptr);
+}
+int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out) {
+    return scratch_get(dev, name, bytes, out, nullptr, true);
 }
 
 // Cleared whenever the slot is (re)allocated — decided by the allocation itself, not by comparing addresses: the

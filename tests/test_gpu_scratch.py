@@ -1,4 +1,7 @@
-"""What the library's scratch does when memory is short: calls that can do without a buffer do without it."""
+"""What the library's scratch does when memory is short: calls that can do without a buffer do without it, and nothing
+that was there is given up for a buffer that does not come."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -7,6 +10,12 @@ from conftest import peak_err
 pytestmark = pytest.mark.gpu
 Q6_K = 14
 K = 2048
+
+
+def _free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 def _device(pkg, monkeypatch, limit=0):
@@ -42,5 +51,35 @@ def test_a_batch_without_room_for_the_decoded_rows_keeps_its_loader(pkg, orc, mo
         yd = g.alloc(m * n)
         g.mm(g.upload(x), g.lin(Q6_K, n, K, _weights(pkg, n)), yd, m, act_mode=pkg.ACT_FLOAT)
         _check(g, yd, n, m, toks, _want(pkg, orc, x[toks]))
+    finally:
+        g.close()
+
+
+def test_a_refused_growth_leaves_the_smaller_buffer(pkg, orc, monkeypatch):
+    """Two layer sizes by turns beside a recorded chain, the larger beyond the limit: every call succeeds, and neither gives
+    the smaller matrix's buffer up (or strands one per turn)."""
+    small, large, m = 8192, 65536, 300
+    g = _device(pkg, monkeypatch, 160 << 20)
+    try:
+        x = pkg.synth.normal_f32(m * K, "scratch", "x", m).reshape(m, K)
+        want = _want(pkg, orc, x[:8])
+        xd, yd = g.upload(x), g.alloc(m * large)
+        lins = {n: g.lin(Q6_K, n, K, _weights(pkg, n)) for n in (small, large)}
+        g.mm(xd, lins[large], yd, m, act_mode=pkg.ACT_FLOAT)
+        g.mm(xd, lins[small], yd, m, act_mode=pkg.ACT_FLOAT)
+        g.capture_begin()
+        g.mm(xd, lins[small], yd, m, act_mode=pkg.ACT_FLOAT)
+        graph = g.capture_end()
+        g.submit()
+        free = _free_bytes()
+        for _ in range(3):
+            for n in (large, small):
+                g.mm(xd, lins[n], yd, m, act_mode=pkg.ACT_FLOAT)
+                _check(g, yd, n, m, slice(0, 8), want)
+                assert _free_bytes() == free, n
+            g.memset0(yd)
+            graph.launch()
+            _check(g, yd, small, m, slice(0, 8), want)
+        graph.free()
     finally:
         g.close()
