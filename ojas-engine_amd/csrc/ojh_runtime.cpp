@@ -179,7 +179,11 @@ extern "C" int ojh_alloc(ojh_device *dev, size_t bytes, ojh_buf **out) {
     if (dev->capturing) return ojh_fail(OJH_ERR_ARG, "ojh_alloc while recording a graph");
     OJH_HIP(hipSetDevice(dev->ordinal));
     void *p = nullptr;
-    OJH_HIP(hipMalloc(&p, bytes ? bytes : 1));
+    hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // (reported here: a caller that goes on without the buffer leaves no error for the next check)
+        return ojh_fail(OJH_ERR_HIP, "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+    }
     ojh_buf *b = new ojh_buf();
     b->ptr = p;
     b->bytes = bytes;

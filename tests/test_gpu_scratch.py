@@ -83,3 +83,11 @@ def test_a_refused_growth_leaves_the_smaller_buffer(pkg, orc, monkeypatch):
         graph.free()
     finally:
         g.close()
+
+
+def test_a_failed_allocation_leaves_no_error_behind(gpu, pkg):
+    """... for whoever asks the runtime next: the failure is the return code's, and a call that goes on without the buffer
+    has succeeded."""
+    with pytest.raises(pkg.OjasHipError, match="hipMalloc"):
+        gpu.alloc_bytes(1 << 50)
+    assert ctypes.CDLL("libamdhip64.so").hipGetLastError() == 0
