@@ -14,6 +14,7 @@ struct ojh_buf {
     void *ptr = nullptr;
     size_t bytes = 0;
     bool owned = false;
+    bool recorded = false;       // scratch handed out while a chain was recorded
 };
 
 struct ojh_lin {
@@ -111,7 +112,8 @@ struct ojh_device {
     bool capture_hip_graph = false;
     std::vector<ojh_command> recorded;
     // Recorded chains hold raw pointers into the scratch buffers.  While any chain of this device is alive, a scratch
-    // buffer that has to grow is parked here instead of freed, and released when the last chain is.
+    // buffer that was handed out to a recording and has to grow is parked here instead of freed, and released when the
+    // last chain is.
     int live_graphs = 0;
     std::vector<ojh_buf *> parked;
     // the single-launch decode chain (ojh_chain.cpp): its counters on the device, the word a wait that gave up sets

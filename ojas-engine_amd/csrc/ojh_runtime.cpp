@@ -276,7 +276,7 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
         if (dev->capturing)
             return ojh_fail(OJH_ERR_ARG, "scratch '%s' would have to grow while recording a graph: run the call once "
                                           "eagerly first", name);
-        const bool park = slot && dev->live_graphs > 0;   // a recorded chain may still replay into it
+        const bool park = slot && slot->recorded && dev->live_graphs > 0;   // a recorded chain may still replay into it
         size_t cap = bytes < 4096 ? 4096 : spare ? bytes : bytes + bytes / 4;
         if (dev->scratch_max) {
             const size_t held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
@@ -304,6 +304,7 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
         if (!slot && (rc = ojh_alloc(dev, cap, &slot))) return rc;
         if (fresh) *fresh = true;
     }
+    if (dev->capturing) slot->recorded = true;
     *out = slot;
     return OJH_OK;
 }

@@ -1,5 +1,5 @@
-"""What the library's scratch does when memory is short: calls that can do without a buffer do without it, and nothing
-that was there is given up for a buffer that does not come."""
+"""What the library's scratch does when memory is short: calls that can do without a buffer do without it, nothing that
+was there is given up for a buffer that does not come, and only what a recorded chain holds is kept beside a larger one."""
 import ctypes
 
 import numpy as np
@@ -91,3 +91,54 @@ def test_a_failed_allocation_leaves_no_error_behind(gpu, pkg):
     with pytest.raises(pkg.OjasHipError, match="hipMalloc"):
         gpu.alloc_bytes(1 << 50)
     assert ctypes.CDLL("libamdhip64.so").hipGetLastError() == 0
+
+
+def test_an_outgrown_buffer_no_chain_holds_is_given_back(pkg, orc, monkeypatch):
+    """A recorded chain that never touched the decoded rows' scratch (a decode step) does not keep what eager prefill outgrows."""
+    m, sizes = 300, (16384, 32768, 65536)
+    g = _device(pkg, monkeypatch)
+    try:
+        x = pkg.synth.normal_f32(m * K, "scratch", "x", m).reshape(m, K)
+        want = _want(pkg, orc, x[:8])
+        xd, yd = g.upload(x), g.alloc(m * sizes[-1])
+        lins = [g.lin(Q6_K, n, K, _weights(pkg, n)) for n in sizes]
+        one = g.lin(Q6_K, 256, K, _weights(pkg, 256))
+        g.mm(xd, one, yd, m, act_mode=pkg.ACT_FLOAT)                       # code objects loaded, the activations' scratch sized
+        g.mm(xd, one, yd, 1, act_mode=pkg.ACT_Q8K)
+        g.capture_begin()
+        g.mm(xd, one, yd, 1, act_mode=pkg.ACT_Q8K)
+        graph = g.capture_end()
+        g.submit()
+        free = _free_bytes()
+        for n, lin in zip(sizes, lins):
+            g.mm(xd, lin, yd, m, act_mode=pkg.ACT_FLOAT)
+            _check(g, yd, n, m, slice(0, 8), want)
+        assert free - _free_bytes() <= sizes[-1] * K * 2 + (16 << 20)      # the largest alone, not the 67 and 134 MB before it
+        graph.free()
+    finally:
+        g.close()
+
+
+def test_a_chain_keeps_the_decoded_rows_it_was_recorded_with(pkg, orc, monkeypatch):
+    """... while one that did replays into its own buffer after eager calls have outgrown it."""
+    m, small, large = 130, 512, 16384
+    g = _device(pkg, monkeypatch)
+    try:
+        x = pkg.synth.normal_f32(m * K, "scratch", "x", m).reshape(m, K)
+        want = _want(pkg, orc, x[:8])
+        xd, yd, yl = g.upload(x), g.alloc(m * small), g.alloc(m * large)
+        lins = {n: g.lin(Q6_K, n, K, _weights(pkg, n)) for n in (small, large)}
+        g.mm(xd, lins[small], yd, m, act_mode=pkg.ACT_FLOAT)
+        eager = g.read(yd, m * small)
+        g.capture_begin()
+        g.mm(xd, lins[small], yd, m, act_mode=pkg.ACT_FLOAT)
+        graph = g.capture_end()
+        for _ in range(3):
+            g.mm(xd, lins[large], yl, m, act_mode=pkg.ACT_FLOAT)
+            g.memset0(yd)
+            graph.launch()
+            assert np.array_equal(g.read(yd, m * small), eager)
+            _check(g, yl, large, m, slice(0, 8), want)
+        graph.free()
+    finally:
+        g.close()
