@@ -13,9 +13,10 @@
 // to cover a trip to memory with (128 x 128: four steps of 32 KB).  The barrier of a step sits before its last K
 // sub-step, whose fragments are in registers by then: its matrix instructions cover the next step's first fragments
 // and the requests for the step that takes over the slot.
-// Tile -> workgroup: workgroups are dealt round robin to the eight XCDs, so the token tiles of one row tile are given
-// numbers eight apart: one L2 fetches a row tile's weights, once.
+// Tile -> workgroup (ojk_spread.h): the token tiles of one row tile stay on one XCD, whose L2 fetches its weights once, and
+// every XCD has its share of the tiles however few the row tiles are.
 #include "ojk_common.h"
+#include "ojk_spread.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
@@ -33,13 +34,13 @@ __device__ __forceinline__ void gemm_f16_body(const ushort* __restrict__ xh, con
     constexpr uint BM = 64u * MI, BN = 64u * NJ, RB = 128u, STAGE = (BM + BN) * RB;                // RB: bytes of a row per K step
     constexpr int XL = 2 * MI, WL = 2 * NJ, NC = XL + WL, Q = MI * NJ;     // copies per wave and step: activations, weights, all; MFMAs per sub-step
     const uint mt = (M + BM - 1u) / BM, nt_ = (N + BN - 1u) / BN;
-    const uint idx = blockIdx.x >> 3, tn = (blockIdx.x & 7u) + 8u * (idx / mt), tm = idx % mt;
-    if (tn >= nt_) return;
+    uint tn, tm, slice;
+    if (!ojk_spread(blockIdx.x, SPLITK ? blockIdx.y : 0u, nt_, mt, SPLITK ? nsplit : 1u, tn, tm, slice)) return;
     const uint n0 = tn * BN, m0 = tm * BM;
     uint s_begin = 0, s_end = K >> 6;
     if (SPLITK) {
         const uint per = (s_end + nsplit - 1u) / nsplit;
-        s_begin = min(blockIdx.y * per, s_end);
+        s_begin = min(slice * per, s_end);
         s_end = min(s_begin + per, s_end);
         if (s_begin >= s_end) return;
     }
