@@ -35,7 +35,8 @@ __device__ __forceinline__ void gemm_f16_body(const ushort* __restrict__ xh, con
     constexpr int XL = 2 * MI, WL = 2 * NJ, NC = XL + WL, Q = MI * NJ;     // copies per wave and step: activations, weights, all; MFMAs per sub-step
     const uint mt = (M + BM - 1u) / BM, nt_ = (N + BN - 1u) / BN;
     uint tn, tm, slice;
-    if (!ojk_spread(blockIdx.x, SPLITK ? blockIdx.y : 0u, nt_, mt, SPLITK ? nsplit : 1u, tn, tm, slice)) return;
+    const uint place = (blockIdx.x >> 3) + (SPLITK ? blockIdx.y * (gridDim.x >> 3) : 0u);
+    if (!ojk_spread(blockIdx.x & 7u, place, nt_, mt, SPLITK ? nsplit : 1u, tn, tm, slice)) return;
     const uint n0 = tn * BN, m0 = tm * BM;
     uint s_begin = 0, s_end = K >> 6;
     if (SPLITK) {
