@@ -497,3 +497,23 @@ def test_decoder_with_activations_converted_beside_it(gpu, orc, pkg, ty, tag, bf
     got = gpu.read(z, nz + 8)
     assert np.all(got[:nz] == 0) and np.all(got[nz:] == 7.5)
     assert np.all(gpu.read(out, n * k // 2 + 8)[-8:] == 7.5)
+
+
+@pytest.mark.parametrize("n,k,m,bf16,accum", [(385, 1024, 130, 0, False), (128, 1280, 129, 1, False), (385, 1024, 257, 1, True)])
+def test_grid_codebook_batch_over_k_slices(gpu, orc, pkg, n, k, m, bf16, accum):
+    """Rows of a format whose decoder converts nothing beside its work: the activations converted and the output cleared in a
+    launch of their own, ahead of K slices that add into it — over an output that held something else, ragged rows and
+    tokens.  f16 operands, K products added in f32: K 2^-24 of the peak (the magnitudes sum to some 0.15 sqrt(K) peaks), and
+    with `accum` the rounding of the sum onto what was there, of the same size."""
+    raw = pkg.synth.weights(18, n, k, "gridsk", n, k)
+    x = pkg.synth.normal_f32(m * k, "gridsk", "x", m)
+    xb = pkg.synth.to_bf16_bits(x) if bf16 else x
+    if bf16:
+        x = pkg.synth.bf16_bits_to_f32(xb)
+    want = orc.matmul_ref(raw, 18, n, k, x.reshape(m, k), wmode=1, xmode=1)
+    y0 = pkg.synth.normal_f32(m * n, "gridsk", "y0") if accum else np.full(m * n, 777.25, np.float32)
+    yd = gpu.upload(np.concatenate([y0, np.full(64, 777.25, np.float32)]))
+    gpu.mm(gpu.upload_bytes(xb.view(np.uint8)), gpu.lin(18, n, k, raw), yd, m, accum, x_dtype=bf16, act_mode=pkg.ACT_FLOAT)
+    got = gpu.read(yd, m * n + 64)
+    assert np.all(got[m * n:] == np.float32(777.25))
+    assert peak_err(got[:m * n].reshape(m, n), want + (y0.reshape(m, n) if accum else 0.0)) <= 2 * k * 2.0 ** -24
