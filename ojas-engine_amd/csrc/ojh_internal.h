@@ -145,6 +145,7 @@ bool ojh_float_rows(uint32_t ggml_type);   // the CPU path reads f32 activations
 size_t ojh_block_align(const ojh_block_format *f);
 uint32_t ojh_matmul_q8row_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M);  // K slices of the row-int8 tile (1: whole)
 uint32_t ojh_gemm_q8k_gs_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M);   // K slices of the Q6_K / Q5_K int8 tile (1: whole)
+uint32_t ojh_gemm_slices(const ojh_device *dev, uint64_t tiles, uint32_t most);   // K slices of an f16 tile
 uint32_t ojh_gemm_sr_slices(uint32_t K, uint32_t nsplit);   // K slices of the `_sr` tiles that hold a super-block
 bool ojh_grid_type(uint32_t ggml_type);    // a grid-codebook format: its kernels live in the family "iq_grid"
 bool ojh_float_only(uint32_t ggml_type);   // ... and only the f32-activation matvecs exist for it

@@ -1338,6 +1338,14 @@ static int check_gemm_q4l(const ojh_kernel_spec *s, const uint32_t *c, const uin
     return OJH_OK;
 }
 
+// K slices until every CU has a tile, `most` at most
+uint32_t ojh_gemm_slices(const ojh_device *dev, uint64_t tiles, uint32_t most) {
+    const uint32_t cus = dev ? (uint32_t)dev->prop.multiProcessorCount : 256u;
+    uint32_t z = tiles ? (uint32_t)(cus / tiles) : 1;   // floor: 224 tiles on 256 CUs are better left whole
+    if (z > most) z = most;
+    if (z > 16) z = 16;
+    return z ? z : 1;
+}
 static int shape_gemm(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M,
                       uint32_t grid[3], uint32_t block[3]) {
     bool sk;
@@ -1347,13 +1355,8 @@ static int shape_gemm(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t 
     grid[1] = (M + bm - 1) / bm;
     grid[2] = 1;
     if (sk) {  // split K until every CU has a tile, at least 4 K-steps per slice
-        uint32_t cus = dev ? (uint32_t)dev->prop.multiProcessorCount : 256u;
-        uint32_t tiles = grid[0] * grid[1], steps = K / 64;
-        uint32_t z = tiles ? cus / tiles : 1;  // floor: 224 tiles on 256 CUs are better left whole
-        if (z > steps / 4) z = steps / 4;
-        if (s->rows_per_wave == 13 && z > steps / 16) z = steps / 16;   // K over the waves: a super-block per wave and slice at least
-        if (z > 16) z = 16;
-        grid[2] = z ? z : 1;
+        const uint32_t steps = K / 64;     // (13: K over the waves, a super-block per wave and slice at least)
+        grid[2] = ojh_gemm_slices(dev, (uint64_t)grid[0] * grid[1], s->rows_per_wave == 13 ? steps / 16 : steps / 4);
     }
     block[0] = 256;
     block[1] = block[2] = 1;
@@ -1391,13 +1394,7 @@ static int shape_gemm_f16d(const ojh_kernel_spec *s, const ojh_device *dev, uint
     const uint32_t nt = (N + bn - 1) / bn, mt = (M + bm - 1) / bm;
     grid[0] = (nt + 7) / 8 * 8 * mt;
     grid[1] = grid[2] = 1;
-    if (s->rows_per_wave & 1024) {   // slices of eight K steps at least, until every CU has one
-        const uint32_t cus = dev ? (uint32_t)dev->prop.multiProcessorCount : 256u, tiles = nt * mt;
-        uint32_t z = tiles ? cus / tiles : 1;
-        if (z > K / 512) z = K / 512;
-        if (z > 16) z = 16;
-        grid[1] = z ? z : 1;
-    }
+    if (s->rows_per_wave & 1024) grid[1] = ojh_gemm_slices(dev, (uint64_t)nt * mt, K / 512);   // (eight K steps each at least)
     block[0] = 256;
     block[1] = block[2] = 1;
     return OJH_OK;

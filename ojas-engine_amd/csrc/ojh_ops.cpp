@@ -546,14 +546,54 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 // tile whose operands the memory system copies (`gemm_f16d_*`) — the same weights (dequant_to_f16's bits) and f16 activations
 // as the tile that decodes on the way into LDS, sums in another order.  That tile's loaders fetch a row's block piecemeal,
 // 64 weights a step (a 210-byte Q6_K block is touched in four cache lines four times over), and decode every weight once per
-// 128 or 256 tokens; the pass reads and writes everything once (0.5 us per 2^20 weights), so it pays from some batch on.
-// Measured, decoding tile -> pass + copying tile, us:
-//   Q6_K   6914 x 2816 at 333 tokens 60 -> 35, 14336 x 4096 at 130 79 -> 71, at 700 200 -> 129, 4096^2 at 700 83 -> 45,
-//          4096 x 14336 at 700 267 -> 145; but 30000 x 2048 at 130 .. 256 tokens 58 .. 61 against 72 .. 75, at 400 114 -> 98
-//   Q5_K   6914 x 2816 at 400 46 -> 38, 4096 x 14336 at 400 108 -> 105, at 700 196 -> 146; 14336 x 4096 at 400 87 against 98,
-//          at 700 170 -> 130, 30000 x 2048 at 400 96 against 99, at 700 144 -> 143 (Q8_0 and IQ4_XS within 6 % of these)
-//   formats decoded ahead of a batch in any case (grid codebooks, Q3_K beyond its cap), against `gemm_mm_f16*`: from 129
-//   tokens 73 -> 65 (Q3_K 14336 x 4096 at 160), 229 -> 171 (30000 x 2048 at 1024); level below.
+// 128 or 256 tokens; the pass reads and writes everything once.  Which is ahead is a matter of rounds of workgroups over the
+// CUs more than of rows or tokens, so both are priced, in us: K steps on the busiest CU times what a step takes (a part
+// that does not depend on how many CUs are busy, and one that grows with them), the atomics that K slices meet in, the
+// pass.  The prices are least squares over 20000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048
+// tokens); what they choose is on average within 0.5 % of the faster route (by tokens and rows alone: 1.7 %).  Both routes measured, decoding tile / pass + copying tile:
+//   Q6_K   6914 x 2816 at 333 tokens 60 / 37, 14336 x 4096 at 130 79 / 71, 4096 x 4096 at 700 83 / 45
+//   IQ4_NL 5330 x 11776 at 333 95 / 85, 8192 x 14336 at 333 162 / 215 (decoded rows beyond 112 MB: read back from memory)
+//   Q5_0   8576 x 4096 at 257 106 / 51, MXFP4 8192 x 14336 at 512 188 / 249, Q4_1 8192 x 1024 at 512 26 / 32
+static uint32_t f16d_tile(const ojh_device *dev, uint32_t N, uint32_t m) {   // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256 tokens x rows
+    // rounds of workgroups over the chip times a tile's time per K step with every CU busy (0.49 / 0.83 / 1.37 us): within
+    // 0.13 % of the fastest of the three on average; 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262;
+    // 4096 x 14336 at 2048 334 / 279 / 388; 6914 x 2816 at 333 35 / 51 / 76
+    const uint64_t cus = (uint64_t)dev->prop.multiProcessorCount;
+    auto rounds = [&](uint32_t bm, uint32_t bn) { return ((uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm) + cus - 1) / cus; };
+    if (dev->f16d_tile > 0) return (uint32_t)dev->f16d_tile - 1u;
+    const uint64_t c1 = 8 * rounds(128, 128), c2 = 13 * rounds(256, 128), c3 = 23 * rounds(256, 256);
+    return c3 <= c1 && c3 <= c2 ? 2u : c2 < c1 ? 1u : 0u;
+}
+// whether the tile that decodes on the way into LDS is 128 tokens tall instead of 256
+static bool gemm_mm_m128(const ojh_device *dev, uint32_t N, uint32_t m, bool decoded) {
+    const uint64_t t256 = (uint64_t)((N + 127) / 128) * ((m + 255) / 256);
+    return dev->gemm_m128 && (m <= (uint32_t)dev->gemm_m128 || 2 * t256 <= (uint32_t)dev->prop.multiProcessorCount || decoded);
+}
+static bool f16d_pays(const ojh_device *dev, const ojh_lin *w, uint32_t m, bool decoded) {
+    const uint32_t K = w->k, N = w->n;
+    const double cus = dev->prop.multiProcessorCount, mi = (double)N * K / (1 << 20);
+    auto walk = [&](uint32_t bm, uint32_t bn, uint32_t most, double round, double fill) {
+        const uint64_t tiles = (uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm);
+        const uint32_t z = dev->gemm_sr ? 1u : ojh_gemm_slices(dev, tiles, most);
+        const double per_cu = tiles * z / cus;
+        return (K / 64 + z - 1) / z * (round * ceil(per_cu) + fill * per_cu) + (z > 1 ? 3.1 * z * m * N / (1 << 20) : 0.0);
+    };
+    const uint32_t tile = f16d_tile(dev, N, m);
+    const double copied = tile == 2 ? 3.0 + walk(256, 256, 1, 1.14, 0.23) : tile == 1 ? 1.5 + walk(256, 128, 1, 0.66, 0.17)
+                                                                                   : walk(128, 128, K / 512, 0.30, 0.19);
+    // (a format that is decoded first in any case: the same pass, conversion included only where its decoder does that)
+    if (decoded) return copied < (ojh_grid_type(w->type) ? 0.0 : 0.5) + walk(128, 128, K / 256, 0.40, 0.20);
+    // a K step of 128 x 128 and of 256 x 128 on the loader
+    double s128 = 0.79, s256 = 1.14;
+    switch (w->type) {
+    case OJH_IQ4_NL: case OJH_Q4_0: case OJH_Q8_0: s128 = 0.71; s256 = 1.06; break;
+    case OJH_Q4_1: s128 = 0.90; s256 = 1.20; break;
+    case OJH_Q5_0: case OJH_Q6_K: s128 = 1.14; s256 = 1.46; break;
+    default: break;
+    }
+    const double loaded = gemm_mm_m128(dev, N, m, false) ? walk(128, 128, K / 256, s128, 0.0) : 2.0 + walk(256, 128, K / 256, s256, 0.0);
+    return 1.5 + 0.42 * mi + (mi > 56 ? 0.45 * (mi - 56) : 0.0) + copied < loaded;
+}
 static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
     const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
     if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || q4kl || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
@@ -565,9 +605,7 @@ static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int 
             return false;
     }
     if (dev->deq_big_m > 1) return m >= dev->deq_big_m;
-    if (decoded) return m >= 129u;
-    if (w->type == OJH_Q6_K) return m >= (w->n > 16384u ? 257u : 129u);
-    return m >= (w->n > 8192u ? 513u : 257u);
+    return m >= 129u && f16d_pays(dev, w, m, decoded);
 }
 // Whether all the route needs is there.  What every form of the call needs comes first, so that the decoded rows' scratch,
 // which a format with a loader can do without, never takes its room: the activations' scratch, and the family of the tiles
@@ -584,24 +622,16 @@ static int f16d_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, bool decode
 }
 static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, uint32_t m,
                        int accum) {
-    const uint32_t K = w->k, N = w->n, cus = (uint32_t)dev->prop.multiProcessorCount;
+    const uint32_t K = w->k, N = w->n, tile = f16d_tile(dev, N, m);
     const bool grid_fmt = ojh_grid_type(w->type);
     int rc;
     ojh_buf *xh, *wdeq;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
     if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;
-    auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm); };
-    auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + cus - 1) / cus; };
-    // rounds of workgroups over the chip times a tile's measured time per K step (0.34 / 0.55 / 0.98 us at 128 x 128, 256 x
-    // 128, 256 x 256): 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 /
-    // 279 / 388; 6914 x 2816 at 333 35 / 51 / 76
-    const char *name = "gemm_f16d_128";
-    const uint64_t c1 = 8 * rounds(128, 128), c2 = 13 * rounds(256, 128), c3 = 23 * rounds(256, 256);
-    if (dev->f16d_tile == 3 || (!dev->f16d_tile && c3 <= c1 && c3 <= c2)) name = "gemm_f16d_256";
-    else if (dev->f16d_tile == 2 || (!dev->f16d_tile && c2 < c1)) name = "gemm_f16d_256x128";
+    const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? "gemm_f16d_256x128" : "gemm_f16d_128";
     uint32_t sg[3], sb[3];
     bool sk = false;
-    if (!strcmp(name, "gemm_f16d_128")) {
+    if (!tile) {
         if ((rc = ojh_launch_shape(dev, "gemm_f16d_128_sk", K, N, m, sg, sb))) return rc;
         sk = sg[1] > 1 && !dev->gemm_sr;
         if (sk) name = "gemm_f16d_128_sk";
@@ -765,10 +795,8 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         std::string base = std::string("gemm_mm_") + (deq_tile ? "f16" : w->type == OJH_Q8_0 ? "q8_0" : f->tag);
         // (the tile that shares the dequantized weights through LDS is 256 tokens tall; its 128-token form up to 128 tokens
         // and wherever the taller one would give at most half of the CUs a tile — 14336 x 4096 at 256 tokens: Q8_0 78 ->
-        // 55 us, Q6_K 100 -> 77; plain f16 rows take it at every size, 322 -> 288 us at 2048 tokens)
-        const uint64_t t256 = (uint64_t)((N + 127) / 128) * ((m + 255) / 256);
-        if (!xl && dev->gemm_m128 && (m <= (uint32_t)dev->gemm_m128 || 2 * t256 <= (uint32_t)dev->prop.multiProcessorCount || deq_tile))
-            base += "_m128";
+        // 55 us, Q6_K 100 -> 77 — and for plain f16 rows, 322 -> 288 us at 2048 tokens)
+        if (!xl && gemm_mm_m128(dev, N, m, deq_tile)) base += "_m128";
         if (xl) {
             // 256-token tiles when they give every CU a tile, or half of them with a K long enough
             // to split in two without the slices' fixed costs showing (measured on MI355X);

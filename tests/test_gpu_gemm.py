@@ -517,3 +517,20 @@ def test_grid_codebook_batch_over_k_slices(gpu, orc, pkg, n, k, m, bf16, accum):
     got = gpu.read(yd, m * n + 64)
     assert np.all(got[m * n:] == np.float32(777.25))
     assert peak_err(got[:m * n].reshape(m, n), want + (y0.reshape(m, n) if accum else 0.0)) <= 2 * k * 2.0 ** -24
+
+
+@pytest.mark.parametrize("ty,n,k,m,copied", [(14, 6914, 2816, 333, True), (6, 8576, 4096, 257, True), (18, 4096, 4096, 300, True), (2, 256, 4096, 700, True),
+                                             (20, 8192, 14336, 333, False), (139, 8192, 14336, 512, False), (14, 8192, 14336, 160, False), (20, 8192, 4096, 128, False)])
+def test_long_batches_take_the_route_that_is_ahead(pkg, ty, n, k, m, copied):
+    """Rows decoded into scratch ahead of the copied tile, or on the way into LDS: sizes where one route measured 10 - 50 %
+    ahead of the other.  A device of its own tells the route by the code objects it had to load."""
+    g = pkg.HipGpu(0)
+    try:
+        lin = g.lin_wrap(ty, n, k, g.alloc_bytes(n * pkg.row_bytes(ty, k)))
+        x = g.alloc(m * k)
+        g.memset0(x)
+        g.mm(x, lin, g.alloc(m * n), m, act_mode=pkg.ACT_FLOAT)
+        g.submit()
+        assert bool(g.has_kernel("gemm_f16d_128")) == copied
+    finally:
+        g.close()
