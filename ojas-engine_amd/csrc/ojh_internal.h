@@ -87,7 +87,7 @@ struct ojh_device {
     uint32_t q8row_split = 1;    // OJAS_HIP_Q8ROW_SPLIT: K slices of that tile (0: never, 1: by shape, n: n)
     uint64_t scratch_max = 0;    // OJAS_HIP_SCRATCH_MAX: bytes of device memory the library's scratch may take (0: no limit of its own)
     int f16d_tile = 0;           // OJAS_HIP_F16D_TILE: that tile's size (0: by shape, 1: 128 x 128, 2: 256 x 128, 3: 256 x 256 tokens x rows)
-    uint32_t deq_big_m = 1;      // OJAS_HIP_DEQ_BIG_M: tokens from which a format with a loader in the f16 tile is decoded into scratch all the same, ahead of the tile that copies both operands (0: never, 1: by shape, n: from n)
+    uint32_t deq_big_m = 1;      // OJAS_HIP_DEQ_BIG_M: tokens from which a format with a loader in the f16 tile is decoded into scratch all the same, ahead of the tile that copies both operands (0: never, 1: by shape, n: from n; Q6_K of 32 Mi weights or more, Q5_K / Q8_0 of as many from 2 n)
     uint32_t deq_min_m = 1;      // OJAS_HIP_DEQ_MIN_M: tokens from which a format without a tile of its own is decoded into scratch and multiplied on the f16 tile (0: never, 1: by matrix size, n: n)
     uint32_t q80_tile_min_m = 1; // OJAS_HIP_Q80_TILE_MIN_M: tokens from which OJH_ACT_AUTO sends Q8_0 rows to the f16 tile (0: GEMM_MIN_M, 1: by shape, n: n)
     int gemm_m128 = 128;         // OJAS_HIP_GEMM_M128: tokens up to which Q5_K / Q6_K / Q8_0 batches take the 128-token f16 tile (0: never)

@@ -604,7 +604,11 @@ static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int 
             slot == dev->scratch.end() || !slot->second || slot->second->bytes < (size_t)w->n * w->k * 2)
             return false;
     }
-    if (dev->deq_big_m > 1) return m >= dev->deq_big_m;
+    if (dev->deq_big_m > 1 && !decoded) {   // asked for: Q6_K and, from twice as many tokens, Q5_K / Q8_0 rows of large matrices
+        const bool kq = w->type == OJH_Q6_K || w->type == OJH_Q5_K || w->type == OJH_Q8_0;
+        if (w->type == OJH_Q4_K || (kq && (uint64_t)w->n * w->k < (32ull << 20))) return false;
+        return m >= (w->type == OJH_Q5_K || w->type == OJH_Q8_0 ? 2 * dev->deq_big_m : dev->deq_big_m);
+    }
     return m >= 129u && f16d_pays(dev, w, m, decoded);
 }
 // Whether all the route needs is there.  What every form of the call needs comes first, so that the decoded rows' scratch,

@@ -534,3 +534,21 @@ def test_long_batches_take_the_route_that_is_ahead(pkg, ty, n, k, m, copied):
         assert bool(g.has_kernel("gemm_f16d_128")) == copied
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("ty,n,k,m,copied", [(14, 4096, 4096, 300, False), (14, 8192, 4096, 300, True), (14, 8192, 4096, 199, False), (8, 8192, 4096, 399, False),
+                                             (8, 8192, 4096, 400, True), (20, 256, 1024, 200, True), (20, 256, 1024, 199, False), (18, 4096, 4096, 300, True)])
+def test_a_pinned_token_count_means_what_it_meant(pkg, monkeypatch, ty, n, k, m, copied):
+    """`OJAS_HIP_DEQ_BIG_M=200`: Q6_K rows of 32 Mi weights from 200 tokens, Q8_0 rows of as many from 400, IQ4_NL rows of any
+    matrix from 200; formats that are decoded in any case are not its business."""
+    monkeypatch.setenv("OJAS_HIP_DEQ_BIG_M", "200")
+    g = pkg.HipGpu(0)
+    try:
+        lin = g.lin_wrap(ty, n, k, g.alloc_bytes(n * pkg.row_bytes(ty, k)))
+        x = g.alloc(m * k)
+        g.memset0(x)
+        g.mm(x, lin, g.alloc(m * n), m, act_mode=pkg.ACT_FLOAT)
+        g.submit()
+        assert bool(g.has_kernel("gemm_f16d_128")) == copied
+    finally:
+        g.close()
