@@ -264,7 +264,7 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     // ... a wave per row tile where 16 tokens of K fit the workgroup's LDS (OJAS_HIP_MOE=4 keeps the workgroup-per-tile form)
     const bool mt_gu = mm && dev->moe_mode != 4 && ojh_moe_mt_lds(d) <= 81920;
     const bool mt_down = mm && dev->moe_mode != 4 && !down5 && ojh_moe_mt_lds(n_ff) <= 81920;
-    const uint32_t b1024[3] = {1024, 1, 1};
+    uint32_t b_mt[3] = {1024, 1, 1};
     // 1. quantize the tokens once, 2. group the (token, slot) assignments by expert: one launch where a token is one
     //    workgroup's work (the grouping rides along as an extra workgroup), two otherwise
     if (dev->moe_fuse && d <= 8192) {
@@ -278,11 +278,11 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     }
     // 3. gate/up + SiLU*mul, one launch over all experts
     {
-        uint32_t g[3] = {mt_gu ? ojh_moe_mt_groups(dev, n_ff, E, 8) : mm ? (n_ff + 15) / 16 : (n_ff + 7) / 8, E, 1};
+        uint32_t g[3] = {mt_gu ? ojh_moe_mt_groups(dev, d, n_ff, E, true, &b_mt[0]) : mm ? (n_ff + 15) / 16 : (n_ff + 7) / 8, E, 1};
         if ((rc = ojh_launch(dev, mt_gu ? "moe_gu_q4k_mt" : mm ? "moe_gu_q4k_mm" : "moe_gu_q4k_m",
                              {xq->ptr, xs->ptr, (char *)gate->raw->ptr + gate->off, (char *)up->raw->ptr + up->off, act->ptr,
                               offsets, list},
-                             {d, n_ff, ksel, NA}, g, mt_gu ? b1024 : b256)))
+                             {d, n_ff, ksel, NA}, g, mt_gu ? b_mt : b256)))
             return rc;
     }
     // 4. quantize every assignment's activation (the CPU path quantizes `act` inside matvec_kq)
@@ -304,11 +304,11 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
             return rc;
     } else {
         const bool dots = down5 || !mm;
-        uint32_t g[3] = {mt_down ? ojh_moe_mt_groups(dev, d, E, 16) : dots && n_ff <= 1024 ? (d + 31) / 32 : (d + 15) / 16, E, 1};
+        uint32_t g[3] = {mt_down ? ojh_moe_mt_groups(dev, n_ff, d, E, false, &b_mt[0]) : dots && n_ff <= 1024 ? (d + 31) / 32 : (d + 15) / 16, E, 1};
         // (Q5_K rows have no matrix-core form: they stay on integer dots at every batch size)
         if ((rc = ojh_launch(dev, down5 ? down_m.c_str() : mt_down ? "moe_down_q4k_mt" : mm ? "moe_down_q4k_mm" : "moe_down_q4k_m",
                              {aq->ptr, as_->ptr, (char *)down->raw->ptr + down->off, dv->ptr, offsets, list},
-                             {n_ff, d, NA}, g, mt_down ? b1024 : b256)))
+                             {n_ff, d, NA}, g, mt_down ? b_mt : b256)))
             return rc;
     }
     // 6. router-weighted sum over slots, in slot order

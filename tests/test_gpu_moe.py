@@ -794,3 +794,25 @@ def test_expert_ffn_rejects_what_it_cannot_run(gpu, pkg):
         gpu.moe_ffn(x, 1, d, nff, E + 1, 2, idx, wgt, lg_, lu_, ld_, y)
     with pytest.raises(pkg.OjasHipError, match="needs"):
         gpu.moe_ffn(x, 2, d, nff, E, 2, idx, wgt, lg_, lu_, ld_, y)
+
+
+@pytest.mark.parametrize("name,k,n,experts,grid,threads", [
+    ("moe_gu_q4k_mt", 2048, 768, 128, 2, 1024), ("moe_down_q4k_mt", 768, 2048, 128, 2, 1024), ("moe_down_q4k_mt", 2816, 512, 8, 4, 512),
+    ("moe_gu_q4k_mt", 512, 256, 8, 4, 512), ("moe_down_q4k_mt", 768, 1024, 32, 8, 512), ("moe_down_q4k_mt", 256, 2816, 96, 2, 1024)])
+def test_grouped_wave_tiles_are_cut_for_the_chip(gpu, name, k, n, experts, grid, threads):
+    """Few experts of few rows: eight waves in twice the workgroups instead of CUs without any; 96 experts of 176 tiles of one
+    super-block: no more workgroups than save a round, since each stages the expert's tokens."""
+    assert gpu.launch_shape(name, k, n, experts) == ([grid, experts, 1], [threads, 1, 1])
+
+
+@pytest.mark.parametrize("T,E,ksel,d,nff", [(48, 8, 4, 512, 2816), (100, 96, 4, 768, 256)])
+def test_expert_ffn_in_both_forms_of_the_wave_tiles(gpu, orc, pkg, T, E, ksel, d, nff):
+    """A layer whose grouped launches take eight waves, and one of sixteen, against the CPU path."""
+    gate, up, down = _experts(pkg, E, d, nff, "forms")
+    x = pkg.synth.normal_f32(T * d, "moe", "x", T, d).reshape(T, d)
+    gi, gw, idx_d, wgt_d = _route(gpu, pkg.synth.normal_f32(T * E, "moe", "lg", T, E).reshape(T, E), ksel)
+    yd = gpu.alloc(T * d)
+    gpu.moe_ffn(gpu.upload(x), T, d, nff, E, ksel, idx_d, wgt_d, gpu.lin(Q4_K, E * nff, d, gate), gpu.lin(Q4_K, E * nff, d, up),
+                gpu.lin(Q4_K, E * d, nff, down), yd, act_mode=pkg.ACT_Q8K)
+    want = orc.moe_ffn(x, gi, gw, gate, up, Q4_K, down, Q4_K, E, nff, mode=0)
+    assert peak_err(gpu.read(yd, T * d).reshape(T, d), want) <= TOL_SEEN
