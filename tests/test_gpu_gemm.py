@@ -330,9 +330,10 @@ def test_formats_without_a_tile_are_decoded_into_scratch_for_a_batch(gpu, orc, p
 
 @pytest.mark.parametrize("ty,m", [(Q6_K, 1024), (Q8_0, 2048)])
 def test_long_batches_decode_the_rows_ahead_of_the_tile(gpu, orc, pkg, ty, m):
-    """Q6_K rows from 1024 tokens (Q5_K / Q8_0 from 2048) of a matrix of 32 Mi weights: `ojh_mm` decodes them into
-    scratch and runs the plain-f16 tile — the same weights (dequant_to_f16's bits) as the tile that dequantizes on the
-    way into LDS, so the two agree to the last bits of an f32 sum; sampled rows against the oracle at the tile's bound."""
+    """`OJAS_HIP_DEQ_BIG_M=1024`: Q6_K rows from 1024 tokens (Q5_K / Q8_0 from 2048) of a matrix of 32 Mi weights are decoded
+    into scratch ahead of the tile that copies both operands — the same weights (dequant_to_f16's bits) as the tile that
+    dequantizes on the way into LDS, so the two agree to the last bits of an f32 sum; sampled rows against the oracle at the
+    tile's bound."""
     n, k = 8192, 4096
     gen = {Q6_K: pkg.synth.q6k_weights, Q8_0: pkg.synth.q80_weights}[ty]
     w = gen(n, k, "big", ty)
@@ -493,7 +494,10 @@ def test_decoder_with_activations_converted_beside_it(gpu, orc, pkg, ty, tag, bf
     gpu.dispatch(gpu.begin(), "dequant_%s_f16_x" % tag, [(gpu.upload_bytes(raw), 0), (out, 0), (gpu.upload_bytes(xb.view(np.uint8)), 0), (xh, 0), (z, 0)],
                  [nb, ne, nz, 3, bf16], grid, block)
     assert np.array_equal(gpu.read(out, n * k, np.uint16), orc.dequant_to_f16(raw, ty, n * k))
-    assert np.array_equal(gpu.read(xh, ne, np.uint16), x.astype(np.float16).view(np.uint16))
+    halves = gpu.read(xh, 2 * (ne // 2 + 9), np.uint16)
+    assert np.array_equal(halves[:ne], x.astype(np.float16).view(np.uint16))
+    before = np.full(ne // 2 + 9, 7.5, np.float32).view(np.uint16)
+    assert np.array_equal(halves[ne:], before[ne:])
     got = gpu.read(z, nz + 8)
     assert np.all(got[:nz] == 0) and np.all(got[nz:] == 7.5)
     assert np.all(gpu.read(out, n * k // 2 + 8)[-8:] == 7.5)
@@ -552,3 +556,30 @@ def test_a_pinned_token_count_means_what_it_meant(pkg, monkeypatch, ty, n, k, m,
         assert bool(g.has_kernel("gemm_f16d_128")) == copied
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("tile", ["1", "2", "3"])
+@pytest.mark.parametrize("n,k,m,bf16,accum", [(385, 1024, 130, 0, False), (1100, 320, 257, 1, False), (385, 1024, 300, 1, True), (129, 64, 513, 0, True)])
+def test_copied_tile_sizes_through_mm(gpu, pkg, monkeypatch, tile, n, k, m, bf16, accum):
+    """`OJAS_HIP_F16D_TILE`: each size of the copied tile behind the decode pass, as `ojh_mm` launches it, against the tile that
+    decodes on the way into LDS: the same weights and activations, K f32 additions in another order each (2 K 2^-24 of the
+    peak, the magnitudes summing to some 0.15 sqrt(K) peaks); nothing written past the last token."""
+    raw = pkg.synth.weights(20, n, k, "tiles", n, k)
+    x = pkg.synth.normal_f32(m * k, "tiles", "x", m)
+    xb = pkg.synth.to_bf16_bits(x) if bf16 else x
+    y0 = pkg.synth.normal_f32(m * n, "tiles", "y0") if accum else np.full(m * n, 777.25, np.float32)
+    outs = []
+    for big in ("2", "0"):
+        monkeypatch.setenv("OJAS_HIP_DEQ_BIG_M", big)
+        monkeypatch.setenv("OJAS_HIP_F16D_TILE", tile)
+        g = pkg.HipGpu(0)
+        try:
+            yd = g.upload(np.concatenate([y0, np.full(64, 777.25, np.float32)]))
+            g.mm(g.upload_bytes(xb.view(np.uint8)), g.lin(20, n, k, raw), yd, m, accum, x_dtype=bf16, act_mode=pkg.ACT_FLOAT)
+            got = g.read(yd, m * n + 64)
+            assert g.has_kernel("gemm_f16d_128") == (big == "2")
+            assert np.all(got[m * n:] == np.float32(777.25))
+            outs.append(got[:m * n])
+        finally:
+            g.close()
+    assert peak_err(outs[0], outs[1]) <= 2 * k * 2.0 ** -24
