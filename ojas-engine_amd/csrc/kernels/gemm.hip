@@ -851,7 +851,8 @@ GEMM_ENTRIES(q3k, LoaderQ3K)
 // either operand holds 8 consecutive positions of K group g.  The order of K inside an instruction is free as long as both
 // operands agree, so lane (n, g) decodes the whole 32-weight block g of the chunk for row n (the per-thread loaders of the
 // tile: one or two wide loads) and feeds it to four instructions, 8 weights each; lane (m, g) reads the matching 64 bytes
-// of token m.  Up to 16 TG tokens per launch (TG accumulators); partial sums of the waves meet in LDS in wave order.
+// of token m.  Up to 16 TG tokens per launch (TG accumulators); partial sums of the waves meet in LDS in wave order (eight
+// waves on four slots: wave w adds wave w + 4's to its own first).
 //   gemm_few_<fmt>{,_r4}_t{1,2,4}(xh, w, y, K, N, accum, M)     grid [ceil(N / 16 RG),1,1] x 256 (or 512 where RG TG <= 8),
 //   K a multiple of 128, M <= 16 TG; `_r4`: RG = 4 groups of 16 rows per workgroup
 // Bound by latency: a wave waits a trip to memory per chunk for its tokens and the next block, and with 64 rows a workgroup

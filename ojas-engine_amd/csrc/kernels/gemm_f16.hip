@@ -21,13 +21,6 @@
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ void gf_copy16(const void* base, uint voff, uint lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(base), "s"(lds_addr)
-                 : "memory");
-}
-
 template <int MI, int NJ, int D, bool SPLITK, bool ACCUM>
 __device__ __forceinline__ void gemm_f16_body(const ushort* __restrict__ xh, const ushort* __restrict__ w, float* __restrict__ y,
                                               uint K, uint N, uint M, uint nsplit, uchar* lds) {
@@ -63,7 +56,7 @@ __device__ __forceinline__ void gemm_f16_body(const ushort* __restrict__ xh, con
     const uchar* const wb = (const uchar*)w + (size_t)s_begin * RB;
     // requests past the last step are clamped onto it: every step issues the same NC copies
 #define GF_COPY(I, T, SLOT)                                                                                   \
-    gf_copy16(((I) < XL ? xb : wb) + (size_t)min((T), last) * RB, off[I],                                   \
+    lds_dma16_s(((I) < XL ? xb : wb) + (size_t)min((T), last) * RB, off[I],                                   \
               ((I) < XL ? xdst + (I) * 1024u : wdst + ((I) - XL) * 1024u) + (SLOT) * STAGE)
 
     const uint wy = wave >> 1, wx = wave & 1u, fr = lane & 31u, kg = lane >> 5, sw = (fr >> 1) & 7u;

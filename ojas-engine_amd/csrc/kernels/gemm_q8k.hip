@@ -590,10 +590,6 @@ quantize_q8k_bf16_sides(const ushort* x, signed char* q, float* scales, float* x
     quantize_q8k_sides_body<true>(x, q, scales, xst, sums, K, M, MP);
 }
 
-__device__ __forceinline__ void gxt_copy16(const void* base, uint voff, uint lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds_addr) : "memory");
-}
-
 // one 16-row tile's super-block: its two planes, and the row's side of the min term for the f32 matrix unit:
 // n0 = -dmin * m[kg], n1 = -dmin * m[kg + 4] (sh = 8 kg)
 __device__ __forceinline__ void gxt_planes(const GqW& w, gq_i4 (&BA)[4], gq_i4 (&BB)[4], float& n0, float& n1, float& d, uint sh) {
@@ -643,12 +639,12 @@ __device__ __forceinline__ void gemm_q8k_q4k_xt_body(const signed char* __restri
         for (int i = 0; i < 4; i++) {
             const uint tk = wave * 16u + (uint)i * 4u + (lo >> 4);
             const uint tg = min(t0 + tk, M - 1u);                  // tokens past M: any row (their sides are zeros)
-            gxt_copy16(xb, tg * K + (((lo & 15u) ^ (tk & 15u)) << 4), x_lds + stage * GXT_STAGE + (uint)i * 1024u);
+            lds_dma16_s(xb, tg * K + (((lo & 15u) ^ (tk & 15u)) << 4), x_lds + stage * GXT_STAGE + (uint)i * 1024u);
         }
-        if (wave < 4u) gxt_copy16((const uchar*)sums + ((size_t)sb * MP + t0) * 32u + wave * 1024u, lane16,
+        if (wave < 4u) lds_dma16_s((const uchar*)sums + ((size_t)sb * MP + t0) * 32u + wave * 1024u, lane16,
                                   lds0 + stage * GXT_STAGE + GXT_TOK * 256u + wave * 1024u);
         else if (wave == 4u) {
-            if (lane < 32u) gxt_copy16(xst + (size_t)sb * MP + t0, lane16, lds0 + stage * GXT_STAGE + GXT_TOK * 288u);
+            if (lane < 32u) lds_dma16_s(xst + (size_t)sb * MP + t0, lane16, lds0 + stage * GXT_STAGE + GXT_TOK * 288u);
         }
     };
     // this lane's row (clamped past N; a 32-bit byte offset from a uniform base: the tensor stays below 4 GiB)

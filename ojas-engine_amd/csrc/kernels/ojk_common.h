@@ -245,11 +245,12 @@ __device__ __forceinline__ uint iq4_levels4(uint idx4) {
 // One instruction moves 16 bytes per lane from base + voff to LDS bytes lds_addr + 16 lane .. (1 KB
 // per wave, contiguous in LDS whatever the global addresses; lds_addr is the same in every lane).
 // Completion is counted by vmcnt.
+// `lds_dma16_s`: lds_addr in a scalar register already.
+__device__ __forceinline__ void lds_dma16_s(const void* base, uint voff, uint lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds_addr) : "memory");
+}
 __device__ __forceinline__ void lds_dma16(const void* base, uint voff, uint lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane((int)lds_addr))
-                 : "memory");
+    lds_dma16_s(base, voff, (uint)__builtin_amdgcn_readfirstlane((int)lds_addr));
 }
 // wait until at most `n` vector memory operations are outstanding (a count not listed waits for all)
 __device__ __forceinline__ void vm_wait(uint n) {

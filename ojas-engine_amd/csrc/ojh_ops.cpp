@@ -755,9 +755,9 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
     // tokens; on 4096 x 4096 28 against 13 / 22 / 31 / 39 at 4 / 8 / 12 / 16)
     const uint32_t deq_min = dev->deq_min_m != 1 ? dev->deq_min_m : (uint64_t)N * K >= (32ull << 20) ? 5u : 9u;
     // IQ4_NL / IQ4_XS rows have loaders in the tile: short of the long batches they skip the decode pass (14336 x 4096:
-    // 53 - 62 -> 32 - 42 us up to 128 tokens, 114 -> 93 at 512; 4096 x 4096 at 16 tokens 29 -> 14; from 1024 tokens
-    // the pass pays for itself as it does for Q6_K) and take the tile from 5 tokens on every shape (the matvec that
-    // walks the rows once per four tokens: 13 / 22 us at 4 / 8 tokens on 4096 x 4096)
+    // 53 - 62 -> 32 - 42 us up to 128 tokens; 4096 x 4096 at 16 tokens 29 -> 14; beyond, f16d_pays weighs the pass again) and
+    // take the tile from 5 tokens on every shape (the matvec that walks the rows once per four tokens: 13 / 22 us at 4 / 8
+    // tokens on 4096 x 4096)
     // (the legacy 32-weight blocks, MXFP4, Q2_K and Q3_K likewise)
     const bool own_loader = w->type == OJH_IQ4_NL || (w->type == OJH_IQ4_XS && K % 256 == 0) || w->type == OJH_Q4_0 ||
                             w->type == OJH_Q4_1 || w->type == OJH_Q5_0 || w->type == OJH_Q5_1 || w->type == OJH_MXFP4 ||
