@@ -550,14 +550,16 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 // CUs more than of rows or tokens, so both are priced, in us: K steps on the busiest CU times what a step takes (a part
 // that does not depend on how many CUs are busy, and one that grows with them), the atomics that K slices meet in, the
 // pass.  The prices are least squares over 20000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048
-// tokens); what they choose is on average within 0.5 % of the faster route (by tokens and rows alone: 1.7 %).  Both routes measured, decoding tile / pass + copying tile:
+// tokens); what they choose is on average within 0.5 % of the faster route (by tokens and rows alone: 1.7 %), and 4 % or
+// more behind the decoding tile in 1 of 125 calls.  Both routes measured, decoding tile / pass + copying tile:
 //   Q6_K   6914 x 2816 at 333 tokens 60 / 37, 14336 x 4096 at 130 79 / 71, 4096 x 4096 at 700 83 / 45
 //   IQ4_NL 5330 x 11776 at 333 95 / 85, 8192 x 14336 at 333 162 / 215 (decoded rows beyond 112 MB: read back from memory)
 //   Q5_0   8576 x 4096 at 257 106 / 51, MXFP4 8192 x 14336 at 512 188 / 249, Q4_1 8192 x 1024 at 512 26 / 32
 static uint32_t f16d_tile(const ojh_device *dev, uint32_t N, uint32_t m) {   // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256 tokens x rows
-    // rounds of workgroups over the chip times a tile's time per K step with every CU busy (0.49 / 0.83 / 1.37 us): within
-    // 0.13 % of the fastest of the three on average; 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262;
-    // 4096 x 14336 at 2048 334 / 279 / 388; 6914 x 2816 at 333 35 / 51 / 76
+    // rounds of workgroups over the chip times a K step of the tile (fitted over 6650 timed calls, launch, decode pass and
+    // stores apart: 0.49 / 0.83 / 1.37 us with every CU busy): within 0.13 % of the fastest of the three on average; 14336 x
+    // 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 / 279 / 388; 6914 x 2816 at
+    // 333 35 / 51 / 76
     const uint64_t cus = (uint64_t)dev->prop.multiProcessorCount;
     auto rounds = [&](uint32_t bm, uint32_t bn) { return ((uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm) + cus - 1) / cus; };
     if (dev->f16d_tile > 0) return (uint32_t)dev->f16d_tile - 1u;
