@@ -549,9 +549,9 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 // 128 or 256 tokens; the pass reads and writes everything once.  Which is ahead is a matter of rounds of workgroups over the
 // CUs more than of rows or tokens, so both are priced, in us: K steps on the busiest CU times what a step takes (a part
 // that does not depend on how many CUs are busy, and one that grows with them), the atomics that K slices meet in, the
-// pass.  The prices are least squares over 20000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048
-// tokens); what they choose is on average within 0.5 % of the faster route (by tokens and rows alone: 1.7 %), and 4 % or
-// more behind the decoding tile in 1 of 125 calls.  Both routes measured, decoding tile / pass + copying tile:
+// pass.  The prices are fitted to 39000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048 tokens): what
+// they choose is on average within 0.4 % of the faster route, and 4 % or more behind the decoding tile in one call of 50
+// (by tokens and rows alone 1.7 %, and one of 40).  Both routes measured, decoding tile / pass + copying tile:
 //   Q6_K   6914 x 2816 at 333 tokens 60 / 37, 14336 x 4096 at 130 79 / 71, 4096 x 4096 at 700 83 / 45
 //   IQ4_NL 5330 x 11776 at 333 95 / 85, 8192 x 14336 at 333 162 / 215 (decoded rows beyond 112 MB: read back from memory)
 //   Q5_0   8576 x 4096 at 257 106 / 51, MXFP4 8192 x 14336 at 512 188 / 249, Q4_1 8192 x 1024 at 512 26 / 32
@@ -578,23 +578,23 @@ static bool f16d_pays(const ojh_device *dev, const ojh_lin *w, uint32_t m, bool 
         const uint64_t tiles = (uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm);
         const uint32_t z = dev->gemm_sr ? 1u : ojh_gemm_slices(dev, tiles, most);
         const double per_cu = tiles * z / cus;
-        return (K / 64 + z - 1) / z * (round * ceil(per_cu) + fill * per_cu) + (z > 1 ? 3.1 * z * m * N / (1 << 20) : 0.0);
+        return (K / 64 + z - 1) / z * (round * ceil(per_cu) + fill * per_cu) + (z > 1 ? 2.2 * z * m * N / (1 << 20) : 0.0);
     };
     const uint32_t tile = f16d_tile(dev, N, m);
-    const double copied = tile == 2 ? 3.0 + walk(256, 256, 1, 1.14, 0.23) : tile == 1 ? 1.5 + walk(256, 128, 1, 0.66, 0.17)
-                                                                                   : walk(128, 128, K / 512, 0.30, 0.19);
+    const double copied = tile == 2 ? 2.75 + walk(256, 256, 1, 1.14, 0.15) : tile == 1 ? 4.0 + walk(256, 128, 1, 0.64, 0.15)
+                                                                                   : 0.75 + walk(128, 128, K / 512, 0.28, 0.19);
     // (a format that is decoded first in any case: the same pass, conversion included only where its decoder does that)
-    if (decoded) return copied < (ojh_grid_type(w->type) ? 0.0 : 0.5) + walk(128, 128, K / 256, 0.40, 0.20);
+    if (decoded) return copied < (ojh_grid_type(w->type) ? 0.75 : 2.75) + walk(128, 128, K / 256, 0.40, 0.20);
     // a K step of 128 x 128 and of 256 x 128 on the loader
-    double s128 = 0.79, s256 = 1.14;
+    double s128 = 0.76, s256 = 1.16;
     switch (w->type) {
-    case OJH_IQ4_NL: case OJH_Q4_0: case OJH_Q8_0: s128 = 0.71; s256 = 1.06; break;
-    case OJH_Q4_1: s128 = 0.90; s256 = 1.20; break;
-    case OJH_Q5_0: case OJH_Q6_K: s128 = 1.14; s256 = 1.46; break;
+    case OJH_IQ4_NL: case OJH_Q4_0: case OJH_Q8_0: s128 = 0.74; s256 = 1.10; break;
+    case OJH_Q4_1: s128 = 0.82; s256 = 1.27; break;
+    case OJH_Q5_0: case OJH_Q6_K: s128 = 1.00; s256 = 1.47; break;
     default: break;
     }
-    const double loaded = gemm_mm_m128(dev, N, m, false) ? walk(128, 128, K / 256, s128, 0.0) : 2.0 + walk(256, 128, K / 256, s256, 0.0);
-    return 1.5 + 0.42 * mi + (mi > 56 ? 0.45 * (mi - 56) : 0.0) + copied < loaded;
+    const double loaded = gemm_mm_m128(dev, N, m, false) ? walk(128, 128, K / 256, s128, 0.0) : 3.5 + walk(256, 128, K / 256, s256, 0.0);
+    return 0.42 * mi + (mi > 56 ? 0.5 * (mi - 56) : 0.0) + copied < loaded;
 }
 static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
     const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
