@@ -550,7 +550,7 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 // CUs more than of rows or tokens, so both are priced, in us: K steps on the busiest CU times what a step takes (a part
 // that does not depend on how many CUs are busy, and one that grows with them), the atomics that K slices meet in, the
 // pass.  The prices are fitted to 39000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048 tokens): what
-// they choose is on average within 0.4 % of the faster route, and 4 % or more behind the decoding tile in one call of 50
+// they choose is on average within 0.8 % of the faster route, and 4 % or more behind the decoding tile in one call of 90
 // (by tokens and rows alone 1.7 %, and one of 40).  Both routes measured, decoding tile / pass + copying tile:
 //   Q6_K   6914 x 2816 at 333 tokens 60 / 37, 14336 x 4096 at 130 79 / 71, 4096 x 4096 at 700 83 / 45
 //   IQ4_NL 5330 x 11776 at 333 95 / 85, 8192 x 14336 at 333 162 / 215 (decoded rows beyond 112 MB: read back from memory)
@@ -581,7 +581,7 @@ static bool f16d_pays(const ojh_device *dev, const ojh_lin *w, uint32_t m, bool 
         return (K / 64 + z - 1) / z * (round * ceil(per_cu) + fill * per_cu) + (z > 1 ? 2.2 * z * m * N / (1 << 20) : 0.0);
     };
     const uint32_t tile = f16d_tile(dev, N, m);
-    const double copied = tile == 2 ? 2.75 + walk(256, 256, 1, 1.14, 0.15) : tile == 1 ? 4.0 + walk(256, 128, 1, 0.64, 0.15)
+    const double copied = tile == 2 ? 2.75 + walk(256, 256, 1, 1.14, 0.15) : tile == 1 ? 4.0 + walk(256, 128, 1, 0.66, 0.15)
                                                                                    : 0.75 + walk(128, 128, K / 512, 0.28, 0.19);
     // (a format that is decoded first in any case: the same pass, conversion included only where its decoder does that)
     if (decoded) return copied < (ojh_grid_type(w->type) ? 0.75 : 2.75) + walk(128, 128, K / 256, 0.40, 0.20);
@@ -611,7 +611,9 @@ static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int 
         if (w->type == OJH_Q4_K || (kq && (uint64_t)w->n * w->k < (32ull << 20))) return false;
         return m >= (w->type == OJH_Q5_K || w->type == OJH_Q8_0 ? 2 * dev->deq_big_m : dev->deq_big_m);
     }
-    return m >= 129u && f16d_pays(dev, w, m, decoded);
+    // (129 to 256 tokens are two tiles of 128, the second part empty: the two routes are within the prices' error of each
+    // other there for the lighter loaders, whose rows then need no scratch)
+    return m >= (decoded || w->type == OJH_Q6_K ? 129u : 257u) && f16d_pays(dev, w, m, decoded);
 }
 // Whether all the route needs is there.  What every form of the call needs comes first, so that the decoded rows' scratch,
 // which a format with a loader can do without, never takes its room: the activations' scratch, and the family of the tiles
