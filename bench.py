@@ -418,7 +418,7 @@ def extras(gpu, pkg, lin_q) -> dict:
                 del xb, y
             lin.free()
         out[f"prefill_gemm_{tag}"] = {"activations": "bf16 N(0,1), converted to f16 into the tile", "accumulate": "f32",
-                                      "peak_tflops": 2500.0, "timed": "conversion + zero fill (split-K) + tile", **fam}
+                                      "peak_tflops": 2500.0, "timed": "conversion + zero fill (split-K) + tile; from 129 (Q6_K) or 257 tokens also the decode pass, where `ojh_mm` takes it", **fam}
     # ---- the same two matrices in the CPU path's arithmetic (quant_q8k activations, int8 MFMA), f32 in
     i8 = {}
     for name, lin in zip(("gate_up_14336x4096", "down_4096x14336"), lin_q):
@@ -528,7 +528,7 @@ def extras(gpu, pkg, lin_q) -> dict:
         del wf
     out["float_rows_gemv_128256x4096"] = {"activations": "f32", "kernels": "gemv_nat_<fmt>_px", **fr}
     # ---- the same formats against a batch (f32 in, OJH_ACT_AUTO): the f16 tile through the formats' own loaders, or the
-    # decode pass into f16 scratch + the plain-f16 tile for those without one
+    # decode pass into f16 scratch + a tile over plain f16 rows for those without one and for long batches
     fb = {}
     nb, kb = 14336, 4096
     for ty, tag in ((pkg.IQ4_XS, "iq4xs"), (pkg.Q4_0, "q40"), (pkg.Q5_1, "q51"), (pkg.MXFP4, "mxfp4"), (pkg.Q3_K, "q3k"),
@@ -539,7 +539,7 @@ def extras(gpu, pkg, lin_q) -> dict:
             us = _time(gpu, lambda i: gpu.mm(xb, wf[i % 2], yb, m), 10, 2)
             fb[f"{tag}_M{m}"] = {"us": round(us, 1), "mfma_frac": round(2.0 * m * nb * kb / us / 1e6 / 2500.0, 4)}
         del wf
-    out["float_rows_batch_14336x4096"] = {"activations": "f32 -> f16", "kernels": "gemm_mm_<fmt>{,_m128}{,_sk} (IQ4_NL / IQ4_XS, Q4_0 .. Q5_1, MXFP4, Q2_K; Q3_K up to 128 tokens) or dequant_<fmt>_f16 + gemm_mm_f16_m128{,_sk} (Q3_K beyond, the grid codebooks)", **fb}
+    out["float_rows_batch_14336x4096"] = {"activations": "f32 -> f16", "kernels": "gemm_few_<fmt>_r4_t1 at 16 tokens, gemm_mm_<fmt>_m128{,_sk} at 128, dequant_<fmt>_f16_x + gemm_f16d_* or gemm_mm_<fmt> at 512; the grid codebooks dequant_<fmt>_f16 + gemm_mm_f16_m128{,_sk} / gemm_f16d_*", **fb}
     # IQ2_XXS as the CPU path multiplies it: int8 activations per 256, integer dots (dot_iq2xxs_q8k)
     wf = [gpu.lin(pkg.IQ2_XXS, n, k, synth.weights(pkg.IQ2_XXS, n, k, "bench", "iq2xxs", "head")) for _ in range(2)]
     us = _time(gpu, lambda i: gpu.mm(x, wf[i % 2], y), 20, 3)
