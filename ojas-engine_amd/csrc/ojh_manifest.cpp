@@ -1363,17 +1363,18 @@ static int shape_gemm(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t 
     return OJH_OK;
 }
 
-// gemm_f16d_{128,256x128,256}(xh, w, y, K, N, accum, M), gemm_f16d_128_sk(xh, w, y, K, N, M, nsplit): plain f16 rows, both
+// gemm_f16d_{128,256x128,256,128_kw,256x128_kw}(xh, w, y, K, N, accum, M), gemm_f16d_128_sk(xh, w, y, K, N, M, nsplit): plain f16 rows, both
 // operands copied into LDS by the memory system; grid [8 ceil(row tiles / 8) x token tiles, 1 | nsplit, 1].
-// `rows_per_wave`: 16 x (tokens / 128) + rows / 128, + 1024 for the split form
+// `rows_per_wave`: 16 x (tokens / 128) + rows / 128, + 1024 for the split form, + 2048 on eight waves
 static int check_gemm_f16d(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3],
                            const uint32_t block[3], size_t need[16], size_t align[16]) {
     const bool sk = s->rows_per_wave & 1024;
+    const uint32_t threads = s->rows_per_wave & 2048 ? 512 : 256;
     const uint32_t bm = 128u * ((uint32_t)s->rows_per_wave >> 4 & 15u), bn = 128u * ((uint32_t)s->rows_per_wave & 15u);
     const uint32_t K = c[0], N = c[1], M = sk ? c[2] : c[3], nsplit = sk ? c[3] : 1;
     if (!K || !N || K % 64) return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u (K a positive multiple of 64)", s->name, K, N);
     if (!M || !nsplit) return ojh_fail(OJH_ERR_ARG, "%s: M and nsplit must be positive", s->name);
-    int rc = check_block(block, 256);
+    int rc = check_block(block, threads);
     if (rc) return rc;
     const uint64_t nt = ((uint64_t)N + bn - 1) / bn, mt = ((uint64_t)M + bm - 1) / bm, want = (nt + 7) / 8 * 8 * mt;
     if (grid[0] != want || grid[1] != nsplit || grid[2] != 1)
@@ -1395,7 +1396,7 @@ static int shape_gemm_f16d(const ojh_kernel_spec *s, const ojh_device *dev, uint
     grid[0] = (nt + 7) / 8 * 8 * mt;
     grid[1] = grid[2] = 1;
     if (s->rows_per_wave & 1024) grid[1] = ojh_gemm_slices(dev, (uint64_t)nt * mt, K / 512);   // (eight K steps each at least)
-    block[0] = 256;
+    block[0] = s->rows_per_wave & 2048 ? 512 : 256;
     block[1] = block[2] = 1;
     return OJH_OK;
 }
@@ -2162,6 +2163,8 @@ static std::vector<ojh_kernel_spec> build_manifest() {
     add("gemm_mm_f16_m128_sk", "gemm", 3, 4, OJH_F16, 15, check_gemm, shape_gemm);
     add("gemm_f16d_128", "gemm_f16", 3, 4, OJH_F16, 16 + 1, check_gemm_f16d, shape_gemm_f16d);
     add("gemm_f16d_256x128", "gemm_f16", 3, 4, OJH_F16, 32 + 1, check_gemm_f16d, shape_gemm_f16d);
+    add("gemm_f16d_128_kw", "gemm_f16", 3, 4, OJH_F16, 2048 + 16 + 1, check_gemm_f16d, shape_gemm_f16d);
+    add("gemm_f16d_256x128_kw", "gemm_f16", 3, 4, OJH_F16, 2048 + 32 + 1, check_gemm_f16d, shape_gemm_f16d);
     add("gemm_f16d_256", "gemm_f16", 3, 4, OJH_F16, 32 + 2, check_gemm_f16d, shape_gemm_f16d);
     add("gemm_f16d_128_sk", "gemm_f16", 3, 4, OJH_F16, 1024 + 16 + 1, check_gemm_f16d, shape_gemm_f16d);
     // Q4L (relaid Q4_K + side arrays) under the reference's names and argument lists

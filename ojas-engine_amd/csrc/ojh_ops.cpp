@@ -557,9 +557,9 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 //   Q5_0   8576 x 4096 at 257 106 / 51, MXFP4 8192 x 14336 at 512 188 / 249, Q4_1 8192 x 1024 at 512 26 / 32
 static uint32_t f16d_tile(const ojh_device *dev, uint32_t N, uint32_t m) {   // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256 tokens x rows
     // rounds of workgroups over the chip times a K step of the tile (fitted over 6650 timed calls, launch, decode pass and
-    // stores apart: 0.49 / 0.83 / 1.37 us with every CU busy): within 0.13 % of the fastest of the three on average; 14336 x
-    // 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 / 279 / 388; 6914 x 2816 at
-    // 333 35 / 51 / 76
+    // stores apart: 0.49 / 0.83 / 1.37 us with every CU busy on four waves): within 0.13 % of the fastest of the three on
+    // average; 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 / 279 / 388;
+    // 6914 x 2816 at 333 35 / 51 / 76.  On eight waves the first two take 6 - 8 % less (0.46 / 0.77)
     const uint64_t cus = (uint64_t)dev->prop.multiProcessorCount;
     auto rounds = [&](uint32_t bm, uint32_t bn) { return ((uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm) + cus - 1) / cus; };
     if (dev->f16d_tile > 0) return (uint32_t)dev->f16d_tile - 1u;
@@ -636,7 +636,11 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     ojh_buf *xh, *wdeq;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
     if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;
-    const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? "gemm_f16d_256x128" : "gemm_f16d_128";
+    // (eight waves pay for their sums' meeting from some 44 K steps on: 128 x 128 tiles, all CUs busy, with the decode pass, four
+    // / eight: 2048 x 1024 at 2048 tokens 25 / 28 us, x 2048 31.5 / 35, x 2560 36.7 / 38.6, x 3072 at 1900 40.9 / 40.0; 6914 x
+    // 2816 at 333 34.3 / 33.2; 4096 x 4096 at 1024 52.5 / 50.2.  256 x 128: 4096 x 2048 at 2048 48.9 / 48.3, 10000 x 1536 at
+    // 700 41.7 / 40.2, 4096 x 1024 at 2048 level)
+    const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? "gemm_f16d_256x128_kw" : K >= 2816 ? "gemm_f16d_128_kw" : "gemm_f16d_128";
     uint32_t sg[3], sb[3];
     bool sk = false;
     if (!tile) {

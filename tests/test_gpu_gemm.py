@@ -475,6 +475,26 @@ def test_copied_f16_tile_by_name(gpu, pkg, kernel, bm, bn, m, k, n, accum):
         gpu.dispatch(gpu.begin(), kernel, [(xd, 0), (wd, 0), (yd, 0)], [k, n, m, 1] if sk else [k, n, 0, m], [tiles + 8, 1, 1], [256, 1, 1])
 
 
+@pytest.mark.parametrize("kernel,bm", [("gemm_f16d_128_kw", 128), ("gemm_f16d_256x128_kw", 256)])
+@pytest.mark.parametrize("m,k,n,accum", [(1, 64, 1, False), (129, 128, 127, True), (257, 192, 1100, False), (300, 1088, 385, True)])
+def test_copied_f16_tile_on_eight_waves(gpu, pkg, kernel, bm, m, k, n, accum):
+    """The halves of a step's K on two groups of waves that meet in LDS: fewer steps than the ring is deep, one row and token
+    past a tile, both halves of the rows a group stores; bound as for four waves."""
+    gpu.ensure_family("gemm_f16")
+    x = pkg.synth.normal_f32(m * k, "f16d", "x", m, k).astype(np.float16)
+    w = pkg.synth.normal_f32(n * k, "f16d", "w", n, k).astype(np.float16)
+    want = x.astype(np.float64).reshape(m, k) @ w.astype(np.float64).reshape(n, k).T
+    y0 = pkg.synth.normal_f32(m * n, "f16d", "y0").reshape(m, n) if accum else np.zeros((m, n), np.float32)
+    yd = gpu.upload(np.concatenate([y0.ravel(), np.full(256, 777.25, np.float32)]))
+    grid, block = gpu.launch_shape(kernel, k, n, m)
+    assert grid[0] == (((n + 127) // 128 + 7) // 8 * 8) * ((m + bm - 1) // bm) and block[0] == 512
+    gpu.dispatch(gpu.begin(), kernel, [(gpu.upload_bytes(x.view(np.uint8)), 0), (gpu.upload_bytes(w.view(np.uint8)), 0), (yd, 0)],
+                 [k, n, int(accum), m], grid, block)
+    got = gpu.read(yd, m * n + 256)
+    assert np.all(got[m * n:] == np.float32(777.25))
+    assert peak_err(got[:m * n].reshape(m, n), want + y0) <= 1e-5
+
+
 @pytest.mark.parametrize("ty,tag", [(8, "q80"), (14, "q6k"), (2, "q40"), (11, "q3k")])
 @pytest.mark.parametrize("bf16", [0, 1])
 def test_decoder_with_activations_converted_beside_it(gpu, orc, pkg, ty, tag, bf16):
