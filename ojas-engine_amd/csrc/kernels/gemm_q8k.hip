@@ -501,12 +501,17 @@ gemm_q8k_q4k_mk(const signed char* xq, const float* xs, const uchar* w, float* y
 #define GXT_ROWS 128u
 #define GXT_STAGE (GXT_TOK * 256u + GXT_TOK * 32u + GXT_TOK * 4u)     // tokens | scaled sums | scales = 37376 bytes
 
-extern "C" __global__ void __launch_bounds__(256)
-q8k_token_sides(const signed char* __restrict__ xq, const float* __restrict__ xs, float* __restrict__ xst,
-                float* __restrict__ sums, uint K, uint M, uint MP) {
+// A token's side array of a super-block, by the tile that reads it: HALF = false: the eight runs' sums of q times the scale,
+// in f32, run r at place 2 (r % 4) + r / 4; HALF = true: sixteen f16, sum / 2 rounded down of runs 0 .. 7, then the sums' last
+// bits (a sum is at most 32 * 127 = 4064: both parts are whole numbers that f16 holds).
+__device__ __forceinline__ ushort gxk_half(int v) { return __half_as_ushort(__int2half_rn(v)); }
+template <bool HALF>
+__device__ __forceinline__ void q8k_token_sides_body(const signed char* __restrict__ xq, const float* __restrict__ xs, float* __restrict__ xst,
+                                                     float* __restrict__ sums, uint K, uint M, uint MP) {
     const uint nsb = K >> 8, sb = blockIdx.x, t = blockIdx.y * 256u + threadIdx.x;
     if (t >= MP) return;
     float f[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    int run[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     float sc = 0.0f;
     if (t < M) {
         sc = xs[(size_t)t * nsb + sb];
@@ -518,13 +523,33 @@ q8k_token_sides(const signed char* __restrict__ xq, const float* __restrict__ xs
             bs = dot4_i8(a.y, 0x01010101u, bs); bs = dot4_i8(a.z, 0x01010101u, bs); bs = dot4_i8(a.w, 0x01010101u, bs);
             bs = dot4_i8(b.x, 0x01010101u, bs); bs = dot4_i8(b.y, 0x01010101u, bs);
             bs = dot4_i8(b.z, 0x01010101u, bs); bs = dot4_i8(b.w, 0x01010101u, bs);
+            run[jj] = bs;
             f[2 * (jj & 3) + (jj >> 2)] = __fmul_rn(sc, (float)bs);
         }
     }
     xst[(size_t)sb * MP + t] = sc;
-    float4* o = (float4*)(sums + ((size_t)sb * MP + t) * 8u);
-    o[0] = make_float4(f[0], f[1], f[2], f[3]);
-    o[1] = make_float4(f[4], f[5], f[6], f[7]);
+    uint4* o = (uint4*)(sums + ((size_t)sb * MP + t) * 8u);
+    if (HALF) {
+        uint h[8];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            h[q] = (uint)gxk_half(run[2 * q] >> 1) | ((uint)gxk_half(run[2 * q + 1] >> 1) << 16);
+            h[4 + q] = (uint)gxk_half(run[2 * q] & 1) | ((uint)gxk_half(run[2 * q + 1] & 1) << 16);
+        }
+        o[0] = make_uint4(h[0], h[1], h[2], h[3]);
+        o[1] = make_uint4(h[4], h[5], h[6], h[7]);
+    } else {
+        o[0] = make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3]));
+        o[1] = make_uint4(__float_as_uint(f[4]), __float_as_uint(f[5]), __float_as_uint(f[6]), __float_as_uint(f[7]));
+    }
+}
+extern "C" __global__ void __launch_bounds__(256)
+q8k_token_sides(const signed char* xq, const float* xs, float* xst, float* sums, uint K, uint M, uint MP) {
+    q8k_token_sides_body<false>(xq, xs, xst, sums, K, M, MP);
+}
+extern "C" __global__ void __launch_bounds__(256)
+q8k_token_sides_h(const signed char* xq, const float* xs, float* xst, float* sums, uint K, uint M, uint MP) {
+    q8k_token_sides_body<true>(xq, xs, xst, sums, K, M, MP);
 }
 
 // The activation quantizer and q8k_token_sides in one launch, for callers that hand over f32 or bf16 tokens:
@@ -533,7 +558,7 @@ q8k_token_sides(const signed char* __restrict__ xq, const float* __restrict__ xs
 // four values per lane: the segment is quantized exactly as quantize_q8k does (amax / 127, 1 for a zero segment, round
 // half away, clamp), and its scale and scaled 32-position sums go to the transposed side arrays as well; the segments of
 // rows M .. MP - 1 write zeros there and nothing else.  No barrier and no LDS: the maximum and the sums travel by DPP.
-template <bool BF16>
+template <bool BF16, bool HALF>
 __device__ __forceinline__ void quantize_q8k_sides_body(const void* __restrict__ xv, signed char* __restrict__ q,
                                                         float* __restrict__ scales, float* __restrict__ xst,
                                                         float* __restrict__ sums, uint K, uint M, uint MP) {
@@ -574,8 +599,13 @@ __device__ __forceinline__ void quantize_q8k_sides_body(const void* __restrict__
     s32 += dpp_i32<OJK_DPP_QUAD_XOR1>(s32);
     s32 += dpp_i32<OJK_DPP_QUAD_XOR2>(s32);
     s32 += dpp_i32<OJK_DPP_ROW_HALF_MIRROR>(s32);
-    // lane 8 j holds the sum of run j, which goes to position 2 (j % 4) + j / 4
-    if ((lane & 7u) == 0) sums[((size_t)sb * MP + m) * 8u + ((lane >> 2) & 6u) + (lane >> 5)] = __fmul_rn(scale, (float)s32);
+    // lane 8 j holds the sum of run j
+    if (HALF && (lane & 7u) == 0) {
+        ushort* const o = (ushort*)(sums + ((size_t)sb * MP + m) * 8u) + (lane >> 3);
+        o[0] = gxk_half(s32 >> 1);
+        o[8] = gxk_half(s32 & 1);
+    }
+    if (!HALF && (lane & 7u) == 0) sums[((size_t)sb * MP + m) * 8u + ((lane >> 2) & 6u) + (lane >> 5)] = __fmul_rn(scale, (float)s32);
     if (lane == 0) {
         scales[seg] = scale;
         xst[(size_t)sb * MP + m] = scale;
@@ -583,11 +613,20 @@ __device__ __forceinline__ void quantize_q8k_sides_body(const void* __restrict__
 }
 extern "C" __global__ void __launch_bounds__(256)
 quantize_q8k_sides(const float* x, signed char* q, float* scales, float* xst, float* sums, uint K, uint M, uint MP) {
-    quantize_q8k_sides_body<false>(x, q, scales, xst, sums, K, M, MP);
+    quantize_q8k_sides_body<false, false>(x, q, scales, xst, sums, K, M, MP);
 }
 extern "C" __global__ void __launch_bounds__(256)
 quantize_q8k_bf16_sides(const ushort* x, signed char* q, float* scales, float* xst, float* sums, uint K, uint M, uint MP) {
-    quantize_q8k_sides_body<true>(x, q, scales, xst, sums, K, M, MP);
+    quantize_q8k_sides_body<true, false>(x, q, scales, xst, sums, K, M, MP);
+}
+
+extern "C" __global__ void __launch_bounds__(256)
+quantize_q8k_sides_h(const float* x, signed char* q, float* scales, float* xst, float* sums, uint K, uint M, uint MP) {
+    quantize_q8k_sides_body<false, true>(x, q, scales, xst, sums, K, M, MP);
+}
+extern "C" __global__ void __launch_bounds__(256)
+quantize_q8k_bf16_sides_h(const ushort* x, signed char* q, float* scales, float* xst, float* sums, uint K, uint M, uint MP) {
+    quantize_q8k_sides_body<true, true>(x, q, scales, xst, sums, K, M, MP);
 }
 
 // one 16-row tile's super-block: its two planes, and the row's side of the min term for the f32 matrix unit:
@@ -600,6 +639,60 @@ __device__ __forceinline__ void gxt_planes(const GqW& w, gq_i4 (&BA)[4], gq_i4 (
     n0 = __fmul_rn(ndmin, (float)((mn_lo >> sh) & 0xFFu));
     n1 = __fmul_rn(ndmin, (float)((mn_hi >> sh) & 0xFFu));
     gq_planes(w, BA, BB);
+}
+
+// K slices of a tile meet in scratch; true for the workgroup that holds the sum and owns y.  NP passes of four values a thread,
+// 512 threads; a slice's place is 32 KB whatever NP is (the tiles of a launch need not have the same).
+template <int NP>
+__device__ __forceinline__ bool gxt_meet(gq_f4 (&acc)[NP], float* __restrict__ part, uint* __restrict__ cnt, uint ns_eff, uchar* lds) {
+    // The partial tile goes out as the registers hold it ([pair][thread]: 512 contiguous bytes per wave and store),
+    // written through and read from behind the L2 (system-scope accesses): a tile's slices run on different XCDs,
+    // whose L2s do not see each other's lines.  The stores are awaited by instruction before the slice is counted.
+    typedef unsigned long long u64;
+    const uint tile = blockIdx.y * gridDim.x + blockIdx.x;
+    const uint te = threadIdx.x;
+    u64* const mine = (u64*)part + ((size_t)tile * ns_eff + blockIdx.z) * 4096u + te;
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            __hip_atomic_store(mine + (size_t)(p * 2 + h) * 512u,
+                               (u64)__float_as_uint(acc[p][2 * h]) | ((u64)__float_as_uint(acc[p][2 * h + 1]) << 32),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __syncthreads();
+    if (te == 0u) *(volatile uint*)lds = atomicAdd(cnt + tile, 1u);
+    __syncthreads();
+    if ((uint)__builtin_amdgcn_readfirstlane((int)*(volatile uint*)lds) != ns_eff - 1u) return false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    // (four slices' loads in flight before the first is added: a trip to memory per four slices, not one per load;
+    // past the last slice the loads repeat it and are dropped)
+    const u64* const all = (const u64*)part + (size_t)tile * ns_eff * 4096u + te;
+    for (uint s0 = 0; s0 < ns_eff; s0 += 4u) {
+        u64 v[4][NP * 2];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint sl = min(s0 + (uint)q, ns_eff - 1u);
+#pragma unroll
+            for (int i = 0; i < NP * 2; i++)
+                v[q][i] = __hip_atomic_load(all + (size_t)sl * 4096u + (uint)i * 512u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (s0 + (uint)q < ns_eff) {
+#pragma unroll
+                for (int i = 0; i < NP * 2; i++) {
+                    const float a = __uint_as_float((uint)v[q][i]), b = __uint_as_float((uint)(v[q][i] >> 32));
+                    const bool first = s0 + (uint)q == 0u;
+                    acc[i / 2][2 * (i % 2)] = first ? a : acc[i / 2][2 * (i % 2)] + a;
+                    acc[i / 2][2 * (i % 2) + 1] = first ? b : acc[i / 2][2 * (i % 2) + 1] + b;
+                }
+            }
+        }
+    }
+    if (te == 0u) cnt[tile] = 0u;                               // ready for the next launch
+    return true;
 }
 
 // TH = 1: eight row tiles (128 rows) per workgroup, a wave takes one of them against all eight passes of 16 tokens;
@@ -711,54 +804,8 @@ __device__ __forceinline__ void gemm_q8k_q4k_xt_body(const signed char* __restri
         }
     }
     if (SPLIT) {
-        // The partial tile goes out as the registers hold it ([pair][thread]: 512 contiguous bytes per wave and store),
-        // written through and read from behind the L2 (system-scope accesses): a tile's slices run on different XCDs,
-        // whose L2s do not see each other's lines.  The stores are awaited by instruction before the slice is counted.
-        typedef unsigned long long u64;
         const uint ns_eff = (nsb + per - 1u) / per;
-        const uint tile = blockIdx.y * gridDim.x + blockIdx.x;
-        const uint te = threadIdx.x;
-        u64* const mine = (u64*)part + ((size_t)tile * ns_eff + blockIdx.z) * (uint)(P * 2) * 512u + te;
-#pragma unroll
-        for (int p = 0; p < P; p++)
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-                __hip_atomic_store(mine + (size_t)(p * 2 + h) * 512u,
-                                   (u64)__float_as_uint(acc[p][2 * h]) | ((u64)__float_as_uint(acc[p][2 * h + 1]) << 32),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (te == 0u) *(volatile uint*)lds = atomicAdd(cnt + tile, 1u);
-        __syncthreads();
-        if ((uint)__builtin_amdgcn_readfirstlane((int)*(volatile uint*)lds) != ns_eff - 1u) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        // (four slices' loads in flight before the first is added: a trip to memory per four slices, not one per load;
-        // past the last slice the loads repeat it and are dropped)
-        const u64* const all = (const u64*)part + (size_t)tile * ns_eff * (uint)(P * 2) * 512u + te;
-        for (uint s0 = 0; s0 < ns_eff; s0 += 4u) {
-            u64 v[4][P * 2];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint sl = min(s0 + (uint)q, ns_eff - 1u);
-#pragma unroll
-                for (int i = 0; i < P * 2; i++)
-                    v[q][i] = __hip_atomic_load(all + ((size_t)sl * (uint)(P * 2) + (uint)i) * 512u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                if (s0 + (uint)q < ns_eff) {
-#pragma unroll
-                    for (int i = 0; i < P * 2; i++) {
-                        const float a = __uint_as_float((uint)v[q][i]), b = __uint_as_float((uint)(v[q][i] >> 32));
-                        const bool first = s0 + (uint)q == 0u;
-                        acc[i / 2][2 * (i % 2)] = first ? a : acc[i / 2][2 * (i % 2)] + a;
-                        acc[i / 2][2 * (i % 2) + 1] = first ? b : acc[i / 2][2 * (i % 2) + 1] + b;
-                    }
-                }
-            }
-        }
-        if (te == 0u) cnt[tile] = 0u;                               // ready for the next launch
+        if (!gxt_meet<P>(acc, part, cnt, ns_eff, lds)) return;
     }
     // (the lane id asked of the hardware again, so that nothing of it has to live through the loop)
     const uint le = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -775,6 +822,169 @@ __device__ __forceinline__ void gemm_q8k_q4k_xt_body(const signed char* __restri
         }
 }
 
+// ... and for the tile below: the two planes, d and dmin, and the mins as the f16 operand that meets the halved sums (lanes
+// kg = 0, 1: 2 m of sub-blocks 4 kg .. + 3) and the last bits (kg = 2, 3: m of 4 (kg - 2) .. + 3)
+typedef _Float16 gxk_h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 gxk_h2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void gxk_planes(const GqW& w, gq_i4 (&BA)[4], gq_i4 (&BB)[4], gxk_h4& mins, float& d, float& dmin, uint kg) {
+    d = f16_bits_to_f32(w.hdr.x & 0xFFFFu);
+    dmin = f16_bits_to_f32(w.hdr.x >> 16);
+    const uint mn_lo = w.hdr.z & 0x3F3F3F3Fu;
+    const uint mn_hi = ((w.hdr.w >> 4) & 0x0F0F0F0Fu) | ((w.hdr.z >> 2) & 0x30303030u);
+    const uint m4 = (kg & 1u) ? mn_hi : mn_lo;
+    // 0x64mm is 1024 + m in f16
+    const gxk_h2 off = {(_Float16)1024.0f, (_Float16)1024.0f}, two = kg < 2u ? (gxk_h2){(_Float16)2.0f, (_Float16)2.0f} : (gxk_h2){(_Float16)1.0f, (_Float16)1.0f};
+    const gxk_h2 a = (__builtin_bit_cast(gxk_h2, __builtin_amdgcn_perm(0x64646464u, m4, 0x04010400u)) - off) * two;
+    const gxk_h2 b = (__builtin_bit_cast(gxk_h2, __builtin_amdgcn_perm(0x64646464u, m4, 0x04030402u)) - off) * two;
+    mins = (gxk_h4){a[0], a[1], b[0], b[1]};
+    gq_planes(w, BA, BB);
+}
+
+// The 64-row tile for grids of at most one workgroup per CU:
+//   gemm_q8k_q4k_xk64(xq, xst, sums, w, y, K, N, M, ACC, MP)                          grid [ceil(N / 64), MP / 128, 1] x 512
+//   gemm_q8k_q4k_xk64_sr(xq, xst, sums, w, y, part, cnt, K, N, M, ACC, MP, NSPLIT)    grid [.., .., slices], as _xt64_sr
+// `sums` from q8k_token_sides_h or quantize_q8k{,_bf16}_sides_h.  The eight waves of gemm_q8k_q4k_xt64 halve the tokens of a
+// super-block, so both build the same planes, wait for copies asked for one super-block before, and issue the next ones ahead
+// of any matrix instruction: 2.3 us a super-block, vector issue and matrix pipe both at 0.35 - 0.4.  With a CU's LDS to
+// itself the tile holds two pairs of super-blocks: four row tiles x two halves of K, a wave walks every other super-block
+// against all NP passes of 16 tokens (planes built once, a barrier every two super-blocks); the next pair's copies go out
+// between the matrix instructions of the first passes; a pass's operands are read one pass ahead and its sums formed one
+// pass behind; and the min term, whole numbers, is one f16 instruction (the sums halved, their last bits beside them: exact
+// in f32) instead of two of the slow f32 ones.  The halves of K meet in LDS once.  NP = 4 where no more than 64 tokens are
+// left.  14336 x 4096, kernel alone: 128 tokens 33.5 -> 24 us (nothing of the min term's part: 26), 48 tokens 31.5 -> 16;
+// copies ahead of the passes instead of between them 28.5; tokens laid out a super-block apart instead of K: no difference.
+// Now bound by issue: matrix pipe and vector ALU share what the barrier leaves of a step.
+// Per (token, row, super-block) the sum takes xs (d isum - dmin msum), both sums exact, even and odd super-blocks apart.
+template <int NP, bool SPLIT>
+__device__ __forceinline__ void gemm_q8k_q4k_xk_body(const signed char* __restrict__ xq, const float* __restrict__ xst,
+                                                     const ushort* __restrict__ sums, const uchar* __restrict__ w,
+                                                     float* __restrict__ y, uint K, uint N, uint M, uint ACC, uint MP, uchar* lds,
+                                                     float* __restrict__ part, uint* __restrict__ cnt, uint nsplit) {
+    const uint tid = threadIdx.x, lane = tid & 63u;
+    const uint wave = (uint)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint rt = wave & 3u, kh = wave >> 2;                     // the wave's 16 rows and its super-blocks' parity
+    const uint nsb = K >> 8, n = lane & 15u, kg = lane >> 4;
+    const uint t0 = blockIdx.y * GXT_TOK, r0 = blockIdx.x * 64u + rt * 16u;
+    const uint lds0 = (uint)(size_t)(__attribute__((address_space(3))) uchar*)lds;
+    const gq_i4 zero = {0, 0, 0, 0};
+    // the super-blocks of this workgroup: all of them, or slice blockIdx.z of ceil(nsb / nsplit) each
+    const uint per = SPLIT ? (nsb + nsplit - 1u) / nsplit : nsb;
+    const uint sb0 = SPLIT ? blockIdx.z * per : 0u, sb1 = SPLIT ? min(nsb, sb0 + per) : nsb, last = sb1 - 1u;
+    constexpr int XC = NP / 2;                                      // copies of a super-block's tokens per wave, four tokens each
+    uint xoff[XC];
+#pragma unroll
+    for (int i = 0; i < XC; i++) {
+        const uint tk = (wave * (uint)XC + (uint)i) * 4u + (lane >> 4);
+        xoff[i] = min(t0 + tk, M - 1u) * K + (((lane & 15u) ^ (tk & 15u)) << 4);
+    }
+    // copy c of super-blocks sb and sb + 1 (one past the end repeats the last) into stages 2 pair and 2 pair + 1: eight of
+    // tokens, one of scaled sums, one of scales
+    auto copy = [&](int c, uint sb, uint pair) {
+        if (c < 2 * XC) {
+            const uint h = (uint)(c / XC);
+            lds_dma16_s((const uchar*)xq + (size_t)min(sb + h, last) * 256u, xoff[c % XC],
+                        lds0 + (2u * pair + h) * GXT_STAGE + (wave * (uint)XC + (uint)(c % XC)) * 1024u);
+            return;
+        }
+        const uint sq = min(sb + kh, last), st = lds0 + (2u * pair + kh) * GXT_STAGE;
+        if (c == 2 * XC) {
+            if (rt < (uint)XC) lds_dma16_s((const uchar*)sums + ((size_t)sq * MP + t0) * 32u + rt * 1024u, lane * 16u, st + GXT_TOK * 256u + rt * 1024u);
+        } else if (rt == 0u && lane < 32u) lds_dma16_s(xst + (size_t)sq * MP + t0, lane * 16u, st + GXT_TOK * 288u);
+    };
+    const uint wrow = min(r0 + n, N - 1u) * nsb * Q4K_BYTES;
+    gq_f4 acc[NP];
+#pragma unroll
+    for (int p = 0; p < NP; p++) acc[p] = (gq_f4){0.0f, 0.0f, 0.0f, 0.0f};
+    uint o0[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) o0[c] = n * 256u + 8u * (kg & 1u) + (((4u * (uint)c + (kg >> 1)) ^ n) << 4);
+    const uint side_lds = GXT_TOK * 256u + n * 32u + 8u * kg, sc_lds = GXT_TOK * 288u + 16u * kg;
+
+    GqW cur = gq_load((w + (size_t)min(sb0 + kh, last) * Q4K_BYTES) + wrow, kg);
+#pragma unroll
+    for (int c = 0; c < 2 * XC + 2; c++) copy(c, sb0, 0u);
+    for (uint sb = sb0; sb < sb1; sb += 2u) {
+        const uint pair = ((sb - sb0) >> 1) & 1u;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();                                            // the pair's stages are complete; the other pair is free
+        const bool more = sb + 2u < sb1;
+        const uchar* st = lds + (2u * pair + kh) * GXT_STAGE;
+        gq_i4 BA[4], BB[4];
+        gxk_h4 mins;
+        float d, dmin;
+        gxk_planes(cur, BA, BB, mins, d, dmin, kg);
+        __builtin_amdgcn_sched_barrier(0);
+        cur = gq_load((w + (size_t)min(sb + 2u + kh, last) * Q4K_BYTES) + wrow, kg);
+        __builtin_amdgcn_sched_barrier(0);
+        if (sb + kh < sb1) {
+            gq_i4 A[2][4], DA[2], DB[2];
+            gxk_h4 am[2];
+            gq_f4 DM[2];
+            float4 sx[2];
+#define GXK_READ(P)                                                                                           \
+            do {                                                                                              \
+                _Pragma("unroll") for (int c = 0; c < 4; c++) {                                               \
+                    const uint2 a0 = *(const uint2*)(st + o0[c] + 4096u * (uint)(P)), a1 = *(const uint2*)(st + (o0[c] ^ 32u) + 4096u * (uint)(P)); \
+                    A[(P) & 1][c] = (gq_i4){(int)a0.x, (int)a0.y, (int)a1.x, (int)a1.y};                       \
+                }                                                                                             \
+                am[(P) & 1] = *(const gxk_h4*)(st + side_lds + 512u * (uint)(P));                              \
+            } while (0)
+#define GXK_SUM(P)                                                                                            \
+            do {                                                                                              \
+                const float sxv[4] = {sx[(P) & 1].x, sx[(P) & 1].y, sx[(P) & 1].z, sx[(P) & 1].w};             \
+                _Pragma("unroll") for (int v = 0; v < 4; v++) acc[P][v] += sxv[v] * (d * (float)(8 * DB[(P) & 1][v] + DA[(P) & 1][v]) - dmin * DM[(P) & 1][v]); \
+            } while (0)
+            GXK_READ(0);
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const int b = p & 1;
+                sx[b] = *(const float4*)(st + sc_lds + 64u * (uint)p);
+                if (p + 1 < NP) GXK_READ(p + 1);
+                DM[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(am[b], mins, (gq_f4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                DA[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b][0], BA[0], zero, 0, 0, 0);
+                DB[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b][0], BB[0], zero, 0, 0, 0);
+                if (more && p <= XC) { copy(2 * p, sb + 2u, pair ^ 1u); copy(2 * p + 1, sb + 2u, pair ^ 1u); }
+#pragma unroll
+                for (int c = 1; c < 4; c++) {
+                    DA[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b][c], BA[c], DA[b], 0, 0, 0);
+                    DB[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[b][c], BB[c], DB[b], 0, 0, 0);
+                }
+                if (p) GXK_SUM(p - 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            GXK_SUM(NP - 1);
+#undef GXK_READ
+#undef GXK_SUM
+        }
+    }
+    // the halves of K meet in LDS: each half's waves leave the passes that the other's store
+    __syncthreads();
+    gq_f4* const box = (gq_f4*)lds + lane;
+#pragma unroll
+    for (int p = 0; p < NP / 2; p++) box[(wave * (NP / 2) + p) * 64u] = kh ? acc[p] : acc[NP / 2 + p];
+    __syncthreads();
+    gq_f4 res[NP / 2];
+#pragma unroll
+    for (int p = 0; p < NP / 2; p++) {
+        const gq_f4 o = box[((wave ^ 4u) * (NP / 2) + p) * 64u];
+        res[p] = kh ? o + acc[NP / 2 + p] : acc[p] + o;
+    }
+    if (SPLIT) {
+        if (!gxt_meet<NP / 2>(res, part, cnt, (nsb + per - 1u) / per, lds)) return;
+    }
+    const uint r = r0 + n;
+#pragma unroll
+    for (int p = 0; p < NP / 2; p++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const uint t = t0 + 8u * NP * kh + 16u * (uint)p + 4u * kg + (uint)v;
+            if (t < M && r < N) {
+                float* q = y + (size_t)t * N + r;
+                *q = ACC ? *q + res[p][v] : res[p][v];
+            }
+        }
+}
+
 extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 gemm_q8k_q4k_xt(const signed char* xq, const float* xst, const float* sums, const uchar* w, float* y, uint K, uint N, uint M,
                 uint ACC, uint MP) {
@@ -786,6 +996,20 @@ gemm_q8k_q4k_xt64(const signed char* xq, const float* xst, const float* sums, co
                   uint ACC, uint MP) {
     __shared__ __attribute__((aligned(1024))) uchar lds_xt[2 * GXT_STAGE];
     gemm_q8k_q4k_xt_body<2>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xt);
+}
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_q8k_q4k_xk64(const signed char* xq, const float* xst, const ushort* sums, const uchar* w, float* y, uint K, uint N, uint M,
+                  uint ACC, uint MP) {
+    __shared__ __attribute__((aligned(1024))) uchar lds_xk[4 * GXT_STAGE];
+    if (M - blockIdx.y * GXT_TOK <= 64u) gemm_q8k_q4k_xk_body<4, false>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xk, nullptr, nullptr, 1u);
+    else gemm_q8k_q4k_xk_body<8, false>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xk, nullptr, nullptr, 1u);
+}
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_q8k_q4k_xk64_sr(const signed char* xq, const float* xst, const ushort* sums, const uchar* w, float* y, float* part, uint* cnt,
+                     uint K, uint N, uint M, uint ACC, uint MP, uint NSPLIT) {
+    __shared__ __attribute__((aligned(1024))) uchar lds_xk[4 * GXT_STAGE];
+    if (M - blockIdx.y * GXT_TOK <= 64u) gemm_q8k_q4k_xk_body<4, true>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xk, part, cnt, NSPLIT);
+    else gemm_q8k_q4k_xk_body<8, true>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xk, part, cnt, NSPLIT);
 }
 // the 64-row tile over K slices, for matrices whose 64-row tiles alone leave most CUs idle:
 //   gemm_q8k_q4k_xt64_sr(xq, xst, sums, w, y, part, cnt, K, N, M, ACC, MP, NSPLIT)

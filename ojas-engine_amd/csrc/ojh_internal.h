@@ -73,6 +73,7 @@ struct ojh_device {
     uint32_t rms_threads = 0;    // OJAS_HIP_RMS_THREADS: block size of rmsnorm_q8k (256 or 1024; 0: by the number of rows)
     uint32_t q4k_xt_split = 1;   // OJAS_HIP_Q4K_XT_SPLIT: K slices of the 64-row int8 tile when its tiles leave CUs idle (0: never, 1: chosen, n: n)
     uint32_t q4k_xt_min_m = 1;   // OJAS_HIP_Q4K_XT_MIN_M: tokens from which Q4_K rows take the 128-token int8 tile (0: never, 1: by shape)
+    bool q4k_xk = true;          // OJAS_HIP_Q4K_XK=0: the 64-row int8 tile never in the form that has a CU to itself
     bool q4k_xt64 = false;       // OJAS_HIP_Q4K_XT64=1: that tile always in its 64-row form
     bool no_scratch = false;     // set around calls that may not allocate (ojh_mm_noalloc): paths that need library scratch are skipped
     uint32_t q8row_mt_min_m = 1; // OJAS_HIP_Q8ROW_MT_MIN_M: tokens from which ojh_matmul_q8 takes the int8 matrix tile (0: never, 1: measured default, n: n)
@@ -195,7 +196,7 @@ int ojh_mm_checks(const char *who, const ojh_lin *w, ojh_buf *y, size_t y_off, c
 int ojh_quant_q8k_launch(ojh_device *dev, const void *x, int x_dtype, uint32_t m, uint32_t k, void *q, void *scales);
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,
                       const ojh_buf *bias, uint32_t m, int accum, bool sides_ready = false);
-bool ojh_q4k_xt_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp);
+bool ojh_q4k_xt_taken(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp);
 int ojh_noalloc_setup(ojh_device *dev);   // resolves the static scratch array on the current GPU (ojh_noalloc.cpp)
 void ojh_gemm_q8k_tiles(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M, uint32_t *rw, uint32_t *rt);   // row tiles per workgroup / per wave of gemm_q8k_q4k_mf
 uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t E, bool gu, uint32_t *threads);   // workgroups per expert of those entries, and their threads

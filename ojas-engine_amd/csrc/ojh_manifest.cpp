@@ -2081,6 +2081,11 @@ static std::vector<ojh_kernel_spec> build_manifest() {
     add("quantize_q8k_bf16_sides", "gemm_q8k", 5, 3, 0, 0, check_quantize_sides, shape_quantize_sides);
     add("gemm_q8k_q4k_xt", "gemm_q8k", 5, 5, OJH_Q4_K, 1, check_gemm_q8k_xt, shape_gemm_q8k_xt);
     add("gemm_q8k_q4k_xt64", "gemm_q8k", 5, 5, OJH_Q4_K, 2, check_gemm_q8k_xt, shape_gemm_q8k_xt);
+    add("q8k_token_sides_h", "gemm_q8k", 4, 3, 0, 0, check_gemm_q8k_xt, shape_gemm_q8k_xt);
+    add("quantize_q8k_sides_h", "gemm_q8k", 5, 3, 0, 0, check_quantize_sides, shape_quantize_sides);
+    add("quantize_q8k_bf16_sides_h", "gemm_q8k", 5, 3, 0, 0, check_quantize_sides, shape_quantize_sides);
+    add("gemm_q8k_q4k_xk64", "gemm_q8k", 5, 5, OJH_Q4_K, 2, check_gemm_q8k_xt, shape_gemm_q8k_xt);
+    add("gemm_q8k_q4k_xk64_sr", "gemm_q8k", 7, 6, OJH_Q4_K, 2, check_gemm_q8k_xt_sr, shape_gemm_q8k_xt_sr);
     add("gemm_q8k_q4k_xt64_sr", "gemm_q8k", 7, 6, OJH_Q4_K, 2, check_gemm_q8k_xt_sr, shape_gemm_q8k_xt_sr);
     add("gemv_q8", "gemv_q8", 4, 2, 0, 0, check_gemv_q8, shape_gemv_q8);
     add("gemv_q8_accum", "gemv_q8", 4, 2, 0, 0, check_gemv_q8, shape_gemv_q8);

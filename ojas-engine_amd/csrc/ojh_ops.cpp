@@ -176,7 +176,23 @@ static uint32_t q4k_xt_slices(const ojh_device *dev, uint32_t K, uint32_t N, uin
     if (z < 2 || tiles * z * 2 < cus) return whole;
     return ojh_gemm_sr_slices(K, z);
 }
-// Tokens from which that tile is taken (measured with the rows streamed from HBM, K = 2048 .. 14336): the tile costs
+// Slices of the form that has a CU to itself (1: whole; 0: not this form): up to one tile per CU in all, of at least four
+// super-blocks, two where four would leave more than half the CUs idle.  Above one tile per CU two workgroups of the other
+// form share it and are as fast or faster.  That form / this one, with the quantizer, us: 14336 x 4096 at 48 tokens 36.5 /
+// 21.4, at 128 38.4 / 28.9; 4096 x 14336 at 512 109.5 / 95; 4096^2 at 512 41.9 / 34; at 128 (four slices) 19.0 / 17.5;
+// 14336 x 4096 at 256 (448 tiles) 57.8 / 57.8, at 512 84 / 111.
+static uint32_t q4k_xk_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
+    const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount, nsb = K / 256;
+    const uint64_t tiles = (uint64_t)((N + 63) / 64) * ((m + 127) / 128);
+    if (!dev->q4k_xk || dev->q4k_xt64 || dev->q4k_xt_split > 1 || tiles > cus) return 0;
+    uint32_t z = std::min<uint32_t>((uint32_t)(cus / tiles), 8u), cap = std::max(nsb / 4, 1u);
+    if (dev->q4k_xt_split == 0 || z < 2) return 1;
+    if (tiles * std::min(z, cap) * 2 < cus) cap = std::max(nsb / 2, 1u);
+    z = std::min(z, cap);
+    return z < 2 ? 1 : ojh_gemm_sr_slices(K, z);
+}
+// Tokens from which that tile is taken whatever the form (measured with the rows streamed from HBM, K = 2048 .. 14336, before
+// the form that has a CU to itself): the tile costs
 // the same from 1 to 128 tokens, the matrix-core kernel below it doubles past 32 tokens.  So from 33 tokens; from 17
 // where K is at least twice the row count (few tiles, each a long walk: 4096 x 14336 takes 38 us here against 45);
 // and only from 65 for a matrix of more than one and a half 64-row tiles per CU, where two 32-token passes of the
@@ -187,11 +203,23 @@ static uint32_t q4k_xt_min_tokens(const ojh_device *dev, uint32_t K, uint32_t N)
     if (2 * (uint64_t)((N + 63) / 64) > 3ull * cus) return 65;
     return K >= 2ull * N ? 17 : 33;
 }
-bool ojh_q4k_xt_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp) {
+// The form that has a CU to itself multiplies no more than 64 tokens where no more are left, and is ahead from 17 of them,
+// where the few-token kernels need a second pass of 16 (before / with it, 24 tokens, us: 14336 x 4096 22.6 / 20.7, 4096^2
+// 16.7 / 12.4, 1024 x 4096 15.3 / 11.4, 4096 x 14336 35.2 / 22.3, 2048^2 10.8 / 9.9; at 12 tokens 17.7 / 20.4, 8.9 / 12.3, 8.5 /
+// 11.4).  The few-token kernels need none of its scratch, so where that is not to be had the call stays with them.
+static bool q4k_xk_early(ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
+    const uint32_t z = m >= 17 && dev->q4k_xt_min_m == 1 ? q4k_xk_slices(dev, K, N, m) : 0;
+    if (!z || ensure(dev, "gemm_q8k")) return false;
+    const size_t mp = (m + 127) / 128 * 128, nsb = K / 256, tiles = (size_t)((N + 63) / 64) * (mp / 128);
+    ojh_buf *b;
+    return !ojh_scratch_spare(dev, "xt_xst", nsb * mp * 4, &b) && !ojh_scratch_spare(dev, "xt_sums", nsb * mp * 32, &b) &&
+           (z == 1 || (!ojh_scratch_spare(dev, "xt_part", tiles * z * 32768, &b) && !ojh_scratch_get_zeroed(dev, "xt_cnt", tiles * 4, &b)));
+}
+bool ojh_q4k_xt_taken(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp) {
     const uint32_t K = w->k, N = w->n;
-    return w->type == OJH_Q4_K && dev->q4k_xt_min_m && m >= q4k_xt_min_tokens(dev, K, N) && !dev->no_scratch &&
-           q4k_xt_slices(dev, K, N, m) >= 1 &&
-           (uint64_t)m * K <= 0xFFFFFFFFull && (uint64_t)w->row_bytes * N <= 0xFFFFFFFFull && (uintptr_t)wp % 16 == 0;
+    return w->type == OJH_Q4_K && dev->q4k_xt_min_m && !dev->no_scratch && q4k_xt_slices(dev, K, N, m) >= 1 &&
+           (uint64_t)m * K <= 0xFFFFFFFFull && (uint64_t)w->row_bytes * N <= 0xFFFFFFFFull && (uintptr_t)wp % 16 == 0 &&
+           (m >= q4k_xt_min_tokens(dev, K, N) || q4k_xk_early(dev, K, N, m));
 }
 
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,
@@ -230,8 +258,21 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
         if ((rc = ojh_scratch_get(dev, "xt_sums", nsb * mp * 32, &sums))) return rc;
         uint32_t sg[3], sb[3];
         if (!sides_ready) {
-            if ((rc = ojh_launch_shape(dev, "q8k_token_sides", K, N, m, sg, sb))) return rc;
-            if ((rc = ojh_launch(dev, "q8k_token_sides", {xq, xs, xst->ptr, sums->ptr}, {K, m, mp}, sg, sb))) return rc;
+            const char *sides = q4k_xk_slices(dev, K, N, m) ? "q8k_token_sides_h" : "q8k_token_sides";
+            if ((rc = ojh_launch_shape(dev, sides, K, N, m, sg, sb))) return rc;
+            if ((rc = ojh_launch(dev, sides, {xq, xs, xst->ptr, sums->ptr}, {K, m, mp}, sg, sb))) return rc;
+        }
+        // at most one 64-row tile per CU: the form that has a CU to itself, over K slices where that leaves CUs idle
+        if (const uint32_t z = q4k_xk_slices(dev, K, N, m)) {
+            const size_t tiles = (size_t)((N + 63) / 64) * (mp / 128);
+            sg[0] = (N + 63) / 64; sg[1] = mp / 128; sg[2] = z;
+            sb[0] = 512; sb[1] = sb[2] = 1;
+            if (z == 1) return ojh_launch(dev, "gemm_q8k_q4k_xk64", {xq, xst->ptr, sums->ptr, wp, yp}, {K, N, m, (uint32_t)(accum != 0), mp}, sg, sb);
+            ojh_buf *part, *cnt;
+            if ((rc = ojh_scratch_get(dev, "xt_part", tiles * z * 32768, &part))) return rc;
+            if ((rc = ojh_scratch_get_zeroed(dev, "xt_cnt", tiles * 4, &cnt))) return rc;
+            return ojh_launch(dev, "gemm_q8k_q4k_xk64_sr", {xq, xst->ptr, sums->ptr, wp, yp, part->ptr, cnt->ptr},
+                              {K, N, m, (uint32_t)(accum != 0), mp, z}, sg, sb);
         }
         // too few 64-row tiles for the chip: K slices of them, summed in slice order by the last to finish
         if (const uint32_t z = q4k_xt_slices(dev, K, N, m); z > 1) {
@@ -935,7 +976,9 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
             if ((rc = ojh_scratch_get(dev, "xt_xst", nsb * mp * 4, &xst))) return rc;
             if ((rc = ojh_scratch_get(dev, "xt_sums", nsb * mp * 32, &sums))) return rc;
             uint32_t qg[3] = {K / 256 * (mp / 4), 1, 1};
-            if ((rc = ojh_launch(dev, x_dtype == OJH_X_BF16 ? "quantize_q8k_bf16_sides" : "quantize_q8k_sides",
+            const std::string quant = std::string(x_dtype == OJH_X_BF16 ? "quantize_q8k_bf16_sides" : "quantize_q8k_sides") +
+                                      (q4k_xk_slices(dev, K, N, m) ? "_h" : "");
+            if ((rc = ojh_launch(dev, quant.c_str(),
                                  {at(x, x_off), xq->ptr, xs->ptr, xst->ptr, sums->ptr}, {K, m, mp}, qg, block)))
                 return rc;
             return ojh_mm_q8k_launch(dev, xq->ptr, xs->ptr, w, f, yp, bias, m, accum, true);

@@ -248,3 +248,109 @@ def test_prefill_tiles_by_name(gpu, orc, pkg, m, n, k):
     with pytest.raises(pkg.OjasHipError, match="rounded up to 128"):
         gpu.dispatch(gpu.begin(), "gemm_q8k_q4k_xt", [(xq, 0), (xst, 0), (sums, 0), (wd, 0), (ymf, 0)], [k, n, m, 0, mp + 128],
                      [(n + 127) // 128, mp // 128, 1], [512, 1, 1])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 256), (40, 130, 512), (64, 65, 2304), (65, 77, 768), (128, 128, 256), (190, 200, 2048), (300, 1000, 1280)])
+def test_tile_with_a_cu_to_itself_by_name(gpu, orc, pkg, m, n, k):
+    """`gemm_q8k_q4k_xk64{,_sr}` and the side arrays they read: one super-block, odd counts (the second half of K idle in the
+    last step), up to 64 tokens in a tile and just past, ragged rows; the sums are `gemm_q8k_q4k_mf`'s terms, two halves of K
+    added once (K / 256 f32 additions: 2e-6 of the peak, as for the other tile)."""
+    w, x = _case(pkg, m, n, k, "xk")
+    gpu.ensure_family("gemm_q8k")
+    gpu.ensure_family("gemv_q8k")
+    nsb, mp = k // 256, (m + 127) // 128 * 128
+    xq, xs, xst, sums = gpu.alloc_bytes(m * k), gpu.alloc(m * nsb), gpu.alloc(nsb * mp), gpu.alloc(nsb * mp * 8)
+    gpu.quant_q8k(gpu.upload(x), m, k, xq, xs)
+    gpu.dispatch(gpu.begin(), "q8k_token_sides_h", [(xq, 0), (xs, 0), (xst, 0), (sums, 0)], [k, m, mp], [nsb, (mp + 255) // 256, 1], [256, 1, 1])
+    # halved run sums and their last bits as f16, zeros past row M; the quantizer that writes them gives the same bytes
+    q = gpu.read(xq, m * k, np.int8).reshape(m, nsb, 8, 32).astype(np.int32).sum(3).transpose(1, 0, 2)
+    sd = gpu.read(sums, nsb * mp * 16, np.float16).reshape(nsb, mp, 16)
+    assert np.array_equal(sd[:, :m, :8], (q >> 1).astype(np.float16)) and np.array_equal(sd[:, :m, 8:], (q & 1).astype(np.float16))
+    assert np.array_equal(2 * sd[:, :m, :8].astype(np.int32) + sd[:, :m, 8:].astype(np.int32), q) and not sd[:, m:].any()
+    xb = (x.view(np.uint32) >> 16).astype(np.uint16)
+    for name, src in (("quantize_q8k_sides_h", x), ("quantize_q8k_bf16_sides_h", xb)):
+        bf = src is xb
+        q1, s1, t1, u1 = gpu.alloc_bytes(m * k), gpu.alloc(m * nsb), gpu.alloc(nsb * mp), gpu.alloc(nsb * mp * 8)
+        gpu.quant_q8k(gpu.upload((xb.astype(np.uint32) << 16).view(np.float32) if bf else x), m, k, q1, s1)
+        gpu.dispatch(gpu.begin(), "q8k_token_sides_h", [(q1, 0), (s1, 0), (t1, 0), (u1, 0)], [k, m, mp], [nsb, (mp + 255) // 256, 1], [256, 1, 1])
+        q2, s2 = gpu.alloc_bytes(m * k), gpu.alloc(m * nsb)
+        t2, u2 = gpu.upload(np.full(nsb * mp, 7.5, np.float32)), gpu.upload(np.full(nsb * mp * 8, 7.5, np.float32))
+        gpu.dispatch(gpu.begin(), name, [(gpu.upload_bytes(xb.view(np.uint8)) if bf else gpu.upload(x), 0), (q2, 0), (s2, 0), (t2, 0), (u2, 0)],
+                     [k, m, mp], [nsb * mp // 4, 1, 1], [256, 1, 1])
+        for a, b, c in ((q1, q2, m * k // 4), (s1, s2, m * nsb), (t1, t2, nsb * mp), (u1, u2, nsb * mp * 8)):
+            assert np.array_equal(gpu.read(a, c, np.uint32), gpu.read(b, c, np.uint32)), name
+    wd, ymf = gpu.upload_bytes(w), gpu.alloc(m * n)
+    gpu.dispatch(gpu.begin(), "gemm_q8k_q4k_mf", [(xq, 0), (xs, 0), (wd, 0), (ymf, 0)], [k, n, m, 0, 4, 1],
+                 [(n + 63) // 64, (m + 63) // 64, 1], [256, 1, 1])
+    ref = gpu.read(ymf, m * n).reshape(m, n)
+    want = np.stack([orc.matvec_kq(w, Q4_K, n, k, x[t]) for t in range(m)])
+    tiles = (n + 63) // 64 * (mp // 128)
+    cnt = gpu.alloc_bytes(tiles * 4)
+    gpu.memset0(cnt)
+    for nsplit in [0] + sorted({min(s, nsb) for s in (2, 3, nsb)}):
+        per = (nsb + nsplit - 1) // nsplit if nsplit else nsb
+        slices = (nsb + per - 1) // per
+        part = gpu.alloc(tiles * slices * 8192)
+        seen = []
+        for acc in (0, 1, 0):
+            y0 = pkg.synth.normal_f32(m * n, "gq", "xk-y0", acc).reshape(m, n)
+            yd = gpu.upload(np.concatenate([y0.ravel(), np.full(n, 4242.5, np.float32)]))
+            bufs = [(xq, 0), (xst, 0), (sums, 0), (wd, 0), (yd, 0)]
+            gpu.dispatch(gpu.begin(), "gemm_q8k_q4k_xk64_sr" if nsplit else "gemm_q8k_q4k_xk64", bufs + [(part, 0), (cnt, 0)] if nsplit else bufs,
+                         [k, n, m, acc, mp, nsplit] if nsplit else [k, n, m, acc, mp], [(n + 63) // 64, mp // 128, slices], [512, 1, 1])
+            got = gpu.read(yd, m * n + n)
+            assert np.all(got[m * n:] == 4242.5), "wrote past the last token"
+            assert not gpu.read(cnt, tiles, np.uint32).any()
+            got = got[:m * n].reshape(m, n)
+            if acc:
+                assert peak_err(got - y0, want) <= TOL_SEEN
+            else:
+                assert peak_err(got, want) <= TOL_SEEN and peak_err(got, ref) <= 2e-6
+                seen.append(got.view(np.uint32).copy())
+        assert np.array_equal(seen[0], seen[1]), nsplit
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 4096, 1024), (33, 1100, 2304), (128, 2048, 4096), (200, 4100, 1280)])
+def test_both_forms_of_the_int8_tile_through_mm(pkg, monkeypatch, m, n, k):
+    """What `OJAS_HIP_Q4K_XK` chooses between, for the sizes the rule sends to the new form: the same terms in another order."""
+    w, x = _case(pkg, m, n, k, "xk-mm")
+    outs = []
+    for xk in ("0", "1"):
+        monkeypatch.setenv("OJAS_HIP_Q4K_XK", xk)
+        g = pkg.HipGpu(0)
+        try:
+            for xd, dt in ((g.upload(x), pkg.X_F32), (g.upload_bytes((x.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8)), pkg.X_BF16)):
+                yd = g.upload(np.full(m * n + 64, 4242.5, np.float32))
+                g.mm(xd, g.lin(Q4_K, n, k, w), yd, m, x_dtype=dt, act_mode=pkg.ACT_Q8K)
+                got = g.read(yd, m * n + 64)
+                assert np.all(got[m * n:] == 4242.5)
+                outs.append(got[:m * n])
+        finally:
+            g.close()
+    assert peak_err(outs[2], outs[0]) <= 2e-6 and peak_err(outs[3], outs[1]) <= 2e-6
+
+
+def test_few_tokens_without_room_for_the_tile_keep_their_kernel(pkg, orc, monkeypatch):
+    """24 tokens of Q4_K rows run on the 64-row tile where its scratch is to be had.  A limit that holds the quantized tokens
+    alone, and a chain recorded before anything ran at that size, leave them on the few-token kernel: the same terms."""
+    m, n, k = 24, 700, 2048
+    w, x = _case(pkg, m, n, k, "early")
+    want = np.stack([orc.matvec_kq(w, Q4_K, n, k, x[t]) for t in range(m)])
+    for limit, first in (("0", m), ("65536", m), ("0", 16)):
+        monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", limit)
+        g = pkg.HipGpu(0)
+        try:
+            xd, lin, yd = g.upload(x), g.lin(Q4_K, n, k, w), g.alloc(m * n)
+            g.ensure_family("gemm_q8k")
+            xq, xs = g.alloc_bytes(m * k), g.alloc(m * k // 256)
+            g.quant_q8k(xd, m, k, xq, xs)
+            g.mm_q8k(xq, xs, lin, yd, first)
+            if first < m:
+                g.submit()
+                g.capture_begin()
+                g.mm_q8k(xq, xs, lin, yd, m)
+                chain = g.capture_end()
+                chain.launch()
+            assert peak_err(g.read(yd, m * n).reshape(m, n), want) <= TOL_SEEN
+        finally:
+            g.close()
