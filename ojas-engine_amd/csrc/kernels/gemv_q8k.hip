@@ -18,6 +18,7 @@
 // (always for the min term; for the scale term unless |sum| >= 2^24, where the reference itself
 // rounds).  The per-row f32 accumulation over super-blocks runs in a different order than the
 // reference's (lanes own different super-blocks), which moves the last ulp only.
+#include <type_traits>
 #include "ojk_common.h"
 #include "ojk_q4k_dot.h"
 #include "ojk_act.h"
@@ -765,9 +766,10 @@ struct Q6kX {          // a lane's share of the activations of one super-block
     float sx;
 };
 
+template <uint SEG = 256u>      // bytes from one super-block's activations to the next's
 __device__ __forceinline__ Q6kX q6k_load_x(const signed char* xq, const float* xs, uint sb, uint hf, uint l0) {
     Q6kX f;
-    const signed char* p = xq + (size_t)sb * 256u + hf * 128u + l0;
+    const signed char* p = xq + (size_t)sb * SEG + hf * 128u + l0;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         f.x[q] = *(const uint4*)(p + 32 * q);
@@ -866,6 +868,122 @@ __device__ __forceinline__ void gemv_q8k_q6k_body(const signed char* __restrict_
 }
 
 GEMV_Q8K_ENTRIES(q6k, gemv_q8k_q6k_body)
+
+// ---- one small projection of one token in one launch ---------------------------------------------
+//   gemv_fq8k_{q4k,q5k,q6k}_one{,_bf16}_{r1,r2}(x, w, y, K, N, NRB, ACC)     x: f32 | bf16 [K], K <= 16384, grid [ceil(N / NRB)] x 1024
+// The quantizer and the matvec of a 1024 x 4096 projection take 2.3 and 2.8 us on the device and 7.7 from call to call: two
+// dependent launches and their issue from the host are the time.  As above every workgroup quantizes x into LDS, the
+// activations asked for first and its first weights second, and walks NRB rows, here of one tensor in any of the three
+// formats and from f32 or bf16 activations.  4.4 us from call to call
+// at 1024 x 4096, 4.6 at 4096^2 (7.8 in two launches); what bounds it is the launch.
+// Each format keeps the lane map and the order of operations of its gemv_q8k_<fmt>, so the bits are those of two launches.
+template <class B>
+struct One8 {                             // eight lanes a super-block: Q4_K, Q5_K
+    static constexpr uint LANES = 8u, BYTES = B::BYTES;
+    B b;
+    typedef Q4kFrag X;
+    __device__ __forceinline__ void load(const uchar* blk, uint u) { b.load(blk, u); }
+    static __device__ __forceinline__ X frag(const signed char* sx, const float* ss, uint sb, uint u) {
+        X f;
+        const signed char* p = sx + sb * FQ_SEG + (u >> 1) * 64u + (u & 1u) * 16u;
+        f.xl = *(const uint4*)p;
+        f.xh = *(const uint4*)(p + 32);
+        f.bl = bytesum4(f.xl);
+        f.bh = bytesum4(f.xh);
+        f.sx = ss[sb];
+        return f;
+    }
+    __device__ __forceinline__ float dot(const X& f, uint u) const { return b.dot(u >> 1, f); }
+};
+struct One6 {                             // four: Q6_K
+    static constexpr uint LANES = 4u, BYTES = Q6K_BYTES;
+    Q6kW b;
+    typedef Q6kX X;
+    __device__ __forceinline__ void load(const uchar* blk, uint u) { b = q6k_load_w(blk, u >> 1, (u & 1u) * 16u); }
+    static __device__ __forceinline__ X frag(const signed char* sx, const float* ss, uint sb, uint u) {
+        return q6k_load_x<FQ_SEG>(sx, ss, sb, u >> 1, (u & 1u) * 16u);
+    }
+    __device__ __forceinline__ float dot(const X& f, uint) const { return q6k_lane_dot(b, f); }
+};
+template <int R, class W, bool BF16>
+__device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, const uchar* __restrict__ w, float* __restrict__ y,
+                                                   uint K, uint N, uint NRB, uint ACC) {
+    __shared__ __attribute__((aligned(16))) signed char sx[(FQ_MAX_K / 256u) * FQ_SEG];
+    __shared__ float ss[FQ_MAX_K / 256u];
+    const uint tid = threadIdx.x, lane = tid & 63u, wave = (uint)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), nw = blockDim.x >> 6;
+    constexpr uint STEP = 64u / W::LANES;
+    const uint nsb = K >> 8, g = lane / W::LANES, l = lane % W::LANES;
+    const uint row_end = min((blockIdx.x + 1u) * NRB, N);
+    uint row0 = blockIdx.x * NRB + wave * R;
+    auto fetch = [&](uint r0, uint sb, W (&o)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; r++) o[r].load(w + ((size_t)min(r0 + r, N - 1u) * nsb + min(sb, nsb - 1u)) * W::BYTES, l);
+    };
+    typedef typename std::conditional<BF16, uint2, float4>::type X4;
+    constexpr int NB = 4;
+    X4 v[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) v[i] = ((const X4*)xv)[min(wave + nw * (uint)i, nsb - 1u) * 64u + lane];
+    __builtin_amdgcn_sched_barrier(0);
+    W cur[R], nxt[R];
+    fetch(row0, g, cur);
+    __builtin_amdgcn_sched_barrier(0);
+    for (uint s0 = 0; s0 < nsb; s0 += nw * NB) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const uint seg = s0 + wave + nw * (uint)i;
+            float4 t;
+            if constexpr (BF16) t = make_float4(__uint_as_float(v[i].x << 16), __uint_as_float(v[i].x & 0xFFFF0000u),
+                                                __uint_as_float(v[i].y << 16), __uint_as_float(v[i].y & 0xFFFF0000u));
+            else t = v[i];
+            if (s0 + nw * NB < nsb) v[i] = ((const X4*)xv)[min(seg + nw * NB, nsb - 1u) * 64u + lane];
+            if (seg < nsb) {
+                const float a = wave_max(amax4(t));
+                const float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
+                *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(t, __fdiv_rn(1.0f, scale));
+                if (lane == 0) ss[seg] = scale;
+            }
+        }
+    }
+    __syncthreads();
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.0f;
+    uint sb = g;
+    while (row0 < row_end) {
+        uint nsb_next = sb + STEP, nrow = row0;
+        const bool last = nsb_next >= nsb + g;    // the group's last step
+        if (last) { nsb_next = g; nrow = row0 + nw * R; }
+        if (nrow < row_end) fetch(nrow, nsb_next, nxt);
+        if (sb < nsb) {
+            const typename W::X f = W::frag(sx, ss, sb, l);
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] += cur[r].dot(f, l);
+        }
+        if (last) {
+            float t = R == 2 ? wave_sum2(acc[0], acc[R - 1], lane) : wave_sum(acc[0]);
+            if (lane < (uint)R && row0 + lane < row_end) {
+                float* o = y + row0 + lane;
+                *o = ACC ? *o + t : t;
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] = 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) cur[r] = nxt[r];
+        sb = nsb_next;
+        row0 = nrow;
+    }
+}
+#define FQ8K_ONE(FMT, W, SUF, BF16, R)                                                                            \
+    extern "C" __global__ void __launch_bounds__(1024) gemv_fq8k_##FMT##_one##SUF##_r##R(                         \
+        const void* x, const uchar* w, float* y, uint K, uint N, uint NRB, uint ACC) {                            \
+        gemv_fq8k_one_body<R, W, BF16>(x, w, y, K, N, NRB, ACC);                                                  \
+    }
+#define FQ8K_ONES(FMT, W) FQ8K_ONE(FMT, W, , false, 1) FQ8K_ONE(FMT, W, , false, 2) FQ8K_ONE(FMT, W, _bf16, true, 1) FQ8K_ONE(FMT, W, _bf16, true, 2)
+FQ8K_ONES(q4k, One8<W4k>)
+FQ8K_ONES(q5k, One8<W5k>)
+FQ8K_ONES(q6k, One6)
 
 // ---- the fused launches for the other K-quants ---------------------------------------------------
 // A Q4_K_M file keeps some tensors of a stage in Q6_K or Q5_K (attention v, the feed-forward down) beside Q4_K ones;

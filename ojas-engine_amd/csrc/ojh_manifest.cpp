@@ -804,6 +804,28 @@ static int check_gemv_fq8k_x4(const ojh_kernel_spec *s, const uint32_t *c, const
     return OJH_OK;
 }
 
+// gemv_fq8k_<fmt>_one{,_bf16}_{r1,r2}(x, w, y, K, N, NRB, ACC): one tensor, f32 or bf16 activations
+static int check_gemv_fq8k_one(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3], const uint32_t block[3],
+                               size_t need[16], size_t align[16]) {
+    const ojh_block_format *f;
+    const uint32_t K = c[0], N = c[1], NRB = c[2], ACC = c[3];
+    int rc = check_kn(s, K, N, &f);
+    if (rc) return rc;
+    if (!block[0] || block[0] % 64 || block[0] > 1024 || block[1] != 1 || block[2] != 1)
+        return ojh_fail(OJH_ERR_ARG, "%s: block must be [x,1,1], x a multiple of 64 up to 1024", s->name);
+    if (K > 16384) return ojh_fail(OJH_ERR_ARG, "%s: K=%u exceeds 16384", s->name, K);
+    if (ACC > 1) return ojh_fail(OJH_ERR_ARG, "%s: ACC=%u", s->name, ACC);
+    if (!NRB) return ojh_fail(OJH_ERR_ARG, "%s: NRB must be positive", s->name);
+    if (grid[1] != 1 || grid[2] != 1 || (uint64_t)grid[0] * NRB < N || (uint64_t)grid[0] * NRB > 0xFFFFFFFFull)
+        return ojh_fail(OJH_ERR_ARG, "%s: grid x NRB does not cover N=%u rows", s->name, N);
+    need[0] = (size_t)K * (strstr(s->name, "bf16") ? 2 : 4);
+    need[1] = (size_t)N * (K / f->weights) * f->bytes;
+    need[2] = (size_t)N * 4;
+    align[1] = ojh_block_align(f);
+    align[2] = 4;
+    return OJH_OK;
+}
+
 // gemv_nat_<fmt>_m(x, w, y, K, N, M, ACC)
 static int check_gemv_nat_m(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3],
                             const uint32_t block[3], size_t need[16], size_t align[16]) {
@@ -2074,6 +2096,9 @@ static std::vector<ojh_kernel_spec> build_manifest() {
             add(fq + "_x4_r2", "gemv_q8k", 9, 7, f.type, 2, check_gemv_fq8k_x4, shape_rows);
         }
     }
+    for (uint32_t ty : {OJH_Q4_K, OJH_Q5_K, OJH_Q6_K})
+        for (const char *x : {"_one_r1", "_one_r2", "_one_bf16_r1", "_one_bf16_r2"})
+            add(std::string("gemv_fq8k_") + ojh_format(ty)->tag + x, "gemv_q8k", 3, 4, ty, x[strlen(x) - 1] - '0', check_gemv_fq8k_one, shape_rows);
     add("gemm_q8k_q4k_mf", "gemm_q8k", 4, 6, OJH_Q4_K, 1, check_gemm_q8k, shape_gemm_q8k);
     add("gemm_q8k_q4k_ml", "gemm_q8k", 4, 4, OJH_Q4_K, 1, check_gemm_q8k_ml, shape_ml);
     add("q8k_token_sides", "gemm_q8k", 4, 3, 0, 0, check_gemm_q8k_xt, shape_gemm_q8k_xt);

@@ -516,6 +516,9 @@ extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_bu
                       {ws[0]->k, ends[0], ends[1], ends[2], ends[3]}, grid, block);
 }
 
+static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w);
+static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum);
+
 // One stage of a decode layer in ONE launch: 1 to 4 projections of one f32 vector, the vector quantized inside the launch.
 extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int count, const ojh_lin *const *ws,
                             ojh_buf *const *ys, const size_t *y_offs, int accum) {
@@ -545,6 +548,8 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     // in flight as the plain matvec's thousands of small ones, and many small ones repeat the quantization too often.
     // OJAS_HIP_FQ_MULTI = 0 never takes it, 2 takes it at every size.
     const bool small_stage = total * K <= 32u * 1024u * 1024u && K <= 4096u;
+    if (count == 1 && !fused && dev->fq_multi && fq_one_taken(dev, ws[0]))
+        return fq_one_launch(dev, at(x, x_off), OJH_X_F32, ws[0], ojh_format(ws[0]->type), at(ys[0], y_offs ? y_offs[0] : 0), accum);
     if (!fused || K > 16384 || dev->fq_multi == 0 || (dev->fq_multi == 1 && !small_stage)) {   // quantize once, then the per-format launches
         size_t nsb = K / 256;
         ojh_buf *xq, *xs;
@@ -713,6 +718,32 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     }
     if (sk) return ojh_launch(dev, name, {xh->ptr, wdeq->ptr, yp}, {K, N, m, sg[1]}, sg, sb);
     return ojh_launch(dev, name, {xh->ptr, wdeq->ptr, yp}, {K, N, (uint32_t)(accum != 0), m}, sg, sb);
+}
+
+// One small K-quant projection of one token: quantizer and matvec in one launch.  It repeats the quantization in every
+// workgroup and keeps fewer bytes in flight than the plain matvec, so it stays with matrices whose second launch costs more.
+// Two launches / one, call to call, us: 1024 x 4096 Q4_K 8.0 / 4.4; 4096^2 Q4_K 7.8 / 4.6, Q5_K 7.9 / 5.1, Q6_K 7.8 / 6.0; 14336
+// x 4096 Q4_K 9.1 / 8.5, Q5_K 11.8 / 9.9, Q6_K 11.4 / 12.9 (8192 x 4096 8.5 / 8.8); 4096 x 8192 Q4_K 7.9 / 7.2, Q5_K 8.1 / 7.9,
+// Q6_K 8.7 / 9.0; 1024 x 8192 Q6_K 8.0 / 6.7; 1024 x 14336 Q4_K 8.0 / 8.2, Q5_K 8.3 / 8.7, Q6_K 8.0 / 9.5; where the host
+// issues a launch in 3 us instead of 4: 1024 x 4096 Q4_K 6.1 / 3.7, 3000 x 6144 6.1 / 5.2, 30000 x 1792 8.5 / 8.8, 12000 x 4096
+// Q5_K 10.6 / 8.9, 2000 x 8192 Q6_K 6.4 / 6.6.
+static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w) {
+    const uint64_t mi = ((uint64_t)w->n * w->k + (1u << 20) - 1) >> 20;
+    if (w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) return false;
+    if (dev->fq_one != 1) return dev->fq_one == 2 && w->k <= 16384u;
+    if (w->n >= 32768u) return false;              // (heads have forms of their own)
+    if (w->type == OJH_Q6_K) return mi <= (w->k <= 4096u ? 16u : w->k <= 8192u ? 8u : 0u);
+    return mi <= (w->k > 8192u ? 0u : w->k > 4096u ? 24u : w->type == OJH_Q5_K ? 56u : 32u);
+}
+static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum) {
+    const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
+    uint32_t nrb = (w->n + cus - 1) / cus;         // a workgroup of sixteen waves per CU; two rows a wave where it has more than one
+    const uint32_t r = nrb > 16 ? 2 : 1;
+    nrb = (nrb + r - 1) / r * r;
+    const uint32_t grid[3] = {(w->n + nrb - 1) / nrb, 1, 1}, block[3] = {1024, 1, 1};
+    const std::string name = std::string("gemv_fq8k_") + f->tag + (x_dtype == OJH_X_BF16 ? "_one_bf16_r" : "_one_r") + (r == 2 ? "2" : "1");
+    int rc = ensure(dev, "gemv_q8k");
+    return rc ? rc : ojh_launch(dev, name.c_str(), {xp, at(w->raw, w->off), yp}, {w->k, w->n, nrb, (uint32_t)(accum != 0)}, grid, block);
 }
 
 extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dtype, const ojh_lin *w, ojh_buf *y,
@@ -962,6 +993,7 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         grid[0] = (N + nrb - 1) / nrb;
         return ojh_launch(dev, name, {at(x, x_off), wp, yp}, {K, N, nrb}, grid, block);
     }
+    if (q8k && m == 1 && !bias && fq_one_taken(dev, w)) return fq_one_launch(dev, at(x, x_off), x_dtype, w, f, yp, accum);
     if (q8k) {
         if ((rc = ensure(dev, "gemv_q8k"))) return rc;
         size_t nsb = K / 256;

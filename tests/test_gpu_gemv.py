@@ -653,3 +653,64 @@ def test_q6k_head_form_keeps_activations_in_registers(gpu, orc, pkg, n, k):
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], got[1:-1])
     with pytest.raises(pkg.OjasHipError, match="8192"):
         gpu.dispatch(gpu.begin(), "gemv_q8k_q6k_px", [(xq, 0), (xs, 0), (wd, 0), (y2, 0)], [16384, n, 0][:2], [8, 1, 1], [256, 1, 1])
+
+
+@pytest.mark.parametrize("ty", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("n,k,nrb", [(1, 256, 1), (130, 2304, 5), (77, 1024, 40), (515, 4096, 33), (9, 16384, 9)])
+def test_one_projection_with_the_quantizer_inside_by_name(gpu, orc, pkg, ty, n, k, nrb):
+    """`gemv_fq8k_<fmt>_one{,_bf16}_{r1,r2}`: one super-block, odd counts, rows past a workgroup's waves, the longest K; plain
+    store and accumulate, NaN and infinities quantized as the quantizer launch does; bit-equal to the two launches."""
+    gpu.ensure_family("gemv_q8k")
+    raw, x = _inputs(pkg, ty, n, k, "one")
+    xb = pkg.synth.to_bf16_bits(x)
+    y0 = pkg.synth.normal_f32(n, "one", "y0")
+    lin, wd = gpu.lin(ty, n, k, raw), gpu.upload_bytes(raw)
+    for bf, odd in ((False, False), (True, False), (False, True)):
+        xf = pkg.synth.bf16_bits_to_f32(xb) if bf else x.copy()
+        if odd:
+            xf[3], xf[k - 5] = np.nan, np.inf
+        xq, xs, y1 = gpu.alloc_bytes(k), gpu.alloc(k // 256), gpu.alloc(n)
+        gpu.quant_q8k(gpu.upload(xf), 1, k, xq, xs)
+        gpu.mm_q8k(xq, xs, lin, y1)
+        two = gpu.read(y1, n)
+        for r in (1, 2):
+            for acc in (0, 1):
+                yd = gpu.upload(np.concatenate([y0, np.full(4, -7.25, np.float32)]))
+                gpu.dispatch(gpu.begin(), "gemv_fq8k_%s_one%s_r%d" % (TAG[ty], "_bf16" if bf else "", r),
+                             [(gpu.upload_bytes(xb.view(np.uint8)) if bf else gpu.upload(xf), 0), (wd, 0), (yd, 0)], [k, n, nrb, acc],
+                             [(n + nrb - 1) // nrb, 1, 1], [1024 if r == 1 else 192, 1, 1])
+                got = gpu.read(yd, n + 4)
+                assert np.all(got[n:] == -7.25)
+                if odd:
+                    assert np.array_equal(np.isfinite(got[:n]), np.isfinite(two))
+                elif acc:
+                    assert peak_err(got[:n] - y0, two) <= TOL_Q8K_SEEN
+                else:
+                    assert np.array_equal(got[:n].view(np.uint32), two.view(np.uint32))
+                    assert peak_err(got[:n], orc.matvec_kq(raw, ty, n, k, xf)) <= TOL_Q8K_SEEN
+
+
+@pytest.mark.parametrize("ty,n,k", [(Q4_K, 700, 4096), (Q5_K, 4100, 1024), (Q6_K, 33, 8192), (Q6_K, 4096, 4096)])
+def test_one_projection_routes_agree(pkg, monkeypatch, ty, n, k):
+    """`OJAS_HIP_FQ_ONE` off and on, f32 and bf16 tokens, through ojh_mm and ojh_mm_multi: the same bits."""
+    raw, x = _inputs(pkg, ty, n, k, "one-mm")
+    xb = pkg.synth.to_bf16_bits(x)
+    outs = []
+    for one in ("0", "1"):
+        monkeypatch.setenv("OJAS_HIP_FQ_ONE", one)
+        g = pkg.HipGpu(0)
+        try:
+            lin, xd, bd = g.lin(ty, n, k, raw), g.upload(x), g.upload_bytes(xb.view(np.uint8))
+            res = []
+            for f in (lambda y: g.mm(xd, lin, y, 1), lambda y: g.mm(bd, lin, y, 1, x_dtype=pkg.X_BF16), lambda y: g.mm_multi(xd, [lin], [y]),
+                      lambda y: g.mm(xd, lin, y, 1, accum=True)):
+                y = g.upload(np.full(n + 4, 0.5, np.float32))
+                f(y)
+                got = g.read(y, n + 4)
+                assert np.all(got[n:] == 0.5)
+                res.append(got[:n])
+            outs.append(res)
+        finally:
+            g.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
