@@ -285,7 +285,7 @@ struct LoaderIQ4NL {
     __device__ __forceinline__ void part() {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const uint lv = iq4_levels4((q[I] >> (4 * s)) & 0x0F0F0F0Fu);
+            const uint lv = s ? iq4_levels_of<1>(q[I]) : iq4_levels_of<0>(q[I]);
             float v0 = __fmul_rn(d, (float)(signed char)(lv)), v1 = __fmul_rn(d, (float)(signed char)(lv >> 8));
             float v2 = __fmul_rn(d, (float)(signed char)(lv >> 16)), v3 = __fmul_rn(d, (float)((int)lv >> 24));
             o[8 * s + 2 * I] = pack2(v0, v1);
@@ -327,7 +327,7 @@ struct LoaderIQ4XS {
     __device__ __forceinline__ void part() {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const uint lv = iq4_levels4((q[I] >> (4 * s)) & 0x0F0F0F0Fu);
+            const uint lv = s ? iq4_levels_of<1>(q[I]) : iq4_levels_of<0>(q[I]);
             float v0 = __fmul_rn(d, (float)(signed char)(lv)), v1 = __fmul_rn(d, (float)(signed char)(lv >> 8));
             float v2 = __fmul_rn(d, (float)(signed char)(lv >> 16)), v3 = __fmul_rn(d, (float)((int)lv >> 24));
             o[8 * s + 2 * I] = pack2(v0, v1);
@@ -631,10 +631,12 @@ struct LoaderQ4L {
 // which row of x and of y token m of the launch is: itself, or (grouped expert products) an entry of a list — the
 // activation row that entry divided by DIV (an assignment's token), the output row the entry itself
 struct GmDense {
+    static constexpr bool FRAG = true;       // (the few-token kernel may read its activations in fragment order)
     __device__ __forceinline__ uint in_row(uint m) const { return m; }
     __device__ __forceinline__ uint out_row(uint m) const { return m; }
 };
 struct GmList {
+    static constexpr bool FRAG = false;
     const uint* lst;
     uint last, div;
     __device__ __forceinline__ uint out_row(uint m) const { return min(lst[m], last); }
@@ -854,12 +856,17 @@ GEMM_ENTRIES(q3k, LoaderQ3K)
 // of token m.  Up to 16 TG tokens per launch (TG accumulators); partial sums of the waves meet in LDS in wave order (eight
 // waves on four slots: wave w adds wave w + 4's to its own first).
 //   gemm_few_<fmt>{,_r4}_t{1,2,4}(xh, w, y, K, N, accum, M)     grid [ceil(N / 16 RG),1,1] x 256 (or 512 where RG TG <= 8),
-//   K a multiple of 128, M <= 16 TG; `_r4`: RG = 4 groups of 16 rows per workgroup
+//   K a multiple of 128, M <= 16 TG; `_r4`: RG = 4 groups of 16 rows per workgroup; accum 1: y += ; accum 2 (or 3): xh in the
+//   order of few_x_{f32,bf16}
 // Bound by latency: a wave waits a trip to memory per chunk for its tokens and the next block, and with 64 rows a workgroup
 // there is less than one workgroup per CU on most matrices.  So `_r4_t2` runs eight waves where there are fewer than two
 // workgroups per CU, each with half the chunks; the kernel alone, four -> eight waves, us: IQ4_XS 14336 x 4096 at 17 / 32 tokens
 // 20.0 -> 16.0 / 22.1 -> 18.9, x 14336 69.9 -> 48.7 / 76.6 -> 56.0, 28672 x 4096 31.2 -> 30.0 / 36.0 -> 35.6; Q8_0, whose
 // bytes bound it sooner, 0 - 2 % (30.4 -> 29.6 at 14336 x 4096), never slower up to 32640 rows.
+// Row by row, a load of the tokens' pieces touches 64 lines for 16 bytes each and the address unit walks them one by one: 7 of
+// the 16 us of 24 tokens.  In fragment order (few_x_*) it is 1 KB in a row, and the next chunk's is asked for while this one's
+// rows are decoded.  With the conversion, us: IQ4_XS 14336 x 4096 at 24 tokens 19.5 -> 17.8, 4096^2 at 24 11.7 -> 8.5, 4096 x
+// 14336 at 16 20.1 -> 15.4, Q8_0 14336 x 4096 at 24 32.4 -> 28.9.  Now bound by the decoding's vector instructions (5 a weight).
 typedef float float4v __attribute__((ext_vector_type(4)));
 template <int J, class L>
 __device__ __forceinline__ half8 gm_frag(const L& ld) {
@@ -882,9 +889,14 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
     const uchar* wrow[RG];
 #pragma unroll
     for (int r = 0; r < RG; r++) wrow[r] = w + (size_t)min(n0 + 16u * r + i16, N - 1u) * rb;
+    // a lane's four pieces of a chunk of its token: 64 bytes of the token's row, or pieces 1 KB apart in fragment order
+    const bool frag = TM::FRAG && (accum & 2u) != 0u;
+    const uint xc = frag ? 2048u * TG : 128u, xj = frag ? 512u : 8u;
+    accum &= 1u;
     const ushort* xrow[TG];
 #pragma unroll
-    for (int tg = 0; tg < TG; tg++) xrow[tg] = xh + (size_t)tm.in_row(min(16u * tg + i16, M - 1u)) * K + g * 32u;
+    for (int tg = 0; tg < TG; tg++)
+        xrow[tg] = frag ? xh + 2048u * tg + 8u * lane : xh + (size_t)tm.in_row(min(16u * tg + i16, M - 1u)) * K + g * 32u;
     float4v acc[RG][TG];
 #pragma unroll
     for (int r = 0; r < RG; r++)
@@ -906,24 +918,24 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
             acc[R][tg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[tg][3], gm_frag<3>(CUR), acc[R][tg], 0, 0, 0);  \
         }                                                                                                         \
     } while (0)
+#define GF_X(XV, C)                                                                                               \
+    _Pragma("unroll") for (int tg = 0; tg < TG; tg++)                                                             \
+        _Pragma("unroll") for (int j = 0; j < 4; j++) XV[tg][j] = *(const half8*)(xrow[tg] + (C) * xc + xj * j)
     uint c = wave;
     if (c < nchunk) ld0.load(wrow[0], c * 128u + g * 32u, 0u);
+    half8 xv[TG][4];
+    if (c < nchunk) GF_X(xv, c);
     for (; c < nchunk; c += nw) {
-        half8 xv[TG][4];
-#pragma unroll
-        for (int tg = 0; tg < TG; tg++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) xv[tg][j] = *(const half8*)(xrow[tg] + c * 128u + 8u * j);
+        half8 xn[TG][4];
+        if (RG > 1 && c + nw < nchunk) GF_X(xn, c + nw);          // (the next chunk's tokens travel while this one's rows are decoded)
         if (RG == 1) {
             // (two chunks per trip so that the loaders alternate by name)
             GF_GROUP(ld0, ld1, 0, wrow[0], c + nw);
             c += nw;
             if (c < nchunk) {
-#pragma unroll
-                for (int tg = 0; tg < TG; tg++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) xv[tg][j] = *(const half8*)(xrow[tg] + c * 128u + 8u * j);
+                GF_X(xv, c);
                 GF_GROUP(ld1, ld0, 0, wrow[0], c + nw);
+                if (c + nw < nchunk) GF_X(xv, c + nw);
             }
         } else {
 #pragma unroll
@@ -931,8 +943,13 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
                 GF_GROUP(ld0, ld1, r, wrow[r + 1 < RG ? r + 1 : 0], c);
                 GF_GROUP(ld1, ld0, r + 1 < RG ? r + 1 : 0, wrow[r + 2 < RG ? r + 2 : 0], r + 2 < RG ? c : c + nw);
             }
+#pragma unroll
+            for (int tg = 0; tg < TG; tg++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) xv[tg][j] = xn[tg][j];
         }
     }
+#undef GF_X
 #undef GF_GROUP
     // D: lane (n = lane % 16, g) holds tokens 4 g + v of its group against row n
 #define GF_SLOT(W) red[W][r * TG + tg][(g * 4u + v) * 16u + i16]
@@ -969,6 +986,29 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
     GEMM_FEW_ENTRY(FMT, LOADER, _r4_t1, 1, 4)                                                                     \
     GEMM_FEW_ENTRY(FMT, LOADER, _r4_t2, 2, 4)                                                                     \
     GEMM_FEW_ENTRY(FMT, LOADER, _r4_t4, 4, 4)
+// few_x_{f32,bf16}(x, xh, K, M, TG): M <= 16 TG tokens to f16 in the order in which a chunk's fragments are read — piece (chunk c,
+// token group tg, j, lane) at ((c TG + tg) 4 + j) 64 + lane holds positions 128 c + 32 (lane / 16) + 8 j .. + 7 of token 16 tg +
+// lane % 16 (the last token again past M).  grid [ceil(K TG / 128)] x 256, a piece a thread.
+template <bool BF16>
+__device__ __forceinline__ void few_x_body(const void* __restrict__ x, ushort* __restrict__ xh, uint K, uint M, uint TG) {
+    const uint p = blockIdx.x * 256u + threadIdx.x, lane = p & 63u, q = p >> 6, j = q & 3u, ct = q >> 2, c = ct / TG, tg = ct - c * TG;
+    if (c >= K >> 7) return;
+    const size_t at = (size_t)min(16u * tg + (lane & 15u), M - 1u) * K + 128u * c + 32u * (lane >> 4) + 8u * j;
+    uint o[4];
+    if (BF16) {
+        const uint4 b = *(const uint4*)((const ushort*)x + at);
+        const uint v[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = pack2(__uint_as_float(v[e] << 16), __uint_as_float(v[e] & 0xFFFF0000u));
+    } else {
+        const float4 a = *(const float4*)((const float*)x + at), b = *(const float4*)((const float*)x + at + 4);
+        o[0] = pack2(a.x, a.y); o[1] = pack2(a.z, a.w); o[2] = pack2(b.x, b.y); o[3] = pack2(b.z, b.w);
+    }
+    *(uint4*)(xh + (size_t)p * 8u) = make_uint4(o[0], o[1], o[2], o[3]);
+}
+extern "C" __global__ void __launch_bounds__(256) few_x_f32(const float* x, ushort* xh, uint K, uint M, uint TG) { few_x_body<false>(x, xh, K, M, TG); }
+extern "C" __global__ void __launch_bounds__(256) few_x_bf16(const ushort* x, ushort* xh, uint K, uint M, uint TG) { few_x_body<true>(x, xh, K, M, TG); }
+
 GEMM_FEW_ENTRIES(q8_0, LoaderQ80)
 GEMM_FEW_ENTRIES(f16, LoaderF16)
 GEMM_FEW_ENTRIES(iq4nl, LoaderIQ4NL)

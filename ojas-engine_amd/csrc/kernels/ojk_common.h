@@ -241,6 +241,19 @@ __device__ __forceinline__ uint iq4_levels4(uint idx4) {
     return (hi & mask) | (lo & ~mask);
 }
 
+// The levels of the four low (HI = 0) or high nibbles of a dword of code bytes, straight from it: a byte-permute that repeats
+// bytes' sign bits makes the mask of the indices from 8 on (selectors 8 .. 11: the signs of bytes 1, 3, 5, 7), seven
+// instructions instead of nine or ten.
+template <int HI>
+__device__ __forceinline__ uint iq4_levels_of(uint q) {
+    const uint sel = (HI ? q >> 4 : q) & 0x07070707u;
+    const uint v = HI ? q : q << 4;                                         // bit 3 of every index as its byte's sign
+    const uint lo = __builtin_amdgcn_perm(0xF6EADDCFu, 0xBFAD9881u, sel);
+    const uint hi = __builtin_amdgcn_perm(0x71594535u, 0x26190D01u, sel);
+    const uint mask = __builtin_amdgcn_perm(v << 8, v, 0x090B080Au);
+    return (hi & mask) | (lo & ~mask);
+}
+
 // ---- global -> LDS copies by the memory system ------------------------------------------------
 // One instruction moves 16 bytes per lane from base + voff to LDS bytes lds_addr + 16 lane .. (1 KB
 // per wave, contiguous in LDS whatever the global addresses; lds_addr is the same in every lane).

@@ -1437,18 +1437,39 @@ static int check_gemm_few(const ojh_kernel_spec *s, const uint32_t *c, const uin
         return rc;
     }
     if (K % 128) return ojh_fail(OJH_ERR_ARG, "%s: K=%u must be a multiple of 128", s->name, K);
+    if (c[2] > 3) return ojh_fail(OJH_ERR_ARG, "%s: accum=%u, takes 0 to 3", s->name, c[2]);
     if (!M || M > 16 * TG) return ojh_fail(OJH_ERR_ARG, "%s: M=%u, takes 1 to %u tokens", s->name, M, 16 * TG);
     if (block[0] != 256 && !(block[0] == 512 && RG * TG <= 8))
         return ojh_fail(OJH_ERR_ARG, "%s: block must be 256%s threads", s->name, RG * TG <= 8 ? " or 512" : "");
     if (block[1] != 1 || block[2] != 1) return ojh_fail(OJH_ERR_ARG, "%s: block must be [x,1,1]", s->name);
     if (grid[0] != (N + 16 * RG - 1) / (16 * RG) || grid[1] != 1 || grid[2] != 1)
         return ojh_fail(OJH_ERR_ARG, "%s: grid must be [%u,1,1]", s->name, (N + 16 * RG - 1) / (16 * RG));
-    need[0] = (size_t)M * K * 2;
+    need[0] = (size_t)(c[2] & 2 ? 16 * TG : M) * K * 2;
     need[1] = (size_t)N * (K / f->weights) * f->bytes;
     need[2] = (size_t)M * N * 4;
     align[0] = 16;
     align[1] = s->type == OJH_F16 ? 16 : ojh_block_align(f);
     align[2] = 4;
+    return OJH_OK;
+}
+// few_x_{f32,bf16}(x, xh, K, M, TG)
+static int check_few_x(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t grid[3], const uint32_t block[3], size_t need[16],
+                       size_t align[16]) {
+    const uint32_t K = c[0], M = c[1], TG = c[2];
+    if (!K || K % 128 || !TG || TG > 4 || !M || M > 16 * TG) return ojh_fail(OJH_ERR_ARG, "%s: K=%u (a multiple of 128) M=%u TG=%u (1 to 4)", s->name, K, M, TG);
+    int rc = check_block(block, 256);
+    if (rc) return rc;
+    if (grid[0] != K / 128 * TG || grid[1] != 1 || grid[2] != 1) return ojh_fail(OJH_ERR_ARG, "%s: grid must be [%u,1,1]", s->name, K / 128 * TG);
+    need[0] = (size_t)M * K * (s->rows_per_wave == 2 ? 2 : 4);
+    need[1] = (size_t)16 * TG * K * 2;
+    align[0] = align[1] = 16;
+    return OJH_OK;
+}
+static int shape_few_x(const ojh_kernel_spec *, const ojh_device *, uint32_t K, uint32_t, uint32_t M, uint32_t grid[3], uint32_t block[3]) {
+    grid[0] = K / 128 * (M <= 16 ? 1 : M <= 32 ? 2 : 4);
+    grid[1] = grid[2] = 1;
+    block[0] = 256;
+    block[1] = block[2] = 1;
     return OJH_OK;
 }
 static int shape_gemm_few(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t, uint32_t N, uint32_t,
@@ -2186,6 +2207,8 @@ static std::vector<ojh_kernel_spec> build_manifest() {
             add(g + "_r4_t" + std::to_string(tg), "gemm", 3, 4, t, 64 + tg, check_gemm_few, shape_gemm_few);
         }
     }
+    add("few_x_f32", "gemm", 2, 3, 0, 4, check_few_x, shape_few_x);
+    add("few_x_bf16", "gemm", 2, 3, 0, 2, check_few_x, shape_few_x);
     // plain f16 rows on the same tile: what every format without a tile of its own is decoded into ahead of a batch
     add("gemm_mm_f16", "gemm", 3, 4, OJH_F16, 0, check_gemm, shape_gemm);
     add("gemm_mm_f16_sk", "gemm", 3, 4, OJH_F16, 1, check_gemm, shape_gemm);

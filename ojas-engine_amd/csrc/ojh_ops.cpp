@@ -873,8 +873,13 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         const bool xl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT &&
                         (uint64_t)w->row_bytes * N <= 0xFFFFFFFFull;  // 32-bit row offsets in that tile
         if ((rc = ensure(dev, "glue")) || (rc = ensure(dev, xl ? "gemm_xl" : "gemm"))) return rc;
+        // (the few-token kernel below reads the tokens' f16 copy in the order of its lanes where there is room for whole
+        // groups of sixteen tokens, row by row otherwise)
+        const uint32_t few_tg = m <= 16 ? 1 : m <= 32 ? 2 : 4;
         ojh_buf *xh;
-        if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
+        const bool few_frag = !xl && !deq_tile && dev->gemm_few && m <= dev->gemm_few && m <= 64 && K % 128 == 0 && (own_loader || w->type == OJH_Q8_0) &&
+                              !ojh_scratch_spare(dev, "xh", (size_t)16 * few_tg * K * 2, &xh);
+        if (!few_frag && (rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
         const uint32_t n_el = m * K, conv_blocks = (n_el / 8 + 255) / 256 + 1;
         std::string base = std::string("gemm_mm_") + (deq_tile ? "f16" : w->type == OJH_Q8_0 ? "q8_0" : f->tag);
         // (the tile that shares the dequantized weights through LDS is 256 tokens tall; its 128-token form up to 128 tokens
@@ -905,20 +910,24 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         // (`gemm_few_*`; 14336 x 4096 at 8 / 16 / 32 tokens, kernel alone: IQ4_XS 14 / 15 / 23 us against 30 of the tile,
         // Q8_0 26 / 28 / 32 against 36; 4096 x 4096 IQ4_XS 7 / 9 / 11 against 12 .. 14).  Four row groups per workgroup where
         // that still gives most CUs a workgroup: the tokens' bytes, re-read by every workgroup, are most of its traffic.
-        // (with 16 rows per workgroup a long K costs more: up to 16 tokens there; Q8_0, twice the bytes per weight, only
-        // where the tile is no better — 4096 x 14336 at 32 tokens: IQ4_XS 34 against 31 us, Q8_0 48 against 36)
+        // (with 16 rows per workgroup a long K costs more, and below 2048 rows there are few of them: up to 16 tokens there, and
+        // none for Q8_0, twice the bytes per weight, nor more for Q3_K, eight loads at 2-byte alignment.  Tile / this kernel
+        // beyond, us: 4096 x 14336 at 24 tokens IQ4_XS 29.1 / 18.4, at 30 Q4_0 30.3 / 23.4, Q5_1 31.6 / 21.4, Q2_K 32.1 / 21.8, MXFP4
+        // 29.7 / 21.3, Q3_K 40.7 / 40.4; 2048 x 8192 IQ4_XS at 24 13.9 / 12.8; 1024 x 8192 at 24 Q4_0 13.4 / 14.6, Q2_K 13.9 / 15.5;
+        // Q8_0 4096^2 at 32 16.9 / 12.2, 2048 x 4096 at 32 13.0 / 11.8, 1024 x 4096 at 24 10.7 / 11.5, 2048 x 8192 at 12 14.4 / 17.5)
         const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
         const bool r4 = (uint64_t)(N + 63) / 64 * 4 >= 3ull * cus;
-        const uint32_t few_cap = r4 ? dev->gemm_few : K > 4096 ? (w->type == OJH_Q8_0 ? 0u : 16u) : w->type == OJH_Q8_0 ? 16u : dev->gemm_few;
+        const bool few_long = N >= 2048 ? w->type != OJH_Q3_K || K <= 4096 : w->type != OJH_Q8_0 && K <= 4096;
+        const uint32_t few_cap = r4 ? dev->gemm_few : w->type == OJH_Q8_0 && K > 4096 ? 0u : few_long ? dev->gemm_few : std::min(dev->gemm_few, 16u);
         if (dev->gemm_few && !xl && !deq_tile && (own_loader || w->type == OJH_Q8_0) && m <= few_cap && m <= 64 && K % 128 == 0) {
             const std::string few = std::string("gemm_few_") + (w->type == OJH_Q8_0 ? "q8_0" : f->tag) + (r4 ? "_r4" : "") +
                                     (m <= 16 ? "_t1" : m <= 32 ? "_t2" : "_t4");
-            uint32_t fg[3], fb[3], eg[3] = {conv_blocks, 1, 1};
+            uint32_t fg[3], fb[3], eg[3] = {few_frag ? K / 128 * few_tg : conv_blocks, 1, 1};
             if ((rc = ojh_launch_shape(dev, few.c_str(), K, N, m, fg, fb))) return rc;
-            if ((rc = ojh_launch(dev, x_dtype == OJH_X_BF16 ? "copy_bf16_half" : "copy_f32_half", {at(x, x_off), xh->ptr},
-                                 {n_el}, eg, block)))
+            if ((rc = few_frag ? ojh_launch(dev, x_dtype == OJH_X_BF16 ? "few_x_bf16" : "few_x_f32", {at(x, x_off), xh->ptr}, {K, m, few_tg}, eg, block)
+                               : ojh_launch(dev, x_dtype == OJH_X_BF16 ? "copy_bf16_half" : "copy_f32_half", {at(x, x_off), xh->ptr}, {n_el}, eg, block)))
                 return rc;
-            return ojh_launch(dev, few.c_str(), {xh->ptr, wp, yp}, {K, N, (uint32_t)(accum != 0), m}, fg, fb);
+            return ojh_launch(dev, few.c_str(), {xh->ptr, wp, yp}, {K, N, (few_frag ? 2u : 0u) | (uint32_t)(accum != 0), m}, fg, fb);
         }
         uint32_t sg[3], sb[3];
         if ((rc = ojh_launch_shape(dev, (base + "_sk").c_str(), K, N, m, sg, sb))) return rc;

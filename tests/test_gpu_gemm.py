@@ -450,6 +450,38 @@ def test_few_token_kernel_with_eight_waves_on_four_slots(gpu, orc, pkg, ty, tag,
     assert peak_err(got, x.astype(np.float64).reshape(m, k) @ wf.T) <= (2e-5 if accum else 2e-6)
 
 
+@pytest.mark.parametrize("suf,rg,tg", [("_t1", 1, 1), ("_t2", 1, 2), ("_r4_t1", 4, 1), ("_r4_t2", 4, 2), ("_r4_t4", 4, 4)])
+@pytest.mark.parametrize("ty,tag", [(23, "iq4xs"), (8, "q8_0"), (2, "q40")])
+@pytest.mark.parametrize("frac,k,n,accum,bf16", [(1, 256, 17, 0, 0), (16, 1280, 130, 1, 1), (9, 2304, 65, 0, 1)])
+def test_few_token_kernel_on_tokens_in_fragment_order(gpu, orc, pkg, suf, rg, tg, ty, tag, frac, k, n, accum, bf16):
+    """`few_x_{f32,bf16}` and `gemm_few_*` with accum 2 / 3: the order itself, the last token repeated past M, nothing written
+    past whole groups of sixteen tokens; and the products, bit-equal to those on tokens row by row."""
+    m = 16 * (tg - 1) + frac
+    gpu.ensure_family("gemm")
+    gpu.ensure_family("glue")
+    raw = pkg.synth.weights(ty, n, k, "frag", tag, n, k)
+    x = pkg.synth.normal_f32(m * k, "frag", "x", m, k)
+    xb = pkg.synth.to_bf16_bits(x) if bf16 else x
+    if bf16:
+        x = pkg.synth.bf16_bits_to_f32(xb)
+    x16 = x.astype(np.float16).reshape(m, k)
+    xh = gpu.upload(np.full(16 * tg * k // 2 + 16, 7.5, np.float32))
+    gpu.dispatch(gpu.begin(), "few_x_bf16" if bf16 else "few_x_f32", [(gpu.upload_bytes(xb.view(np.uint8)), 0), (xh, 0)], [k, m, tg], [k // 128 * tg, 1, 1], [256, 1, 1])
+    whole = np.concatenate([x16, np.repeat(x16[-1:], 16 * tg - m, 0)])
+    order = whole.reshape(tg, 16, k // 128, 4, 4, 8).transpose(2, 0, 4, 3, 1, 5)      # [chunk][group][j][k group][token][8]
+    assert np.array_equal(gpu.read(xh, 16 * tg * k, np.uint16), order.ravel().view(np.uint16))
+    assert np.all(gpu.read(xh, 16 * tg * k // 2 + 16)[-16:] == 7.5)
+    wd, rows = gpu.upload_bytes(raw), gpu.upload_bytes(x16.view(np.uint8).ravel())
+    outs = []
+    for xd, flag in ((rows, 0), (xh, 2)):
+        y0 = pkg.synth.normal_f32(m * n, "frag", "y0")
+        yd = gpu.upload(np.concatenate([y0, np.full(n, 4242.5, np.float32)]))
+        gpu.dispatch(gpu.begin(), "gemm_few_%s%s" % (tag, suf), [(xd, 0), (wd, 0), (yd, 0)], [k, n, flag | accum, m], [(n + 16 * rg - 1) // (16 * rg), 1, 1], [256, 1, 1])
+        outs.append(gpu.read(yd, m * n + n))
+        assert np.all(outs[-1][m * n:] == np.float32(4242.5))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("kernel,bm,bn", [("gemm_f16d_128", 128, 128), ("gemm_f16d_256x128", 256, 128), ("gemm_f16d_256", 256, 256),
                                           ("gemm_f16d_128_sk", 128, 128)])
 @pytest.mark.parametrize("m,k,n,accum", [(1, 64, 1, False), (129, 128, 127, True), (257, 192, 1100, False), (300, 1088, 385, True)])
