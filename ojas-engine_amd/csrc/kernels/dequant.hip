@@ -101,6 +101,27 @@ __device__ __forceinline__ void decode_q4k(const uchar* __restrict__ w, ushort* 
     store8_f16(out + b * 256u + c * 64u + hi * 32u + part * 8u, h);
 }
 
+// ... with the weights of the Q4_K prefill tiles (the reference GPU kernel's, crates/ojas-formats/src/quant.rs:192-222): one f16
+// fma q qa + qb a weight, qa = f16(d * sc), qb = f16(-dmin * m).
+__device__ __forceinline__ void decode_q4kl(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
+    size_t b = tid >> 5;
+    if (b >= nblocks) return;
+    const uint t = (uint)tid & 31u, c = t >> 3, hi = (t >> 2) & 1u, part = t & 3u;
+    const uint* hdr = (const uint*)(w + b * Q4K_BYTES);
+    const uint dd = hdr[0];
+    const float d = f16_bits_to_f32(dd & 0xFFFFu), ndm = -f16_bits_to_f32(dd >> 16);
+    uint sc, mn;
+    q4k_scale_min_pair(hdr[1], hdr[2], hdr[3], c, sc, mn);
+    const __half qa = __ushort_as_half(f32_to_f16_bits(__fmul_rn(d, (float)(hi ? sc >> 8 : sc & 0xFFu))));
+    const __half qb = __ushort_as_half(f32_to_f16_bits(__fmul_rn(ndm, (float)(hi ? mn >> 8 : mn & 0xFFu))));
+    const uint q0 = (hdr[4u + c * 8u + 2u * part] >> (4u * hi)) & 0x0F0F0F0Fu;
+    const uint q1 = (hdr[5u + c * 8u + 2u * part] >> (4u * hi)) & 0x0F0F0F0Fu;
+    ushort h[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = __half_as_ushort(__hfma(__ushort2half_rn((ushort)byte_of(q0, q1, i)), qa, qb));
+    store8_f16(out + b * 256u + c * 64u + hi * 32u + part * 8u, h);
+}
+
 __device__ __forceinline__ void decode_q5k(const uchar* __restrict__ w, ushort* __restrict__ out, uint nblocks, size_t tid) {
     // As Q4_K, plus the fifth bit: bit 2 c + hi of qh[l], l the byte's place among the chunk's 32.
     size_t b = tid >> 5;
@@ -347,6 +368,7 @@ __device__ __forceinline__ void decode_beside(F decode, const void* __restrict__
     }
 DEQUANT_ENTRIES(q80, decode_q80)
 DEQUANT_ENTRIES(q4k, decode_q4k)
+DEQUANT_ENTRIES(q4kl, decode_q4kl)
 DEQUANT_ENTRIES(q5k, decode_q5k)
 DEQUANT_ENTRIES(q6k, decode_q6k)
 DEQUANT_ENTRIES(iq4nl, decode_iq4nl)

@@ -2058,6 +2058,10 @@ static std::vector<ojh_kernel_spec> build_manifest() {
         const char *fam_nat = grid_fmt ? "iq_grid" : "gemv", *fam_q8k = grid_fmt ? "iq_grid" : "gemv_q8k";
         add("dequant_" + t + "_f16", grid_fmt ? "iq_grid" : "dequant", 2, 1, f.type, 0, check_dequant, shape_dequant);
         if (!grid_fmt) add("dequant_" + t + "_f16_x", "dequant", 5, 5, f.type, 0, check_dequant_x, shape_dequant_x);
+        if (f.type == OJH_Q4_K) {
+            add("dequant_q4kl_f16", "dequant", 2, 1, f.type, 0, check_dequant, shape_dequant);
+            add("dequant_q4kl_f16_x", "dequant", 5, 5, f.type, 0, check_dequant_x, shape_dequant_x);
+        }
         if (f.type == OJH_Q5_K) {   // Q5_K: the decoder, the CPU path's int8-activation matvec
             std::string q5 = "gemv_q8k_" + t;
             add(q5, "gemv_q8k", 4, 2, f.type, 4, check_gemv_q8k, shape_rows);

@@ -642,9 +642,41 @@ static bool f16d_pays(const ojh_device *dev, const ojh_lin *w, uint32_t m, bool 
     const double loaded = gemm_mm_m128(dev, N, m, false) ? walk(128, 128, K / 256, s128, 0.0) : 3.5 + walk(256, 128, K / 256, s256, 0.0);
     return 0.42 * mi + (mi > 56 ? 0.5 * (mi - 56) : 0.0) + copied < loaded;
 }
+// Q4_K rows have tiles that dequantize straight into the matrix operand, far cheaper loaders than the other formats': decoding
+// first pays where those tiles leave CUs idle or K slices have to meet through atomics, mostly below 3000 rows, and where a
+// long K amortizes the pass.  Both priced as above, the terms fitted to 3031 pairs of timed calls (512 - 32768 rows, K 1024 -
+// 14336, 200 - 2048 tokens; median error 2 - 5 %), and taken where ahead by a twentieth: 652 of the pairs, on average 16 %
+// faster, six of them more than 3 % slower.  Tiles / pass + copying tile, us: 1088 x 2304 at 1944 tokens 39.8 / 26.9, 2752 x
+// 6912 at 768 78.7 / 54.7, 4096 x 4096 at 1024 56.7 / 49.4, 4096 x 14336 at 2048 264 / 250, 6914 x 2816 at 333 39.2 / 33.1;
+// kept: 14336 x 4096 at 512 70 / 93, at 2048 235 / 255, 28534 x 12288 at 241 202 / 427.  The pass forms the tiles' weights
+// (dequant_q4kl_f16_x: f16 q qa + qb).
+static bool f16d_pays_q4k(const ojh_device *dev, uint32_t N, uint32_t K, uint32_t m) {
+    const double cus = dev->prop.multiProcessorCount, mi = (double)N * K / (1 << 20), mk = (double)m * K / (1 << 20), mn = (double)m * N / (1 << 20);
+    struct Price { double fixed, acts, round, fill, meet, out, start; };
+    auto price = [&](uint32_t bm, uint32_t bn, uint32_t most, const Price &p) {
+        const uint64_t tiles = (uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm);
+        const uint32_t z = most ? ojh_gemm_slices(dev, tiles, most) : 1u;
+        const double per_cu = tiles * z / cus, steps = (K / 64 + z - 1) / z;
+        return p.fixed + p.acts * mk + steps * (p.round * ceil(per_cu) + p.fill * per_cu) + (z > 1 ? p.meet * z * mn : 0.0) + p.out * mn + p.start * ceil(per_cu);
+    };
+    const double over = mi > 56 ? mi - 56 : 0.0;
+    const uint32_t tile = f16d_tile(dev, N, m);
+    const double copied = tile == 2   ? 0.345 * mi + 0.481 * over + price(256, 256, 0, {2.2, 0.24, 0.827, 0.802, 0.0, 0.50, 8.9})
+                          : tile == 1 ? 0.263 * mi + 0.735 * over + price(256, 128, 0, {6.5, 0.06, 0.306, 0.547, 0.0, 0.68, 5.8})
+                                      : 0.422 * mi + 0.684 * over + price(128, 128, K / 512, {7.5, 0.77, 0.173, 0.218, 3.59, 1.92, 0.35});
+    // the tile that ojh_mm takes otherwise
+    const uint64_t t256 = (uint64_t)((N + 255) / 256) * ((m + 255) / 256), t128 = (uint64_t)((N + 255) / 256) * ((m + 127) / 128);
+    const uint32_t z128 = (uint32_t)((uint64_t)cus / t128);
+    const bool tall = t256 >= (uint64_t)cus || (2 * t256 >= (uint64_t)cus && K >= 8192);
+    const double loaded = !tall && K >= 1024 && z128 >= 2 && (K <= 8192 || z128 >= 4) ? price(128, 64, K / 1024, {4.4, 1.26, 0.215, 0.037, 3.01, 1.33, 4.7})
+                          : tall ? price(256, 256, K / 256, {5.3, 0.64, 1.059, 0.683, 2.29, 0.39, 5.2})
+                                 : price(128, 256, K / 256, {11.4, 0.75, 0.436, 0.509, 2.24, 0.15, 0.0});
+    return 1.05 * copied < loaded;
+}
 static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
     const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
-    if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || q4kl || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
+    if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
+    if (q4kl && (dev->deq_big_m != 1 || dev->gemm_bdk != 1 || dev->gemm_sr || m < 257 || w->n < 512 || w->k < 1024 || !f16d_pays_q4k(dev, w->n, w->k, m))) return false;
     // while a graph is recorded nothing can be loaded or grown: what is not there yet leaves the call on the tile it has
     if (dev->capturing) {
         const auto slot = dev->scratch.find("wdeq");
@@ -657,6 +689,7 @@ static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int 
         if (w->type == OJH_Q4_K || (kq && (uint64_t)w->n * w->k < (32ull << 20))) return false;
         return m >= (w->type == OJH_Q5_K || w->type == OJH_Q8_0 ? 2 * dev->deq_big_m : dev->deq_big_m);
     }
+    if (q4kl) return true;                                     // (priced above)
     // (129 to 256 tokens are two tiles of 128, the second part empty: the two routes are within the prices' error of each
     // other there for the lighter loaders, whose rows then need no scratch)
     return m >= (decoded || w->type == OJH_Q6_K ? 129u : 257u) && f16d_pays(dev, w, m, decoded);
@@ -675,7 +708,7 @@ static int f16d_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, bool decode
     return OJH_OK;
 }
 static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, uint32_t m,
-                       int accum) {
+                       int accum, bool q4kl) {
     const uint32_t K = w->k, N = w->n, tile = f16d_tile(dev, N, m);
     const bool grid_fmt = ojh_grid_type(w->type);
     int rc;
@@ -698,7 +731,7 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     const uint32_t n_el = m * K, nz = sk && !accum ? m * N : 0, nb = (uint32_t)((uint64_t)N * K / f->weights);
     const uint32_t cb = (uint32_t)(((uint64_t)n_el / 8 + nz / 4 + 255) / 256 + 1);
     uint32_t dg[3], db[3];
-    const std::string dq = std::string("dequant_") + f->tag + "_f16";
+    const std::string dq = std::string("dequant_") + f->tag + (q4kl ? "l_f16" : "_f16");
     if (!grid_fmt) {
         if ((rc = ojh_launch_shape(dev, (dq + "_x").c_str(), cb, nb, 0, dg, db))) return rc;
         if ((rc = ojh_launch(dev, (dq + "_x").c_str(), {at(w->raw, w->off), wdeq->ptr, xp, xh->ptr, yp},
@@ -853,7 +886,7 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
     if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) {
         bool ready;
         if ((rc = f16d_ready(dev, w, m, deq_tile, &ready))) return rc;
-        if (ready) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum);
+        if (ready) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum, w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT);
     }
     void *tile_w = wp;
     if (deq_tile) {

@@ -592,6 +592,33 @@ def test_long_batches_take_the_route_that_is_ahead(pkg, ty, n, k, m, copied):
         g.close()
 
 
+@pytest.mark.parametrize("n,k,m,copied", [(1100, 2304, 1900, True), (2752, 1024, 770, True), (4096, 1024, 300, False), (1100, 2304, 256, False)])
+def test_q4k_long_batches_by_price(orc, pkg, n, k, m, copied):
+    """Q4_K rows on their own tiles or decoded ahead of the copied tile, by price; f16 q qa + qb either way (the decoder's bits
+    first), f16 activations, K products added in f32: K 2^-24 of the peak (the magnitudes sum to some 0.15 sqrt(K) peaks)."""
+    raw = pkg.synth.q4k_weights(n, k, "q4kl", n, k)
+    bits = orc.q4l_weights_f16(raw, k, n)
+    x = pkg.synth.normal_f32(m * k, "q4kl", "x", m)
+    g = pkg.HipGpu(0)
+    try:
+        g.ensure_family("dequant")
+        nb, out, wd = n * k // 256, g.upload(np.full(n * k // 2 + 8, 7.5, np.float32)), g.upload_bytes(raw)
+        grid, block = g.launch_shape("dequant_q4kl_f16", 0, nb, 0)
+        g.dispatch(g.begin(), "dequant_q4kl_f16", [(wd, 0), (out, 0)], [nb], grid, block)
+        assert np.array_equal(g.read(out, n * k, np.uint16), np.asarray(bits).ravel().view(np.uint16))
+        assert np.all(g.read(out, n * k // 2 + 8)[-8:] == 7.5)
+        yd = g.upload(np.full(m * n + 64, 777.25, np.float32))
+        g.mm(g.upload(x), g.lin(Q4_K, n, k, raw), yd, m, act_mode=pkg.ACT_AUTO)
+        got = g.read(yd, m * n + 64)
+        assert bool(g.has_kernel("gemm_f16d_128")) == copied
+        assert np.all(got[m * n:] == np.float32(777.25))
+        rows = np.r_[0:3, n // 2, n - 2:n]
+        want = x.astype(np.float16).astype(np.float64).reshape(m, k) @ np.asarray(bits).view(np.float16).astype(np.float64).reshape(n, k)[rows].T
+        assert peak_err(got[:m * n].reshape(m, n)[:, rows], want) <= 2 * k * 2.0 ** -24
+    finally:
+        g.close()
+
+
 @pytest.mark.parametrize("ty,n,k,m,copied", [(14, 4096, 4096, 300, False), (14, 8192, 4096, 300, True), (14, 8192, 4096, 199, False), (8, 8192, 4096, 399, False),
                                              (8, 8192, 4096, 400, True), (20, 256, 1024, 200, True), (20, 256, 1024, 199, False), (18, 4096, 4096, 300, True)])
 def test_a_pinned_token_count_means_what_it_meant(pkg, monkeypatch, ty, n, k, m, copied):
