@@ -51,6 +51,12 @@ template <int N>
 __device__ __forceinline__ void gx_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
+// ... and every LDS read issued so far has its data: where no barrier (which waits for them) stands between the last reads
+// of a stage and the copies that overwrite it
+template <int N>
+__device__ __forceinline__ void gx_wait_reads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
+}
 
 // One thread's share of a weight slab: 64 weights of one row = one 32-byte chunk c of a Q4_K
 // super-block (low nibbles: sub-block 2c, high nibbles: sub-block 2c+1) plus the header.
@@ -528,8 +534,8 @@ __device__ __forceinline__ void gemm_bd_body(const ushort* __restrict__ xh, cons
         c0 = r0.frag<3>(magic); c1 = r1.frag<3>(magic);                                                \
         GB_MIX(5);                                                                                     \
         __builtin_amdgcn_sched_barrier(0);                                                             \
-        gx_wait<(C) == 2 ? 4 : 2>();                                                                   \
-        if (!KW) __syncthreads();                                                                      \
+        if (KW) gx_wait_reads<(C) == 2 ? 4 : 2>();                                                     \
+        else { gx_wait<(C) == 2 ? 4 : 2>(); __syncthreads(); }                                         \
         copy_x((T) + 2u);                                                                              \
         copy_nib((T) + 3u);                                                                            \
         if ((C) == 1) copy_hdr((T) + 3u);                                                              \

@@ -228,6 +228,24 @@ def test_tile_with_weights_dequantized_into_registers(gpu, orc, pkg, m, k, n):
     assert peak_err(outs["gemm_mm_q4kl_bdk", 0], outs["gemm_mm_q4kl_bd", 0]) <= 2e-6
 
 
+@pytest.mark.parametrize("m", [35, 100])
+def test_waves_that_split_k_reuse_their_stages(gpu, pkg, m):
+    """`gemm_mm_q4kl_bdk`: no barrier stands in its loop, so a wave itself must have read a stage before its copies
+    overwrite it.  385 rows repeated 64 times: a row's sums are the same instructions on the same bytes wherever the row
+    stands, so its 64 outputs are equal bit for bit — on buffers that no launch has touched before, as on the second pass."""
+    k, rows, rep = 6400, 385, 64
+    gpu.ensure_family("gemm_xl")
+    n = rows * rep
+    w = np.tile(np.asarray(pkg.synth.q4k_weights(rows, k, "stages")).view(np.uint8).reshape(rows, -1), (rep, 1))
+    for fresh in range(3):
+        x = pkg.synth.normal_f32(m * k, "stages", fresh).astype(np.float16)
+        xh, wd, yd = gpu.upload_bytes(x), gpu.upload_bytes(w), gpu.upload(np.zeros(m * n, np.float32))
+        for run in range(2):
+            gpu.dispatch(gpu.begin(), "gemm_mm_q4kl_bdk", [(xh, 0), (wd, 0), (yd, 0)], [k, n, 0, m], [n // 64, (m + 127) // 128, 1], [256, 1, 1])
+            got = gpu.read(yd, m * n).reshape(m, rep, rows)
+            assert np.array_equal(got, np.broadcast_to(got[:, :1], got.shape)), (fresh, run)
+
+
 def test_q4l_entries_by_their_reference_names(gpu, orc, pkg):
     """`gemm_mm_q4l` (f32 x), `gemm_mm_q4l_hb` (f16 x) and `gemm_mm_q4l_sk` with the reference's argument lists
     (crates/ojas-cuda/src/kernels/gemm_q.rs:26-38: x, w4, y, qa, qb; K, N, accum, M | K, N, M, nsplit) on weights relaid
