@@ -647,9 +647,13 @@ static bool f16d_pays(const ojh_device *dev, const ojh_lin *w, uint32_t m, bool 
 // long K amortizes the pass.  Both priced as above, the terms fitted to 3031 pairs of timed calls (512 - 32768 rows, K 1024 -
 // 14336, 200 - 2048 tokens; median error 2 - 5 %), and taken where ahead by a twentieth: 652 of the pairs, on average 16 %
 // faster, six of them more than 3 % slower.  Tiles / pass + copying tile, us: 1088 x 2304 at 1944 tokens 39.8 / 26.9, 2752 x
-// 6912 at 768 78.7 / 54.7, 4096 x 4096 at 1024 56.7 / 49.4, 4096 x 14336 at 2048 264 / 250, 6914 x 2816 at 333 39.2 / 33.1;
+// 6912 at 768 78.7 / 54.7, 4096 x 4096 at 1024 56.7 / 49.4, 6914 x 2816 at 333 39.2 / 33.1;
 // kept: 14336 x 4096 at 512 70 / 93, at 2048 235 / 255, 28534 x 12288 at 241 202 / 427.  The pass forms the tiles' weights
 // (dequant_q4kl_f16_x: f16 q qa + qb).
+// Not beyond K = 8192: what the pass wrote has to come from the caches, and in the first call after other work it does not.
+// Repeated / first call, us: 4096 x 14336 at 2048 263 -> 250 / 282 -> 294, at 1536 218 -> 210 / 221 -> 275, at 1024 150 -> 158 / 164 -> 192,
+// 4096 x 11008 at 1024 120 -> 125 / 135 -> 135; against 4096 x 8192 at 2048 178 -> 150 / 197 -> 160, at 1024 93 -> 87 / 110 -> 107, 2048 x
+// 8192 at 1536 86 -> 74 / 101 -> 90.
 static bool f16d_pays_q4k(const ojh_device *dev, uint32_t N, uint32_t K, uint32_t m) {
     const double cus = dev->prop.multiProcessorCount, mi = (double)N * K / (1 << 20), mk = (double)m * K / (1 << 20), mn = (double)m * N / (1 << 20);
     struct Price { double fixed, acts, round, fill, meet, out, start; };
@@ -676,7 +680,7 @@ static bool f16d_pays_q4k(const ojh_device *dev, uint32_t N, uint32_t K, uint32_
 static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int act_mode, bool decoded) {
     const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;   // (tiles of its own, other weight bits)
     if (!dev->deq_big_m || dev->no_scratch || dev->gemm_split_override || (uint64_t)w->n * w->k > 0x7FFFFFFFull) return false;
-    if (q4kl && (dev->deq_big_m != 1 || dev->gemm_bdk != 1 || dev->gemm_sr || m < 257 || w->n < 512 || w->k < 1024 || !f16d_pays_q4k(dev, w->n, w->k, m))) return false;
+    if (q4kl && (dev->deq_big_m != 1 || dev->gemm_bdk != 1 || dev->gemm_sr || m < 257 || w->n < 512 || w->k < 1024 || w->k > 8192 || !f16d_pays_q4k(dev, w->n, w->k, m))) return false;
     // while a graph is recorded nothing can be loaded or grown: what is not there yet leaves the call on the tile it has
     if (dev->capturing) {
         const auto slot = dev->scratch.find("wdeq");
