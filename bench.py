@@ -433,10 +433,9 @@ def extras(gpu, pkg, lin_q) -> dict:
     out["verify_prefill_q4k_int8"] = {"arithmetic": "quant_q8k activations, int8 x u4 dots on the int8 matrix cores, the CPU "
                                                     "reference's scale algebra (results within 2e-5 of matvec_kq)",
                                       "peak_tops": 5000.0,
-                                      "timed": "quantizer + the tile: from 33 tokens (17 where K >= 2 N: down) quantize_q8k_sides + gemm_q8k_q4k_xt{,64} "
-                                               "(128-token tiles, scales folded into int8 planes, v_mfma_i32_16x16x64_i8; where the "
-                                               "64-row tiles alone leave CUs idle or singly occupied — down up to M = 512 — gemm_q8k_q4k_xt64_sr: K slices "
-                                               "summed in slice order by the last to finish); below, "
+                                      "timed": "quantizer + the tile: from 17 tokens quantize_q8k_sides_h + gemm_q8k_q4k_xk64 up to one 64-row x 128-token tile "
+                                               "per CU (down up to M = 512, with K slices summed in slice order by the last to finish: _sr), beyond "
+                                               "quantize_q8k_sides + gemm_q8k_q4k_xt{,64} (scales folded into int8 planes, v_mfma_i32_16x16x64_i8); below, "
                                                "gemm_q8k_q4k_mf (down at M = 8: gemm_q8k_q4k_mk)", **i8}
     # ---- the same arithmetic over Q6_K and Q5_K rows (a Q4_K_M / Q5_K_M file mixes them in), f32 in
     for ty, tag, gen in ((pkg.Q6_K, "q6k", synth.q6k_weights), (pkg.Q5_K, "q5k", synth.q5k_weights)):
@@ -539,7 +538,7 @@ def extras(gpu, pkg, lin_q) -> dict:
             us = _time(gpu, lambda i: gpu.mm(xb, wf[i % 2], yb, m), 10, 2)
             fb[f"{tag}_M{m}"] = {"us": round(us, 1), "mfma_frac": round(2.0 * m * nb * kb / us / 1e6 / 2500.0, 4)}
         del wf
-    out["float_rows_batch_14336x4096"] = {"activations": "f32 -> f16", "kernels": "gemm_few_<fmt>_r4_t1 at 16 tokens, gemm_mm_<fmt>_m128{,_sk} at 128, dequant_<fmt>_f16_x + gemm_f16d_* or gemm_mm_<fmt> at 512; the grid codebooks dequant_<fmt>_f16 + gemm_mm_f16_m128{,_sk} / gemm_f16d_*", **fb}
+    out["float_rows_batch_14336x4096"] = {"activations": "f32 -> f16", "kernels": "few_x_f32 + gemm_few_<fmt>_r4_t1 at 16 tokens, gemm_mm_<fmt>_m128{,_sk} at 128, dequant_<fmt>_f16_x + gemm_f16d_* or gemm_mm_<fmt> at 512; the grid codebooks dequant_<fmt>_f16 + gemm_mm_f16_m128{,_sk} / gemm_f16d_*", **fb}
     # IQ2_XXS as the CPU path multiplies it: int8 activations per 256, integer dots (dot_iq2xxs_q8k)
     wf = [gpu.lin(pkg.IQ2_XXS, n, k, synth.weights(pkg.IQ2_XXS, n, k, "bench", "iq2xxs", "head")) for _ in range(2)]
     us = _time(gpu, lambda i: gpu.mm(x, wf[i % 2], y), 20, 3)
