@@ -864,9 +864,9 @@ GEMM_ENTRIES(q3k, LoaderQ3K)
 // 20.0 -> 16.0 / 22.1 -> 18.9, x 14336 69.9 -> 48.7 / 76.6 -> 56.0, 28672 x 4096 31.2 -> 30.0 / 36.0 -> 35.6; Q8_0, whose
 // bytes bound it sooner, 0 - 2 % (30.4 -> 29.6 at 14336 x 4096), never slower up to 32640 rows.
 // Row by row, a load of the tokens' pieces touches 64 lines for 16 bytes each and the address unit walks them one by one: 7 of
-// the 16 us of 24 tokens.  In fragment order (few_x_*) it is 1 KB in a row, and the next chunk's is asked for while this one's
-// rows are decoded.  With the conversion, us: IQ4_XS 14336 x 4096 at 24 tokens 19.5 -> 17.8, 4096^2 at 24 11.7 -> 8.5, 4096 x
-// 14336 at 16 20.1 -> 15.4, Q8_0 14336 x 4096 at 24 32.4 -> 28.9.  Now bound by the decoding's vector instructions (5 a weight).
+// the 16 us of 24 tokens.  In fragment order (few_x_*) it is 1 KB in a row.  With the conversion, us: IQ4_XS 14336 x 4096 at 24
+// tokens 19.5 -> 17.2, 4096^2 at 24 11.3 -> 8.6, 4096 x 14336 at 16 19.9 -> 15.8, Q8_0 14336 x 4096 at 24 31.9 -> 29.1.  Now bound by
+// the decoding's vector instructions (5 a weight).
 typedef float float4v __attribute__((ext_vector_type(4)));
 template <int J, class L>
 __device__ __forceinline__ half8 gm_frag(const L& ld) {
@@ -923,11 +923,13 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
         _Pragma("unroll") for (int j = 0; j < 4; j++) XV[tg][j] = *(const half8*)(xrow[tg] + (C) * xc + xj * j)
     uint c = wave;
     if (c < nchunk) ld0.load(wrow[0], c * 128u + g * 32u, 0u);
-    half8 xv[TG][4];
-    if (c < nchunk) GF_X(xv, c);
+    // A chunk's tokens are not asked for a chunk ahead: that gains nothing (0.1 % over 450 calls of 5 - 16 tokens) and its registers
+    // cost occupancy.  `_r4_t2` 121 -> 152 of them, one workgroup of eight waves a CU instead of two: Q5_1 24094 x 7936 at 17 tokens
+    // 61 -> 73 us, IQ4_XS 14336 x 4096 at 24 17.2 -> 18.1; `moe_few_iq4xs` 136 -> 172, two waves a SIMD instead of three: 128 experts
+    // top-8, IQ4_XS gate/up + IQ4_NL down, 256 tokens 194 -> 228.
     for (; c < nchunk; c += nw) {
-        half8 xn[TG][4];
-        if (RG > 1 && c + nw < nchunk) GF_X(xn, c + nw);          // (the next chunk's tokens travel while this one's rows are decoded)
+        half8 xv[TG][4];
+        GF_X(xv, c);
         if (RG == 1) {
             // (two chunks per trip so that the loaders alternate by name)
             GF_GROUP(ld0, ld1, 0, wrow[0], c + nw);
@@ -935,7 +937,6 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
             if (c < nchunk) {
                 GF_X(xv, c);
                 GF_GROUP(ld1, ld0, 0, wrow[0], c + nw);
-                if (c + nw < nchunk) GF_X(xv, c + nw);
             }
         } else {
 #pragma unroll
@@ -943,10 +944,6 @@ __device__ __forceinline__ void gemm_few_body(const ushort* __restrict__ xh, con
                 GF_GROUP(ld0, ld1, r, wrow[r + 1 < RG ? r + 1 : 0], c);
                 GF_GROUP(ld1, ld0, r + 1 < RG ? r + 1 : 0, wrow[r + 2 < RG ? r + 2 : 0], r + 2 < RG ? c : c + nw);
             }
-#pragma unroll
-            for (int tg = 0; tg < TG; tg++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) xv[tg][j] = xn[tg][j];
         }
     }
 #undef GF_X
