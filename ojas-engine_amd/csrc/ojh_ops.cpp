@@ -700,12 +700,12 @@ static bool f16d_taken(const ojh_device *dev, const ojh_lin *w, uint32_t m, int 
 }
 // Whether all the route needs is there.  What every form of the call needs comes first, so that the decoded rows' scratch,
 // which a format with a loader can do without, never takes its room: the activations' scratch, and the family of the tiles
-// that a recorded call of fewer tokens would take (nothing can be loaded then).
-static int f16d_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, bool decoded, bool *ready) {
+// that a recorded call of fewer tokens, or one that finds no room for its decoded rows, would take (nothing can be loaded then).
+static int f16d_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, bool decoded, bool q4kl, bool *ready) {
     int rc;
     ojh_buf *b;
     *ready = false;
-    if ((rc = ensure(dev, "glue")) || (!dev->capturing && (rc = ensure(dev, "gemm")))) return rc;
+    if ((rc = ensure(dev, "glue")) || (!dev->capturing && (rc = ensure(dev, q4kl ? "gemm_xl" : "gemm")))) return rc;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * w->k * 2, &b))) return rc;
     *ready = !ensure(dev, ojh_grid_type(w->type) ? "iq_grid" : "dequant") && !ensure(dev, "gemm_f16") &&
              !(decoded ? ojh_scratch_get : ojh_scratch_spare)(dev, "wdeq", (size_t)w->n * w->k * 2, &b);
@@ -888,9 +888,10 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
     const bool tile_fits = K % 64 == 0 && (uint64_t)m * K < 0x7FFFFFFFull && (uint64_t)m * N < 0x7FFFFFFFull;
     const bool tile_taken = (deq_tile || iq4_own || (m >= tile_min && act_mode != OJH_ACT_Q8K && !iq4 && !grid_fmt)) && tile_fits;
     if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) {
+        const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;
         bool ready;
-        if ((rc = f16d_ready(dev, w, m, deq_tile, &ready))) return rc;
-        if (ready) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum, w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT);
+        if ((rc = f16d_ready(dev, w, m, deq_tile, q4kl, &ready))) return rc;
+        if (ready) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum, q4kl);
     }
     void *tile_w = wp;
     if (deq_tile) {

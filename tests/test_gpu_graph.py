@@ -148,3 +148,31 @@ def test_a_smaller_batch_is_recorded_after_eager_long_ones(orc, pkg, ty):
         graph.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("n2,few", [(1100, 100), (1180, 1900)])
+def test_q4k_batches_are_recorded_after_eager_ones_that_were_decoded_first(orc, pkg, n2, few):
+    """1900 tokens of 1100 Q4_K rows are decoded ahead of the copied tile, whose family alone they need.  A recorded batch of fewer
+    tokens, and one of more rows than the decoded rows' scratch holds, run on the tiles that read Q4_K rows."""
+    n, k, many = 1100, 2304, 1900
+    x = pkg.synth.normal_f32(many * k, "graph", "x8").reshape(many, k)
+    w, w2 = pkg.synth.q4k_weights(n, k, "graph", "w8"), pkg.synth.q4k_weights(n2, k, "graph", "w9")
+    g = pkg.HipGpu(0)
+    try:
+        lin, lin2, xd, yd = g.lin(Q4_K, n, k, w), g.lin(Q4_K, n2, k, w2), g.upload(x), g.alloc(many * n2)
+        g.mm(xd, lin, yd, many, act_mode=pkg.ACT_AUTO)
+        assert g.has_kernel("gemm_f16d_128")
+        g.capture_begin()
+        g.mm(xd, lin2, yd, few, act_mode=pkg.ACT_AUTO)
+        graph = g.capture_end()
+        rows = np.r_[0:3, n2 // 2, n2 - 2:n2]
+        bits = np.asarray(orc.q4l_weights_f16(w2, k, n2)).view(np.float16).astype(np.float64).reshape(n2, k)[rows]
+        want = x[:few].astype(np.float16).astype(np.float64) @ bits.T
+        for _ in range(3):
+            g.memset0(yd)
+            graph.launch()
+            # f16 operands, K products added in f32: K 2^-24 of the peak (the magnitudes sum to some 0.15 sqrt(K) peaks)
+            assert peak_err(g.read(yd, few * n2).reshape(few, n2)[:, rows], want) <= 2 * k * 2.0 ** -24
+        graph.free()
+    finally:
+        g.close()
