@@ -181,8 +181,9 @@ const ojh_kernel_spec *ojh_find_kernel(const char *name);
 
 // ---- helpers -----------------------------------------------------------------------------------
 int ojh_scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out);
-// ... one the caller can do without: fails, and leaves the slot as it is, where memory is short
-int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out);
+// ... one the caller can do without: fails, and leaves the slot as it is, where memory is short; `ahead`: with the quarter of
+// growing room that ojh_scratch_get adds, where there is room for it
+int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool ahead = false);
 // ... a slot whose kernels leave zeros behind: cleared whenever it is (re)allocated
 int ojh_scratch_get_zeroed(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out);
 int ojh_launch(ojh_device *dev, const char *name, const std::vector<void *> &ptrs,

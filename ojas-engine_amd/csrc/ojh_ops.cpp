@@ -267,6 +267,12 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
             const size_t tiles = (size_t)((N + 63) / 64) * (mp / 128);
             sg[0] = (N + 63) / 64; sg[1] = mp / 128; sg[2] = z;
             sb[0] = 512; sb[1] = sb[2] = 1;
+            // fewer tokens may want more slices than these do, and a recorded call can ask for nothing: the places that the form
+            // with two workgroups a CU would leave behind are asked for beside, where there is room
+            if (const uint32_t zt = q4k_xt_slices(dev, K, N, m); zt > z && m >= q4k_xt_min_tokens(dev, K, N) && !dev->capturing) {
+                ojh_buf *b;
+                if (!ojh_scratch_spare(dev, "xt_part", tiles * zt * 32768, &b, true)) (void)ojh_scratch_get_zeroed(dev, "xt_cnt", tiles * 4, &b);
+            }
             if (z == 1) return ojh_launch(dev, "gemm_q8k_q4k_xk64", {xq, xst->ptr, sums->ptr, wp, yp}, {K, N, m, (uint32_t)(accum != 0), mp}, sg, sb);
             ojh_buf *part, *cnt;
             if ((rc = ojh_scratch_get(dev, "xt_part", tiles * z * 32768, &part))) return rc;
@@ -708,7 +714,7 @@ static int f16d_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, bool decode
     if ((rc = ensure(dev, "glue")) || (!dev->capturing && (rc = ensure(dev, q4kl ? "gemm_xl" : "gemm")))) return rc;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * w->k * 2, &b))) return rc;
     *ready = !ensure(dev, ojh_grid_type(w->type) ? "iq_grid" : "dequant") && !ensure(dev, "gemm_f16") &&
-             !(decoded ? ojh_scratch_get : ojh_scratch_spare)(dev, "wdeq", (size_t)w->n * w->k * 2, &b);
+             !(decoded ? ojh_scratch_get(dev, "wdeq", (size_t)w->n * w->k * 2, &b) : ojh_scratch_spare(dev, "wdeq", (size_t)w->n * w->k * 2, &b));
     return OJH_OK;
 }
 static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, uint32_t m,

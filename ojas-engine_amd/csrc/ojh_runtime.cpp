@@ -269,9 +269,9 @@ static size_t scratch_held(const ojh_device *dev) {
 }
 
 // `fresh` (optional) tells whether the slot was (re)allocated by this call: its contents are then undefined.
-// `spare`: a buffer the caller can do without.  It is not allocated ahead of its size, nor where it would leave less memory
-// free than it takes, and a smaller one in the slot is given up only once the larger is there.
-static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool *fresh, bool spare = false) {
+// `spare`: a buffer the caller can do without.  It is not allocated where it would leave less memory free than it takes, nor
+// ahead of its size unless `ahead`, and a smaller one in the slot is given up only once the larger is there.
+static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool *fresh, bool spare = false, bool ahead = true) {
     ojh_buf *&slot = dev->scratch[name];
     if (fresh) *fresh = false;
     if (!slot || slot->bytes < bytes) {
@@ -279,7 +279,7 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
             return ojh_fail(OJH_ERR_ARG, "scratch '%s' would have to grow while recording a graph: run the call once "
                                           "eagerly first", name);
         const bool park = slot && slot->recorded && dev->live_graphs > 0;   // a recorded chain may still replay into it
-        size_t cap = bytes < 4096 ? 4096 : spare ? bytes : bytes + bytes / 4;
+        size_t cap = bytes < 4096 ? 4096 : ahead ? bytes + bytes / 4 : bytes;
         if (dev->scratch_max) {
             const size_t held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
             if (held + cap > dev->scratch_max) cap = bytes;
@@ -292,6 +292,7 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
             size_t left = 0, total = 0;
             OJH_HIP(hipSetDevice(dev->ordinal));
             OJH_HIP(hipMemGetInfo(&left, &total));
+            if (left / 2 < cap) cap = std::max<size_t>(bytes, 4096);
             if (left / 2 < cap) return ojh_fail(OJH_ERR_HIP, "scratch '%s' of %zu bytes: %zu left on the device", name, bytes, left);
             if ((rc = ojh_alloc(dev, cap, &grown))) return rc;
         }
@@ -314,8 +315,8 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
 int ojh_scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out) {
     return scratch_get(dev, name, bytes, out, nullptr);
 }
-int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out) {
-    return scratch_get(dev, name, bytes, out, nullptr, true);
+int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool ahead) {
+    return scratch_get(dev, name, bytes, out, nullptr, true, ahead);
 }
 
 // Cleared whenever the slot is (re)allocated — decided by the allocation itself, not by comparing addresses: the

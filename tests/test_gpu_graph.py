@@ -176,3 +176,27 @@ def test_q4k_batches_are_recorded_after_eager_ones_that_were_decoded_first(orc, 
         graph.free()
     finally:
         g.close()
+
+
+def test_int8_batch_recorded_after_an_eager_longer_one_has_its_slices_places(orc, pkg):
+    """256 int8 tokens of 8192 Q4_K rows fill the chip with whole tiles; 100 need two K slices of them, which meet in scratch.  The
+    longer call leaves that scratch behind for a shorter one that is recorded."""
+    n, k, many, few = 8192, 8192, 256, 100
+    rows = pkg.synth.q4k_weights(256, k, "graph", "w10")
+    x = pkg.synth.normal_f32(many * k, "graph", "x10").reshape(many, k)
+    g = pkg.HipGpu(0)
+    try:
+        lin, xd, yd = g.lin(Q4_K, n, k, np.tile(rows, n // 256)), g.upload(x), g.alloc(many * n)
+        g.mm(xd, lin, yd, many, act_mode=pkg.ACT_Q8K)
+        g.capture_begin()
+        g.mm(xd, lin, yd, few, act_mode=pkg.ACT_Q8K)
+        graph = g.capture_end()
+        toks = [0, 63, few - 1]
+        want = np.stack([np.tile(orc.matvec_kq(rows, Q4_K, 256, k, x[t]), n // 256) for t in toks])
+        for _ in range(3):
+            g.memset0(yd)
+            graph.launch()
+            assert peak_err(g.read(yd, few * n).reshape(few, n)[toks], want) <= 2e-5
+        graph.free()
+    finally:
+        g.close()
