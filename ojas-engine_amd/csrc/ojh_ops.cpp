@@ -786,6 +786,9 @@ static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *
     const uint32_t grid[3] = {(w->n + nrb - 1) / nrb, 1, 1}, block[3] = {1024, 1, 1};
     const std::string name = std::string("gemv_fq8k_") + f->tag + (x_dtype == OJH_X_BF16 ? "_one_bf16_r" : "_one_r") + (r == 2 ? "2" : "1");
     int rc = ensure(dev, "gemv_q8k");
+    // (a recorded call of the two launches — more rows, or a bias — can ask for nothing: what they need is left behind, some KB)
+    ojh_buf *b;
+    if (!dev->capturing && !ojh_scratch_spare(dev, "xq", w->k, &b, true)) (void)ojh_scratch_spare(dev, "xs", w->k / 64, &b, true);
     return rc ? rc : ojh_launch(dev, name.c_str(), {xp, at(w->raw, w->off), yp}, {w->k, w->n, nrb, (uint32_t)(accum != 0)}, grid, block);
 }
 

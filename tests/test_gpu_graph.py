@@ -200,3 +200,33 @@ def test_int8_batch_recorded_after_an_eager_longer_one_has_its_slices_places(orc
         graph.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("multi", [False, True])
+@pytest.mark.parametrize("ty", [12, 13])
+def test_one_token_recorded_after_a_small_matrix_quantized_inside_its_launch(orc, pkg, ty, multi):
+    """A small matrix of one token quantizes inside its launch; a larger one of the same K, and the same with a bias, quantize ahead
+    of it into scratch, which the small one's eager call leaves behind."""
+    k, small, large = 8192, 64, 8192
+    rows = pkg.synth.weights(ty, small, k, "graph", "w11")
+    x, b = pkg.synth.normal_f32(k, "graph", "x11"), pkg.synth.normal_f32(small, "graph", "b11")
+    g = pkg.HipGpu(0)
+    try:
+        ls, ll = g.lin(ty, small, k, rows), g.lin(ty, large, k, np.tile(rows, large // small))
+        xd, bd, ys, yl = g.upload(x), g.upload(b), g.alloc(small), g.alloc(large)
+        call = (lambda lin, y: g.mm_multi(xd, [lin], [y])) if multi else (lambda lin, y: g.mm(xd, lin, y, 1, act_mode=pkg.ACT_Q8K))
+        call(ls, ys)
+        g.capture_begin()
+        call(ll, yl)
+        g.mm(xd, ls, ys, 1, bias=bd, act_mode=pkg.ACT_Q8K)
+        graph = g.capture_end()
+        want = orc.matvec_kq(rows, ty, small, k, x)
+        for _ in range(3):
+            g.memset0(yl)
+            g.memset0(ys)
+            graph.launch()
+            assert peak_err(g.read(yl, large), np.tile(want, large // small)) <= 2e-5
+            assert peak_err(g.read(ys, small), want + b) <= 2e-5
+        graph.free()
+    finally:
+        g.close()
