@@ -921,11 +921,11 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
                         (uint64_t)w->row_bytes * N <= 0xFFFFFFFFull;  // 32-bit row offsets in that tile
         if ((rc = ensure(dev, "glue")) || (rc = ensure(dev, xl ? "gemm_xl" : "gemm"))) return rc;
         // (the few-token kernel below reads the tokens' f16 copy in the order of its lanes where there is room for whole
-        // groups of sixteen tokens, row by row otherwise)
+        // groups of sixteen tokens, row by row otherwise; with the growing room that a recorded batch of a few more may count on)
         const uint32_t few_tg = m <= 16 ? 1 : m <= 32 ? 2 : 4;
         ojh_buf *xh;
         const bool few_frag = !xl && !deq_tile && dev->gemm_few && m <= dev->gemm_few && m <= 64 && K % 128 == 0 && (own_loader || w->type == OJH_Q8_0) &&
-                              !ojh_scratch_spare(dev, "xh", (size_t)16 * few_tg * K * 2, &xh);
+                              !ojh_scratch_spare(dev, "xh", (size_t)16 * few_tg * K * 2, &xh, true);
         if (!few_frag && (rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
         const uint32_t n_el = m * K, conv_blocks = (n_el / 8 + 255) / 256 + 1;
         std::string base = std::string("gemm_mm_") + (deq_tile ? "f16" : w->type == OJH_Q8_0 ? "q8_0" : f->tag);

@@ -230,3 +230,27 @@ def test_one_token_recorded_after_a_small_matrix_quantized_inside_its_launch(orc
         graph.free()
     finally:
         g.close()
+
+
+def test_a_batch_of_a_few_more_tokens_is_recorded_after_an_eager_one(orc, pkg):
+    """Scratch that grows takes a quarter more than was asked for: 36 tokens are recorded after 30, which the few-token kernel reads
+    in groups of sixteen."""
+    n, k, first, more = 96, 512, 30, 36
+    w = pkg.synth.weights(23, n, k, "graph", "w12")
+    x = pkg.synth.normal_f32(more * k, "graph", "x12").reshape(more, k)
+    g = pkg.HipGpu(0)
+    try:
+        lin, xd, yd = g.lin(23, n, k, w), g.upload(x), g.alloc(more * n)
+        g.mm(xd, lin, yd, first, act_mode=pkg.ACT_FLOAT)
+        g.capture_begin()
+        g.mm(xd, lin, yd, more, act_mode=pkg.ACT_FLOAT)
+        graph = g.capture_end()
+        want = orc.matmul_ref(w, 23, n, k, x, wmode=1, xmode=1)
+        for _ in range(3):
+            g.memset0(yd)
+            graph.launch()
+            # f16 operands, K products added in f32: K 2^-24 of the peak (the magnitudes sum to some 0.15 sqrt(K) peaks)
+            assert peak_err(g.read(yd, more * n).reshape(more, n), want) <= k * 2.0 ** -24
+        graph.free()
+    finally:
+        g.close()
