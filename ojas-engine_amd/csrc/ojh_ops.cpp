@@ -23,6 +23,10 @@ static int span_ok(const char *what, const ojh_buf *b, size_t off, size_t bytes,
 
 static inline void *at(const ojh_buf *b, size_t off) { return (char *)b->ptr + off; }
 
+static inline bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+    return (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+
 // ---- Lin ---------------------------------------------------------------------------------------
 static int lin_check(uint32_t type, uint32_t n, uint32_t k, size_t *row_bytes) {
     const ojh_block_format *f = ojh_format(type);
@@ -522,7 +526,7 @@ extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_bu
                       {ws[0]->k, ends[0], ends[1], ends[2], ends[3]}, grid, block);
 }
 
-static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w);
+static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y);
 static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum);
 
 // One stage of a decode layer in ONE launch: 1 to 4 projections of one f32 vector, the vector quantized inside the launch.
@@ -554,7 +558,7 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     // in flight as the plain matvec's thousands of small ones, and many small ones repeat the quantization too often.
     // OJAS_HIP_FQ_MULTI = 0 never takes it, 2 takes it at every size.
     const bool small_stage = total * K <= 32u * 1024u * 1024u && K <= 4096u;
-    if (count == 1 && !fused && dev->fq_multi && fq_one_taken(dev, ws[0]))
+    if (count == 1 && !fused && dev->fq_multi && fq_one_taken(dev, ws[0], at(x, x_off), (size_t)K * 4, at(ys[0], y_offs ? y_offs[0] : 0)))
         return fq_one_launch(dev, at(x, x_off), OJH_X_F32, ws[0], ojh_format(ws[0]->type), at(ys[0], y_offs ? y_offs[0] : 0), accum);
     if (!fused || K > 16384 || dev->fq_multi == 0 || (dev->fq_multi == 1 && !small_stage)) {   // quantize once, then the per-format launches
         size_t nsb = K / 256;
@@ -770,9 +774,10 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
 // Q6_K 8.7 / 9.0; 1024 x 8192 Q6_K 8.0 / 6.7; 1024 x 14336 Q4_K 8.0 / 8.2, Q5_K 8.3 / 8.7, Q6_K 8.0 / 9.5; where the host
 // issues a launch in 3 us instead of 4: 1024 x 4096 Q4_K 6.1 / 3.7, 3000 x 6144 6.1 / 5.2, 30000 x 1792 8.5 / 8.8, 12000 x 4096
 // Q5_K 10.6 / 8.9, 2000 x 8192 Q6_K 6.4 / 6.6.
-static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w) {
+// Not where y lies over x: a workgroup may store its rows before another has read the token.
+static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y) {
     const uint64_t mi = ((uint64_t)w->n * w->k + (1u << 20) - 1) >> 20;
-    if (w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) return false;
+    if ((w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) || overlap(x, x_bytes, y, (size_t)w->n * 4)) return false;
     if (dev->fq_one != 1) return dev->fq_one == 2 && w->k <= 16384u;
     if (w->n >= 32768u) return false;              // (heads have forms of their own)
     if (w->type == OJH_Q6_K) return mi <= (w->k <= 4096u ? 16u : w->k <= 8192u ? 8u : 0u);
@@ -1049,7 +1054,7 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         grid[0] = (N + nrb - 1) / nrb;
         return ojh_launch(dev, name, {at(x, x_off), wp, yp}, {K, N, nrb}, grid, block);
     }
-    if (q8k && m == 1 && !bias && fq_one_taken(dev, w)) return fq_one_launch(dev, at(x, x_off), x_dtype, w, f, yp, accum);
+    if (q8k && m == 1 && !bias && fq_one_taken(dev, w, at(x, x_off), K * esz, yp)) return fq_one_launch(dev, at(x, x_off), x_dtype, w, f, yp, accum);
     if (q8k) {
         if ((rc = ensure(dev, "gemv_q8k"))) return rc;
         size_t nsb = K / 256;

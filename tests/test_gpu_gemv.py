@@ -714,3 +714,23 @@ def test_one_projection_routes_agree(pkg, monkeypatch, ty, n, k):
             g.close()
     for a, b in zip(*outs):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("ty,multi", [(Q4_K, False), (Q5_K, False), (Q6_K, False), (Q5_K, True), (Q6_K, True)])
+@pytest.mark.parametrize("y_off", [0, 4 * 700, 4 * 1000])
+def test_one_projection_written_over_its_token(gpu, pkg, ty, multi, y_off):
+    """y over x, over its second half, over its last values: a launch that quantized inside could store rows before all of the token
+    is read, so the token is quantized ahead; the bits are those of a y of its own."""
+    n, k = 1024, 1024
+    raw, x = _inputs(pkg, ty, n, k, "over")
+    lin = gpu.lin(ty, n, k, raw)
+    xd, yd, both = gpu.upload(x), gpu.alloc(n), gpu.upload(np.concatenate([x, np.zeros(1024, np.float32)]))
+    if multi:
+        gpu.mm_multi(xd, [lin], [yd])
+        gpu.mm_multi(both, [lin], [both], [y_off])
+    else:
+        gpu.mm(xd, lin, yd, 1)
+        gpu.mm(both, lin, both, 1, y_off=y_off)
+    got = gpu.read(both, 2048)
+    assert np.array_equal(got[y_off // 4:y_off // 4 + n].view(np.uint32), gpu.read(yd, n).view(np.uint32))
+    assert np.array_equal(got[:y_off // 4], x[:y_off // 4])
