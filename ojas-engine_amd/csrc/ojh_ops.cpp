@@ -901,8 +901,9 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
                           !dev->no_scratch && K % 64 == 0 && (uint64_t)N * K / f->weights <= 0x7FFFFFFFu / 64;
     const bool tile_fits = K % 64 == 0 && (uint64_t)m * K < 0x7FFFFFFFull && (uint64_t)m * N < 0x7FFFFFFFull;
     const bool tile_taken = (deq_tile || iq4_own || (m >= tile_min && act_mode != OJH_ACT_Q8K && !iq4 && !grid_fmt)) && tile_fits;
-    if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile)) {
-        const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;
+    const bool q4kl = w->type == OJH_Q4_K && !dev->gemm_exact && act_mode != OJH_ACT_FLOAT_EXACT;
+    // (Q4_K rows not where y lies over x: the pass may clear y while it converts x, which their own tiles, whole, do not)
+    if (tile_taken && f16d_taken(dev, w, m, act_mode, deq_tile) && !(q4kl && overlap(at(x, x_off), (size_t)m * K * esz, yp, (size_t)m * N * 4))) {
         bool ready;
         if ((rc = f16d_ready(dev, w, m, deq_tile, q4kl, &ready))) return rc;
         if (ready) return f16d_launch(dev, at(x, x_off), x_dtype, w, f, yp, m, accum, q4kl);

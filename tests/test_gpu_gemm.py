@@ -680,3 +680,27 @@ def test_copied_tile_sizes_through_mm(gpu, pkg, monkeypatch, tile, n, k, m, bf16
         finally:
             g.close()
     assert peak_err(outs[0], outs[1]) <= 2 * k * 2.0 ** -24
+
+
+def test_q4k_batch_written_over_its_tokens(orc, pkg):
+    """512 x 1024 at 400 tokens is decoded first, over K slices that add into a y cleared beside the activations' conversion; with y
+    over x it runs on the tile that converts first and stores whole sums."""
+    n, k, m = 512, 1024, 400
+    raw = pkg.synth.q4k_weights(n, k, "q4kl", "over")
+    x = pkg.synth.normal_f32(m * k, "q4kl", "over-x", m)
+    g = pkg.HipGpu(0)
+    try:
+        lin, xd = g.lin(Q4_K, n, k, raw), g.upload(x)
+        g.mm(xd, lin, xd, m, act_mode=pkg.ACT_AUTO)
+        assert not g.has_kernel("gemm_f16d_128")
+        got = g.read(xd, m * n).reshape(m, n)
+        yd = g.alloc(m * n)
+        g.mm(g.upload(x), lin, yd, m, act_mode=pkg.ACT_AUTO)
+        assert g.has_kernel("gemm_f16d_128")
+        rows = np.r_[0:3, n // 2, n - 2:n]
+        bits = np.asarray(orc.q4l_weights_f16(raw, k, n)).view(np.float16).astype(np.float64).reshape(n, k)[rows]
+        want = x.astype(np.float16).astype(np.float64).reshape(m, k) @ bits.T
+        # f16 operands, K products added in f32: K 2^-24 of the peak, as above
+        assert peak_err(got[:, rows], want) <= 2 * k * 2.0 ** -24 and peak_err(g.read(yd, m * n).reshape(m, n)[:, rows], want) <= 2 * k * 2.0 ** -24
+    finally:
+        g.close()
