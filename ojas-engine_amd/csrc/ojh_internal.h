@@ -4,6 +4,7 @@
 
 #include <cstdarg>
 #include <cstdint>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -184,6 +185,8 @@ int ojh_scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **o
 // ... one the caller can do without: fails, and leaves the slot as it is, where memory is short; `ahead`: with the quarter of
 // growing room that ojh_scratch_get adds, where there is room for it
 int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool ahead = false);
+// ... whether several such fit what they are limited to together, asked before the first of them takes its room
+bool ojh_scratch_fits(const ojh_device *dev, std::initializer_list<std::pair<const char *, size_t>> wanted);
 // ... a slot whose kernels leave zeros behind: cleared whenever it is (re)allocated
 int ojh_scratch_get_zeroed(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out);
 int ojh_launch(ojh_device *dev, const char *name, const std::vector<void *> &ptrs,
@@ -197,8 +200,7 @@ int ojh_mm_checks(const char *who, const ojh_lin *w, ojh_buf *y, size_t y_off, c
                   const ojh_block_format **fmt);
 int ojh_quant_q8k_launch(ojh_device *dev, const void *x, int x_dtype, uint32_t m, uint32_t k, void *q, void *scales);
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,
-                      const ojh_buf *bias, uint32_t m, int accum, bool sides_ready = false);
-bool ojh_q4k_xt_taken(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp);
+                      const ojh_buf *bias, uint32_t m, int accum, int xt = -1);
 int ojh_noalloc_setup(ojh_device *dev);   // resolves the static scratch array on the current GPU (ojh_noalloc.cpp)
 void ojh_gemm_q8k_tiles(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M, uint32_t *rw, uint32_t *rt);   // row tiles per workgroup / per wave of gemm_q8k_q4k_mf
 uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t E, bool gu, uint32_t *threads);   // workgroups per expert of those entries, and their threads

@@ -210,24 +210,33 @@ static uint32_t q4k_xt_min_tokens(const ojh_device *dev, uint32_t K, uint32_t N)
 // The form that has a CU to itself multiplies no more than 64 tokens where no more are left, and is ahead from 17 of them,
 // where the few-token kernels need a second pass of 16 (before / with it, 24 tokens, us: 14336 x 4096 22.6 / 20.7, 4096^2
 // 16.7 / 12.4, 1024 x 4096 15.3 / 11.4, 4096 x 14336 35.2 / 22.3, 2048^2 10.8 / 9.9; at 12 tokens 17.7 / 20.4, 8.9 / 12.3, 8.5 /
-// 11.4).  The few-token kernels need none of its scratch, so where that is not to be had the call stays with them.
-static bool q4k_xk_early(ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
-    const uint32_t z = m >= 17 && dev->q4k_xt_min_m == 1 ? q4k_xk_slices(dev, K, N, m) : 0;
-    if (!z || ensure(dev, "gemm_q8k")) return false;
-    const size_t mp = (m + 127) / 128 * 128, nsb = K / 256, tiles = (size_t)((N + 63) / 64) * (mp / 128);
-    ojh_buf *b;
-    return !ojh_scratch_spare(dev, "xt_xst", nsb * mp * 4, &b) && !ojh_scratch_spare(dev, "xt_sums", nsb * mp * 32, &b) &&
-           (z == 1 || (!ojh_scratch_spare(dev, "xt_part", tiles * z * 32768, &b) && !ojh_scratch_get_zeroed(dev, "xt_cnt", tiles * 4, &b)));
+// 11.4).
+static bool q4k_xk_early(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
+    return m >= 17 && dev->q4k_xt_min_m == 1 && q4k_xk_slices(dev, K, N, m);
 }
-bool ojh_q4k_xt_taken(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp) {
+// What a Q4_K product of m tokens does about that tile.  From q4k_xt_min_tokens it takes it.  The few-token kernels need none of
+// its scratch, so a product of fewer tokens takes it only where all of that is to be had (and takes none where some is not),
+// which is asked for here, once a product.
+enum { XT_ASK = -1, XT_NO, XT_TAKE, XT_SIDES };    // XT_SIDES: taken, its side arrays written by the quantizer
+static int q4k_xt_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp) {
     const uint32_t K = w->k, N = w->n;
-    return w->type == OJH_Q4_K && dev->q4k_xt_min_m && !dev->no_scratch && q4k_xt_slices(dev, K, N, m) >= 1 &&
-           (uint64_t)m * K <= 0xFFFFFFFFull && (uint64_t)w->row_bytes * N <= 0xFFFFFFFFull && (uintptr_t)wp % 16 == 0 &&
-           (m >= q4k_xt_min_tokens(dev, K, N) || q4k_xk_early(dev, K, N, m));
+    if (w->type != OJH_Q4_K || !dev->q4k_xt_min_m || dev->no_scratch || !q4k_xt_slices(dev, K, N, m) || (uint64_t)m * K > 0xFFFFFFFFull ||
+        (uint64_t)w->row_bytes * N > 0xFFFFFFFFull || (uintptr_t)wp % 16)
+        return XT_NO;
+    if (m >= q4k_xt_min_tokens(dev, K, N)) return XT_TAKE;
+    if (!q4k_xk_early(dev, K, N, m) || ensure(dev, "gemm_q8k")) return XT_NO;
+    const size_t z = q4k_xk_slices(dev, K, N, m), mp = (m + 127) / 128 * 128, nsb = K / 256, tiles = (size_t)((N + 63) / 64) * (mp / 128);
+    const size_t xst = nsb * mp * 4, sums = nsb * mp * 32, part = tiles * z * 32768, cnt = tiles * 4;
+    ojh_buf *b;
+    if (z == 1 ? !ojh_scratch_fits(dev, {{"xt_xst", xst}, {"xt_sums", sums}})
+               : !ojh_scratch_fits(dev, {{"xt_xst", xst}, {"xt_sums", sums}, {"xt_part", part}, {"xt_cnt", cnt}}))
+        return XT_NO;
+    return (z == 1 || (!ojh_scratch_spare(dev, "xt_part", part, &b) && !ojh_scratch_get_zeroed(dev, "xt_cnt", cnt, &b))) &&
+           !ojh_scratch_spare(dev, "xt_sums", sums, &b) && !ojh_scratch_spare(dev, "xt_xst", xst, &b) ? XT_TAKE : XT_NO;
 }
 
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,
-                         const ojh_buf *bias, uint32_t m, int accum, bool sides_ready) {
+                         const ojh_buf *bias, uint32_t m, int accum, int xt) {
     const uint32_t K = w->k, N = w->n;
     void *wp = at(w->raw, w->off);
     uint32_t grid[3] = {1, 1, 1}, block[3] = {256, 1, 1};
@@ -252,7 +261,8 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
     // Q4_K rows against a prefill-sized batch: 128 x 128 tiles, the tokens copied into LDS by the memory system
     // (needs two side arrays, built by one small launch into the library's scratch — or by the quantizer itself when
     // ojh_mm quantizes: it then comes here with the side arrays ready)
-    if (ojh_q4k_xt_taken(dev, w, m, wp)) {
+    if (xt == XT_ASK) xt = q4k_xt_ready(dev, w, m, wp);
+    if (xt != XT_NO) {
         int rc = ensure(dev, "gemm_q8k");
         if (rc) return rc;
         const uint32_t mp = (m + 127) / 128 * 128;
@@ -261,7 +271,7 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
         if ((rc = ojh_scratch_get(dev, "xt_xst", nsb * mp * 4, &xst))) return rc;
         if ((rc = ojh_scratch_get(dev, "xt_sums", nsb * mp * 32, &sums))) return rc;
         uint32_t sg[3], sb[3];
-        if (!sides_ready) {
+        if (xt != XT_SIDES) {
             const char *sides = q4k_xk_slices(dev, K, N, m) ? "q8k_token_sides_h" : "q8k_token_sides";
             if ((rc = ojh_launch_shape(dev, sides, K, N, m, sg, sb))) return rc;
             if ((rc = ojh_launch(dev, sides, {xq, xs, xst->ptr, sums->ptr}, {K, m, mp}, sg, sb))) return rc;
@@ -297,9 +307,9 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
         }
         // 128-row tiles when they give every CU one, 64-row tiles otherwise
         const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
-        const char *xt = (uint64_t)((N + 127) / 128) * (mp / 128) >= cus && !dev->q4k_xt64 ? "gemm_q8k_q4k_xt" : "gemm_q8k_q4k_xt64";
-        if ((rc = ojh_launch_shape(dev, xt, K, N, m, sg, sb))) return rc;
-        return ojh_launch(dev, xt, {xq, xst->ptr, sums->ptr, wp, yp}, {K, N, m, (uint32_t)(accum != 0), mp}, sg, sb);
+        const char *tile = (uint64_t)((N + 127) / 128) * (mp / 128) >= cus && !dev->q4k_xt64 ? "gemm_q8k_q4k_xt" : "gemm_q8k_q4k_xt64";
+        if ((rc = ojh_launch_shape(dev, tile, K, N, m, sg, sb))) return rc;
+        return ojh_launch(dev, tile, {xq, xst->ptr, sums->ptr, wp, yp}, {K, N, m, (uint32_t)(accum != 0), mp}, sg, sb);
     }
     // Q4_K rows against several tokens: the int8 matrix cores, in the shape measured fastest on K = 4096 and 14336.
     // A long matrix (six 16-row tiles per CU and wave: 24576 rows on this GPU) against 2 .. 16 tokens: a wave
@@ -1063,7 +1073,8 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         if ((rc = ojh_scratch_get(dev, "xq", (size_t)m * nsb * 256, &xq))) return rc;
         if ((rc = ojh_scratch_get(dev, "xs", (size_t)m * nsb * 4, &xs))) return rc;
         // ahead of the 128-token int8 tile the quantizer writes that tile's side arrays too (one launch less)
-        if (ojh_q4k_xt_taken(dev, w, m, wp) && K % 256 == 0 && (uintptr_t)at(x, x_off) % (x_dtype == OJH_X_BF16 ? 8 : 16) == 0) {
+        const int xt = q4k_xt_ready(dev, w, m, wp);
+        if (xt != XT_NO) {
             if ((rc = ensure(dev, "gemm_q8k"))) return rc;
             const uint32_t mp = (m + 127) / 128 * 128;
             ojh_buf *xst, *sums;
@@ -1075,10 +1086,10 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
             if ((rc = ojh_launch(dev, quant.c_str(),
                                  {at(x, x_off), xq->ptr, xs->ptr, xst->ptr, sums->ptr}, {K, m, mp}, qg, block)))
                 return rc;
-            return ojh_mm_q8k_launch(dev, xq->ptr, xs->ptr, w, f, yp, bias, m, accum, true);
+            return ojh_mm_q8k_launch(dev, xq->ptr, xs->ptr, w, f, yp, bias, m, accum, XT_SIDES);
         }
         if ((rc = ojh_quant_q8k_launch(dev, at(x, x_off), x_dtype, m, K, xq->ptr, xs->ptr))) return rc;
-        return ojh_mm_q8k_launch(dev, xq->ptr, xs->ptr, w, f, yp, bias, m, accum);
+        return ojh_mm_q8k_launch(dev, xq->ptr, xs->ptr, w, f, yp, bias, m, accum, xt);
     }
 
     // floating-point activations: the matvec kernels read f32

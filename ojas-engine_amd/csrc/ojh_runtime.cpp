@@ -319,6 +319,20 @@ int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf *
     return scratch_get(dev, name, bytes, out, nullptr, true, ahead);
 }
 
+bool ojh_scratch_fits(const ojh_device *dev, std::initializer_list<std::pair<const char *, size_t>> wanted) {
+    size_t held = scratch_held(dev);
+    bool grows = false;
+    for (const auto &w : wanted) {
+        const auto it = dev->scratch.find(w.first);
+        const ojh_buf *slot = it == dev->scratch.end() ? nullptr : it->second;
+        if (slot && slot->bytes >= w.second) continue;
+        const bool park = slot && slot->recorded && dev->live_graphs > 0;
+        grows = true;
+        held += std::max<size_t>(w.second, 4096) - (slot && !park ? slot->bytes : 0);
+    }
+    return !grows || (!dev->capturing && (!dev->scratch_max || held <= dev->scratch_max));
+}
+
 // Cleared whenever the slot is (re)allocated — decided by the allocation itself, not by comparing addresses: the
 // allocator may hand a grown slot the address the freed one had.
 int ojh_scratch_get_zeroed(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out) {

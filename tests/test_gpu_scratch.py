@@ -142,3 +142,26 @@ def test_a_chain_keeps_the_decoded_rows_it_was_recorded_with(pkg, orc, monkeypat
         graph.free()
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("room", [-4096, 4096])
+def test_a_batch_that_cannot_have_all_its_scratch_takes_none(pkg, orc, monkeypatch, room):
+    """24 tokens of Q4_K rows run on the 64-row int8 tile where its four scratch buffers are to be had.  Where the limit holds the
+    small ones, or the largest, but not all, the call stays with the few-token kernel, and none of them is left to take room from other calls."""
+    m, n = 24, 2112
+    w = pkg.synth.q4k_weights(n, 4096, "scratch", "w24")
+    x = pkg.synth.normal_f32(m * 4096, "scratch", "x24").reshape(m, 4096)
+    part = 33 * 4 * 32768                                    # 33 64-row tiles over four slices of K
+    g = _device(pkg, monkeypatch, part + room)
+    try:
+        lin, xd, yd = g.lin(12, n, 4096, w), g.upload(x), g.alloc(m * n)
+        xq, xs = g.alloc_bytes(m * 4096), g.alloc(m * 16)
+        g.quant_q8k(xd, m, 4096, xq, xs)
+        g.ensure_family("gemm_q8k")
+        other = g.lin(Q6_K, 256, K, _weights(pkg, 256))
+        xo, yo = g.upload(np.zeros(4096 * K, np.float32)), g.alloc(4096 * 256)
+        g.mm_q8k(xq, xs, lin, yd, m)
+        assert peak_err(g.read(yd, m * n).reshape(m, n), np.stack([orc.matvec_kq(w, 12, n, 4096, x[t]) for t in range(m)])) <= 2e-5
+        g.mm(xo, other, yo, (part + room - 4096) // (K * 2), act_mode=pkg.ACT_FLOAT)      # f16 activations that fill the limit but for 4 KB
+    finally:
+        g.close()
