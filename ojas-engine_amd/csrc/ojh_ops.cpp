@@ -209,10 +209,13 @@ static uint32_t q4k_xt_min_tokens(const ojh_device *dev, uint32_t K, uint32_t N)
 }
 // The form that has a CU to itself multiplies no more than 64 tokens where no more are left, and is ahead from 17 of them,
 // where the few-token kernels need a second pass of 16 (before / with it, 24 tokens, us: 14336 x 4096 22.6 / 20.7, 4096^2
-// 16.7 / 12.4, 1024 x 4096 15.3 / 11.4, 4096 x 14336 35.2 / 22.3, 2048^2 10.8 / 9.9; at 12 tokens 17.7 / 20.4, 8.9 / 12.3, 8.5 /
-// 11.4).
+// 16.7 / 12.4, 1024 x 4096 15.3 / 11.4, 4096 x 14336 35.2 / 22.3; at 12 tokens 17.7 / 20.4, 8.9 / 12.3, 8.5 / 11.4).  Not for
+// short rows, where its fixed part shows (6000 x 1024 8.9 / 9.8, 4000 x 1792 10.0 / 10.4, 3500 x 2048 level, 2000 x 2048 10.9 / 9.9),
+// unless more 64-row tiles than half the CUs make the few-token kernel walk two tiles a wave (8400 x 1024 11.1 / 8.6, x 2048
+// 18.9 / 12.3).
 static bool q4k_xk_early(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
-    return m >= 17 && dev->q4k_xt_min_m == 1 && q4k_xk_slices(dev, K, N, m);
+    const bool ahead = K > 2048 || (K == 2048 && N <= 2560) || (N + 63) / 64 * 2 > (uint32_t)dev->prop.multiProcessorCount;
+    return ahead && m >= 17 && dev->q4k_xt_min_m == 1 && q4k_xk_slices(dev, K, N, m);
 }
 // What a Q4_K product of m tokens does about that tile.  From q4k_xt_min_tokens it takes it.  The few-token kernels need none of
 // its scratch, so a product of fewer tokens takes it only where all of that is to be had (and takes none where some is not),

@@ -354,3 +354,26 @@ def test_few_tokens_without_room_for_the_tile_keep_their_kernel(pkg, orc, monkey
             assert peak_err(g.read(yd, m * n).reshape(m, n), want) <= TOL_SEEN
         finally:
             g.close()
+
+
+def _bits_of_both_forms(pkg, monkeypatch, m, n, k):
+    """ojh_mm on int8 activations with the form that has a CU to itself switched off and as chosen"""
+    w, x = _case(pkg, m, n, k, "xk-route")
+    outs = []
+    for xk in ("0", "1"):
+        monkeypatch.setenv("OJAS_HIP_Q4K_XK", xk)
+        g = pkg.HipGpu(0)
+        try:
+            yd = g.alloc(m * n)
+            g.mm(g.upload(x), g.lin(Q4_K, n, k, w), yd, m, act_mode=pkg.ACT_Q8K)
+            outs.append(g.read(yd, m * n).view(np.uint32))
+        finally:
+            g.close()
+    return outs
+
+
+@pytest.mark.parametrize("m,n,k,taken", [(24, 6000, 1024, False), (24, 3500, 2048, False), (24, 2100, 2048, True), (24, 4000, 2304, True), (24, 8300, 1024, True)])
+def test_few_tokens_take_the_tile_on_long_or_many_rows(pkg, monkeypatch, m, n, k, taken):
+    """On short rows the few-token kernel stays ahead unless it walks two tiles a wave; seen by the order of the sums."""
+    old, new = _bits_of_both_forms(pkg, monkeypatch, m, n, k)
+    assert np.array_equal(old, new) != taken
