@@ -184,11 +184,14 @@ static uint32_t q4k_xt_slices(const ojh_device *dev, uint32_t K, uint32_t N, uin
 // super-blocks, two where four would leave more than half the CUs idle.  Above one tile per CU two workgroups of the other
 // form share it and are as fast or faster.  That form / this one, with the quantizer, us: 14336 x 4096 at 48 tokens 36.5 /
 // 21.4, at 128 38.4 / 28.9; 4096 x 14336 at 512 109.5 / 95; 4096^2 at 512 41.9 / 34; at 128 (four slices) 19.0 / 17.5;
-// 14336 x 4096 at 256 (448 tiles) 57.8 / 57.8, at 512 84 / 111.
+// 14336 x 4096 at 256 (448 tiles) 57.8 / 57.8, at 512 84 / 111.  Nor where the other form takes three slices of tiles that cover
+// little more than half the CUs here: 4352 x 12800 at 200 tokens (136 tiles) 63.5 / 72, 9600 x 13568 at 120 (150) 65.5 / 75, against
+// 12288 x 12800 at 120 (192 tiles, two slices) 85 / 71; up to 64 tokens, half a tile, 9600 x 13568 at 60 63 / 52.
 static uint32_t q4k_xk_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
     const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount, nsb = K / 256;
     const uint64_t tiles = (uint64_t)((N + 63) / 64) * ((m + 127) / 128);
     if (!dev->q4k_xk || dev->q4k_xt64 || dev->q4k_xt_split > 1 || tiles > cus) return 0;
+    if (tiles * 2 > cus && m > 64 && q4k_xt_slices(dev, K, N, m) > 2) return 0;
     uint32_t z = std::min<uint32_t>((uint32_t)(cus / tiles), 8u), cap = std::max(nsb / 4, 1u);
     if (dev->q4k_xt_split == 0 || z < 2) return 1;
     if (tiles * std::min(z, cap) * 2 < cus) cap = std::max(nsb / 2, 1u);

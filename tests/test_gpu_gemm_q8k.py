@@ -358,7 +358,8 @@ def test_few_tokens_without_room_for_the_tile_keep_their_kernel(pkg, orc, monkey
 
 def _bits_of_both_forms(pkg, monkeypatch, m, n, k):
     """ojh_mm on int8 activations with the form that has a CU to itself switched off and as chosen"""
-    w, x = _case(pkg, m, n, k, "xk-route")
+    w, x = _case(pkg, m, 64, k, "xk-route")
+    w = np.tile(w.reshape(64, -1), (n // 64 + 1, 1))[:n].ravel()
     outs = []
     for xk in ("0", "1"):
         monkeypatch.setenv("OJAS_HIP_Q4K_XK", xk)
@@ -375,5 +376,12 @@ def _bits_of_both_forms(pkg, monkeypatch, m, n, k):
 @pytest.mark.parametrize("m,n,k,taken", [(24, 6000, 1024, False), (24, 3500, 2048, False), (24, 2100, 2048, True), (24, 4000, 2304, True), (24, 8300, 1024, True)])
 def test_few_tokens_take_the_tile_on_long_or_many_rows(pkg, monkeypatch, m, n, k, taken):
     """On short rows the few-token kernel stays ahead unless it walks two tiles a wave; seen by the order of the sums."""
+    old, new = _bits_of_both_forms(pkg, monkeypatch, m, n, k)
+    assert np.array_equal(old, new) != taken
+
+
+@pytest.mark.parametrize("m,n,k,taken", [(70, 8300, 12288, False), (60, 8300, 12288, True), (70, 11000, 12288, True)])
+def test_three_slices_of_whole_tiles_stay_with_two_workgroups_a_cu(pkg, monkeypatch, m, n, k, taken):
+    """130 tiles of more than 64 tokens over three slices of K keep the form that shares a CU; 64 tokens, and two slices, do not."""
     old, new = _bits_of_both_forms(pkg, monkeypatch, m, n, k)
     assert np.array_equal(old, new) != taken
