@@ -786,18 +786,21 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
 // One small K-quant projection of one token: quantizer and matvec in one launch.  It repeats the quantization in every
 // workgroup and keeps fewer bytes in flight than the plain matvec, so it stays with matrices whose second launch costs more.
 // Two launches / one, call to call, us: 1024 x 4096 Q4_K 8.0 / 4.4; 4096^2 Q4_K 7.8 / 4.6, Q5_K 7.9 / 5.1, Q6_K 7.8 / 6.0; 14336
-// x 4096 Q4_K 9.1 / 8.5, Q5_K 11.8 / 9.9, Q6_K 11.4 / 12.9 (8192 x 4096 8.5 / 8.8); 4096 x 8192 Q4_K 7.9 / 7.2, Q5_K 8.1 / 7.9,
-// Q6_K 8.7 / 9.0; 1024 x 8192 Q6_K 8.0 / 6.7; 1024 x 14336 Q4_K 8.0 / 8.2, Q5_K 8.3 / 8.7, Q6_K 8.0 / 9.5; where the host
-// issues a launch in 3 us instead of 4: 1024 x 4096 Q4_K 6.1 / 3.7, 3000 x 6144 6.1 / 5.2, 30000 x 1792 8.5 / 8.8, 12000 x 4096
-// Q5_K 10.6 / 8.9, 2000 x 8192 Q6_K 6.4 / 6.6.
+// x 4096 Q4_K 9.1 / 8.5, Q5_K 11.8 / 9.9; where the host issues a launch in 3 us instead of 4: 1024 x 4096 Q4_K 6.1 / 3.7, 30000 x
+// 1792 8.5 / 8.8, 12000 x 4096 Q5_K 10.6 / 8.9, 2000 x 6144 6.6 / 5.9.
+// Beyond sixteen rows a CU, one a wave, the waves take a second pair of rows while others idle: that pays for a short walk over K only
+// (K > 4096: 4468 x 5632 Q5_K 7.2 / 8.3, 4311 x 4864 Q4_K 6.6 / 6.9), and for Q6_K, four lanes a super-block, not at all (9216 x 1024
+// 6.8 / 7.8, 6144 x 2048 6.7 / 7.2, 4369 x 3840 6.7 / 7.7).  A longer K costs steps: 2800 x 8192 Q4_K 6.6 / 6.8, 2304 x 8192 Q5_K
+// 6.7 / 7.3, 1500 x 8192 6.6 / 6.9, 1024 x 14336 Q4_K 8.0 / 8.2, Q6_K 8.0 / 9.5.
 // Not where y lies over x: a workgroup may store its rows before another has read the token.
 static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y) {
-    const uint64_t mi = ((uint64_t)w->n * w->k + (1u << 20) - 1) >> 20;
+    const uint32_t K = w->k, mi = (uint32_t)(((uint64_t)w->n * K + (1u << 20) - 1) >> 20);
     if ((w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) || overlap(x, x_bytes, y, (size_t)w->n * 4)) return false;
-    if (dev->fq_one != 1) return dev->fq_one == 2 && w->k <= 16384u;
-    if (w->n >= 32768u) return false;              // (heads have forms of their own)
-    if (w->type == OJH_Q6_K) return mi <= (w->k <= 4096u ? 16u : w->k <= 8192u ? 8u : 0u);
-    return mi <= (w->k > 8192u ? 0u : w->k > 4096u ? 24u : w->type == OJH_Q5_K ? 56u : 32u);
+    if (dev->fq_one != 1) return dev->fq_one == 2 && K <= 16384u;
+    if (w->n >= 32768u || K > 8192u) return false; // (heads have forms of their own)
+    if (w->type != OJH_Q6_K && K <= 4096u) return mi <= (w->type == OJH_Q5_K ? 56u : 32u);
+    if (w->n > 16u * (uint32_t)dev->prop.multiProcessorCount) return false;
+    return mi <= (w->type == OJH_Q6_K ? (K <= 4096u ? 16u : 8u) : w->type == OJH_Q4_K ? 18u : K <= 6144u ? 14u : 8u);
 }
 static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum) {
     const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;

@@ -734,3 +734,23 @@ def test_one_projection_written_over_its_token(gpu, pkg, ty, multi, y_off):
     got = gpu.read(both, 2048)
     assert np.array_equal(got[y_off // 4:y_off // 4 + n].view(np.uint32), gpu.read(yd, n).view(np.uint32))
     assert np.array_equal(got[:y_off // 4], x[:y_off // 4])
+
+
+@pytest.mark.parametrize("ty,n,k,one", [(Q6_K, 4096, 1024, True), (Q6_K, 4100, 1024, False), (Q5_K, 4100, 4096, True), (Q5_K, 4100, 4352, False),
+                                        (Q5_K, 1024, 8192, True), (Q5_K, 1100, 8192, False), (Q4_K, 2300, 8192, True), (Q4_K, 2400, 8192, False)])
+def test_one_launch_where_it_is_ahead(pkg, monkeypatch, ty, n, k, one):
+    """One row a wave beyond K = 4096 and for Q6_K, and fewer weights the longer K is.  The two launches stage the token in scratch,
+    which the one launch can do without: a limit too small for it tells them apart."""
+    monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", "1")
+    raw, x = _inputs(pkg, ty, 64, k, "one-rule")
+    raw = np.tile(np.asarray(raw).reshape(64, -1), (n // 64 + 1, 1))[:n].ravel()
+    g = pkg.HipGpu(0)
+    try:
+        xd, lin, y = g.upload(x), g.lin(ty, n, k, raw), g.alloc(n)
+        if one:
+            g.mm(xd, lin, y, 1, act_mode=pkg.ACT_Q8K)
+        else:
+            with pytest.raises(pkg.OjasHipError, match="OJAS_HIP_SCRATCH_MAX"):
+                g.mm(xd, lin, y, 1, act_mode=pkg.ACT_Q8K)
+    finally:
+        g.close()
