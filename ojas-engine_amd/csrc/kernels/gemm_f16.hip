@@ -14,7 +14,8 @@
 // to cover a trip to memory with (128 x 128: four steps of 32 KB).  The barrier of a step sits before its last K
 // sub-step, whose fragments are in registers by then: its matrix instructions cover the next step's first fragments
 // and the requests for the step that takes over the slot.
-// `_kw` (what ojh_mm launches from K = 2816, and of 256 x 128 always): one wave a SIMD waits out every copy and fragment read that is late, and a
+// `_kw` (what ojh_mm launches but for a short K, and for few tokens on grids that fill the chip: f16d_eight_waves): one wave a SIMD
+// waits out every copy and fragment read that is late, and a
 // second wave with a tile of its own finds no room in LDS.  Two waves on the same tile, two of a step's four sub-steps each,
 // read no more of LDS and fill each other's gaps; their sums meet once, through LDS.  With the decode pass: Q8_0 4096 x 14336
 // at 2048 tokens 254 -> 238 us, at 1024 155 -> 149; IQ4_XS 8192^2 at 384 96 -> 92; Q6_K 6914 x 2816 at 333 34.3 -> 33.0.

@@ -638,6 +638,18 @@ static uint32_t f16d_tile(const ojh_device *dev, uint32_t N, uint32_t m) {   // 
     const uint64_t c1 = 8 * rounds(128, 128), c2 = 13 * rounds(256, 128), c3 = 23 * rounds(256, 256);
     return c3 <= c1 && c3 <= c2 ? 2u : c2 < c1 ? 1u : 0u;
 }
+// Whether that tile (0 or 1) runs on eight waves, which pay for their sums' meeting by filling each other's gaps.  Whole calls on four
+// / eight, mean and worst of random ones beyond 256 tokens: 128 x 128 from K = 2304 0.96 / 0.98 in one round of workgroups over the CUs
+// as in several, below that 1.00 - 1.03 / 1.08 in several; 256 x 128 in one round 0.94 / 1.03 from K = 1024, in several 1.04 / 1.10 at
+// K = 1024, 1.00 / 1.03 at 1280, 0.95 - 0.98 / 1.02 from 1536.  Up to 256 tokens a row of weights meets two tiles or one, and what
+// fetches it bounds: 0.96 / 1.05 up to three quarters of the CUs (128 x 128; 256 x 128 where the decoded rows stay in the caches, 0.93 -
+// 0.95), 1.01 - 1.08 / 1.11 otherwise.  us: Q8_0 4096 x 2816 at 1900 tokens 57.2 / 54.1, Q6_K 9500 x 8192 at 200 101 / 96, IQ3_XXS 23484 x
+// 7936 at 251 252 / 277, IQ4_NL 26621 x 1024 at 1241 116 / 126.
+static bool f16d_eight_waves(const ojh_device *dev, uint32_t N, uint32_t K, uint32_t m, uint32_t tile) {
+    const uint64_t cus = (uint64_t)dev->prop.multiProcessorCount, bm = tile ? 256 : 128, tiles = (uint64_t)((N + 127) / 128) * ((m + bm - 1) / bm);
+    if (tile ? K < 1536 && tiles > cus : K < 2304) return false;
+    return m > 256 || (4 * tiles <= 3 * cus && (!tile || (uint64_t)N * K <= 56u << 20));
+}
 // whether the tile that decodes on the way into LDS is 128 tokens tall instead of 256
 static bool gemm_mm_m128(const ojh_device *dev, uint32_t N, uint32_t m, bool decoded) {
     const uint64_t t256 = (uint64_t)((N + 127) / 128) * ((m + 255) / 256);
@@ -745,11 +757,8 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     ojh_buf *xh, *wdeq;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
     if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;
-    // (eight waves pay for their sums' meeting from some 44 K steps on: 128 x 128 tiles, all CUs busy, with the decode pass, four
-    // / eight: 2048 x 1024 at 2048 tokens 25 / 28 us, x 2048 31.5 / 35, x 2560 36.7 / 38.6, x 3072 at 1900 40.9 / 40.0; 6914 x
-    // 2816 at 333 34.3 / 33.2; 4096 x 4096 at 1024 52.5 / 50.2.  256 x 128: 4096 x 2048 at 2048 48.9 / 48.3, 10000 x 1536 at
-    // 700 41.7 / 40.2, 4096 x 1024 at 2048 level)
-    const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? "gemm_f16d_256x128_kw" : K >= 2816 ? "gemm_f16d_128_kw" : "gemm_f16d_128";
+    const bool kw = f16d_eight_waves(dev, N, K, m, tile);
+    const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? (kw ? "gemm_f16d_256x128_kw" : "gemm_f16d_256x128") : kw ? "gemm_f16d_128_kw" : "gemm_f16d_128";
     uint32_t sg[3], sb[3];
     bool sk = false;
     if (!tile) {

@@ -704,3 +704,26 @@ def test_q4k_batch_written_over_its_tokens(orc, pkg):
         assert peak_err(got[:, rows], want) <= 2 * k * 2.0 ** -24 and peak_err(g.read(yd, m * n).reshape(m, n)[:, rows], want) <= 2 * k * 2.0 ** -24
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("n,k,m,kernel", [(4352, 2304, 500, "gemm_f16d_128_kw"), (4352, 2048, 500, "gemm_f16d_128"), (8320, 2304, 250, "gemm_f16d_128_kw"),
+                                          (12800, 2304, 250, "gemm_f16d_128"), (16512, 1024, 250, "gemm_f16d_256x128_kw"), (25000, 1024, 250, "gemm_f16d_256x128"),
+                                          (10123, 1024, 1958, "gemm_f16d_256x128"), (10123, 1536, 1958, "gemm_f16d_256x128_kw")])
+def test_copied_tile_takes_eight_waves_by_size(pkg, n, k, m, kernel):
+    """Short K, and few tokens on grids that fill the chip, keep four waves.  The expected kernel on the decoded rows gives ojh_mm's
+    bits; the others add in another order."""
+    block = n // 32 + 1
+    raw = np.tile(np.asarray(pkg.synth.weights(18, 32, k, "kw", k)).view(np.uint8).reshape(32, -1), (block, 1))[:n].ravel()
+    x = pkg.synth.normal_f32(m * k, "kw", "x", m, k)
+    g = pkg.HipGpu(0)
+    try:
+        lin, wd, yd, y2 = g.lin(18, n, k, raw), g.upload_bytes(raw), g.alloc(m * n), g.alloc(m * n)
+        g.mm(g.upload(x), lin, yd, m, act_mode=pkg.ACT_AUTO)
+        assert g.has_kernel("gemm_f16d_128")
+        xh, w16 = g.upload_bytes(x.astype(np.float16).view(np.uint8)), g.alloc_bytes(n * k * 2)
+        g.dequant_f16(18, wd, n * k, w16)
+        grid, threads = g.launch_shape(kernel, k, n, m)
+        g.dispatch(g.begin(), kernel, [(xh, 0), (w16, 0), (y2, 0)], [k, n, 0, m], grid, threads)
+        assert np.array_equal(g.read(yd, m * n).view(np.uint32), g.read(y2, m * n).view(np.uint32))
+    finally:
+        g.close()
