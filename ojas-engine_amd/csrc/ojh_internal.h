@@ -16,6 +16,7 @@ struct ojh_buf {
     size_t bytes = 0;
     bool owned = false;
     bool recorded = false;       // scratch handed out while a chain was recorded
+    bool spare = false;          // scratch that no call has needed since it was allocated (ojh_scratch_spare)
 };
 
 struct ojh_lin {
@@ -183,7 +184,8 @@ const ojh_kernel_spec *ojh_find_kernel(const char *name);
 // ---- helpers -----------------------------------------------------------------------------------
 int ojh_scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out);
 // ... one the caller can do without: fails, and leaves the slot as it is, where memory is short; `ahead`: with the quarter of
-// growing room that ojh_scratch_get adds, where there is room for it
+// growing room that ojh_scratch_get adds, where there is room for it.  Given back when ojh_scratch_get would be refused, so a call
+// asks for what it needs before what it can do without
 int ojh_scratch_spare(ojh_device *dev, const char *name, size_t bytes, ojh_buf **out, bool ahead = false);
 // ... whether several such fit what they are limited to together, asked before the first of them takes its room
 bool ojh_scratch_fits(const ojh_device *dev, std::initializer_list<std::pair<const char *, size_t>> wanted);

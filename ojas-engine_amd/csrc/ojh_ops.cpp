@@ -237,8 +237,12 @@ static int q4k_xt_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, const voi
     if (z == 1 ? !ojh_scratch_fits(dev, {{"xt_xst", xst}, {"xt_sums", sums}})
                : !ojh_scratch_fits(dev, {{"xt_xst", xst}, {"xt_sums", sums}, {"xt_part", part}, {"xt_cnt", cnt}}))
         return XT_NO;
-    return (z == 1 || (!ojh_scratch_spare(dev, "xt_part", part, &b) && !ojh_scratch_get_zeroed(dev, "xt_cnt", cnt, &b))) &&
+    return (z == 1 || (!ojh_scratch_get_zeroed(dev, "xt_cnt", cnt, &b) && !ojh_scratch_spare(dev, "xt_part", part, &b))) &&
            !ojh_scratch_spare(dev, "xt_sums", sums, &b) && !ojh_scratch_spare(dev, "xt_xst", xst, &b) ? XT_TAKE : XT_NO;
+}
+
+static int xt_scratch(ojh_device *dev, const ojh_lin *w, uint32_t m, const char *name, size_t bytes, ojh_buf **out) {
+    return m >= q4k_xt_min_tokens(dev, w->k, w->n) ? ojh_scratch_get(dev, name, bytes, out) : ojh_scratch_spare(dev, name, bytes, out);
 }
 
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,
@@ -274,8 +278,7 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
         const uint32_t mp = (m + 127) / 128 * 128;
         const size_t nsb = K / 256;
         ojh_buf *xst, *sums;
-        if ((rc = ojh_scratch_get(dev, "xt_xst", nsb * mp * 4, &xst))) return rc;
-        if ((rc = ojh_scratch_get(dev, "xt_sums", nsb * mp * 32, &sums))) return rc;
+        if ((rc = xt_scratch(dev, w, m, "xt_xst", nsb * mp * 4, &xst)) || (rc = xt_scratch(dev, w, m, "xt_sums", nsb * mp * 32, &sums))) return rc;
         uint32_t sg[3], sb[3];
         if (xt != XT_SIDES) {
             const char *sides = q4k_xk_slices(dev, K, N, m) ? "q8k_token_sides_h" : "q8k_token_sides";
@@ -295,7 +298,7 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
             }
             if (z == 1) return ojh_launch(dev, "gemm_q8k_q4k_xk64", {xq, xst->ptr, sums->ptr, wp, yp}, {K, N, m, (uint32_t)(accum != 0), mp}, sg, sb);
             ojh_buf *part, *cnt;
-            if ((rc = ojh_scratch_get(dev, "xt_part", tiles * z * 32768, &part))) return rc;
+            if ((rc = xt_scratch(dev, w, m, "xt_part", tiles * z * 32768, &part))) return rc;
             if ((rc = ojh_scratch_get_zeroed(dev, "xt_cnt", tiles * 4, &cnt))) return rc;
             return ojh_launch(dev, "gemm_q8k_q4k_xk64_sr", {xq, xst->ptr, sums->ptr, wp, yp, part->ptr, cnt->ptr},
                               {K, N, m, (uint32_t)(accum != 0), mp, z}, sg, sb);
@@ -756,7 +759,7 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     int rc;
     ojh_buf *xh, *wdeq;
     if ((rc = ojh_scratch_get(dev, "xh", (size_t)m * K * 2, &xh))) return rc;
-    if ((rc = ojh_scratch_get(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;
+    if ((rc = ojh_scratch_spare(dev, "wdeq", (size_t)N * K * 2, &wdeq))) return rc;   // (there: f16d_ready)
     const bool kw = f16d_eight_waves(dev, N, K, m, tile);
     const char *name = tile == 2 ? "gemm_f16d_256" : tile == 1 ? (kw ? "gemm_f16d_256x128_kw" : "gemm_f16d_256x128") : kw ? "gemm_f16d_128_kw" : "gemm_f16d_128";
     uint32_t sg[3], sb[3];
@@ -1096,8 +1099,7 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
             if ((rc = ensure(dev, "gemm_q8k"))) return rc;
             const uint32_t mp = (m + 127) / 128 * 128;
             ojh_buf *xst, *sums;
-            if ((rc = ojh_scratch_get(dev, "xt_xst", nsb * mp * 4, &xst))) return rc;
-            if ((rc = ojh_scratch_get(dev, "xt_sums", nsb * mp * 32, &sums))) return rc;
+            if ((rc = xt_scratch(dev, w, m, "xt_xst", nsb * mp * 4, &xst)) || (rc = xt_scratch(dev, w, m, "xt_sums", nsb * mp * 32, &sums))) return rc;
             uint32_t qg[3] = {K / 256 * (mp / 4), 1, 1};
             const std::string quant = std::string(x_dtype == OJH_X_BF16 ? "quantize_q8k_bf16_sides" : "quantize_q8k_sides") +
                                       (q4k_xk_slices(dev, K, N, m) ? "_h" : "");

@@ -268,6 +268,16 @@ static size_t scratch_held(const ojh_device *dev) {
     return held;
 }
 
+// What calls can do without is given back, but for what a recorded chain holds.
+static void give_back_spare(ojh_device *dev, const ojh_buf *but) {
+    for (auto &slot : dev->scratch) {
+        ojh_buf *&b = slot.second;
+        if (!b || b == but || !b->spare || (b->recorded && dev->live_graphs > 0)) continue;
+        ojh_free(dev, b);
+        b = nullptr;
+    }
+}
+
 // `fresh` (optional) tells whether the slot was (re)allocated by this call: its contents are then undefined.
 // `spare`: a buffer the caller can do without.  It is not allocated where it would leave less memory free than it takes, nor
 // ahead of its size unless `ahead`, and a smaller one in the slot is given up only once the larger is there.
@@ -281,8 +291,12 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
         const bool park = slot && slot->recorded && dev->live_graphs > 0;   // a recorded chain may still replay into it
         size_t cap = bytes < 4096 ? 4096 : ahead ? bytes + bytes / 4 : bytes;
         if (dev->scratch_max) {
-            const size_t held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
+            size_t held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
             if (held + cap > dev->scratch_max) cap = bytes;
+            if (held + cap > dev->scratch_max && !spare) {
+                give_back_spare(dev, slot);
+                held = scratch_held(dev) - (slot && !park ? slot->bytes : 0);
+            }
             if (held + cap > dev->scratch_max)
                 return ojh_fail(OJH_ERR_HIP, "scratch '%s' of %zu bytes beside %zu exceeds OJAS_HIP_SCRATCH_MAX", name, bytes, held);
         }
@@ -304,9 +318,14 @@ static int scratch_get(ojh_device *dev, const char *name, size_t bytes, ojh_buf 
             return rc;
         }
         slot = grown;
-        if (!slot && (rc = ojh_alloc(dev, cap, &slot))) return rc;
+        if (!slot && ojh_alloc(dev, cap, &slot)) {
+            give_back_spare(dev, nullptr);
+            if ((rc = ojh_alloc(dev, cap, &slot))) return rc;
+        }
+        slot->spare = spare;
         if (fresh) *fresh = true;
     }
+    if (!spare) slot->spare = false;
     if (dev->capturing) slot->recorded = true;
     *out = slot;
     return OJH_OK;

@@ -165,3 +165,33 @@ def test_a_batch_that_cannot_have_all_its_scratch_takes_none(pkg, orc, monkeypat
         g.mm(xo, other, yo, (part + room - 4096) // (K * 2), act_mode=pkg.ACT_FLOAT)      # f16 activations that fill the limit but for 4 KB
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("first", ["decoded", "int8", "few"])
+def test_scratch_that_a_call_could_do_without_is_given_back(pkg, orc, monkeypatch, first):
+    """A limit that holds what two calls need one after the other: what the first took beside, for speed, does not refuse the second."""
+    n, k, m = 1100, 2304, 1900
+    w = pkg.synth.q4k_weights(n, k, "scratch", "back")
+    x = pkg.synth.normal_f32(m * k, "scratch", "x-back", m)
+    need = 2000 * K * 2                                      # f16 activations of the second call
+    room = {"decoded": m * k * 5 // 2 + n * k * 2 + 4096, "int8": need + 128 * 1024, "few": need}[first]
+    monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", str(room))
+    g = pkg.HipGpu(0)
+    try:
+        xd, yd = g.upload(x), g.alloc(m * n)
+        if first == "decoded":                               # the decoded rows beside the activations
+            g.mm(xd, g.lin(12, n, k, w), yd, m, act_mode=pkg.ACT_AUTO)
+            assert g.has_kernel("gemm_f16d_128")
+            need = room - 1024 * 1024
+        elif first == "int8":                                # the side arrays of the 64-row tile
+            w4 = pkg.synth.q4k_weights(2112, 4096, "scratch", "back")
+            g.mm(xd, g.lin(12, 2112, 4096, w4), yd, 24, act_mode=pkg.ACT_Q8K)
+        else:                                                # one token's int8 copy
+            g.mm(xd, g.lin(12, n, k, w), yd, 1, act_mode=pkg.ACT_Q8K)
+        toks = need // (K * 2)
+        xo = pkg.synth.normal_f32(toks * K, "scratch", "x-back2").reshape(toks, K)
+        yo = g.alloc(toks * 256)
+        g.mm(g.upload(xo), g.lin(Q6_K, 256, K, _weights(pkg, 256)), yo, toks, act_mode=pkg.ACT_FLOAT)
+        _check(g, yo, 256, toks, slice(0, 4), _want(pkg, orc, xo[:4]))
+    finally:
+        g.close()
