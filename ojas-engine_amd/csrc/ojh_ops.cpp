@@ -165,6 +165,8 @@ static int pick_rows(const ojh_device *dev, uint32_t n) {
 // workgroups per CU is the aim, with at most eight slices of at least four super-blocks each (two, where four would
 // leave more than half the CUs idle); a grid that already covers more than half the CUs is sliced only when a slice
 // keeps sixteen super-blocks.  1 = unsliced; 0 = even sliced, most CUs would idle: another kernel takes the product.
+// By default the form that has a CU to itself (q4k_xk_slices) runs these grids but for three slices of more than half the CUs'
+// tiles: for the others this says whether the int8 tile is taken at all, and what scratch is left behind for recorded calls.
 static uint32_t q4k_xt_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
     const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount, nsb = K / 256;
     const uint64_t tiles = (uint64_t)((N + 63) / 64) * ((m + 127) / 128);
@@ -624,17 +626,20 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
 // 128 or 256 tokens; the pass reads and writes everything once.  Which is ahead is a matter of rounds of workgroups over the
 // CUs more than of rows or tokens, so both are priced, in us: K steps on the busiest CU times what a step takes (a part
 // that does not depend on how many CUs are busy, and one that grows with them), the atomics that K slices meet in, the
-// pass.  The prices are fitted to 39000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048 tokens): what
-// they choose is on average within 0.8 % of the faster route, and 4 % or more behind the decoding tile in one call of 90
-// (by tokens and rows alone 1.7 %, and one of 40).  Both routes measured, decoding tile / pass + copying tile:
+// pass.  The prices are fitted to 39000 timed calls (14 formats, 128 - 152064 rows, K 512 - 14336, 129 - 2048 tokens) with the
+// copying tile on four waves: what they choose was on average within 0.8 % of the faster route, and 4 % or more behind the
+// decoding tile in one call of 90 (by tokens and rows alone 1.7 %, and one of 40).  On eight waves that tile takes some 5 % less
+// than it is priced at, so that near the line a call may stay with the decoding one.  Both routes measured then, decoding tile /
+// pass + copying tile:
 //   Q6_K   6914 x 2816 at 333 tokens 60 / 37, 14336 x 4096 at 130 79 / 71, 4096 x 4096 at 700 83 / 45
 //   IQ4_NL 5330 x 11776 at 333 95 / 85, 8192 x 14336 at 333 162 / 215 (decoded rows beyond 112 MB: read back from memory)
 //   Q5_0   8576 x 4096 at 257 106 / 51, MXFP4 8192 x 14336 at 512 188 / 249, Q4_1 8192 x 1024 at 512 26 / 32
 static uint32_t f16d_tile(const ojh_device *dev, uint32_t N, uint32_t m) {   // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256 tokens x rows
-    // rounds of workgroups over the chip times a K step of the tile (fitted over 6650 timed calls, launch, decode pass and
-    // stores apart: 0.49 / 0.83 / 1.37 us with every CU busy on four waves): within 0.13 % of the fastest of the three on
-    // average; 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 / 279 / 388;
-    // 6914 x 2816 at 333 35 / 51 / 76.  On eight waves the first two take 6 - 8 % less (0.46 / 0.77)
+    // rounds of workgroups over the chip times a K step of the tile, fitted over 6650 timed calls with all three on four waves
+    // (launch, decode pass and stores apart: 0.49 / 0.83 / 1.37 us with every CU busy; within 0.13 % of the fastest of the three on
+    // average): 14336 x 4096 at 512 tokens 108 / 100 / 122 us, at 2048 308 / 294 / 262; 4096 x 14336 at 2048 334 / 279 / 388; 6914 x
+    // 2816 at 333 35 / 51 / 76.  Where the first two run on eight waves (f16d_eight_waves) they take 6 - 8 % less, which these
+    // weights do not know
     const uint64_t cus = (uint64_t)dev->prop.multiProcessorCount;
     auto rounds = [&](uint32_t bm, uint32_t bn) { return ((uint64_t)((N + bn - 1) / bn) * ((m + bm - 1) / bm) + cus - 1) / cus; };
     if (dev->f16d_tile > 0) return (uint32_t)dev->f16d_tile - 1u;
@@ -709,11 +714,11 @@ static bool f16d_pays_q4k(const ojh_device *dev, uint32_t N, uint32_t K, uint32_
     const double copied = tile == 2   ? 0.345 * mi + 0.481 * over + price(256, 256, 0, {2.2, 0.24, 0.827, 0.802, 0.0, 0.50, 8.9})
                           : tile == 1 ? 0.263 * mi + 0.735 * over + price(256, 128, 0, {6.5, 0.06, 0.306, 0.547, 0.0, 0.68, 5.8})
                                       : 0.422 * mi + 0.684 * over + price(128, 128, K / 512, {7.5, 0.77, 0.173, 0.218, 3.59, 1.92, 0.35});
-    // the tile that ojh_mm takes otherwise
+    // the tile that ojh_mm takes otherwise (1024 <= K <= 8192 here)
     const uint64_t t256 = (uint64_t)((N + 255) / 256) * ((m + 255) / 256), t128 = (uint64_t)((N + 255) / 256) * ((m + 127) / 128);
     const uint32_t z128 = (uint32_t)((uint64_t)cus / t128);
     const bool tall = t256 >= (uint64_t)cus || (2 * t256 >= (uint64_t)cus && K >= 8192);
-    const double loaded = !tall && K >= 1024 && z128 >= 2 && (K <= 8192 || z128 >= 4) ? price(128, 64, K / 1024, {4.4, 1.26, 0.215, 0.037, 3.01, 1.33, 4.7})
+    const double loaded = !tall && z128 >= 2 ? price(128, 64, K / 1024, {4.4, 1.26, 0.215, 0.037, 3.01, 1.33, 4.7})
                           : tall ? price(256, 256, K / 256, {5.3, 0.64, 1.059, 0.683, 2.29, 0.39, 5.2})
                                  : price(128, 256, K / 256, {11.4, 0.75, 0.436, 0.509, 2.24, 0.15, 0.0});
     return 1.05 * copied < loaded;
