@@ -6,6 +6,8 @@
 // (MOE_FORMATS), and the name -> family registry in crates/ojas-cuda/src/kernels/mod.rs:111-145.
 #include <cstring>
 #include <deque>
+#include <string_view>
+#include <unordered_map>
 
 #include "ojh_internal.h"
 
@@ -2325,11 +2327,16 @@ const std::vector<ojh_kernel_spec> &ojh_manifest_table() {
     return table;
 }
 
+// (every eager call that asks for a launch shape comes here; row by row the last of 493 names took 1.3 us, a third of a launch)
 const ojh_kernel_spec *ojh_find_kernel(const char *name) {
+    static const std::unordered_map<std::string_view, const ojh_kernel_spec *> index = [] {
+        std::unordered_map<std::string_view, const ojh_kernel_spec *> by_name;
+        for (const auto &s : ojh_manifest_table()) by_name.emplace(s.name, &s);
+        return by_name;
+    }();
     if (!name) return nullptr;
-    for (const auto &s : ojh_manifest_table())
-        if (!strcmp(s.name, name)) return &s;
-    return nullptr;
+    const auto it = index.find(name);
+    return it == index.end() ? nullptr : it->second;
 }
 
 extern "C" const char *ojh_kernel_family(const char *name) {

@@ -107,3 +107,22 @@ def test_open_without_a_gpu_fails_loudly(pkg):
     with pytest.raises(pkg.OjasHipError) as e:
         pkg.HipGpu(0)
     assert "no CPU fallback" in str(e.value) or "device" in str(e.value).lower()
+
+
+def test_finding_a_kernel_takes_no_longer_at_the_end_of_the_manifest(pkg):
+    """Eager calls look their kernels up, so the cost must not grow with the table: the last name is found as fast as the
+    first.  Row by row it took 4 times as long, call overhead included; the bound lies halfway."""
+    import time
+    lib = pkg.load_library()
+
+    def seconds(name):
+        best = 1.0
+        for _ in range(9):
+            t = time.perf_counter()
+            for _ in range(2000):
+                lib.ojh_kernel_family(name)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    m = pkg.manifest()
+    assert seconds(m[-1][0].encode()) < 2 * seconds(m[0][0].encode())
