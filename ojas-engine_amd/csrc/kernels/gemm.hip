@@ -858,15 +858,16 @@ GEMM_ENTRIES(q3k, LoaderQ3K)
 //   gemm_few_<fmt>{,_r4}_t{1,2,4}(xh, w, y, K, N, accum, M)     grid [ceil(N / 16 RG),1,1] x 256 (or 512 where RG TG <= 8),
 //   K a multiple of 128, M <= 16 TG; `_r4`: RG = 4 groups of 16 rows per workgroup; accum 1: y += ; accum 2 (or 3): xh in the
 //   order of few_x_{f32,bf16}
-// Bound by latency: a wave waits a trip to memory per chunk for its tokens and the next block, and with 64 rows a workgroup
-// there is less than one workgroup per CU on most matrices.  So `_r4_t2` runs eight waves where there are fewer than two
+// Bound by the decoding's vector instructions (5 a weight; IQ4_XS 14336 x 4096 at 24 tokens: two thirds of the issue slots of a
+// SIMD with its two waves), and behind them by memory, which a wave waits for 42 % of its time: once per chunk for its tokens and
+// the next block.  With 64 rows a workgroup there is less than one workgroup per CU on most matrices, so that four waves leave the
+// slots empty while they wait: `_r4_t2` runs eight where there are fewer than two
 // workgroups per CU, each with half the chunks; the kernel alone, four -> eight waves, us: IQ4_XS 14336 x 4096 at 17 / 32 tokens
 // 20.0 -> 16.0 / 22.1 -> 18.9, x 14336 69.9 -> 48.7 / 76.6 -> 56.0, 28672 x 4096 31.2 -> 30.0 / 36.0 -> 35.6; Q8_0, whose
 // bytes bound it sooner, 0 - 2 % (30.4 -> 29.6 at 14336 x 4096), never slower up to 32640 rows.
 // Row by row, a load of the tokens' pieces touches 64 lines for 16 bytes each and the address unit walks them one by one: 7 of
 // the 16 us of 24 tokens.  In fragment order (few_x_*) it is 1 KB in a row.  With the conversion, us: IQ4_XS 14336 x 4096 at 24
-// tokens 19.5 -> 17.2, 4096^2 at 24 11.3 -> 8.6, 4096 x 14336 at 16 19.9 -> 15.8, Q8_0 14336 x 4096 at 24 31.9 -> 29.1.  Now bound by
-// the decoding's vector instructions (5 a weight).
+// tokens 19.5 -> 17.2, 4096^2 at 24 11.3 -> 8.6, 4096 x 14336 at 16 19.9 -> 15.8, Q8_0 14336 x 4096 at 24 31.9 -> 29.1.
 typedef float float4v __attribute__((ext_vector_type(4)));
 template <int J, class L>
 __device__ __forceinline__ half8 gm_frag(const L& ld) {
