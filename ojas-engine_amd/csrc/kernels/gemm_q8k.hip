@@ -1021,115 +1021,118 @@ gemm_q8k_q4k_xt64_sr(const signed char* xq, const float* xst, const float* sums,
     gemm_q8k_q4k_xt_body<2, true>(xq, xst, sums, w, y, K, N, M, ACC, MP, lds_xt, part, cnt, NSPLIT);
 }
 
-// ---- Q6_K and Q5_K rows against batches of tokens: one matrix instruction per scale group ---------------------------
+// ---- Q6_K and Q5_K rows against batches of tokens: scales folded into two int8 digits ------------------------------
 //   gemm_q8k_{q6k,q5k}_gs(xq, xs, w, y, K, N, M, ACC)                      block 256, grid [ceil(N / 128), ceil(M / 64), 1]
 //   gemm_q8k_{q6k,q5k}_gs_sr(xq, xs, w, y, part, cnt, K, N, M, ACC, NSPLIT)       grid [.., .., slices]
 // The CPU path's arithmetic (dot_q6k / dot_q5k over quant_q8k activations, crates/ojas-cpu/src/cpu_math.rs:638-722) for
-// batches from a handful of tokens to prefill sizes.  A Q6_K scale covers 16 weights and is a full int8, so it cannot be
-// folded into int8 codes the way the Q4_K tile above folds its 6-bit scales; instead v_mfma_i32_32x32x16_i8, whose 16
-// positions are exactly one scale group, gives the group's integer dots for 32 tokens x 32 rows, and the scale enters
-// with one v_mad_i32_i24 per D register (the row is lane-constant in D).  Q5_K: one v_mfma_i32_32x32x32_i8 per 32-weight
-// sub-block (codes 0..31 are one int8 plane), the 6-bit scale likewise, and sum_j m_j bsum_j from two more
-// instructions per super-block over the sub-block sums split as 64 hi + lo (the workgroup splits them while it stages
-// the tokens).
+// batches from a handful of tokens to prefill sizes.  A weight's whole integer, scale x (code - 32) or scale x code, fits 14
+// bits: one packed 16-bit multiply-add forms twice that integer for two weights, and its bytes are the two signed digits
+// (gs_digits) that two accumulating v_mfma_i32_32x32x32_i8 take as they are — 256 D_hi + D_lo is twice the super-block's
+// integer sum, exactly, whatever the scales' groups.  Q5_K: sum_j m_j bsum_j from two more instructions per super-block over
+// the sub-block sums split as 64 hi + lo (the workgroup splits them while it stages the tokens).
 // A workgroup owns 128 rows x 64 tokens: wave w takes rows 32 w .. against both blocks of 32 tokens (only the first where
-// the last token tile holds no more).  B (weights): lane (n, kg) = (lane % 32, lane / 32) builds the codes of
-// positions 8 kg .. 8 kg + 7 of every group of row n from the raw bytes it loads itself, one super-block ahead — no two
-// waves of a workgroup build the same codes.  A (tokens): a super-block's 64 x 256 int8 wait in LDS, rows 264 bytes
-// apart (32 tokens' 8-byte reads then cover all banks), two stages, one barrier per super-block.  Integer sums are
-// exact; per super-block acc += sx * d * (float) isum, super-blocks in order.
+// the last token tile holds no more).  A wave's 32 rows of a super-block come in as 16-byte pieces, neighbouring lanes side
+// by side in a row, and pass through the wave's own part of LDS into operand order: lane (n, kg) = (lane % 32, lane / 32)
+// holds half kg of row n (Q6_K) or positions 16 kg .. of every sub-block (Q5_K).  A (tokens): a super-block's 64 x 256 int8
+// wait in LDS, rows 272 bytes apart (16 lanes' 16-byte reads then cover all banks), two stages, one barrier per super-block.
+// Per super-block acc += sx * d * (float) isum, super-blocks in order.
+// What bounded the form before (one instruction per scale group, the scale multiplied onto every result; a lane loading
+// 8-byte pieces of its own row) was neither its 937 vector instructions a step nor the matrix pipe but the address unit, 3100
+// cycles a step for sixteen rows per load: halving the instructions alone changed nothing (9638 x 3584 at 264 tokens 74.4 ->
+// 75.0 us), the pieces side by side 53.0 (2200 cycles, 543 vector instructions).  Now with the quantizer, Q6_K: 14336 x 4096
+// at 64 tokens 31.0 -> 26.5, 4096 x 4096 at 512 51.5 -> 41.5, 12992 x 10240 at 903 552 -> 445; Q5_K, whose aligned rows took
+// fewer loads: 14336 x 4096 at 512 138.8 -> 121.3, at 64 29.8 -> 27.0.  The same bits as before.
 // `_sr`: K slices whose partial tiles meet in `part` (tiles x slices x 32 KB), added in slice order by the last to arrive.
 #include "ojk_q6k_mfma.h"
 
 typedef int gs_i16 __attribute__((ext_vector_type(16)));
-#define GS_STRIDE 264u
+#define GS_STRIDE 272u
 #define GS_SX (64u * GS_STRIDE)         // the stage's 64 token scales
 #define GS_BS (GS_SX + 256u)            // Q5_K: the split sub-block sums, 16 bytes per token (lo_0..7, hi_0..7)
 #define GS_STAGE (GS_BS + 1024u)
+#define GS_ROWS 512u                    // a wave's 32 rows: bytes per piece of 16
 
-// A running integer sum, pinned after every group: integer additions may be reassociated, and left to itself the
-// compiler turns sixteen groups' multiply-adds into one tree at the end of the super-block, every group's sixteen result
-// registers alive until then (hundreds of spills).
-__device__ __forceinline__ int gs_pin(int v) {
-    asm("" : "+v"(v));
-    return v;
+// Two signed digits of twice a product, four products at a time: ev and od hold p + 128 in their 16-bit halves (products
+// 0, 2 and 1, 3), p even.  hi takes their upper bytes and lo their lower bytes with the sign bit flipped, so that
+// p = 256 hi + lo with both in int8, exactly.
+__device__ __forceinline__ void gs_digits(uint ev, uint od, int& hi, int& lo) {
+    hi = (int)__builtin_amdgcn_perm(od, ev, 0x07030501u);
+    lo = (int)(__builtin_amdgcn_perm(od, ev, 0x06020400u) ^ 0x80808080u);
+}
+// four codes (a byte each) times f, plus b
+__device__ __forceinline__ void gs_scale4(uint codes, gq_u16x2 f, gq_u16x2 b, int& hi, int& lo) {
+    const gq_u16x2 ev = __builtin_bit_cast(gq_u16x2, codes & 0x00FF00FFu) * f + b;
+    const gq_u16x2 od = __builtin_bit_cast(gq_u16x2, __builtin_amdgcn_perm(0u, codes, 0x0C030C01u)) * f + b;
+    gs_digits(__builtin_bit_cast(uint, ev), __builtin_bit_cast(uint, od), hi, lo);
 }
 
 struct GsQ6K {
     static constexpr uint BYTES = Q6K_BYTES;
+    static constexpr uint PIECES = 13u;         // of 16 bytes; the two bytes behind them are d
     static constexpr bool BSUMS = false;
     struct Raw {
-        u32x2_a2 la[2][2], lb[2][2], qh[2][2];   // [half][group of the quarter]: ql[16 h + 8 kg ..], ql[32 + ..], qh[..]
-        u32x4_a2 sc;
+        uint4 ql[4], qh[2];         // the lane's half of the super-block, kg: 64 bytes of nibbles, 32 of bit pairs
+        uint2 sc;                   // its eight scales
         uint d16;
     };
-    static __device__ __forceinline__ Raw load(const uchar* blk, uint kg) {
+    static __device__ __forceinline__ uint tail(const uchar* blk) { return *(const ushort*)(blk + 208u); }
+    static __device__ __forceinline__ Raw unpack(const uchar* row, uint kg, uint d16) {
         Raw r;
-        const uint sh = ((uint)(size_t)blk & 2u) << 3;
-        const uchar* b4 = blk - ((size_t)blk & 2u);
 #pragma unroll
-        for (int hf = 0; hf < 2; hf++)
+        for (int i = 0; i < 4; i++) r.ql[i] = *(const uint4*)(row + 64u * kg + 16u * (uint)i);
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                r.la[hf][h] = q6k_ld8(b4 + 64u * hf + 16u * h + 8u * kg, sh);
-                r.lb[hf][h] = q6k_ld8(b4 + 64u * hf + 32u + 16u * h + 8u * kg, sh);
-                r.qh[hf][h] = q6k_ld8(b4 + 128u + 32u * hf + 16u * h + 8u * kg, sh);
-            }
-        const uint* ps = (const uint*)(b4 + 192u);
-        const uint s0 = ps[0], s1 = ps[1], s2 = ps[2], s3 = ps[3], s4 = ps[4];
-        r.sc.x = __builtin_amdgcn_alignbit(s1, s0, sh);
-        r.sc.y = __builtin_amdgcn_alignbit(s2, s1, sh);
-        r.sc.z = __builtin_amdgcn_alignbit(s3, s2, sh);
-        r.sc.w = __builtin_amdgcn_alignbit(s4, s3, sh);
-        r.d16 = (s4 >> sh) & 0xFFFFu;
+        for (int i = 0; i < 2; i++) r.qh[i] = *(const uint4*)(row + 128u + 32u * kg + 16u * (uint)i);
+        r.sc = *(const uint2*)(row + 192u + 8u * kg);
+        r.d16 = d16;
         return r;
     }
-    // st: the stage; tok0: the wave's first token in it
+    // The digits of 2 sc (code - 32) for group g = 2 q + h of the lane's half: quarter q, positions 16 h .. 16 h + 15.
+    static __device__ __forceinline__ void planes(const Raw& r, int g, gq_i4& hi, gq_i4& lo) {
+        const int q = g >> 1, h = g & 1;
+        const uint4 l4 = r.ql[2 * (q & 1) + h], h4 = r.qh[h];
+        const int s2 = 2 * (int)(signed char)((g < 4 ? r.sc.x : r.sc.y) >> (8 * (g & 3)));
+        const gq_u16x2 f = {(ushort)s2, (ushort)s2};
+        const ushort bb = (ushort)(128 - 32 * s2);
+        const gq_u16x2 b = {bb, bb};
+        const uint ls[4] = {l4.x, l4.y, l4.z, l4.w}, hs[4] = {h4.x, h4.y, h4.z, h4.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint nib = (q & 2) ? ls[i] >> 4 : ls[i];
+            const uint two = q == 3 ? hs[i] >> 2 : q == 2 ? hs[i] : q == 1 ? hs[i] << 2 : hs[i] << 4;
+            int a, c;
+            gs_scale4((nib & 0x0F0F0F0Fu) | (two & 0x30303030u), f, b, a, c);
+            hi[i] = a;
+            lo[i] = c;
+        }
+    }
+    // st: the stage
     template <int NB>   // NB: how many of the wave's two 32-token blocks hold tokens
-    static __device__ __forceinline__ void superblock(const Raw& r, const uchar* st, uint tok0, uint fr, uint kg,
-                                                      float (&acc)[2][16]) {
-        const uchar* xa = st + (tok0 + fr) * GS_STRIDE + 8u * kg;            // the lane's token row of block 0, its 8 positions
-        const float* sx = (const float*)(st + GS_SX) + tok0 + 4u * kg;       // scales of its D registers' tokens: + 32 i + 8 (v / 4) + v % 4
-        int isum[NB][16];
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) isum[i][v] = 0;
+    static __device__ __forceinline__ void superblock(const Raw& r, const uchar* st, uint fr, uint kg, float (&acc)[2][16]) {
+        const uchar* xa = st + fr * GS_STRIDE + 128u * kg;                   // the lane's token row of block 0, its half
+        const float* sx = (const float*)(st + GS_SX) + 4u * kg;              // scales of its D registers' tokens: + 32 i + 8 (v / 4) + v % 4
         const gs_i16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        // group g = 8 hf + 2 q + h: quarter q of half hf, its positions 16 h .. 16 h + 15; scale byte g
-        auto codes = [&](int g) -> long {
-            const int hf = g >> 3, q = (g >> 1) & 3, h = g & 1;
-            const u32x2_a2 ql = (q & 1) ? r.lb[hf][h] : r.la[hf][h];
-            return q6k_signed8(ql.x, ql.y, r.qh[hf][h].x, r.qh[hf][h].y, q);
+        gs_i16 DH[NB], DL[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) DH[i] = zero, DL[i] = zero;
+        // the next group's operands are built under this group's matrix instructions
+        gq_i4 BH, BL, A[NB];
+        auto tokens = [&](int g) {
+#pragma unroll
+            for (int i = 0; i < NB; i++) A[i] = *(const gq_i4*)(xa + (uint)i * 32u * GS_STRIDE + 16u * (uint)g);
         };
-        auto tokens = [&](int g, int i) -> long {
-            return *(const long*)(xa + (uint)i * 32u * GS_STRIDE + 16u * (uint)g);
-        };
-        // the next group's operands are fetched and built under this group's matrix instructions, ahead of its multiply-adds
-        long B = codes(0), A0 = tokens(0, 0), A1 = NB == 2 ? tokens(0, 1) : 0;
+        planes(r, 0, BH, BL);
+        tokens(0);
 #pragma unroll
-        for (int g = 0; g < 16; g++) {
-            const uint sw = g < 4 ? r.sc.x : g < 8 ? r.sc.y : g < 12 ? r.sc.z : r.sc.w;
-            const int s = (int)(signed char)(sw >> (8 * (g & 3)));
-            const gs_i16 D0 = __builtin_amdgcn_mfma_i32_32x32x16_i8(A0, B, zero, 0, 0, 0);
-            gs_i16 D1 = zero;
-            if (NB == 2) D1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(A1, B, zero, 0, 0, 0);
-            if (g < 15) {
-                A0 = tokens(g + 1, 0);
-                if (NB == 2) A1 = tokens(g + 1, 1);
-                B = codes(g + 1);
+        for (int g = 0; g < 8; g++) {
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                DH[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], BH, DH[i], 0, 0, 0);
+                DL[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], BL, DL[i], 0, 0, 0);
             }
-#pragma unroll
-            for (int v = 0; v < 16; v++) isum[0][v] = gs_pin(isum[0][v] + __mul24(s, D0[v]));
-            if (NB == 2) {
-#pragma unroll
-                for (int v = 0; v < 16; v++) isum[NB - 1][v] = gs_pin(isum[NB - 1][v] + __mul24(s, D1[v]));
-            }
-            // (keeps the groups apart: let loose, the scheduler issues every group's matrix instructions first and
-            // spills their results)
+            if (g < 7) tokens(g + 1), planes(r, g + 1, BH, BL);
             __builtin_amdgcn_sched_barrier(0);
         }
-        const float d = f16_bits_to_f32(r.d16);
+        const float d = 0.5f * f16_bits_to_f32(r.d16);                       // (the digits are of twice the products)
 #pragma unroll
         for (int i = 0; i < NB; i++)
 #pragma unroll
@@ -1137,97 +1140,96 @@ struct GsQ6K {
                 // (spelled out: left to contract `acc += sx * d * isum` as it likes, the compiler fuses the last product
                 // into the addition for one token block and not for the other, and a token's bits depend on its block)
                 const float4 x4 = *(const float4*)(sx + 32 * i + 8 * g);
-                acc[i][4 * g] = __fmaf_rn(__fmul_rn(x4.x, d), (float)isum[i][4 * g], acc[i][4 * g]);
-                acc[i][4 * g + 1] = __fmaf_rn(__fmul_rn(x4.y, d), (float)isum[i][4 * g + 1], acc[i][4 * g + 1]);
-                acc[i][4 * g + 2] = __fmaf_rn(__fmul_rn(x4.z, d), (float)isum[i][4 * g + 2], acc[i][4 * g + 2]);
-                acc[i][4 * g + 3] = __fmaf_rn(__fmul_rn(x4.w, d), (float)isum[i][4 * g + 3], acc[i][4 * g + 3]);
+                const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int v = 4 * g + e;
+                    acc[i][v] = __fmaf_rn(__fmul_rn(xv[e], d), (float)(DH[i][v] * 256 + DL[i][v]), acc[i][v]);
+                    asm volatile("" : "+v"(acc[i][v]));     // (here: sunk below the staging, the integer results live on)
+                }
             }
     }
 };
 
 struct GsQ5K {
     static constexpr uint BYTES = Q5K_BYTES;
+    static constexpr uint PIECES = 11u;
     static constexpr bool BSUMS = true;
     struct Raw {
         uint4 hdr;          // d, dmin, the 12 scale bytes
-        uint2 qh[2];        // fifth bits of positions 16 h + 8 kg .. + 7 (bit j: sub-block j)
-        uint2 qs[4][2];     // [chunk][h]: nibbles of the same positions (low: sub-block 2 c, high: 2 c + 1)
+        uint4 qh;           // fifth bits of positions 16 kg .. 16 kg + 15 (bit j: sub-block j)
+        uint4 qs[4];        // nibbles of the same positions, chunk by chunk (low: sub-block 2 c, high: 2 c + 1)
     };
-    static __device__ __forceinline__ Raw load(const uchar* blk, uint kg) {
+    static __device__ __forceinline__ uint tail(const uchar*) { return 0u; }
+    static __device__ __forceinline__ Raw unpack(const uchar* row, uint kg, uint) {
         Raw r;
-        r.hdr = *(const uint4*)blk;
+        r.hdr = *(const uint4*)row;
+        r.qh = *(const uint4*)(row + 16u + 16u * kg);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            r.qh[h] = *(const uint2*)(blk + 16u + 16u * h + 8u * kg);
-#pragma unroll
-            for (int c = 0; c < 4; c++) r.qs[c][h] = *(const uint2*)(blk + 48u + 32u * c + 16u * h + 8u * kg);
-        }
+        for (int c = 0; c < 4; c++) r.qs[c] = *(const uint4*)(row + 48u + 32u * c + 16u * kg);
         return r;
     }
+    // The digits of 2 sc code for sub-block j
+    static __device__ __forceinline__ void planes(const Raw& r, uint sc_lo, uint sc_hi, int j, gq_i4& hi, gq_i4& lo) {
+        const uint s2 = 2u * (((j < 4 ? sc_lo : sc_hi) >> (8 * (j & 3))) & 0xFFu);
+        const gq_u16x2 f = {(ushort)s2, (ushort)s2}, b = {128, 128};
+        const uint4 qs = r.qs[j >> 1];
+        const uint ls[4] = {qs.x, qs.y, qs.z, qs.w}, hs[4] = {r.qh.x, r.qh.y, r.qh.z, r.qh.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint nib = (j & 1) ? ls[i] >> 4 : ls[i];
+            const uint bit = j < 4 ? hs[i] << (4 - j) : hs[i] >> (j - 4);
+            int a, c;
+            gs_scale4((nib & 0x0F0F0F0Fu) | (bit & 0x10101010u), f, b, a, c);
+            hi[i] = a;
+            lo[i] = c;
+        }
+    }
     template <int NB>   // NB: how many of the wave's two 32-token blocks hold tokens
-    static __device__ __forceinline__ void superblock(const Raw& r, const uchar* st, uint tok0, uint fr, uint kg,
-                                                      float (&acc)[2][16]) {
-        const uchar* xa = st + (tok0 + fr) * GS_STRIDE + 8u * kg;            // the lane's token row of block 0, its 8 positions
-        const float* sx = (const float*)(st + GS_SX) + tok0 + 4u * kg;       // scales of its D registers' tokens: + 32 i + 8 (v / 4) + v % 4
-        int isum[NB][16];
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) isum[i][v] = 0;
+    static __device__ __forceinline__ void superblock(const Raw& r, const uchar* st, uint fr, uint kg, float (&acc)[2][16]) {
+        const uchar* xa = st + fr * GS_STRIDE + 16u * kg;                    // the lane's token row of block 0, its 16 positions
+        const float* sx = (const float*)(st + GS_SX) + 4u * kg;              // scales of its D registers' tokens: + 32 i + 8 (v / 4) + v % 4
         const gs_i16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         // the eight 6-bit scales and mins, a byte each (get_scale_min_k4, crates/ojas-formats/src/gguf.rs:1132-1140)
         const uint sc_lo = r.hdr.y & 0x3F3F3F3Fu, mn_lo = r.hdr.z & 0x3F3F3F3Fu;
         const uint sc_hi = (r.hdr.w & 0x0F0F0F0Fu) | ((r.hdr.y >> 2) & 0x30303030u);
         const uint mn_hi = ((r.hdr.w >> 4) & 0x0F0F0F0Fu) | ((r.hdr.z >> 2) & 0x30303030u);
-        // sub-block j, half h: the codes of positions 16 h + 8 kg .. of chunk j / 2 (low or high nibbles) under fifth bit j
-        auto codes = [&](int j, int h) -> long {
-            const uint2 p = r.qs[j >> 1][h];
-            const uint n0 = (j & 1) ? (p.x >> 4) & 0x0F0F0F0Fu : p.x & 0x0F0F0F0Fu;
-            const uint n1 = (j & 1) ? (p.y >> 4) & 0x0F0F0F0Fu : p.y & 0x0F0F0F0Fu;
-            const uint b0 = j < 4 ? (r.qh[h].x << (4 - j)) & 0x10101010u : (r.qh[h].x >> (j - 4)) & 0x10101010u;
-            const uint b1 = j < 4 ? (r.qh[h].y << (4 - j)) & 0x10101010u : (r.qh[h].y >> (j - 4)) & 0x10101010u;
-            return gq_pack(n0 | b0, n1 | b1);
+        gs_i16 DH[NB], DL[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) DH[i] = zero, DL[i] = zero;
+        // the next sub-block's operands are built under this one's matrix instructions
+        gq_i4 BH, BL, A[NB];
+        auto tokens = [&](int j) {
+#pragma unroll
+            for (int i = 0; i < NB; i++) A[i] = *(const gq_i4*)(xa + (uint)i * 32u * GS_STRIDE + 32u * (uint)j);
         };
-        auto tokens = [&](int j, int h, int i) -> long {
-            return *(const long*)(xa + (uint)i * 32u * GS_STRIDE + 32u * (uint)j + 16u * (uint)h);
-        };
-        // the next sub-block's operands are fetched and built under this one's matrix instructions
-        long B[2] = {codes(0, 0), codes(0, 1)};
-        long A[2][2] = {{tokens(0, 0, 0), NB == 2 ? tokens(0, 0, 1) : 0}, {tokens(0, 1, 0), NB == 2 ? tokens(0, 1, 1) : 0}};
+        planes(r, sc_lo, sc_hi, 0, BH, BL);
+        tokens(0);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const int s = (int)(((j < 4 ? sc_lo : sc_hi) >> (8 * (j & 3))) & 0xFFu);
-            // (one instruction over all 32 positions of the sub-block: a lane's sixteen are 8 kg .. and 16 + 8 kg ..)
-            gs_i16 D[NB];
-            const gq_i4 Bj = {(int)B[0], (int)(B[0] >> 32), (int)B[1], (int)(B[1] >> 32)};
 #pragma unroll
             for (int i = 0; i < NB; i++) {
-                const gq_i4 Aj = {(int)A[0][i], (int)(A[0][i] >> 32), (int)A[1][i], (int)(A[1][i] >> 32)};
-                D[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(Aj, Bj, zero, 0, 0, 0);
+                DH[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], BH, DH[i], 0, 0, 0);
+                DL[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], BL, DL[i], 0, 0, 0);
             }
-            if (j < 7) {
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    B[h] = codes(j + 1, h);
-                    A[h][0] = tokens(j + 1, h, 0);
-                    if (NB == 2) A[h][1] = tokens(j + 1, h, 1);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < NB; i++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) isum[i][v] = gs_pin(isum[i][v] + __mul24(s, D[i][v]));
+            if (j < 7) tokens(j + 1), planes(r, sc_lo, sc_hi, j + 1, BH, BL);
             __builtin_amdgcn_sched_barrier(0);
         }
-        // sum_j m_j bsum_j, bsum = 64 hi + lo: positions 0..7 of A carry the lo parts, 8..15 the hi parts, B the mins twice:
-        // D1 = sum m lo + sum m hi; with the lo half of A blanked D2 = sum m hi; the term is D1 + 63 D2
+        // sum_j m_j bsum_j, bsum = 64 hi + lo: positions 0..7 of A carry the lo parts, 8..15 the hi parts, B the mins twice;
+        // with either half of A blanked D1 = sum m lo, D2 = sum m hi
         const long Bm = gq_pack(mn_lo, mn_hi);
         const long km = kg ? -1l : 0l;
-        const float d = f16_bits_to_f32(r.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(r.hdr.x >> 16);
+        const float d = 0.5f * f16_bits_to_f32(r.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(r.hdr.x >> 16);   // (the digits are of twice the products)
+        float part[NB][16];                                 // (ahead of the mins' results: all of them at once spill)
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) part[i][v] = __fmul_rn(d, (float)(DH[i][v] * 256 + DL[i][v]));
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < NB; i++) {
-            const long A1 = *(const long*)(st + GS_BS + (tok0 + 32u * (uint)i + fr) * 16u + 8u * kg);
-            const gs_i16 D1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(A1, Bm, zero, 0, 0, 0);
+            const long A1 = *(const long*)(st + GS_BS + (32u * (uint)i + fr) * 16u + 8u * kg);
+            const gs_i16 D1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(A1 & ~km, Bm, zero, 0, 0, 0);
             const gs_i16 D2 = __builtin_amdgcn_mfma_i32_32x32x16_i8(A1 & km, Bm, zero, 0, 0, 0);
 #pragma unroll
             for (int g = 0; g < 4; g++) {
@@ -1236,14 +1238,16 @@ struct GsQ5K {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int v = 4 * g + e;
-                    const float inner = __fmaf_rn(-dmin, (float)(D1[v] + 63 * D2[v]), __fmul_rn(d, (float)isum[i][v]));
-                    acc[i][v] = __fmaf_rn(xv[e], inner, acc[i][v]);
+                    acc[i][v] = __fmaf_rn(xv[e], __fmaf_rn(-dmin, (float)(D2[v] * 64 + D1[v]), part[i][v]), acc[i][v]);
+                    asm volatile("" : "+v"(acc[i][v]));     // (here: sunk below the staging, the integer results live on and spill)
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 };
 
+template <int NB> struct GsBlocks { static constexpr int value = NB; };
 // which row of xq / xs / y token m of the launch is: itself, or (grouped expert products) an entry of a list
 struct GsDense {
     __device__ __forceinline__ uint row(uint m) const { return m; }
@@ -1266,43 +1270,69 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
     if (SPLIT && sb0 >= sb1) return;                      // (the host launches only slices that hold a super-block)
     constexpr uint TPG = 64u, RPG = 128u;                     // tokens and rows per workgroup
     const uint m0 = ty * TPG, fr = lane & 31u, kg = lane >> 5;
-    const uint row = min(blockIdx.x * RPG + 32u * wave + fr, N - 1u);
-    const uint tok0 = 0u;
     // 32-token blocks that hold tokens: the last token tile may need only the first
     const uint nblk = M - m0 > 32u ? 2u : 1u;
-    const uchar* wr = w + (size_t)row * nsb * F::BYTES;
+    // The wave's 32 rows of a super-block: 16-byte pieces, neighbouring lanes side by side in a row, through registers into
+    // the wave's own part of LDS (no barrier), read back in operand order.  (rows past N repeat the last)
+    constexpr uint NQ = (32u * F::PIECES + 63u) / 64u;
+    const uint row0 = min(blockIdx.x * RPG + 32u * wave, N - 1u), top = N - 1u - row0;
+    const uchar* const w0 = w + (size_t)row0 * nsb * F::BYTES;
+    uint woff[NQ];
+#pragma unroll
+    for (uint i = 0; i < NQ; i++) {
+        const uint p = min(lane + 64u * i, 32u * F::PIECES - 1u), r = p / F::PIECES;
+        woff[i] = min(r, top) * nsb * F::BYTES + (p - r * F::PIECES) * 16u;
+    }
+    const uint doff = min(fr, top) * nsb * F::BYTES;
+    uchar* const mine = lds + 2u * GS_STAGE + wave * (GS_ROWS * F::PIECES + 64u);
+    typedef gq_i4 __attribute__((aligned(2))) piece;        // (Q6_K rows are only 2-byte aligned)
+    gq_i4 wv[NQ];
+    uint wd = 0u;
+    auto ask = [&](uint sb) {
+        const uchar* const b = w0 + (size_t)sb * F::BYTES;
+#pragma unroll
+        for (uint i = 0; i < NQ; i++) wv[i] = *(const piece*)(b + woff[i]);
+        wd = F::tail(b + doff);
+    };
+    auto take = [&]() -> typename F::Raw {
+#pragma unroll
+        for (uint i = 0; i < NQ; i++)
+            if (64u * (i + 1u) <= 32u * F::PIECES || lane < 32u * F::PIECES - 64u * i)
+                *(gq_i4*)(mine + (lane + 64u * i) * 16u) = wv[i];
+        if (F::PIECES * 16u < F::BYTES) ((ushort*)(mine + GS_ROWS * F::PIECES))[fr] = (ushort)wd;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        return F::unpack(mine + fr * (F::PIECES * 16u), kg, ((const ushort*)(mine + GS_ROWS * F::PIECES))[fr]);
+    };
 
     // staging: thread -> chunk tid % 16 (16 bytes) of tokens tid / 16 + 16 p, p = 0 .. 3
     constexpr int NP = 4;
     const uint s_tok = tid >> 4, s_ch = tid & 15u;
-    uint4 tv[NP];
+    gq_i4 tv[NP];
     float tsx = 0.0f;
-    // the rows of this thread's tokens (one lookup per tile, not per super-block)
+    // the rows of this thread's tokens (one lookup per tile, not per super-block); past the last token they repeat it, and
+    // what is multiplied by them is not stored
     uint trow[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) trow[p] = tm.row(min(m0 + s_tok + 16u * (uint)p, M - 1u));
-    const uint xrow = tm.row(min(m0 + tid, M - 1u));
+    const uint xrow = tm.row(min(m0 + (tid & (TPG - 1u)), M - 1u));
     auto fetch = [&](uint sb) {
 #pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const uint m = m0 + s_tok + 16u * (uint)p;
-            tv[p] = make_uint4(0u, 0u, 0u, 0u);
-            if (m < M) tv[p] = *(const uint4*)(xq + (size_t)trow[p] * K + (size_t)sb * 256u + s_ch * 16u);
-        }
-        if (tid < TPG) tsx = m0 + tid < M ? xs[(size_t)xrow * nsb + sb] : 0.0f;
+        for (int p = 0; p < NP; p++) tv[p] = *(const gq_i4*)(xq + (size_t)trow[p] * K + (size_t)sb * 256u + s_ch * 16u);
+        tsx = xs[(size_t)xrow * nsb + sb];
     };
     auto put = [&](uchar* st) {
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             uchar* o = st + (s_tok + 16u * (uint)p) * GS_STRIDE + s_ch * 16u;
-            *(uint2*)o = make_uint2(tv[p].x, tv[p].y);
-            *(uint2*)(o + 8) = make_uint2(tv[p].z, tv[p].w);
+            *(gq_i4*)o = tv[p];
             if (F::BSUMS) {
                 // half a sub-block per thread; its neighbour holds the other half
-                int s = dot4_i8(tv[p].x, 0x01010101u, 0);
-                s = dot4_i8(tv[p].y, 0x01010101u, s);
-                s = dot4_i8(tv[p].z, 0x01010101u, s);
-                s = dot4_i8(tv[p].w, 0x01010101u, s);
+                int s = dot4_i8((uint)tv[p][0], 0x01010101u, 0);
+                s = dot4_i8((uint)tv[p][1], 0x01010101u, s);
+                s = dot4_i8((uint)tv[p][2], 0x01010101u, s);
+                s = dot4_i8((uint)tv[p][3], 0x01010101u, s);
                 s += dpp_i32<OJK_DPP_QUAD_XOR1>(s);
                 if (!(s_ch & 1u)) {
                     uchar* b = st + GS_BS + (s_tok + 16u * (uint)p) * 16u + (s_ch >> 1);
@@ -1311,7 +1341,7 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
                 }
             }
         }
-        if (tid < TPG) ((float*)(st + GS_SX))[tid] = tsx;
+        ((float*)(st + GS_SX))[tid & (TPG - 1u)] = tsx;      // (by all: under a branch its load would sink there, and be waited for with the rows)
     };
 
     float acc[2][16];
@@ -1321,20 +1351,24 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
         for (int v = 0; v < 16; v++) acc[i][v] = 0.0f;
 
     fetch(sb0);
-    typename F::Raw nx = F::load(wr + (size_t)sb0 * F::BYTES, kg);
+    ask(sb0);
     put(lds);
     __syncthreads();
-    for (uint sb = sb0; sb < sb1; sb++) {
-        const typename F::Raw cur = nx;
-        const uint nb = min(sb + 1u, sb1 - 1u);
-        nx = F::load(wr + (size_t)nb * F::BYTES, kg);
-        fetch(nb);
-        const uchar* st = lds + ((sb - sb0) & 1u) * GS_STAGE;
-        if (nblk == 2u) F::template superblock<2>(cur, st, tok0, fr, kg, acc);
-        else F::template superblock<1>(cur, st, tok0, fr, kg, acc);
-        put(lds + (((sb - sb0) & 1u) ^ 1u) * GS_STAGE);
-        __syncthreads();
-    }
+    auto walk = [&](auto nb_) {
+        for (uint sb = sb0; sb < sb1; sb++) {
+            const typename F::Raw cur = take();
+            // tokens first: what waits for them at the end of the step leaves the younger row loads in flight
+            const uint nb = min(sb + 1u, sb1 - 1u);
+            fetch(nb);
+            ask(nb);
+            F::template superblock<decltype(nb_)::value>(cur, lds + ((sb - sb0) & 1u) * GS_STAGE, fr, kg, acc);
+            asm volatile("" ::: "memory");                       // (left to itself the compiler waits for the tokens early in the step)
+            put(lds + (((sb - sb0) & 1u) ^ 1u) * GS_STAGE);
+            __syncthreads();
+        }
+    };
+    if (nblk == 2u) walk(GsBlocks<2>());
+    else walk(GsBlocks<1>());
 
     if (SPLIT) {
         // partial tiles out as the registers hold them ([pair][thread]), written through and read from behind the L2
@@ -1342,12 +1376,12 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
         typedef unsigned long long u64;
         const uint ns_eff = (nsb + per - 1u) / per;
         const uint tile = blockIdx.y * gridDim.x + blockIdx.x;
-        u64* const mine = (u64*)part + ((size_t)tile * ns_eff + blockIdx.z) * 16u * 256u + tid;
+        u64* const own = (u64*)part + ((size_t)tile * ns_eff + blockIdx.z) * 16u * 256u + tid;
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int h = 0; h < 8; h++)
-                __hip_atomic_store(mine + (size_t)(i * 8 + h) * 256u,
+                __hip_atomic_store(own + (size_t)(i * 8 + h) * 256u,
                                    (u64)__float_as_uint(acc[i][2 * h]) | ((u64)__float_as_uint(acc[i][2 * h + 1]) << 32),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1388,7 +1422,7 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-            const uint t = m0 + tok0 + 32u * (uint)i + 8u * (uint)(v >> 2) + 4u * kg + (uint)(v & 3);
+            const uint t = m0 + 32u * (uint)i + 8u * (uint)(v >> 2) + 4u * kg + (uint)(v & 3);
             if (t < M && n < N) {
                 float* o = y + (size_t)tm.row(t) * N + n;
                 *o = ACC ? *o + acc[i][v] : acc[i][v];
@@ -1399,13 +1433,13 @@ __device__ __forceinline__ void gemm_q8k_gs_body(const signed char* __restrict__
 #define GEMM_Q8K_GS(FMT, F)                                                                                              \
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))                         \
     gemm_q8k_##FMT##_gs(const signed char* xq, const float* xs, const uchar* w, float* y, uint K, uint N, uint M, uint ACC) { \
-        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE];                                              \
+        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE + 4 * (GS_ROWS * F::PIECES + 64)];                                              \
         gemm_q8k_gs_body<F, false>(xq, xs, w, y, K, N, M, ACC, lds_gs);                                                  \
     }                                                                                                                    \
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))                         \
     gemm_q8k_##FMT##_gs_sr(const signed char* xq, const float* xs, const uchar* w, float* y, float* part, uint* cnt,     \
                            uint K, uint N, uint M, uint ACC, uint NSPLIT) {                                              \
-        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE];                                              \
+        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE + 4 * (GS_ROWS * F::PIECES + 64)];                                              \
         gemm_q8k_gs_body<F, true>(xq, xs, w, y, K, N, M, ACC, lds_gs, part, cnt, NSPLIT);                                \
     }
 GEMM_Q8K_GS(q6k, GsQ6K)
@@ -1420,7 +1454,7 @@ GEMM_Q8K_GS(q5k, GsQ5K)
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))                         \
     moe_down_##FMT##_gs(const signed char* aq, const float* as_, const uchar* wd, float* dv, const uint* offsets,        \
                         const uint* list, uint K, uint N, uint NA) {                                                     \
-        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE];                                              \
+        __shared__ __attribute__((aligned(16))) uchar lds_gs[2 * GS_STAGE + 4 * (GS_ROWS * F::PIECES + 64)];                                              \
         const uint e = blockIdx.z;                                                                                       \
         const uint a0 = min(offsets[e], NA), a1 = min(offsets[e + 1], NA);                                               \
         if (a0 >= a1) return;                                                                                            \

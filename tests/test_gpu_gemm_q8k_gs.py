@@ -98,3 +98,46 @@ def test_router_path_matches_the_cpu_reference(gpu, orc, pkg, ty, m, n, k, accum
         gpu.mm(gpu.upload(x[t]), lin, one, 1, act_mode=pkg.ACT_Q8K)
         assert peak_err(gpu.read(one, n), got[t * n:(t + 1) * n] - y0[t]) <= TOL_SEEN
     lin.free()
+
+
+@pytest.mark.parametrize("ty,m,n,k", [(Q6_K, 17, 4100, 512), (Q6_K, 32, 130, 4352), (Q6_K, 9, 300, 14336), (Q6_K, 16, 4096, 14336)])
+def test_few_tokens_from_which_the_tile_is_ahead(gpu, orc, pkg, ty, m, n, k):
+    """Both sides of the row and K bounds of the early crossover, through `ojh_mm`."""
+    w, x = _case(pkg, ty, m, n, k, "early")
+    lin = gpu.lin(ty, n, k, w)
+    yd = gpu.upload(np.full(m * n + n, 4242.5, np.float32))
+    gpu.mm(gpu.upload(x), lin, yd, m, False, act_mode=pkg.ACT_Q8K)
+    got = gpu.read(yd, m * n + n)
+    assert np.all(got[m * n:] == 4242.5), "wrote past the last token"
+    for t in range(m):
+        assert peak_err(got[t * n:(t + 1) * n], orc.matvec_kq(w, ty, n, k, x[t])) <= TOL_SEEN
+    lin.free()
+
+
+@pytest.mark.parametrize("ty", [Q6_K, Q5_K])
+@pytest.mark.parametrize("m", [32, 64])
+def test_the_digits_at_the_ends_of_their_range(gpu, orc, pkg, ty, m):
+    """Rows of the extreme scales (-128 / 127, 63) under the extreme codes (0 / 63, 31) against activations of +-127 codes: the
+    largest integers that the two digits and a super-block's sums have to hold."""
+    n, k = 128, 512
+    w = _case(pkg, ty, 1, n, k, "ends")[0].reshape(n * 2, -1).copy()
+    rows = np.arange(n * 2)
+    if ty == Q6_K:
+        w[:, :192] = np.where(rows[:, None] % 2, 0xFF, 0)            # codes 63 / 0
+        w[:, 192:208] = np.where(rows[:, None] // 2 % 2, 0x80, 0x7F)  # scales -128 / 127
+    else:
+        w[:, 4:] = np.where(rows[:, None] % 2, 0xFF, 0xF0)           # scales and mins 63, codes 31 / 15
+    x = np.ones((m, k), np.float32)
+    x[1::2, ::2] = -1.0
+    x[2::4] *= -1.0
+    lin = gpu.lin(ty, n, k, w.ravel())
+    yd = gpu.alloc(m * n)
+    gpu.ensure_family("gemm_q8k")
+    xq, xs = gpu.alloc_bytes(m * k), gpu.alloc(m * 2)
+    gpu.quant_q8k(gpu.upload(x), m, k, xq, xs)
+    gpu.dispatch(gpu.begin(), f"gemm_q8k_{FMT[ty]}_gs", [(xq, 0), (xs, 0), (gpu.upload_bytes(w.ravel()), 0), (yd, 0)], [k, n, m, 0],
+                 [1, 1, 1], [256, 1, 1])
+    got = gpu.read(yd, m * n).reshape(m, n)
+    for t in range(m):
+        assert peak_err(got[t], orc.matvec_kq(w.ravel(), ty, n, k, x[t])) <= TOL_SEEN
+    lin.free()
