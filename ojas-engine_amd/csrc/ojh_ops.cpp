@@ -356,33 +356,46 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
     }
     const size_t w_bytes = w->row_bytes * N;
     const bool dwords_ok = (uintptr_t)wp % 4 == 0 && (w_bytes % 4 == 0 || w->off + w_bytes + 2 <= w->raw->bytes);
-    // Q6_K / Q5_K rows against a batch: 128-row x 64-token tiles, one matrix instruction per scale group;
+    // Q6_K / Q5_K rows against a batch: 128-row x 64-token tiles, scales folded into two int8 digits;
     // over K slices where the tiles alone would leave CUs idle (partial tiles in library scratch, added in slice order)
-    // (from where it was measured ahead of what it replaces, rows streamed from HBM.  Q6_K: from 17 tokens on large
-    // matrices — 14336 x 4096 at 24 tokens 28.6 against 39 us for two launches of 16, 4096 x 14336 32.6 against 50 — and
-    // from 33 on small ones, where two launches still win (4096 x 4096: 18 against 19.4).  Q5_K, whose few-token form is
-    // the integer-dot kernel: from 5 tokens on large matrices (14336 x 4096 at 8 tokens 25.5 against 31.8), from 9 on
-    // small ones (4096 x 4096 at 12 tokens 17.8 against 20.5).)
+    // (from where it was measured ahead of what it replaces, rows streamed from HBM.  Q6_K: from 17 tokens on matrices of
+    // more than 4096 rows or a longer K than that — 7168 x 2048 at 24 tokens 14.6 against 20.4 us for two launches of 16,
+    // 730 x 5632 17.7 against 21.2, 14336 x 4096 24.2 against 39 — from 33 on the others, where two launches are level or
+    // ahead (4096 x 4096: 18.2 against 17.8, 2048 x 1536 13.2 against 12.9), and from 9 where 16 tokens no longer fit the
+    // few-row kernel (4096 x 14336 at 12 tokens 26.3 against 33.4 for two launches of 8).  Q5_K, whose few-token form is
+    // the integer-dot kernel: from 5 tokens on large matrices (14336 x 4096 at 5 tokens 22.6, at 3 22.6 against 17.7 there),
+    // from 9 on small ones (4096 x 4096 at 8 tokens 17.4 against 12.4, 730 x 5632 17.7 against 13.5).)
+    // Below the second threshold a call takes the tile only where all it needs is to be had (a recorded call may ask for
+    // nothing), and leaves its scratch to calls that cannot do without.
     const bool gs_large = N >= 8192 || K > 8192;
+    const bool q6k_few = (N + 15) / 16 <= 2u * (uint32_t)dev->prop.multiProcessorCount && ojh_q6k_mk_lds(K, 16) > 163840;
     const uint32_t gs_min = dev->kq_gs_min_m != 1 ? dev->kq_gs_min_m
                             : w->type == OJH_Q6_K ? (gs_large ? 17u : 33u) : (gs_large ? 5u : 9u);
-    if ((w->type == OJH_Q6_K || w->type == OJH_Q5_K) && gs_min && m >= gs_min && K % 256 == 0 &&
+    const uint32_t gs_early = dev->kq_gs_min_m != 1 || w->type != OJH_Q6_K || dev->no_scratch ? gs_min
+                              : q6k_few ? 9u : N > 4096 || K > 4096 ? 17u : 33u;
+    if ((w->type == OJH_Q6_K || w->type == OJH_Q5_K) && gs_min && m >= gs_early && K % 256 == 0 &&
         (uintptr_t)xq % 16 == 0 && (w->type == OJH_Q6_K ? dwords_ok : (uintptr_t)wp % 16 == 0)) {
-        int rc = ensure(dev, "gemm_q8k");
-        if (rc) return rc;
+        int rc;
+        const bool early = m < gs_min;
         const std::string gs = std::string("gemm_q8k_") + f->tag + "_gs";
         uint32_t sg[3] = {(N + 127) / 128, (m + 63) / 64, 1}, sb[3] = {256, 1, 1};
         const uint32_t z = dev->no_scratch ? 1 : ojh_gemm_q8k_gs_slices(dev, K, N, m);
-        if (z > 1) {
-            const size_t tiles = (size_t)sg[0] * sg[1];
-            ojh_buf *part, *cnt;
-            if ((rc = ojh_scratch_get(dev, "gs_part", tiles * z * 32768, &part))) return rc;
-            if ((rc = ojh_scratch_get_zeroed(dev, "gs_cnt", tiles * 4, &cnt))) return rc;
+        const size_t tiles = (size_t)sg[0] * sg[1], part_bytes = tiles * z * 32768, cnt_bytes = tiles * 4;
+        const bool taken = !early || ((dev->modules.count("gemm_q8k") || !dev->capturing) &&
+                                      (z < 2 || ojh_scratch_fits(dev, {{"gs_part", part_bytes}, {"gs_cnt", cnt_bytes}})));
+        ojh_buf *part = nullptr, *cnt = nullptr;
+        if (taken && z > 1) {
+            rc = early ? ojh_scratch_spare(dev, "gs_part", part_bytes, &part) : ojh_scratch_get(dev, "gs_part", part_bytes, &part);
+            if (!rc) rc = ojh_scratch_get_zeroed(dev, "gs_cnt", cnt_bytes, &cnt);
+            if (rc && !early) return rc;
+        }
+        if (taken && (z < 2 || cnt)) {
+            if ((rc = ensure(dev, "gemm_q8k"))) return rc;
+            if (z < 2) return ojh_launch(dev, gs.c_str(), {xq, xs, wp, yp}, {K, N, m, (uint32_t)(accum != 0)}, sg, sb);
             sg[2] = z;
             return ojh_launch(dev, (gs + "_sr").c_str(), {xq, xs, wp, yp, part->ptr, cnt->ptr},
                               {K, N, m, (uint32_t)(accum != 0), z}, sg, sb);
         }
-        return ojh_launch(dev, gs.c_str(), {xq, xs, wp, yp}, {K, N, m, (uint32_t)(accum != 0)}, sg, sb);
     }
     // Q6_K rows against 2 or more tokens on the int8 matrix cores (beyond 16 tokens as launches of 16 or 8:
     // each streams the rows once, which the per-token loop of the general entry does sixteen times
