@@ -1027,7 +1027,7 @@ gemm_q8k_q4k_xt64_sr(const signed char* xq, const float* xst, const float* sums,
 // The CPU path's arithmetic (dot_q6k / dot_q5k over quant_q8k activations, crates/ojas-cpu/src/cpu_math.rs:638-722) for
 // batches from a handful of tokens to prefill sizes.  A weight's whole integer, scale x (code - 32) or scale x code, fits 14
 // bits: one packed 16-bit multiply-add forms twice that integer for two weights, and its bytes are the two signed digits
-// (gs_digits) that two accumulating v_mfma_i32_32x32x32_i8 take as they are — 256 D_hi + D_lo is twice the super-block's
+// (gq_digits) that two accumulating v_mfma_i32_32x32x32_i8 take as they are — 256 D_hi + D_lo is twice the super-block's
 // integer sum, exactly, whatever the scales' groups.  Q5_K: sum_j m_j bsum_j from two more instructions per super-block over
 // the sub-block sums split as 64 hi + lo (the workgroup splits them while it stages the tokens).
 // A workgroup owns 128 rows x 64 tokens: wave w takes rows 32 w .. against both blocks of 32 tokens (only the first where
@@ -1051,20 +1051,6 @@ typedef int gs_i16 __attribute__((ext_vector_type(16)));
 #define GS_BS (GS_SX + 256u)            // Q5_K: the split sub-block sums, 16 bytes per token (lo_0..7, hi_0..7)
 #define GS_STAGE (GS_BS + 1024u)
 #define GS_ROWS 512u                    // a wave's 32 rows: bytes per piece of 16
-
-// Two signed digits of twice a product, four products at a time: ev and od hold p + 128 in their 16-bit halves (products
-// 0, 2 and 1, 3), p even.  hi takes their upper bytes and lo their lower bytes with the sign bit flipped, so that
-// p = 256 hi + lo with both in int8, exactly.
-__device__ __forceinline__ void gs_digits(uint ev, uint od, int& hi, int& lo) {
-    hi = (int)__builtin_amdgcn_perm(od, ev, 0x07030501u);
-    lo = (int)(__builtin_amdgcn_perm(od, ev, 0x06020400u) ^ 0x80808080u);
-}
-// four codes (a byte each) times f, plus b
-__device__ __forceinline__ void gs_scale4(uint codes, gq_u16x2 f, gq_u16x2 b, int& hi, int& lo) {
-    const gq_u16x2 ev = __builtin_bit_cast(gq_u16x2, codes & 0x00FF00FFu) * f + b;
-    const gq_u16x2 od = __builtin_bit_cast(gq_u16x2, __builtin_amdgcn_perm(0u, codes, 0x0C030C01u)) * f + b;
-    gs_digits(__builtin_bit_cast(uint, ev), __builtin_bit_cast(uint, od), hi, lo);
-}
 
 struct GsQ6K {
     static constexpr uint BYTES = Q6K_BYTES;
@@ -1100,7 +1086,7 @@ struct GsQ6K {
             const uint nib = (q & 2) ? ls[i] >> 4 : ls[i];
             const uint two = q == 3 ? hs[i] >> 2 : q == 2 ? hs[i] : q == 1 ? hs[i] << 2 : hs[i] << 4;
             int a, c;
-            gs_scale4((nib & 0x0F0F0F0Fu) | (two & 0x30303030u), f, b, a, c);
+            gq_scale4((nib & 0x0F0F0F0Fu) | (two & 0x30303030u), f, b, a, c);
             hi[i] = a;
             lo[i] = c;
         }
@@ -1180,7 +1166,7 @@ struct GsQ5K {
             const uint nib = (j & 1) ? ls[i] >> 4 : ls[i];
             const uint bit = j < 4 ? hs[i] << (4 - j) : hs[i] >> (j - 4);
             int a, c;
-            gs_scale4((nib & 0x0F0F0F0Fu) | (bit & 0x10101010u), f, b, a, c);
+            gq_scale4((nib & 0x0F0F0F0Fu) | (bit & 0x10101010u), f, b, a, c);
             hi[i] = a;
             lo[i] = c;
         }

@@ -33,6 +33,7 @@
 #include "ojk_q4k_dot.h"
 #include "ojk_gq.h"
 #include "ojk_moe_rows.h"
+#include <type_traits>
 
 // ------------------------------------------------------------------ router
 template <int NI>
@@ -1028,14 +1029,133 @@ moe_down_q4k_mm(const signed char* __restrict__ aq, const float* __restrict__ as
 #define MT_UNIT 2304u
 #define MT_DEPTH 2
 #define MT_RING (16u * MT_DEPTH * MT_UNIT)
-// A pass stages 16 P assignments; P = 2 where 32 token rows fit (32 (K + 32) + 5 K / 2 + 384 <= 81920): an expert with
-// 17 .. 32 assignments then has its rows read and unpacked once instead of twice (at 256 tokens over 128 experts with
-// 8 slots each, 16 per expert on average, that is every other expert).
-template <bool GU, int P>
+// Down tensors in Q6_K and Q5_K (moe_down_{q6k,q5k}_mt) take the same walk.  Their integers, scale x (code - 32) or scale x
+// code, enter as two signed digits (gq_scale4), and their rows, 210 bytes apart or 176, pass through registers: 16-byte
+// pieces, neighbouring lanes side by side in a row, one unit ahead, into the wave's own part of LDS and out of it in operand
+// order.  Lane (n, kg) holds of row n: Q6_K the 16-position column kg % 2 of the four quarters of half kg / 2; Q5_K positions
+// 16 (kg % 2) .. of the sub-blocks of parity kg / 2.
+struct MtQ4K {};
+struct MtQ6K {
+    static constexpr uint BYTES = Q6K_BYTES, PIECES = 13u;
+    static constexpr bool MINS = false;
+    uint4 a, b, qh;
+    uint2 sc;
+    uint d16;
+    static __device__ __forceinline__ uint tail(const uchar* blk) { return *(const ushort*)(blk + 208u); }
+    static __device__ __forceinline__ uint token_at(uint kg) { return 128u * (kg >> 1) + 16u * (kg & 1u); }
+    static constexpr uint STEP = 32u;           // a token's bytes of the next instruction
+    __device__ __forceinline__ void read(const uchar* row, uint kg, uint d) {
+        const uint hf = kg >> 1, h = kg & 1u;
+        a = *(const uint4*)(row + 64u * hf + 16u * h);
+        b = *(const uint4*)(row + 64u * hf + 32u + 16u * h);
+        qh = *(const uint4*)(row + 128u + 32u * hf + 16u * h);
+        sc = *(const uint2*)(row + 192u + 8u * hf);
+        d16 = d;
+    }
+    __device__ __forceinline__ void planes(uint kg, gq_i4 (&BH)[4], gq_i4 (&BL)[4]) const {
+        const uint s8 = 8u * (kg & 1u), hs[4] = {qh.x, qh.y, qh.z, qh.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint4 l = (q & 1) ? b : a;
+            const uint ls[4] = {l.x, l.y, l.z, l.w};
+            const int s2 = 2 * (int)(signed char)((q < 2 ? sc.x : sc.y) >> (16u * (uint)(q & 1) + s8));
+            const ushort bb = (ushort)(128 - 32 * s2);
+            const gq_u16x2 f = {(ushort)s2, (ushort)s2}, c = {bb, bb};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint nib = (q & 2) ? ls[i] >> 4 : ls[i];
+                const uint two = q == 3 ? hs[i] >> 2 : q == 2 ? hs[i] : q == 1 ? hs[i] << 2 : hs[i] << 4;
+                int hi, lo;
+                gq_scale4((nib & 0x0F0F0F0Fu) | (two & 0x30303030u), f, c, hi, lo);
+                BH[q][i] = hi;
+                BL[q][i] = lo;
+            }
+        }
+    }
+    __device__ __forceinline__ float d() const { return f16_bits_to_f32(d16); }
+    __device__ __forceinline__ float dmin() const { return 0.0f; }
+    __device__ __forceinline__ long mins(uint) const { return 0; }
+};
+struct MtQ5K {
+    static constexpr uint BYTES = Q5K_BYTES, PIECES = 11u;
+    static constexpr bool MINS = true;
+    uint4 hdr, qh, qs[4];
+    static __device__ __forceinline__ uint tail(const uchar*) { return 0u; }
+    static __device__ __forceinline__ uint token_at(uint kg) { return 16u * kg; }
+    static constexpr uint STEP = 64u;
+    __device__ __forceinline__ void read(const uchar* row, uint kg, uint) {
+        const uint h = 16u * (kg & 1u);
+        hdr = *(const uint4*)row;
+        qh = *(const uint4*)(row + 16u + h);
+#pragma unroll
+        for (int c = 0; c < 4; c++) qs[c] = *(const uint4*)(row + 48u + 32u * (uint)c + h);
+    }
+    __device__ __forceinline__ void planes(uint kg, gq_i4 (&BH)[4], gq_i4 (&BL)[4]) const {
+        const uint par = kg >> 1, sc_lo = hdr.y & 0x3F3F3F3Fu, sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+        const uint hs[4] = {qh.x >> par, qh.y >> par, qh.z >> par, qh.w >> par};    // sub-block 2 c + par: bit 2 c
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint s2 = 2u * (((c < 2 ? sc_lo : sc_hi) >> (16u * (uint)(c & 1) + 8u * par)) & 0xFFu);
+            const gq_u16x2 f = {(ushort)s2, (ushort)s2}, o = {128, 128};
+            const uint ls[4] = {qs[c].x, qs[c].y, qs[c].z, qs[c].w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint bit = c == 0 ? hs[i] << 4 : c == 1 ? hs[i] << 2 : c == 2 ? hs[i] : hs[i] >> 2;
+                int hi, lo;
+                gq_scale4(((ls[i] >> (4u * par)) & 0x0F0F0F0Fu) | (bit & 0x10101010u), f, o, hi, lo);
+                BH[c][i] = hi;
+                BL[c][i] = lo;
+            }
+        }
+    }
+    __device__ __forceinline__ float d() const { return f16_bits_to_f32(hdr.x & 0xFFFFu); }
+    __device__ __forceinline__ float dmin() const { return f16_bits_to_f32(hdr.x >> 16); }
+    __device__ __forceinline__ long mins(uint kg) const {
+        const uint mn_lo = hdr.z & 0x3F3F3F3Fu, mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+        return kg == 0u ? gq_pack(mn_lo, mn_hi) : 0;
+    }
+};
+template <class W> struct MtRing { static constexpr uint WAVE = 16u * 16u * W::PIECES + 32u; };      // one unit and its d's
+template <> struct MtRing<MtQ4K> { static constexpr uint WAVE = (uint)MT_DEPTH * MT_UNIT; };
+template <class W> struct MtBytes { static constexpr uint N = W::BYTES; };
+template <> struct MtBytes<MtQ4K> { static constexpr uint N = Q4K_BYTES; };
+// One pass of 16 tokens against those digits, as gq_planes_pass
+template <class W>
+__device__ __forceinline__ void mt_digits_pass(const gq_i4 (&BH)[4], const gq_i4 (&BL)[4], long Bm, float dh, float dmin, const uchar* xp,
+                                               const uchar* pq, const float* sx16, uint kg, float (&acc)[4]) {
+    const gq_i4 zero = {0, 0, 0, 0};
+    gq_i4 DH = zero, DL = zero, Dlo = zero, Dhi = zero;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const gq_i4 A = *(const gq_i4*)(xp + W::STEP * (uint)c);
+        DH = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, BH[c], DH, 0, 0, 0);
+        DL = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, BL[c], DL, 0, 0, 0);
+    }
+    if (W::MINS) {
+        const gq_i4 lh = *(const gq_i4*)pq;
+        Dlo = __builtin_amdgcn_mfma_i32_16x16x32_i8(gq_pack((uint)lh[0], (uint)lh[1]), Bm, zero, 0, 0, 0);
+        Dhi = __builtin_amdgcn_mfma_i32_16x16x32_i8(gq_pack((uint)lh[2], (uint)lh[3]), Bm, zero, 0, 0, 0);
+    }
+    const float4 sx = *(const float4*)(sx16 + 4u * kg);
+    const float sxv[4] = {sx.x, sx.y, sx.z, sx.w};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const float isum = (float)(DH[v] * 256 + DL[v]);
+        acc[v] = W::MINS ? __fmaf_rn(sxv[v], __fmaf_rn(-dmin, (float)(Dhi[v] * 64 + Dlo[v]), __fmul_rn(dh, isum)), acc[v])
+                         : __fmaf_rn(__fmul_rn(sxv[v], dh), isum, acc[v]);
+    }
+}
+// A pass stages 16 P assignments: as many tiles as the expert has, up to four and to what fits (16 P (K + 32) + 5 P K / 4 + 64 P
+// + 256 <= 81920).  An expert's rows are read and unpacked once per pass (2048 x 768, 256 tokens over 128 experts with 8 slots
+// each, 16 per expert on average: with one tile of 16 a pass every other expert was read twice; 512 tokens 181 -> 164 us the
+// layer with the down rows read once where two tiles read them twice).  A wider pass than the expert fills costs (32 experts
+// of 512 x 1536 at 19 each, the layer 36.0 us at the width that fits the count, 37.8 at the widest that fits LDS).
+template <class W, bool GU, int P>
 __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, const float* __restrict__ xs,
                                             const uchar* __restrict__ w0, const uchar* __restrict__ w1, float* __restrict__ out,
                                             const uint* __restrict__ offsets, const uint* __restrict__ list,
                                             uint K, uint N, uint KSEL, uint NA, uchar* lds) {
+    constexpr bool DMA = std::is_same<W, MtQ4K>::value;
     constexpr uint TP = 16u * P;
     constexpr int D = MT_DEPTH;
     const uint e = blockIdx.y;
@@ -1050,7 +1170,7 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
     uint* lav = (uint*)(lds + o_av);               // [TP] the pass's assignments
     if (tid < 64u) ((uint*)(lds + o_zero))[tid] = 0u;
     const uint n = lane & 15u, kg = lane >> 4;
-    const size_t rb = (size_t)nsb * Q4K_BYTES;
+    const size_t rb = (size_t)nsb * MtBytes<W>::N;
     const uint tiles = (N + 15u) >> 4;
     // copies of a unit: nine lanes per row, seven rows per copy (rows 14 and 15 in the third)
     const uint cq = lane / 9u, cpc16 = (lane - cq * 9u) * 16u, c_off = cq * (uint)rb + cpc16;
@@ -1059,8 +1179,14 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
     const uint first = group * gridDim.x + blockIdx.x, rounds = (tiles + stride - 1u) / stride;
     const uint my_tiles = first < tiles ? (tiles - first + stride - 1u) / stride : 0u;
     const uchar* const w = GU && (wave & 1u) ? w1 : w0;
-    const uint ring = (uint)(size_t)(__attribute__((address_space(3))) uchar*)lds + MT_LDS + wave * ((uint)D * MT_UNIT);
-    const uchar* const rd = lds + MT_LDS + wave * ((uint)D * MT_UNIT) + n * Q4K_BYTES;
+    uchar* const own = lds + MT_LDS + wave * MtRing<W>::WAVE;
+    const uint ring = (uint)(size_t)(__attribute__((address_space(3))) uchar*)lds + MT_LDS + wave * MtRing<W>::WAVE;
+    const uchar* const rd = own + n * Q4K_BYTES;
+    // the pieces of a unit that go through registers (past the last they repeat it)
+    constexpr uint PC = DMA ? 1u : MtRing<W>::WAVE / 256u, NQ = (16u * PC + 63u) / 64u;
+    typedef gq_i4 __attribute__((aligned(2))) piece;
+    gq_i4 wv[NQ];
+    uint wd = 0u;
     for (uint tt = a0; tt < a1; tt += TP) {
         const uint cnt = min(TP, a1 - tt);
         // This wave's tiles as one stream of units (16 rows at one super-block), copied by the memory system into the wave's
@@ -1068,30 +1194,40 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
         const uint units = my_tiles * nsb;
         uint i_u = 0u, i_sb = 0u, i_tile = first, i_slot = 0u;
         auto issue_next = [&]() {
-            const size_t at = (size_t)w + ((size_t)e * N + i_tile * 16u) * rb + (size_t)i_sb * Q4K_BYTES;
+            const size_t at = (size_t)w + ((size_t)e * N + i_tile * 16u) * rb + (size_t)i_sb * MtBytes<W>::N;
             const uchar* base = (const uchar*)(((size_t)(uint)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
                                                (uint)__builtin_amdgcn_readfirstlane((int)(uint)at));   // (the copy wants it in scalar registers)
-            const uint dst = ring + i_slot * MT_UNIT;
-            uint o0 = c_off, o1 = c_off + 7u * (uint)rb, o2 = c_off + 14u * (uint)rb;
-            if (N - i_tile * 16u < 16u) {                          // the last tile of a ragged matrix: no row past N
-                const uint top = N - i_tile * 16u - 1u;
-                o0 = min(cq, top) * (uint)rb + cpc16;
-                o1 = min(7u + cq, top) * (uint)rb + cpc16;
-                o2 = min(14u + cq, top) * (uint)rb + cpc16;
+            if constexpr (DMA) {
+                const uint dst = ring + i_slot * MT_UNIT;
+                uint o0 = c_off, o1 = c_off + 7u * (uint)rb, o2 = c_off + 14u * (uint)rb;
+                if (N - i_tile * 16u < 16u) {                          // the last tile of a ragged matrix: no row past N
+                    const uint top = N - i_tile * 16u - 1u;
+                    o0 = min(cq, top) * (uint)rb + cpc16;
+                    o1 = min(7u + cq, top) * (uint)rb + cpc16;
+                    o2 = min(14u + cq, top) * (uint)rb + cpc16;
+                }
+                if (lane < 63u) {
+                    lds_dma16(base, o0, dst);
+                    lds_dma16(base, o1, dst + 1008u);
+                }
+                if (lane < 18u) lds_dma16(base, o2, dst + 2016u);
+                i_slot = i_slot + 1u == (uint)D ? 0u : i_slot + 1u;
+            } else {
+                const uint top = min(15u, N - i_tile * 16u - 1u);
+#pragma unroll
+                for (uint q = 0; q < NQ; q++) {
+                    const uint p = min(lane + 64u * q, 16u * PC - 1u), r = p / PC;
+                    wv[q] = *(const piece*)(base + (min(r, top) * (uint)rb + (p - r * PC) * 16u));
+                }
+                wd = W::tail(base + min(n, top) * (uint)rb);
             }
-            if (lane < 63u) {
-                lds_dma16(base, o0, dst);
-                lds_dma16(base, o1, dst + 1008u);
-            }
-            if (lane < 18u) lds_dma16(base, o2, dst + 2016u);
             i_u++;
-            i_slot = i_slot + 1u == (uint)D ? 0u : i_slot + 1u;
             if (++i_sb == nsb) {
                 i_sb = 0u;
                 i_tile += stride;
             }
         };
-        for (uint k = 0; k < (uint)D; k++)
+        for (uint k = 0; k < (DMA ? (uint)D : 1u); k++)
             if (i_u < units) issue_next();
         __syncthreads();                           // the previous pass is done with the staged tokens
         if (tid < TP) lav[tid] = min(list[min(tt + tid, a1 - 1u)], NA - 1u);
@@ -1113,9 +1249,13 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
                 bs = dot4_i8(v[q].y, 0x01010101u, bs); bs = dot4_i8(v[q].z, 0x01010101u, bs); bs = dot4_i8(v[q].w, 0x01010101u, bs);
                 bs += dpp_i32<OJK_DPP_QUAD_XOR1>(bs);
                 if (i < total) {
-                    uchar* const x = lds + (size_t)t * S + (o & ~63u) + ((o & 16u) << 1) + ((o & 32u) >> 2);
-                    *(uint2*)x = make_uint2(v[q].x, v[q].y);
-                    *(uint2*)(x + 16u) = make_uint2(v[q].z, v[q].w);
+                    if constexpr (DMA) {
+                        uchar* const x = lds + (size_t)t * S + (o & ~63u) + ((o & 16u) << 1) + ((o & 32u) >> 2);
+                        *(uint2*)x = make_uint2(v[q].x, v[q].y);
+                        *(uint2*)(x + 16u) = make_uint2(v[q].z, v[q].w);
+                    } else {
+                        *(uint4*)(lds + (size_t)t * S + o) = v[q];
+                    }
                     lbq[((o >> 8) * TP + t) * 16u + 8u * (tid & 1u) + ((o >> 5) & 7u)] = (uchar)((tid & 1u) ? bs >> 6 : bs & 63);
                 }
             }
@@ -1131,7 +1271,9 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
 #pragma unroll
         for (int p = 0; p < P; p++) {
             const bool on = n + 16u * p < cnt;
-            xa[p] = on ? lds + (size_t)(n + 16u * p) * S + 16u * kg : lds + o_zero + 16u * kg;
+            uint at = 16u * kg;
+            if constexpr (!DMA) at = W::token_at(kg);
+            xa[p] = on ? lds + (size_t)(n + 16u * p) * S + at : lds + o_zero + at;
             xstep[p] = on ? 256u : 0u;
         }
         uint c_tile = first, c_slot = 0u, u = 0u;
@@ -1144,29 +1286,50 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
             const bool has = c_tile < tiles;
             if (has)
                 for (uint sb = 0; sb < nsb; sb++, u++) {
-                    if (units - u >= (uint)D) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(3 * (D - 1)) : "memory");
-                    else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-                    const uchar* blk = rd + c_slot * MT_UNIT;
-                    c_slot = c_slot + 1u == (uint)D ? 0u : c_slot + 1u;
-                    GqW c;
-                    c.hdr = *(const uint4*)blk;
+                    if constexpr (DMA) {
+                        if (units - u >= (uint)D) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(3 * (D - 1)) : "memory");
+                        else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+                        const uchar* blk = rd + c_slot * MT_UNIT;
+                        c_slot = c_slot + 1u == (uint)D ? 0u : c_slot + 1u;
+                        GqW c;
+                        c.hdr = *(const uint4*)blk;
+    #pragma unroll
+                        for (int q = 0; q < 4; q++) c.q[q] = *(const uint2*)(blk + 16u + 32u * q + 8u * kg);
+                        gq_i4 BA[4], BB[4];
+                        const float d = f16_bits_to_f32(c.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(c.hdr.x >> 16);
+                        const uint mn_lo = c.hdr.z & 0x3F3F3F3Fu;
+                        const uint mn_hi = ((c.hdr.w >> 4) & 0x0F0F0F0Fu) | ((c.hdr.z >> 2) & 0x30303030u);
+                        const long Bm = kg == 0u ? gq_pack(mn_lo, mn_hi) : 0;
+                        gq_planes(c, BA, BB);
+                        // the unit is in registers: its slot takes the unit D ahead
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                        if (i_u < units) issue_next();
+                        __builtin_amdgcn_sched_barrier(0);
+    #pragma unroll
+                        for (int p = 0; p < P; p++)
+                            if ((uint)p < np)
+                                gq_planes_pass(BA, BB, Bm, d, dmin, xa[p] + sb * xstep[p], lbq + ((size_t)sb * TP + 16u * p + n) * 16u,
+                                               lsx + sb * TP + 16u * p, kg, acc[p]);
+                    } else {
 #pragma unroll
-                    for (int q = 0; q < 4; q++) c.q[q] = *(const uint2*)(blk + 16u + 32u * q + 8u * kg);
-                    gq_i4 BA[4], BB[4];
-                    const float d = f16_bits_to_f32(c.hdr.x & 0xFFFFu), dmin = f16_bits_to_f32(c.hdr.x >> 16);
-                    const uint mn_lo = c.hdr.z & 0x3F3F3F3Fu;
-                    const uint mn_hi = ((c.hdr.w >> 4) & 0x0F0F0F0Fu) | ((c.hdr.z >> 2) & 0x30303030u);
-                    const long Bm = kg == 0u ? gq_pack(mn_lo, mn_hi) : 0;
-                    gq_planes(c, BA, BB);
-                    // the unit is in registers: its slot takes the unit D ahead
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    if (i_u < units) issue_next();
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (uint q = 0; q < NQ; q++) *(gq_i4*)(own + min(lane + 64u * q, 16u * PC - 1u) * 16u) = wv[q];
+                        if (16u * PC < MtBytes<W>::N) ((ushort*)(own + 256u * PC))[n] = (ushort)wd;
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                        W c;
+                        c.read(own + n * (16u * PC), kg, ((const ushort*)(own + 256u * PC))[n]);
+                        if (i_u < units) issue_next();
+                        gq_i4 BH[4], BL[4];
+                        c.planes(kg, BH, BL);
+                        const float dh = 0.5f * c.d(), dmin = c.dmin();      // (the digits are of twice the integers)
+                        const long Bm = c.mins(kg);
 #pragma unroll
-                    for (int p = 0; p < P; p++)
-                        if ((uint)p < np)
-                            gq_planes_pass(BA, BB, Bm, d, dmin, xa[p] + sb * xstep[p], lbq + ((size_t)sb * TP + 16u * p + n) * 16u,
-                                           lsx + sb * TP + 16u * p, kg, acc[p]);
+                        for (int p = 0; p < P; p++)
+                            if ((uint)p < np)
+                                mt_digits_pass<W>(BH, BL, Bm, dh, dmin, xa[p] + sb * xstep[p], lbq + ((size_t)sb * TP + 16u * p + n) * 16u,
+                                                  lsx + sb * TP + 16u * p, kg, acc[p]);
+                    }
                 }
             // D register v of lane (n, kg): assignment 16 p + 4 kg + v of the pass, row n of the tile
             const bool mine = has && c_tile * 16u + n < N;
@@ -1201,26 +1364,34 @@ __device__ __forceinline__ void moe_mt_body(const signed char* __restrict__ xq, 
     }
 }
 
-#define MT_RUN(GU, X, S, W0, W1, OUT, KS)                                                                              \
+#define MT_FITS(P) (16u * P * (K + 32u) + 5u * P * (K >> 2) + 64u * P + 256u <= MT_LDS)
+#define MT_RUN(W, GU, X, S, W0, W1, OUT, KS)                                                                           \
     do {                                                                                                              \
-        if (32u * (K + 32u) + 5u * (K >> 1) + 384u <= MT_LDS) moe_mt_body<GU, 2>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt); \
-        else moe_mt_body<GU, 1>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt);                              \
+        const uint n_ = min(offsets[blockIdx.y + 1u], NA) - min(offsets[blockIdx.y], NA);                             \
+        if (n_ > 48u && MT_FITS(4u)) moe_mt_body<W, GU, 4>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt);   \
+        else if (n_ > 32u && MT_FITS(3u)) moe_mt_body<W, GU, 3>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt); \
+        else if (n_ > 16u && MT_FITS(2u)) moe_mt_body<W, GU, 2>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt); \
+        else moe_mt_body<W, GU, 1>(X, S, W0, W1, OUT, offsets, list, K, N, KS, NA, lds_mt);                           \
     } while (0)
 extern "C" __global__ void __launch_bounds__(1024)
 moe_gu_q4k_mt(const signed char* __restrict__ xq, const float* __restrict__ xs, const uchar* __restrict__ wg,
               const uchar* __restrict__ wu, float* __restrict__ act, const uint* __restrict__ offsets,
               const uint* __restrict__ list, uint K, uint N, uint KSEL, uint NA) {
     __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS + MT_RING + 8192u];
-    MT_RUN(true, xq, xs, wg, wu, act, KSEL);
+    MT_RUN(MtQ4K, true, xq, xs, wg, wu, act, KSEL);
 }
 
-extern "C" __global__ void __launch_bounds__(1024)
-moe_down_q4k_mt(const signed char* __restrict__ aq, const float* __restrict__ as_, const uchar* __restrict__ wd,
-                float* __restrict__ dv, const uint* __restrict__ offsets, const uint* __restrict__ list,
-                uint K, uint N, uint NA) {
-    __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS + MT_RING];
-    MT_RUN(false, aq, as_, wd, wd, dv, 1u);
-}
+#define MOE_DOWN_MT(FMT, W)                                                                                            \
+    extern "C" __global__ void __launch_bounds__(1024)                                                                \
+    moe_down_##FMT##_mt(const signed char* __restrict__ aq, const float* __restrict__ as_, const uchar* __restrict__ wd, \
+                        float* __restrict__ dv, const uint* __restrict__ offsets, const uint* __restrict__ list,       \
+                        uint K, uint N, uint NA) {                                                                     \
+        __shared__ __attribute__((aligned(16))) uchar lds_mt[MT_LDS + 16u * MtRing<W>::WAVE];                          \
+        MT_RUN(W, false, aq, as_, wd, wd, dv, 1u);                                                                     \
+    }
+MOE_DOWN_MT(q4k, MtQ4K)
+MOE_DOWN_MT(q5k, MtQ5K)
+MOE_DOWN_MT(q6k, MtQ6K)
 #undef MT_RUN
 
 // ------------------------------------------------------------------ combine

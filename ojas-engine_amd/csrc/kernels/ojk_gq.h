@@ -112,3 +112,17 @@ __device__ __forceinline__ void gq_planes_pass(const gq_i4 (&BA)[4], const gq_i4
 #pragma unroll
     for (int v = 0; v < 4; v++) acc[v] += sxv[v] * (d * (float)(8 * DB[v] + DA[v]) - dmin * (float)(64 * Dhi[v] + Dlo[v]));
 }
+
+// Two signed digits of twice a product, four products at a time: ev and od hold p + 128 in their 16-bit halves (products
+// 0, 2 and 1, 3), p even.  hi takes their upper bytes and lo their lower bytes with the sign bit flipped, so that
+// p = 256 hi + lo with both in int8, exactly.
+__device__ __forceinline__ void gq_digits(uint ev, uint od, int& hi, int& lo) {
+    hi = (int)__builtin_amdgcn_perm(od, ev, 0x07030501u);
+    lo = (int)(__builtin_amdgcn_perm(od, ev, 0x06020400u) ^ 0x80808080u);
+}
+// four codes (a byte each) times f, plus b
+__device__ __forceinline__ void gq_scale4(uint codes, gq_u16x2 f, gq_u16x2 b, int& hi, int& lo) {
+    const gq_u16x2 ev = __builtin_bit_cast(gq_u16x2, codes & 0x00FF00FFu) * f + b;
+    const gq_u16x2 od = __builtin_bit_cast(gq_u16x2, __builtin_amdgcn_perm(0u, codes, 0x0C030C01u)) * f + b;
+    gq_digits(__builtin_bit_cast(uint, ev), __builtin_bit_cast(uint, od), hi, lo);
+}

@@ -2261,6 +2261,8 @@ static std::vector<ojh_kernel_spec> build_manifest() {
     add("moe_gu_q4k_slots", "moe", 6, 6, OJH_Q4_K, 10, check_moe, shape_moe);
     add("moe_down_q4k_slots", "moe", 5, 5, OJH_Q4_K, 11, check_moe, shape_moe);
     add("moe_down_q5k_m", "moe", 6, 3, OJH_Q5_K, 4, check_moe, shape_moe);
+    add("moe_down_q5k_mt", "moe", 6, 3, OJH_Q5_K, 13, check_moe, shape_moe);
+    add("moe_down_q6k_mt", "moe", 6, 3, OJH_Q6_K, 13, check_moe, shape_moe);
     add("moe_down_q5k_gs", "gemm_q8k", 6, 3, OJH_Q5_K, 22, check_moe, shape_moe);
     add("moe_down_q6k_gs", "gemm_q8k", 6, 3, OJH_Q6_K, 22, check_moe, shape_moe);
     add("moe_down_q5k_dec", "moe", 5, 5, OJH_Q5_K, 9, check_moe, shape_moe);

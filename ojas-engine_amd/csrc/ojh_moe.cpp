@@ -211,6 +211,7 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     const bool down5 = down->type != OJH_Q4_K;   // Q5_K or Q6_K down tensors: integer dots at every batch size
     const std::string down_dec = std::string("moe_down_") + ojh_format(down->type)->tag + "_dec";
     const std::string down_m = std::string("moe_down_") + ojh_format(down->type)->tag + "_m";
+    const std::string down_mt = std::string("moe_down_") + ojh_format(down->type)->tag + "_mt";
     if (d % 256 || n_ff % 256) return ojh_fail(OJH_ERR_ARG, "moe_ffn: d=%u and n_ff=%u must be multiples of 256", d, n_ff);
     if (gate->k != d || up->k != d || gate->n != (uint64_t)E * n_ff || up->n != gate->n || down->k != n_ff ||
         down->n != (uint64_t)E * d)
@@ -263,7 +264,7 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
                     (dev->moe_mode == 0 && (uint64_t)NA >= (uint64_t)4 * E);
     // ... a wave per row tile where 16 tokens of K fit the workgroup's LDS (OJAS_HIP_MOE=4 keeps the workgroup-per-tile form)
     const bool mt_gu = mm && dev->moe_mode != 4 && ojh_moe_mt_lds(d) <= 81920;
-    const bool mt_down = mm && dev->moe_mode != 4 && !down5 && ojh_moe_mt_lds(n_ff) <= 81920;
+    const bool mt_down = mm && dev->moe_mode != 4 && ojh_moe_mt_lds(n_ff) <= 81920;
     uint32_t b_mt[3] = {1024, 1, 1};
     // 1. quantize the tokens once, 2. group the (token, slot) assignments by expert: one launch where a token is one
     //    workgroup's work (the grouping rides along as an extra workgroup), two otherwise
@@ -289,10 +290,11 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     {
         if ((rc = ojh_quant_q8k_launch(dev, act->ptr, OJH_X_F32, NA, n_ff, aq->ptr, as_->ptr))) return rc;
     }
-    // 5. down, one launch over all experts.  Q5_K / Q6_K down tensors: once experts see a handful of tokens each, the
-    //    int8 matrix tile of the dense path (one scale group per instruction) over each expert's assignments; the
-    //    integer-dot form below keeps an expert's rows in registers and walks its assignments one by one
-    const uint32_t gs_from = dev->moe_down_gs != 1 ? dev->moe_down_gs : 10u;
+    // 5. down, one launch over all experts.  Q5_K / Q6_K down tensors of many experts take the wave tiles as Q4_K ones do; the
+    //    int8 matrix tile of the dense path over each expert's assignments has those of few experts once they see ten each (8
+    //    experts of 4096 x 2048 at 12 each, whole layer, Q6_K 54 against 61 us on the wave tiles, at 100 181 against 210) and
+    //    of any number from 192 each (32 experts of 1024 x 512 at 256 each 132 against 139; at 128 level, at 64 67 against 56)
+    const uint32_t gs_from = dev->moe_down_gs != 1 ? dev->moe_down_gs : E <= 12 ? 10u : 192u;
     if (down5 && gs_from && (uint64_t)NA >= (uint64_t)gs_from * E && dev->moe_mode != 2) {
         if ((rc = ensure(dev, "gemm_q8k"))) return rc;
         const std::string down_gs = std::string("moe_down_") + ojh_format(down->type)->tag + "_gs";
@@ -303,10 +305,9 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
                              {n_ff, d, NA}, g, b256)))
             return rc;
     } else {
-        const bool dots = down5 || !mm;
+        const bool dots = !mt_down && (down5 || !mm);
         uint32_t g[3] = {mt_down ? ojh_moe_mt_groups(dev, n_ff, d, E, false, &b_mt[0]) : dots && n_ff <= 1024 ? (d + 31) / 32 : (d + 15) / 16, E, 1};
-        // (Q5_K rows have no matrix-core form: they stay on integer dots at every batch size)
-        if ((rc = ojh_launch(dev, down5 ? down_m.c_str() : mt_down ? "moe_down_q4k_mt" : mm ? "moe_down_q4k_mm" : "moe_down_q4k_m",
+        if ((rc = ojh_launch(dev, mt_down ? down_mt.c_str() : dots ? down_m.c_str() : "moe_down_q4k_mm",
                              {aq->ptr, as_->ptr, (char *)down->raw->ptr + down->off, dv->ptr, offsets, list},
                              {n_ff, d, NA}, g, mt_down ? b_mt : b256)))
             return rc;

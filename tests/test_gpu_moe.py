@@ -253,6 +253,40 @@ def test_grouped_wave_tiles_by_name(gpu, orc, pkg, k, n):
             assert peak_err(got[i], want[i]) <= 2e-5, (name, i)
 
 
+@pytest.mark.parametrize("dty", [Q4_K, 13, 14])
+@pytest.mark.parametrize("k,n", [(256, 40), (1024, 24), (1280, 20), (1536, 8), (2048, 33), (4608, 17)])
+def test_grouped_wave_tiles_of_every_pass_width_by_name(gpu, orc, pkg, k, n, dty):
+    """`moe_down_{q4k,q5k,q6k}_mt` over K on both sides of the passes of 64, 48, 32 and 16 assignments, experts whose counts
+    end a pass or go one beyond: every assignment against matvec_kq, whatever the workgroups per expert and their waves."""
+    tag = {Q4_K: "q4k", 13: "q5k", 14: "q6k"}[dty]
+    counts = [0, 16, 17, 48, 49, 64, 65, 1]
+    E, na, nsb = len(counts), sum(counts), k // 256
+    w = pkg.synth.weights(dty, E * n, k, "moemtp", "w", dty, k, n)
+    act = pkg.synth.normal_f32(na * k, "moemtp", "act", k).reshape(na, k)
+    perm = pkg.synth.rng("moemtp", "perm").permutation(na).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    gpu.ensure_family("moe")
+    gpu.ensure_family("gemv_q8k")
+    aq, as_ = gpu.alloc_bytes(na * k), gpu.alloc(na * nsb)
+    gpu.quant_q8k(gpu.upload(act), na, k, aq, as_)
+    wd, od, ld = gpu.upload_bytes(w), gpu.upload_bytes(offsets), gpu.upload_bytes(perm)
+    rb = len(w) // (E * n)
+    seen = []
+    for rg, block in ((1, 1024), (min(3, (n + 15) // 16), 1024), (1, 512)):
+        dv = gpu.upload(np.full(na * n + n, 777.25, np.float32))
+        gpu.dispatch(gpu.begin(), f"moe_down_{tag}_mt", [(aq, 0), (as_, 0), (wd, 0), (dv, 0), (od, 0), (ld, 0)], [k, n, na],
+                     [rg, E, 1], [block, 1, 1])
+        got = gpu.read(dv, na * n + n)
+        assert np.all(got[na * n:] == np.float32(777.25))
+        seen.append(got[:na * n].view(np.uint32).copy())
+    assert np.array_equal(seen[0], seen[1]) and np.array_equal(seen[0], seen[2])
+    got = seen[0].view(np.float32).reshape(na, n)
+    for e in range(E):
+        for i in range(offsets[e], offsets[e + 1]):
+            a = int(perm[i])
+            assert peak_err(got[a], orc.matvec_kq(w[e * n * rb:(e + 1) * n * rb], dty, n, k, act[a])) <= 2e-5, (e, a)
+
+
 @pytest.mark.parametrize("dty", [13, 14])
 def test_grouped_int8_tile_by_name(gpu, orc, pkg, dty):
     """`moe_down_{q5k,q6k}_gs(aq, as, wd, dv, offsets, list, K, N, NA)`: every assignment's row against matvec_kq of its
