@@ -99,11 +99,11 @@ struct ojh_device {
     uint32_t q4k_mf_min_m = 5;   // OJAS_HIP_Q4K_MF_MIN_M: tokens from which Q4_K rows go to the int8 matrix cores
     int moe_mode = 0;            // OJAS_HIP_MOE: 0 = by batch size, 1 = matrix cores always, 2 = grouped integer dots always,
                                  // 3 = per-assignment decode form always, 4 = matrix cores in the workgroup-per-tile form always
-    uint32_t moe_dec_tokens = 2; // OJAS_HIP_MOE_DEC_TOKENS: the decode form serves up to this many tokens (128 experts, top 8, weights from HBM: 2 tokens 21.0 against 23.3 us grouped, 3 tokens 27.4 against 25.9, 8 tokens 59 against 38)
+    int moe_dec_tokens = -1;     // OJAS_HIP_MOE_DEC_TOKENS: the decode form serves up to this many tokens (-1: by what their assignments' experts take, ojh_moe.cpp)
     int gemm_bdk = 1;            // OJAS_HIP_GEMM_BDK: 0 never takes the 64-row tile whose waves split K, 2 takes it wherever the 128-token tile would run
     bool gemm_sr = false;        // OJAS_HIP_GEMM_SR=1: K slices of the prefill tile meet in scratch, added in slice order (reproducible bits), instead of in f32 atomics
     bool moe_route_fuse = true;  // OJAS_HIP_MOE_ROUTE_FUSE=0: ojh_moe_ffn_routed keeps the router a launch of its own
-    bool moe_fuse = true;        // OJAS_HIP_MOE_FUSE=0: the grouped pipeline keeps its quantizer and grouping launches apart
+    bool moe_fuse = true;        // OJAS_HIP_MOE_FUSE=0: the grouped pipeline keeps its router, quantizer and grouping launches apart
     bool gemm_exact = false;     // OJAS_HIP_GEMM_EXACT: Q4_K prefill through the tile that holds dequant_to_f16 bits
     bool fused_quant = false;    // OJAS_HIP_FUSED_QUANT=1: ojh_mm (m = 1, Q4_K) quantizes x inside the matvec launch
     uint32_t fq_blocks_per_cu = 8; // OJAS_HIP_FQ_BLOCKS: blocks per CU the fused-quantizer matvec aims for
@@ -206,6 +206,8 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
 int ojh_noalloc_setup(ojh_device *dev);   // resolves the static scratch array on the current GPU (ojh_noalloc.cpp)
 void ojh_gemm_q8k_tiles(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M, uint32_t *rw, uint32_t *rt);   // row tiles per workgroup / per wave of gemm_q8k_q4k_mf
 uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t E, bool gu, uint32_t *threads);   // workgroups per expert of those entries, and their threads
+constexpr uint32_t OJH_MOE_FOUND = 4096, OJH_MOE_FOUND_BITS = 512;   // most assignments that the _ti (_mi, _mj) expert products look through themselves
+uint64_t ojh_moe_ti_lds(uint32_t K, uint32_t NA);   // LDS bytes of moe_{gu,down}_*_ti where one expert has every assignment
 uint64_t ojh_moe_mt_lds(uint32_t K);                // LDS bytes of moe_{gu,down}_q4k_mt (ojh_manifest.cpp)
 uint64_t ojh_gemm_q8k_mk_lds(uint32_t K, uint32_t M);   // LDS bytes of gemm_q8k_q4k_mk (ojh_manifest.cpp)
 uint64_t ojh_gemm_q8k_ml_lds(uint32_t K);           // LDS bytes of gemm_q8k_q4k_ml (ojh_manifest.cpp)

@@ -1486,6 +1486,7 @@ static int shape_gemm_few(const ojh_kernel_spec *s, const ojh_device *dev, uint3
 }
 
 // LDS of the moe_*_mt entries: 16 token rows, their scales and split sums, a block of zeros, the pass's assignments
+uint64_t ojh_moe_ti_lds(uint32_t K, uint32_t NA) { return 16 * ((uint64_t)K + 32) + K / 4 + K + 256 + ((NA * 2ull + 15) & ~15ull); }   // of the _ti entries: the expert's list beside
 uint64_t ojh_moe_mt_lds(uint32_t K) { return 16 * ((uint64_t)K + 32) + K / 4 + K + 256 + 64; }
 
 // The MoE family; the number of tokens of the batched entries is read off the grid.
@@ -1613,6 +1614,68 @@ static int check_moe(const ojh_kernel_spec *s, const uint32_t *c, const uint32_t
         need[4] = (size_t)(E + 1) * 4;
         need[5] = (size_t)NA * 4;
         align[0] = align[2] = 16;
+        return OJH_OK;
+    }
+    case 23: {  // moe_topk_quant(lg, idx, wgt, x, xq, xs, E, KSEL, K)   grid [T,1,1]
+        uint32_t E = c[0], KS = c[1], K = c[2], T = grid[0];
+        if ((rc = check_block(block, 512))) return rc;
+        if (!E || E > 1024 || !KS || KS > E || KS > 64 || !K || K % 256) return ojh_fail(OJH_ERR_ARG, "%s: E=%u KSEL=%u K=%u out of range", s->name, E, KS, K);
+        if (!T || grid[1] != 1 || grid[2] != 1) return ojh_fail(OJH_ERR_ARG, "%s: grid must be [tokens,1,1]", s->name);
+        need[0] = (size_t)T * E * 4;
+        need[1] = need[2] = (size_t)T * KS * 4;
+        need[3] = (size_t)T * K * 4;
+        need[4] = (size_t)T * K;
+        need[5] = (size_t)T * (K / 256) * 4;
+        align[3] = align[4] = 16;
+        return OJH_OK;
+    }
+    case 24: case 25: {  // moe_gu_q4k_{mi,mil,ti}(xq, xs, wg, wu, act, idx, K, N, KSEL, NA, E)
+        const bool ti = s->rows_per_wave == 25;
+        uint32_t K = c[0], N = c[1], KS = c[2], NA = c[3], E = c[4];
+        if ((rc = check_block(block, !ti ? 256 : block[0] == 512 ? 512 : 1024))) return rc;
+        const uint32_t most = ti ? OJH_MOE_FOUND : OJH_MOE_FOUND_BITS;
+        if (!K || K % 256 || !N || !KS || !NA || NA % KS || NA > most || !E)
+            return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u KSEL=%u NA=%u (<= %u)", s->name, K, N, KS, NA, most);
+        if (ti) {
+            if (ojh_moe_ti_lds(K, NA) > 81920) return ojh_fail(OJH_ERR_ARG, "%s: 16 tokens of K=%u and a list of %u do not fit its 80 KB of LDS", s->name, K, NA);
+            if (!grid[0] || grid[0] > (N + 15) / 16 || grid[1] != std::min(E, NA) || grid[2] != 1)
+                return ojh_fail(OJH_ERR_ARG, "%s: grid must be [1 .. ceil(N/16), min(E, NA), 1]", s->name);
+        } else {
+            const uint32_t per = K <= 1024 ? 16 : 8;
+            if ((K > 2048) != !strcmp(s->name, "moe_gu_q4k_mil"))
+                return ojh_fail(OJH_ERR_UNSUPPORTED, "%s: K=%u (moe_gu_q4k_mi takes up to 2048, moe_gu_q4k_mil more)", s->name, K);
+            if (grid[0] != (N + per - 1) / per || grid[1] != std::min(E, NA) || grid[2] != 1)
+                return ojh_fail(OJH_ERR_ARG, "%s: grid must be [ceil(N/%u), min(E, NA), 1]", s->name, per);
+        }
+        need[0] = (size_t)(NA / KS) * K;
+        need[1] = (size_t)(NA / KS) * (K / 256) * 4;
+        need[2] = need[3] = (size_t)E * N * (K / 256) * 144;
+        need[4] = (size_t)NA * N * 4;
+        need[5] = (size_t)NA * 4;
+        align[0] = align[2] = align[3] = 16;
+        return OJH_OK;
+    }
+    case 26: case 27: {  // moe_down_{q4k,q5k,q6k}_{mi,ti}(act, wd, dv, idx, K, N, NA, E)
+        const bool ti = s->rows_per_wave == 27;
+        uint32_t K = c[0], N = c[1], NA = c[2], E = c[3];
+        const uint32_t most = ti ? OJH_MOE_FOUND : OJH_MOE_FOUND_BITS;
+        if ((rc = check_block(block, !ti ? 256 : block[0] == 512 ? 512 : 1024))) return rc;
+        if (!K || K % 256 || !N || !NA || NA > most || !E) return ojh_fail(OJH_ERR_ARG, "%s: K=%u N=%u NA=%u (<= %u)", s->name, K, N, NA, most);
+        if (ti) {
+            if (ojh_moe_ti_lds(K, NA) > 81920) return ojh_fail(OJH_ERR_ARG, "%s: 16 tokens of K=%u and a list of %u do not fit its 80 KB of LDS", s->name, K, NA);
+            if (!grid[0] || grid[0] > (N + 15) / 16 || grid[1] != std::min(E, NA) || grid[2] != 1)
+                return ojh_fail(OJH_ERR_ARG, "%s: grid must be [1 .. ceil(N/16), min(E, NA), 1]", s->name);
+        } else {
+            const uint32_t per = K <= 512 ? 64 : K <= 1024 ? 32 : 16;
+            if (K > 2048) return ojh_fail(OJH_ERR_UNSUPPORTED, "%s: K=%u exceeds the 2048 (eight super-blocks) a wave takes side by side", s->name, K);
+            if (grid[0] != (N + per - 1) / per || grid[1] != std::min(E, NA) || grid[2] != 1)
+                return ojh_fail(OJH_ERR_ARG, "%s: grid must be [ceil(N/%u), min(E, NA), 1]", s->name, per);
+        }
+        need[0] = (size_t)NA * K * 4;
+        need[1] = (size_t)E * N * (K / 256) * ojh_format(s->type)->bytes;
+        need[2] = (size_t)NA * N * 4;
+        need[3] = (size_t)NA * 4;
+        align[0] = align[1] = 16;
         return OJH_OK;
     }
     case 8: {   // moe_gu_q4k_dec(x, wg, wu, act, idx, K, N, KSEL, NA, E)
@@ -1804,7 +1867,13 @@ static int shape_moe(const ojh_kernel_spec *s, const ojh_device *dev, uint32_t K
     case 6: case 7: grid[0] = (N + 15) / 16; grid[1] = M ? M : 1; break;
     case 14: case 16: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = slots, one token
     case 15: case 17: grid[0] = (N + 3) / 4; break;                           // one token
-    case 12: case 13: grid[0] = ojh_moe_mt_groups(dev, K, N, M ? M : 1, s->rows_per_wave == 12, &block[0]); grid[1] = M ? M : 1; break;  // M = experts
+    case 12: case 13: case 25: case 27:   // M = experts
+        grid[0] = ojh_moe_mt_groups(dev, K, N, M ? M : 1, s->rows_per_wave == 12 || s->rows_per_wave == 25, &block[0]);
+        grid[1] = M ? M : 1;
+        break;
+    case 23: block[0] = 512; grid[0] = M ? M : 1; break;   // M = tokens
+    case 24: grid[0] = K <= 1024 ? (N + 15) / 16 : (N + 7) / 8; grid[1] = M ? M : 1; break;   // M = min(experts, assignments)
+    case 26: grid[0] = K <= 512 ? (N + 63) / 64 : K <= 1024 ? (N + 31) / 32 : (N + 15) / 16; grid[1] = M ? M : 1; break;
     case 8: case 10: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = assignments
     case 9: case 11: grid[0] = (N + 7) / 8; grid[1] = M ? M : 1; break;    // M = tokens
     default: grid[0] = (uint32_t)(((uint64_t)M * N + 255) / 256); break;  // N = D, M = tokens
@@ -2248,6 +2317,14 @@ static std::vector<ojh_kernel_spec> build_manifest() {
     add("moe_topk_m", "moe", 3, 2, 0, 1, check_moe, shape_moe);
     add("moe_group", "moe", 4, 2, 0, 2, check_moe, shape_moe);
     add("moe_quant_group", "moe", 7, 4, 0, 20, check_moe, shape_moe);
+    add("moe_topk_quant", "moe", 6, 3, 0, 23, check_moe, shape_moe);
+    add("moe_gu_q4k_mi", "moe", 6, 5, OJH_Q4_K, 24, check_moe, shape_moe);
+    add("moe_gu_q4k_mil", "moe", 6, 5, OJH_Q4_K, 24, check_moe, shape_moe);
+    add("moe_gu_q4k_ti", "moe", 6, 5, OJH_Q4_K, 25, check_moe, shape_moe);
+    for (uint32_t ty : {OJH_Q4_K, OJH_Q5_K, OJH_Q6_K}) {
+        add(std::string("moe_down_") + ojh_format(ty)->tag + "_mi", "moe", 4, 4, ty, 26, check_moe, shape_moe);
+        add(std::string("moe_down_") + ojh_format(ty)->tag + "_ti", "moe", 4, 4, ty, 27, check_moe, shape_moe);
+    }
     add("moe_gu_q4k_m", "moe", 7, 4, OJH_Q4_K, 3, check_moe, shape_moe);
     add("moe_down_q4k_m", "moe", 6, 3, OJH_Q4_K, 4, check_moe, shape_moe);
     add("moe_combine", "moe", 3, 4, 0, 5, check_moe, shape_moe);

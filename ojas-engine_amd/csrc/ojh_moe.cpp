@@ -3,6 +3,7 @@
 // graph_decode.rs:441-499, prefill graph_chunk.rs:564-628; CPU crates/ojas-cpu/src/cpu_glm.rs:519-597):
 // router -> group assignments by expert -> gate/up (+SiLU*mul) -> quantize -> down -> weighted sum.
 #include "ojh_internal.h"
+#include <cmath>
 #include <cstring>
 #include <string>
 
@@ -32,6 +33,57 @@ extern "C" int ojh_moe_route(ojh_device *dev, const ojh_buf *logits, uint32_t n_
     return ojh_launch(dev, "moe_topk_m", {logits->ptr, idx->ptr, wgt->ptr}, {n_expert, ksel}, grid, block);
 }
 
+// Whether Q5_K / Q6_K down products go to the int8 matrix tile of the dense path: over few experts once they see ten assignments
+// each (8 experts of 4096 x 2048 at 12 each, whole layer, Q6_K 54 against 61 us on the wave tiles, at 100 181 against 210),
+// over any number from 192 each (32 experts of 1024 x 512 at 256 each 132 against 139; at 128 level, at 64 67 against 56).
+static bool moe_dense_tile(const ojh_device *dev, uint64_t NA, uint32_t E, uint32_t down_type) {
+    const uint32_t from = dev->moe_down_gs != 1 ? dev->moe_down_gs : E <= 12 ? 10u : 192u;
+    return down_type != OJH_Q4_K && from && NA >= (uint64_t)from * E && dev->moe_mode != 2;
+}
+// Experts that NA assignments reach, on average
+static double moe_busy(uint64_t NA, uint32_t E) { return E * -std::expm1((double)NA * std::log1p(-1.0 / (E > 1 ? E : 1.0000001))); }
+static double moe_expert_bytes(uint32_t d, uint32_t n_ff, uint32_t down_type) {
+    return (double)n_ff * d / 256 * (2 * 144 + ojh_format(down_type)->bytes);
+}
+// Expert products on the matrix cores, in the launches that are given lists
+static bool moe_tiles(const ojh_device *dev, uint64_t NA, uint32_t E) {
+    return dev->moe_mode == 1 || dev->moe_mode == 4 || (dev->moe_mode == 0 && NA >= (uint64_t)4 * E);
+}
+// Whether a few tokens run in the decode form, two launches addressed by assignment: one token always, more while an expert's
+// bytes for each of their assignments are few — each is read by itself, and every workgroup quantizes its token (whole layer,
+// decode form against the grouped launches: 2 tokens, 24 MB 16.7 against 17.4 us, 42 MB 21.5 against 18.2; 3 - 6 tokens, 11
+// MB 11.4 against 14.2, 15 MB 12.3 against 14.2, 21 MB 17.9 against 14.9).
+static bool moe_decodes(const ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t ksel, uint32_t down_type) {
+    // what the two launches stage in LDS; the down launch keeps one partial sum per slot and lane group for up to 64 slots
+    if (!(d <= 8192 && n_ff <= 2048 && ksel <= 64 && (uint64_t)ksel * n_ff <= 32768)) return false;
+    if (dev->moe_mode) return dev->moe_mode == 3;
+    if (dev->moe_dec_tokens >= 0) return T <= (uint32_t)dev->moe_dec_tokens;
+    return T == 1 || (double)T * ksel * moe_expert_bytes(d, n_ff, down_type) <= (T == 2 ? 32e6 : 16e6);
+}
+// How the grouped products of K-quant experts that find their assignments in idx themselves run, four launches instead of six:
+// on the wave tiles from 3.4 - 0.75 d / 1024 assignments per expert, from 1.1 where a row of gate and up is longer than the dots'
+// one step of 2048 (whole layer, integer dots against tiles: 1024 x 512 at 1 each 20.9 against 27.8 us, at 3 33 against 30.6;
+// 2048 x 768 at 1 66 against 77, at 1.75 80.5 against 81.8, at 2 97 against 83; 2816 x 768 at 1 86 against 102; 2560 x 512 at
+// 1.4 106 against 82; 3072 x 1024 at 1.1 99 against 91), on integer dots below.  Not where a launch needs the lists in
+// memory (the dense tile, the tiles whose K is split), nor beyond what the kernels hold, nor where dots over rows of one step
+// have more than 150 MB to read: finding the assignments costs every wave what a list costs a workgroup (2048 x 768, 128
+// experts, 16 tokens: 66 us against 61, at 8 tokens 42 against 43).
+enum { MOE_LISTS, MOE_FIND_DOTS, MOE_FIND_TILES };
+static int moe_finds(const ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, uint32_t down_type) {
+    const uint64_t NA = (uint64_t)T * ksel;
+    if (!dev->moe_fuse || dev->moe_mode == 3 || dev->moe_mode == 4 || NA > OJH_MOE_FOUND || d % 256 || n_ff % 256 ||
+        moe_dense_tile(dev, NA, E, down_type))
+        return MOE_LISTS;
+    const bool fits = ojh_moe_ti_lds(d, (uint32_t)NA) <= 81920 && ojh_moe_ti_lds(n_ff, (uint32_t)NA) <= 81920;
+    const double from = d > 2048 ? 1.1 : 3.4 - 0.75 * d / 1024;
+    if (dev->moe_mode == 1 || (dev->moe_mode == 0 && fits && NA >= from * E)) return fits ? MOE_FIND_TILES : MOE_LISTS;
+    if (NA > OJH_MOE_FOUND_BITS || n_ff > 2048 || moe_tiles(dev, NA, E)) return MOE_LISTS;
+    return dev->moe_mode == 0 && d <= 2048 && moe_busy(NA, E) * moe_expert_bytes(d, n_ff, down_type) > 150e6 ? MOE_LISTS : MOE_FIND_DOTS;
+}
+static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, const ojh_buf *idx,
+               const ojh_buf *wgt, const ojh_lin *gate, const ojh_lin *up, const ojh_lin *down, ojh_buf *y, int accum, int act_mode,
+               const ojh_buf *logits);
+
 // Router + expert FFN.  A few tokens over Q4_K gate / up experts: the router runs inside the gate/up launch of the
 // decode form (every workgroup routes its token itself; idx / wgt are written for the down launch and for the
 // caller) — two launches per layer instead of three; otherwise ojh_moe_route, then ojh_moe_ffn.
@@ -43,11 +95,15 @@ extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T,
         return ojh_fail(OJH_ERR_ARG, "moe_ffn_routed: tokens=%u experts=%u (<= 1024) ksel=%u (<= 64, <= experts) out of range", T, E, ksel);
     const bool kq = gate->type == OJH_Q4_K && up->type == OJH_Q4_K &&
                     (down->type == OJH_Q4_K || down->type == OJH_Q5_K || down->type == OJH_Q6_K);
-    const bool dec_fits = d && n_ff && d % 256 == 0 && n_ff % 256 == 0 && d <= 8192 && n_ff <= 2048 && (uint64_t)ksel * n_ff <= 32768;
-    const bool fused = kq && act_mode != OJH_ACT_FLOAT && act_mode != OJH_ACT_FLOAT_EXACT && dec_fits &&
-                       (dev->moe_mode == 3 || (dev->moe_mode == 0 && T <= dev->moe_dec_tokens)) && dev->moe_route_fuse;
+    const bool fused = kq && act_mode != OJH_ACT_FLOAT && act_mode != OJH_ACT_FLOAT_EXACT && d && n_ff && d % 256 == 0 && n_ff % 256 == 0 &&
+                       moe_decodes(dev, T, d, n_ff, ksel, down->type) && dev->moe_route_fuse;
     int rc;
     if (!fused) {
+        if (kq && act_mode != OJH_ACT_FLOAT && d && n_ff && !moe_decodes(dev, T, d, n_ff, ksel, down->type) &&
+            moe_finds(dev, T, d, n_ff, E, ksel, down->type) != MOE_LISTS) {
+            if ((rc = span("moe_route: logits", logits, (size_t)T * E * 4, 4))) return rc;
+            return ffn(dev, x, T, d, n_ff, E, ksel, idx, wgt, gate, up, down, y, accum, act_mode, logits);
+        }
         if ((rc = ojh_moe_route(dev, logits, T, E, ksel, idx, wgt))) return rc;
         return ojh_moe_ffn(dev, x, T, d, n_ff, E, ksel, idx, wgt, gate, up, down, y, accum, act_mode);
     }
@@ -77,6 +133,13 @@ extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T,
 extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E,
                            uint32_t ksel, const ojh_buf *idx, const ojh_buf *wgt, const ojh_lin *gate,
                            const ojh_lin *up, const ojh_lin *down, ojh_buf *y, int accum, int act_mode) {
+    return ffn(dev, x, T, d, n_ff, E, ksel, idx, wgt, gate, up, down, y, accum, act_mode, nullptr);
+}
+
+// `logits`: the router runs first (idx and wgt are written), in the launch that quantizes the tokens; moe_finds has to hold
+static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, const ojh_buf *idx,
+               const ojh_buf *wgt, const ojh_lin *gate, const ojh_lin *up, const ojh_lin *down, ojh_buf *y, int accum, int act_mode,
+               const ojh_buf *logits) {
     if (!dev || !gate || !up || !down) return ojh_fail(OJH_ERR_ARG, "ojh_moe_ffn: NULL argument");
     if (!T || !E || E > 1024 || !ksel || ksel > E || T > 65535u / ksel)
         return ojh_fail(OJH_ERR_ARG, "moe_ffn: tokens=%u experts=%u ksel=%u out of range", T, E, ksel);
@@ -229,11 +292,9 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     // A few tokens: two launches addressed by assignment, activations quantized in registers,
     // weighted sum inside the down launch (bit-identical to the grouped integer-dot pipeline).
     // Measured on MI355X the grouped pipeline takes over once tokens start sharing experts.
-    // what the two launches stage in LDS; the down launch keeps one partial sum per slot and lane group for up to 64 slots
-    const bool dec_fits = d <= 8192 && n_ff <= 2048 && ksel <= 64 && (uint64_t)ksel * n_ff <= 32768;
-    if (dev->moe_mode == 3 || (dev->moe_mode == 0 && T <= dev->moe_dec_tokens && dec_fits)) {
-        if (!dec_fits)
-            return ojh_fail(OJH_ERR_UNSUPPORTED, "moe_ffn: the decode form serves d <= 8192, n_ff <= 2048, ksel <= 64 and ksel * n_ff <= 32768");
+    if (dev->moe_mode == 3 && !moe_decodes(dev, T, d, n_ff, ksel, down->type))
+        return ojh_fail(OJH_ERR_UNSUPPORTED, "moe_ffn: the decode form serves d <= 8192, n_ff <= 2048, ksel <= 64 and ksel * n_ff <= 32768");
+    if (moe_decodes(dev, T, d, n_ff, ksel, down->type)) {
         ojh_buf *act;
         if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
         uint32_t g1[3] = {(n_ff + 7) / 8, NA, 1};
@@ -244,6 +305,40 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
         uint32_t g2[3] = {(d + 7) / 8, T, 1};
         return ojh_launch(dev, down_dec.c_str(), {act->ptr, (char *)down->raw->ptr + down->off, idx->ptr, wgt->ptr, y->ptr},
                           {n_ff, d, ksel, E, (uint32_t)(accum != 0)}, g2, b256);
+    }
+    if (const int found = moe_finds(dev, T, d, n_ff, E, ksel, down->type); found != MOE_LISTS) {
+        // 1. the tokens quantized (and routed), 2. gate / up with SiLU * mul, 3. down over activations it quantizes itself
+        // (the CPU path quantizes `act` inside matvec_kq), 4. the router-weighted sum over slots, in slot order
+        const bool tiles = found == MOE_FIND_TILES;
+        const uint32_t ny = std::min(E, NA);
+        const void *wg = (char *)gate->raw->ptr + gate->off, *wu = (char *)up->raw->ptr + up->off, *wd = (char *)down->raw->ptr + down->off;
+        ojh_buf *xq, *xs, *act, *dv;
+        if ((rc = ojh_scratch_get(dev, "moe_xq", (size_t)T * d, &xq))) return rc;
+        if ((rc = ojh_scratch_get(dev, "moe_xs", (size_t)T * nsb_d * 4, &xs))) return rc;
+        if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
+        if ((rc = ojh_scratch_get(dev, "moe_dv", (size_t)NA * d * 4, &dv))) return rc;
+        if (logits) {
+            uint32_t g[3] = {T, 1, 1}, b[3] = {512, 1, 1};
+            rc = ojh_launch(dev, "moe_topk_quant", {logits->ptr, idx->ptr, wgt->ptr, x->ptr, xq->ptr, xs->ptr}, {E, ksel, d}, g, b);
+        } else {
+            rc = ojh_quant_q8k_launch(dev, x->ptr, OJH_X_F32, T, d, xq->ptr, xs->ptr);
+        }
+        if (rc) return rc;
+        // (the wave tiles' grid is cut for the experts that are likely to have an assignment, with a quarter to spare: a CU that
+        // holds a tile has room for no other, and the busy ones do not fall evenly onto the eight dies — 128 experts of 2048 x
+        // 768 at 16 tokens, some 81 busy: two workgroups each 77 us the layer, three 98)
+        const uint32_t busy = std::min<uint32_t>(E, (uint32_t)(1.25 * moe_busy(NA, E)) + 1u);
+        uint32_t g[3], b[3];
+        const char *gu = tiles ? "moe_gu_q4k_ti" : d > 2048 ? "moe_gu_q4k_mil" : "moe_gu_q4k_mi";
+        if ((rc = ojh_launch_shape(dev, gu, d, n_ff, tiles ? busy : ny, g, b))) return rc;
+        g[1] = ny;
+        if ((rc = ojh_launch(dev, gu, {xq->ptr, xs->ptr, (void *)wg, (void *)wu, act->ptr, idx->ptr}, {d, n_ff, ksel, NA, E}, g, b))) return rc;
+        const std::string dn = std::string("moe_down_") + ojh_format(down->type)->tag + (tiles ? "_ti" : "_mi");
+        if ((rc = ojh_launch_shape(dev, dn.c_str(), n_ff, d, tiles ? busy : ny, g, b))) return rc;
+        g[1] = ny;
+        if ((rc = ojh_launch(dev, dn.c_str(), {act->ptr, (void *)wd, dv->ptr, idx->ptr}, {n_ff, d, NA, E}, g, b))) return rc;
+        uint32_t gs[3] = {(uint32_t)(((uint64_t)T * d + 255) / 256), 1, 1};
+        return ojh_launch(dev, "moe_combine", {dv->ptr, wgt->ptr, y->ptr}, {T, ksel, d, (uint32_t)(accum != 0)}, gs, b256);
     }
     ojh_buf *xq, *xs, *act, *aq, *as_, *dv, *grp;
     if ((rc = ojh_scratch_get(dev, "moe_xq", (size_t)T * d, &xq))) return rc;
@@ -260,8 +355,7 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
     // MI355X, 128 experts of 2048 x 768: 4 assignments per expert — 48 tokens of top-8 take 105 us on dots and 115 on
     // the matrix cores, 64 tokens 120 and 116), on integer dots below that.  The two
     // forms round their f32 sums in different orders (last ulp).
-    const bool mm = dev->moe_mode == 1 || dev->moe_mode == 4 ||
-                    (dev->moe_mode == 0 && (uint64_t)NA >= (uint64_t)4 * E);
+    const bool mm = moe_tiles(dev, NA, E);
     // ... a wave per row tile where 16 tokens of K fit the workgroup's LDS (OJAS_HIP_MOE=4 keeps the workgroup-per-tile form)
     const bool mt_gu = mm && dev->moe_mode != 4 && ojh_moe_mt_lds(d) <= 81920;
     const bool mt_down = mm && dev->moe_mode != 4 && ojh_moe_mt_lds(n_ff) <= 81920;
@@ -291,11 +385,8 @@ extern "C" int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32
         if ((rc = ojh_quant_q8k_launch(dev, act->ptr, OJH_X_F32, NA, n_ff, aq->ptr, as_->ptr))) return rc;
     }
     // 5. down, one launch over all experts.  Q5_K / Q6_K down tensors of many experts take the wave tiles as Q4_K ones do; the
-    //    int8 matrix tile of the dense path over each expert's assignments has those of few experts once they see ten each (8
-    //    experts of 4096 x 2048 at 12 each, whole layer, Q6_K 54 against 61 us on the wave tiles, at 100 181 against 210) and
-    //    of any number from 192 each (32 experts of 1024 x 512 at 256 each 132 against 139; at 128 level, at 64 67 against 56)
-    const uint32_t gs_from = dev->moe_down_gs != 1 ? dev->moe_down_gs : E <= 12 ? 10u : 192u;
-    if (down5 && gs_from && (uint64_t)NA >= (uint64_t)gs_from * E && dev->moe_mode != 2) {
+    //    dense int8 tile has those of few experts and of the largest batches
+    if (moe_dense_tile(dev, NA, E, down->type)) {
         if ((rc = ensure(dev, "gemm_q8k"))) return rc;
         const std::string down_gs = std::string("moe_down_") + ojh_format(down->type)->tag + "_gs";
         uint32_t tiles = (T + 63) / 64;

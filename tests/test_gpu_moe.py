@@ -850,3 +850,48 @@ def test_expert_ffn_in_both_forms_of_the_wave_tiles(gpu, orc, pkg, T, E, ksel, d
                 gpu.lin(Q4_K, E * d, nff, down), yd, act_mode=pkg.ACT_Q8K)
     want = orc.moe_ffn(x, gi, gw, gate, up, Q4_K, down, Q4_K, E, nff, mode=0)
     assert peak_err(gpu.read(yd, T * d).reshape(T, d), want) <= TOL_SEEN
+
+
+@pytest.mark.parametrize("mode", ["1", "2"])
+@pytest.mark.parametrize("T,E,ksel,d,nff,dty", [(3, 64, 4, 1024, 512, 13), (5, 128, 8, 768, 768, 14), (16, 16, 8, 2048, 1280, Q4_K),
+                                                (17, 200, 8, 2304, 256, 14), (64, 100, 8, 256, 1024, 13), (40, 7, 7, 2816, 2048, Q4_K),
+                                                (9, 1000, 3, 512, 768, Q4_K), (4, 2, 2, 4096, 512, 14), (70, 12, 5, 1536, 512, Q4_K)])
+def test_products_that_find_their_assignments_against_lists(gpu, orc, pkg, monkeypatch, mode, T, E, ksel, d, nff, dty):
+    """The four-launch forms (integer dots `_mi` / `_mil`, wave tiles `_ti`) against the grouping's lists, bit for bit: fewer and more
+    assignments than experts, 128 and 512 of them and one more, rows of half, one and two steps of the dots, an expert with
+    more than 64, one with none; idx and wgt as the router alone writes them, y accumulated onto."""
+    gate = pkg.synth.q4k_weights(E * nff, d, "moefind", "g", E, d, nff)
+    up = pkg.synth.q4k_weights(E * nff, d, "moefind", "u", E, d, nff)
+    down = pkg.synth.weights(dty, E * d, nff, "moefind", "d", dty, E, d, nff)
+    x = pkg.synth.normal_f32(T * d, "moefind", "x", T, d).reshape(T, d)
+    lg = pkg.synth.normal_f32(T * E, "moefind", "lg", T, E).reshape(T, E)
+    lg[: T * 9 // 10, 0] += 30.0
+    if E > ksel:
+        lg[:, E - 1] -= 50.0
+    y0 = pkg.synth.normal_f32(T * d, "moefind", "y0").reshape(T, d)
+    outs = {}
+    monkeypatch.setenv("OJAS_HIP_MOE", mode)
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("OJAS_HIP_MOE_FUSE", fuse)
+        monkeypatch.setenv("OJAS_HIP_MOE_DOWN_GS", "0")
+        g = pkg.HipGpu(0)
+        try:
+            lg_, lu_, ld_ = g.lin(Q4_K, E * nff, d, gate), g.lin(Q4_K, E * nff, d, up), g.lin(dty, E * d, nff, down)
+            idx, wgt = g.upload_bytes(np.full(T * ksel + 2, 0xFFFFFFFF, np.uint32)), g.upload(np.full(T * ksel + 2, 777.0, np.float32))
+            yd = g.upload(np.concatenate([y0.ravel(), np.full(d, 12345.5, np.float32)]))
+            g.moe_ffn_routed(g.upload(x), T, d, nff, E, ksel, g.upload(lg), idx, wgt, lg_, lu_, ld_, yd, accum=True)
+            ya = g.upload(y0)
+            g.moe_ffn(g.upload(x), T, d, nff, E, ksel, idx, wgt, lg_, lu_, ld_, ya, accum=True)
+            got = g.read(yd, T * d + d)
+            assert np.array_equal(g.read(ya, T * d).view(np.uint32), got[:T * d].view(np.uint32))
+            outs[fuse] = (got, g.read(idx, T * ksel + 2, np.uint32), g.read(wgt, T * ksel + 2))
+        finally:
+            g.close()
+    for a, b in zip(outs["1"], outs["0"]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    got, gi, gw = outs["1"]
+    assert np.all(got[T * d:] == 12345.5)
+    for t in (0, T - 1):
+        want = orc.moe_ffn(x[t:t + 1], gi[t * ksel:(t + 1) * ksel].reshape(1, -1), gw[t * ksel:(t + 1) * ksel].reshape(1, -1), gate, up, Q4_K, down, dty, E, nff,
+                           mode=0)
+        assert peak_err(got[t * d:(t + 1) * d] - y0[t], want[0]) <= TOL, t
