@@ -37,11 +37,16 @@
 #include <type_traits>
 
 // ------------------------------------------------------------------ router
+// KSEL dependent rounds, each a maximum over the wave, are what the router waits for.  Probabilities are never negative, so
+// their bits order like integers: the maxima are integer ones (no canonicalising, the last three steps on the scalar unit),
+// and the winner is a vote on equality.  A NaN or infinite logit makes every probability NaN: then nothing is chosen (index
+// ~0, weights 1 / KSEL).
 template <int NI>
 __device__ __forceinline__ void moe_topk_lanes(const float* __restrict__ lg, uint* __restrict__ idx,
                                                float* __restrict__ wgt, uint E, uint KSEL) {
     // one wave per token; lane l owns experts l, l+64, ... (E <= 64 NI)
     const uint lane = threadIdx.x & 63u;
+    const int NONE = 0xBF800000;    // -1.0f: taken, or no expert
     float p[NI];
     float mx = -3.4028235e38f;
 #pragma unroll
@@ -59,33 +64,34 @@ __device__ __forceinline__ void moe_topk_lanes(const float* __restrict__ lg, uin
         if (e < E) sum += p[i];
     }
     sum = wave_sum(sum);
+    int key[NI];
 #pragma unroll
-    for (int i = 0; i < NI; i++)
-        if (lane + 64u * i < E) p[i] = p[i] / sum;
+    for (int i = 0; i < NI; i++) {
+        const float q = p[i] / sum;
+        key[i] = lane + 64u * i < E && q >= 0.0f ? __float_as_int(q) : NONE;
+    }
     float wsum = 0.0f, mine = 0.0f;
     uint mine_idx = 0;
     for (uint j = 0; j < KSEL; j++) {
-        float bv = -1.0f;
-        uint bi = 0xFFFFFFFFu;
+        int best = key[0];
 #pragma unroll
-        for (int i = 0; i < NI; i++) {  // ascending expert index within the lane: '>' keeps the lowest
-            if (p[i] > bv) { bv = p[i]; bi = lane + 64u * i; }
-        }
-        float m2 = wave_max(bv);
-        // lowest index among the lanes holding the maximum: an expert's index is lane + 64 i, so the lowest i with any
+        for (int i = 1; i < NI; i++) best = max(best, key[i]);
+        const int m2 = wave_max_i32(best);
+        // lowest index among the experts holding the maximum: an expert's index is lane + 64 i, so the lowest i with any
         // such lane decides, and within it the lowest lane — one vote per i and scalar bit scans instead of a second
         // reduction across the wave
         uint win = 0xFFFFFFFFu;
 #pragma unroll
         for (int i = NI - 1; i >= 0; i--) {
-            const unsigned long long vote = __ballot(bv == m2 && bi == lane + 64u * (uint)i);
+            const unsigned long long vote = __ballot(key[i] == m2);
             if (vote) win = (uint)__builtin_ctzll(vote) + 64u * (uint)i;
         }
-        wsum += m2;
-        if (lane == j) { mine = m2; mine_idx = win; }
+        if (m2 < 0) win = 0xFFFFFFFFu;
+        wsum += __int_as_float(m2);
+        if (lane == j) { mine = __int_as_float(m2); mine_idx = win; }
 #pragma unroll
         for (int i = 0; i < NI; i++)
-            if (lane + 64u * i == win) p[i] = -1.0f;
+            if (lane + 64u * i == win) key[i] = NONE;
     }
     if (lane < KSEL) {
         idx[lane] = mine_idx;
@@ -456,13 +462,26 @@ __device__ __forceinline__ uint2 oct_quant_q8k(float4 a, float4 b, float& scale)
     const float inv = __fdiv_rn(1.0f, scale);
     return make_uint2(q8k_pack4(a, inv), q8k_pack4(b, inv));
 }
-// (or threads `first` .. of them: a multiple of 32, as is their number `nt`)
+// (or threads `first` .. of them: a multiple of 32, as is their number `nt`)  DEPTH: trips whose loads are asked for at once
+template <int DEPTH = 1>
 __device__ __forceinline__ void block_quant_q8k(const float* __restrict__ x, uint n, signed char* q, float* s, uint first = 0u, uint nt = 256u) {
-    for (uint base = (threadIdx.x - first) * 8u; base < n; base += 8u * nt) {
-        float scale;
-        const uint2 c = oct_quant_q8k(*(const float4*)(x + base), *(const float4*)(x + base + 4u), scale);
-        *(uint2*)(q + base) = c;
-        if ((threadIdx.x & 31u) == 0) s[base >> 8] = scale;
+    for (uint base = (threadIdx.x - first) * 8u; base < n; base += 8u * nt * DEPTH) {
+        float4 a[DEPTH], b[DEPTH];
+#pragma unroll
+        for (int i = 0; i < DEPTH; i++) {
+            const uint at = min(base + 8u * nt * i, n - 8u);
+            a[i] = *(const float4*)(x + at);
+            b[i] = *(const float4*)(x + at + 4u);
+        }
+#pragma unroll
+        for (int i = 0; i < DEPTH; i++) {
+            const uint at = base + 8u * nt * i;
+            if (at >= n) break;
+            float scale;
+            const uint2 c = oct_quant_q8k(a[i], b[i], scale);
+            *(uint2*)(q + at) = c;
+            if ((threadIdx.x & 31u) == 0) s[at >> 8] = scale;
+        }
     }
 }
 
@@ -480,8 +499,11 @@ __device__ __forceinline__ size_t expert_base(const void* sel, uint a, bool slot
 }
 
 // Block (rb, a): 4 waves x 2 rows of gate and up of assignment a's expert against token a / KSEL.
-// ROUTE: the workgroup routes its token itself first — wave 0 runs the router over lg[t], the slot's expert is read
-// from LDS, and one workgroup per token writes idx / wgt out for the down launch (sel_g / sel_u are not read).
+// ROUTE: the workgroup routes its token itself first — wave 0 runs the router over lg[t] while the others quantize the
+// token, the slot's expert is read from LDS, and one workgroup per token writes idx / wgt out for the down launch (sel_g /
+// sel_u are not read).  A serial chain of trips to memory bounds the launch, not its bytes: the logits, the router's rounds, the
+// weights they name (128 experts of 2048 x 768, top 8, one token, traced: 9.0 -> 7.0 us with the token quantized beside the
+// router, the rounds on integers and a row's next step asked for before the present one is multiplied).
 template <bool SLOTS, bool ROUTE = false>
 __device__ __forceinline__ void moe_gu_dec_body(const float* __restrict__ x, const uchar* __restrict__ wg,
                                                 const uchar* __restrict__ wu, float* __restrict__ act,
@@ -497,11 +519,8 @@ __device__ __forceinline__ void moe_gu_dec_body(const float* __restrict__ x, con
     const uint t = a / KSEL;
     if (ROUTE) {
         if (threadIdx.x < 64u) moe_topk_body(lg + (size_t)t * EG, r_idx, r_wgt, EG, KSEL);
+        else block_quant_q8k<2>(x + (size_t)t * K, K, xq, xs, 64u, 192u);
         __syncthreads();
-        if (blockIdx.x == 0u && a == t * KSEL && threadIdx.x < KSEL) {
-            idx_out[a + threadIdx.x] = r_idx[threadIdx.x];
-            wgt_out[a + threadIdx.x] = r_wgt[threadIdx.x];
-        }
         sel_g = sel_u = r_idx;
         a -= t * KSEL;              // the slot: index into the token's own table
     }
@@ -513,35 +532,41 @@ __device__ __forceinline__ void moe_gu_dec_body(const float* __restrict__ x, con
     const uchar* u0 = wu + expert_base(sel_u, a, SLOTS, EU, (size_t)N * rb) + (size_t)row0 * rb;
     const bool two = row0 + 1u < N;
     const size_t r1 = two ? rb : 0;
-    // the first step's weights are on their way while the activations are quantized
-    const size_t o0 = (size_t)min(g, nsb - 1u) * Q4K_BYTES, q0 = o0 + 16u + l * 16u;
-    uint4 hg0 = *(const uint4*)(g0 + o0), qg0 = *(const uint4*)(g0 + q0);
-    uint4 hg1 = *(const uint4*)(g0 + r1 + o0), qg1 = *(const uint4*)(g0 + r1 + q0);
-    uint4 hu0 = *(const uint4*)(u0 + o0), qu0 = *(const uint4*)(u0 + q0);
-    uint4 hu1 = *(const uint4*)(u0 + r1 + o0), qu1 = *(const uint4*)(u0 + r1 + q0);
-    block_quant_q8k(x + (size_t)t * K, K, xq, xs);
-    __syncthreads();
-    float vg0 = 0.0f, vg1 = 0.0f, vu0 = 0.0f, vu1 = 0.0f;
-    for (uint sb = g; sb < nsb; sb += 8u) {
-        const Q4kFrag f = q4k_load_frag(xq, xs, sb, l);
-        vg0 += q4k_lane_dot(hg0, qg0, c, f);
-        vg1 += q4k_lane_dot(hg1, qg1, c, f);
-        vu0 += q4k_lane_dot(hu0, qu0, c, f);
-        vu1 += q4k_lane_dot(hu1, qu1, c, f);
-        if (sb + 8u < nsb) {
-            const size_t o = (size_t)(sb + 8u) * Q4K_BYTES, oq = o + 16u + l * 16u;
-            hg0 = *(const uint4*)(g0 + o); qg0 = *(const uint4*)(g0 + oq);
-            hg1 = *(const uint4*)(g0 + r1 + o); qg1 = *(const uint4*)(g0 + r1 + oq);
-            hu0 = *(const uint4*)(u0 + o); qu0 = *(const uint4*)(u0 + oq);
-            hu1 = *(const uint4*)(u0 + r1 + o); qu1 = *(const uint4*)(u0 + r1 + oq);
+    W4k wg0, wg1, wu0, wu1;
+    const size_t o0 = (size_t)min(g, nsb - 1u) * Q4K_BYTES;
+    wg0.load(g0 + o0, l); wg1.load(g0 + r1 + o0, l);
+    wu0.load(u0 + o0, l); wu1.load(u0 + r1 + o0, l);
+    if (ROUTE) {
+        if (blockIdx.x == 0u && a == 0u && threadIdx.x < KSEL) {
+            idx_out[(size_t)t * KSEL + threadIdx.x] = r_idx[threadIdx.x];
+            wgt_out[(size_t)t * KSEL + threadIdx.x] = r_wgt[threadIdx.x];
         }
+    } else {   // the first step's weights are on their way while the activations are quantized
+        block_quant_q8k(x + (size_t)t * K, K, xq, xs);
+        __syncthreads();
     }
-    vg0 = wave_sum(vg0); vg1 = wave_sum(vg1); vu0 = wave_sum(vu0); vu1 = wave_sum(vu1);
-    if (lane == 0) {
-        float* o_ = act + (size_t)blockIdx.y * N + row0;
-        o_[0] = (vg0 / (1.0f + expf(-vg0))) * vu0;
-        if (two) o_[1] = (vg1 / (1.0f + expf(-vg1))) * vu1;
+    float vg0 = 0.0f, vg1 = 0.0f, vu0 = 0.0f, vu1 = 0.0f;
+    for (uint s0 = 0; s0 < nsb; s0 += 8u) {
+        const uint sb = s0 + g;
+        W4k ng0 = wg0, ng1 = wg1, nu0 = wu0, nu1 = wu1;
+        if (s0 + 8u < nsb) {
+            const size_t o = (size_t)min(sb + 8u, nsb - 1u) * Q4K_BYTES;
+            ng0.load(g0 + o, l); ng1.load(g0 + r1 + o, l);
+            nu0.load(u0 + o, l); nu1.load(u0 + r1 + o, l);
+        }
+        if (sb < nsb) {
+            const Q4kFrag f = q4k_load_frag(xq, xs, sb, l);
+            vg0 += wg0.dot(c, f);
+            vg1 += wg1.dot(c, f);
+            vu0 += wu0.dot(c, f);
+            vu1 += wu1.dot(c, f);
+        }
+        wg0 = ng0; wg1 = ng1; wu0 = nu0; wu1 = nu1;
     }
+    // lanes 0 / 1 end with the gate sums of the two rows, lanes 2 / 3 with the up sums
+    const float tot = wave_sum4(vg0, vg1, vu0, vu1, lane);
+    const float upv = dpp_f32<OJK_DPP_QUAD_XOR2>(tot);
+    if (lane < (two ? 2u : 1u)) act[(size_t)blockIdx.y * N + row0 + lane] = (tot / (1.0f + expf(-tot))) * upv;
 }
 extern "C" __global__ void __launch_bounds__(256)
 moe_gu_q4k_dec(const float* x, const uchar* wg, const uchar* wu, float* act, const uint* idx, uint K, uint N, uint KSEL,
@@ -568,6 +593,9 @@ moe_gu_q4k_slots(const float* x, const uchar* arena_g, const uchar* arena_u, flo
 // pairs side by side instead of one slot at a time: group sums go through LDS, lane j rebuilds
 // slot j's dot with the association of wave_sum, and the slots are added in order,
 //     y[t][row] (=, +=) sum_j wgt[t][j] * (Wd_{idx[t][j]} act[t][j])[row].
+// One wave a SIMD and a few KB a wave: trips to memory one behind the other bound it, so everything that the launch reads
+// is asked for at its start (the activations four trips at a time, three passes of weights, the slots' weights): the same
+// layer 6.8 -> 5.8 us traced.  A wait for the experts' offsets behind the weights' loads, on one wave, had cost all of that.
 template <class W, bool SLOTS>
 __device__ __forceinline__ void moe_down_dec_body(const float* __restrict__ act, const uchar* __restrict__ wd,
                                                   const void* __restrict__ sel, const float* __restrict__ wgt,
@@ -576,35 +604,86 @@ __device__ __forceinline__ void moe_down_dec_body(const float* __restrict__ act,
     __shared__ float as_[MOE_DEC_DOWN_ACT / 256u];
     __shared__ size_t s_base[64];
     __shared__ __align__(16) float part[4][2][64][8];   // [wave][row][slot][super-block] group sums
+    constexpr uint D = 3u, AD = 4u;
     const uint t = blockIdx.y, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint row0 = min(blockIdx.x * 8u + wave * 2u, N - 1u);   // surplus waves repeat the last row
     const bool two = row0 + 1u < N;
     const uint nsb = K >> 8, G = lane >> 3, l = lane & 7u, c = l >> 1;
     const size_t rb = (size_t)nsb * W::BYTES, r1 = two ? rb : 0;
     const uint U = KSEL * nsb;
-    // the first pass's weights are on their way while the activations are quantized
-    uint u = min(G, U - 1u), j = u / nsb, sb = u - j * nsb;
-    const uchar* w = wd + expert_base(sel, t * KSEL + j, SLOTS, E, (size_t)N * rb) + ((size_t)row0 * nsb + sb) * W::BYTES;
-    W w0, w1;
-    w0.load(w, l);
-    w1.load(w + r1, l);
-    if (threadIdx.x < KSEL) s_base[threadIdx.x] = expert_base(sel, t * KSEL + threadIdx.x, SLOTS, E, (size_t)N * rb);
-    block_quant_q8k(act + (size_t)t * KSEL * K, KSEL * K, aq, as_);
-    __syncthreads();
-    for (uint u0 = 0; u0 < U; u0 += 8u) {
-        const bool on = u0 + G < U;
-        const uint un = min(u0 + 8u + G, U - 1u), jn = un / nsb, sbn = un - jn * nsb;
-        const uchar* wn = wd + s_base[jn] + ((size_t)row0 * nsb + sbn) * W::BYTES;
-        W n0, n1;
-        n0.load(wn, l);
-        n1.load(wn + r1, l);
-        const Q4kFrag f = q4k_load_frag(aq + (size_t)j * K, as_ + (size_t)j * nsb, sb, l);
-        const float v0 = oct_sum(w0.dot(c, f)), v1 = oct_sum(w1.dot(c, f));
-        if (on && l == 0) {
-            part[wave][0][j][sb] = v0;
-            part[wave][1][j][sb] = v1;
+    // the pair a lane group takes in each pass: eight further on than in the one before (past the last: the last)
+    const uint step_j = 8u / nsb, step_s = 8u - step_j * nsb;
+    uint un = G, jn = G / nsb, sn = G - jn * nsb;
+    const auto advance = [&]() {
+        un += 8u; jn += step_j; sn += step_s;
+        if (sn >= nsb) { sn -= nsb; jn++; }
+    };
+    uint j[D], sb[D];
+    size_t eb[D];
+#pragma unroll
+    for (uint i = 0; i < D; i++) {
+        j[i] = un < U ? jn : KSEL - 1u;
+        sb[i] = un < U ? sn : nsb - 1u;
+        eb[i] = expert_base(sel, t * KSEL + j[i], SLOTS, E, (size_t)N * rb);
+        advance();
+    }
+    const size_t eb_lane = expert_base(sel, t * KSEL + min(threadIdx.x, KSEL - 1u), SLOTS, E, (size_t)N * rb);
+    const float wl = wgt[(size_t)t * KSEL + min(lane, KSEL - 1u)];
+    float acc0 = 0.0f, acc1 = 0.0f;
+    if (ACC) {
+        acc0 = y[(size_t)t * N + row0];
+        acc1 = y[(size_t)t * N + row0 + (two ? 1u : 0u)];
+    }
+    const float* at = act + (size_t)t * KSEL * K;
+    float4 xa[AD], xb[AD];
+#pragma unroll
+    for (uint i = 0; i < AD; i++) {
+        const uint p = min(threadIdx.x * 8u + 2048u * i, KSEL * K - 8u);
+        xa[i] = *(const float4*)(at + p);
+        xb[i] = *(const float4*)(at + p + 4u);
+    }
+    if (threadIdx.x < KSEL) s_base[threadIdx.x] = eb_lane;
+    W w0[D], w1[D];
+    const uchar* const wrow = wd + (size_t)row0 * rb;
+#pragma unroll
+    for (uint i = 0; i < D; i++) {
+        const uchar* w = wrow + eb[i] + (size_t)sb[i] * W::BYTES;
+        w0[i].load(w, l);
+        w1[i].load(w + r1, l);
+    }
+#pragma unroll
+    for (uint i = 0; i < AD; i++) {
+        const uint p = threadIdx.x * 8u + 2048u * i;
+        if (p < KSEL * K) {
+            float scale;
+            const uint2 q = oct_quant_q8k(xa[i], xb[i], scale);
+            *(uint2*)(aq + p) = q;
+            if ((threadIdx.x & 31u) == 0) as_[p >> 8] = scale;
         }
-        j = jn; sb = sbn; w0 = n0; w1 = n1;
+    }
+    if (KSEL * K > 2048u * AD)
+        block_quant_q8k(at + 2048u * AD, KSEL * K - 2048u * AD, aq + 2048u * AD, as_ + 8u * AD);
+    __syncthreads();
+    for (uint u0 = 0; u0 < U; u0 += 8u * D) {
+#pragma unroll
+        for (uint i = 0; i < D; i++) {
+            const uint ui = u0 + 8u * i;
+            if (ui >= U) break;
+            const Q4kFrag f = q4k_load_frag(aq + (size_t)j[i] * K, as_ + (size_t)j[i] * nsb, sb[i], l);
+            const float v0 = oct_sum(w0[i].dot(c, f)), v1 = oct_sum(w1[i].dot(c, f));
+            if (ui + G < U && l == 0) {
+                part[wave][0][j[i]][sb[i]] = v0;
+                part[wave][1][j[i]][sb[i]] = v1;
+            }
+            if (ui + 8u * D < U) {
+                j[i] = un < U ? jn : KSEL - 1u;
+                sb[i] = un < U ? sn : nsb - 1u;
+                const uchar* w = wrow + s_base[j[i]] + (size_t)sb[i] * W::BYTES;
+                w0[i].load(w, l);
+                w1[i].load(w + r1, l);
+                advance();
+            }
+        }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -612,22 +691,21 @@ __device__ __forceinline__ void moe_down_dec_body(const float* __restrict__ act,
     // lane j: slot j's two dots, summed like wave_sum sums the eight groups of a wave
     float d0 = 0.0f, d1 = 0.0f;
     if (lane < KSEL) {
-        float s0[8], s1[8];
+        float4 p[4];
+        p[0] = *(const float4*)&part[wave][0][lane][0]; p[1] = *(const float4*)&part[wave][0][lane][4];
+        p[2] = *(const float4*)&part[wave][1][lane][0]; p[3] = *(const float4*)&part[wave][1][lane][4];
+        float s0[8] = {p[0].x, p[0].y, p[0].z, p[0].w, p[1].x, p[1].y, p[1].z, p[1].w};
+        float s1[8] = {p[2].x, p[2].y, p[2].z, p[2].w, p[3].x, p[3].y, p[3].z, p[3].w};
 #pragma unroll
-        for (uint k = 0; k < 8; k++) {
-            s0[k] = k < nsb ? part[wave][0][lane][k] : 0.0f;
-            s1[k] = k < nsb ? part[wave][1][lane][k] : 0.0f;
+        for (uint k = 1; k < 8; k++) {      // past the row: never written
+            s0[k] = k < nsb ? s0[k] : 0.0f;
+            s1[k] = k < nsb ? s1[k] : 0.0f;
         }
         d0 = ((s0[0] + s0[1]) + (s0[2] + s0[3])) + ((s0[4] + s0[5]) + (s0[6] + s0[7]));
         d1 = ((s1[0] + s1[1]) + (s1[2] + s1[3])) + ((s1[4] + s1[5]) + (s1[6] + s1[7]));
     }
-    float acc0 = 0.0f, acc1 = 0.0f;
-    if (ACC) {
-        acc0 = y[(size_t)t * N + row0];
-        acc1 = y[(size_t)t * N + row0 + (two ? 1u : 0u)];
-    }
     for (uint k = 0; k < KSEL; k++) {
-        const float wk = wgt[(size_t)t * KSEL + k];
+        const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wl), k));
         acc0 += wk * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d0), k));
         acc1 += wk * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d1), k));
     }

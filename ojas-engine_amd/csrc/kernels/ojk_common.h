@@ -183,6 +183,15 @@ __device__ __forceinline__ float wave_max(float v) {
     float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
+// The same over integers: one instruction a step, the last steps on the scalar unit.
+__device__ __forceinline__ int wave_max_i32(int v) {
+    v = max(v, dpp_i32<OJK_DPP_QUAD_XOR1>(v));
+    v = max(v, dpp_i32<OJK_DPP_QUAD_XOR2>(v));
+    v = max(v, dpp_i32<OJK_DPP_ROW_HALF_MIRROR>(v));
+    v = max(v, dpp_i32<OJK_DPP_ROW_MIRROR>(v));
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
 __device__ __forceinline__ int wave_sum_i32(int v) {
     v += dpp_i32<OJK_DPP_QUAD_XOR1>(v);
     v += dpp_i32<OJK_DPP_QUAD_XOR2>(v);

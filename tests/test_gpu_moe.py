@@ -61,6 +61,23 @@ def test_router_ties_take_the_lowest_index(gpu):
     assert list(gi[1]) == [3, 70, 127, 0]
 
 
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf, -3.0e38])
+@pytest.mark.parametrize("E", [7, 100, 200, 700])
+def test_router_on_non_finite_logits(gpu, orc, pkg, E, bad):
+    """A NaN or +inf logit makes every probability NaN and nothing is chosen (index ~0, weights 1 / KSEL); -inf and very
+    low ones are probabilities of zero; the token beside it is routed as ever."""
+    lg = pkg.synth.normal_f32(2 * E, "moe", "bad", E).reshape(2, E)
+    lg[0, E // 2] = bad
+    gi, gw, _, _ = _route(gpu, lg, 6)
+    wi, ww = orc.moe_topk(lg[1:], 6)
+    assert np.array_equal(gi[1:], wi) and np.max(np.abs(gw[1:] - ww)) < 1e-5
+    if np.isfinite(bad) or bad < 0:
+        wi, ww = orc.moe_topk(np.where(np.isfinite(lg[:1]), lg[:1], np.float32(-3e38)), 6)
+        assert np.array_equal(gi[:1], wi) and np.max(np.abs(gw[:1] - ww)) < 1e-5
+    else:
+        assert np.all(gi[0] == 0xFFFFFFFF) and np.all(gw[0] == np.float32(1) / 6)
+
+
 @pytest.mark.parametrize("T,E,ksel", [(1, 64, 6), (9, 160, 6), (4, 256, 8), (3, 1000, 5), (2, 7, 7)])
 def test_other_routers_by_their_reference_names(gpu, orc, pkg, T, E, ksel):
     """moe_topk_nonorm (raw softmax probabilities) and moe_topk_v3 (sigmoid scores, bias-corrected choice, renormalised
