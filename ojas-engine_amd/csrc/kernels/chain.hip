@@ -198,15 +198,13 @@ __device__ __forceinline__ void ch_quantizer(ChArgs a, uint s, uint q, double* p
     // ---- quant_q8k of the two segments: the codes past the caches, then — once they are acknowledged — the scales
     float sc0 = 1.0f;
     auto quantize = [&](const float (&v)[4], uint seg, float& scale) {
-        const float amax = wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        const float amax = wave_amax(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
         scale = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
         const float inv = __fdiv_rn(1.0f, scale);
-        const int q0 = (int)sat127(roundf(__fmul_rn(v[0], inv)));
-        const int q1 = (int)sat127(roundf(__fmul_rn(v[1], inv)));
-        const int q2 = (int)sat127(roundf(__fmul_rn(v[2], inv)));
-        const int q3 = (int)sat127(roundf(__fmul_rn(v[3], inv)));
+        const int q0 = code_i8(__fmul_rn(v[0], inv)), q1 = code_i8(__fmul_rn(v[1], inv));
+        const int q2 = code_i8(__fmul_rn(v[2], inv)), q3 = code_i8(__fmul_rn(v[3], inv));
         __hip_atomic_store((uint*)(a->st[s].xq + (size_t)seg * 256u + lane * 4u),
-                           (uint)(q0 & 0xFF) | ((uint)(q1 & 0xFF) << 8) | ((uint)(q2 & 0xFF) << 16) | ((uint)(q3 & 0xFF) << 24),
+                           pack_i8(q0, q1, q2, q3),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     if (has0) quantize(v0, seg0, sc0);

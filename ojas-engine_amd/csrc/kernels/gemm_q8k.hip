@@ -583,17 +583,11 @@ __device__ __forceinline__ void quantize_q8k_sides_body(const void* __restrict__
         const float4 f = *(const float4*)((const float*)xv + i);
         v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
     }
-    const float mx = wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    const float mx = wave_amax(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
     const float scale = mx > 0.0f ? __fdiv_rn(mx, 127.0f) : 1.0f;
     const float inv = __fdiv_rn(1.0f, scale);
-    int s32 = 0;
-    uint pk = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int r = (int)sat127(roundf(__fmul_rn(v[e], inv)));
-        s32 += r;
-        pk |= ((uint)r & 0xFFu) << (8 * e);
-    }
+    const uint pk = q8k_pack4(make_float4(v[0], v[1], v[2], v[3]), inv);
+    int s32 = dot4_i8(pk, 0x01010101u, 0);
     *(uint*)(q + i) = pk;
     // eight lanes hold one run of 32 positions
     s32 += dpp_i32<OJK_DPP_QUAD_XOR1>(s32);

@@ -68,13 +68,11 @@ __device__ __forceinline__ void quantize_q8k_body(const void* __restrict__ xv, s
             for (int j = 0; j < 4; j++) if (i + (uint)j < K) v[j] = p[j];
         }
     }
-    const float mx = wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    const float mx = wave_amax(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
     // scale = amax/127 (1 when the segment is all zero); q = clamp(round_half_away(v * (1/scale)))
     const float scale = mx > 0.0f ? __fdiv_rn(mx, 127.0f) : 1.0f;
     const float inv = __fdiv_rn(1.0f, scale);
-    uint packed = 0u;
-#pragma unroll
-    for (int j = 0; j < 4; j++) packed |= ((uint)(int)sat127(roundf(__fmul_rn(v[j], inv))) & 0xFFu) << (8 * j);
+    const uint packed = q8k_pack4(make_float4(v[0], v[1], v[2], v[3]), inv);
     // the padded tail of a ragged last segment is written as zero
     *(uint*)(q + ((size_t)m * nsb + sb) * 256u + 4u * lane) = packed;
     if (lane == 0) scales[(size_t)m * nsb + sb] = scale;
@@ -455,16 +453,14 @@ rmsnorm_q8k(const float* __restrict__ x, const float* __restrict__ gamma, signed
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) t[e] = i0 + e < K ? __fmul_rn(__fmul_rn(v[e], inv), gm[e]) : 0.0f;
-        const float a = wave_max(fmaxf(fmaxf(fabsf(t[0]), fabsf(t[1])), fmaxf(fabsf(t[2]), fabsf(t[3]))));
+        const float a = wave_amax(fmaxf(fmaxf(fabsf(t[0]), fabsf(t[1])), fmaxf(fabsf(t[2]), fabsf(t[3]))));
         const float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
         const float is = __fdiv_rn(1.0f, scale);
-        uint packed = 0;
+        const uint packed = q8k_pack4(make_float4(t[0], t[1], t[2], t[3]), is);
+        if (WRITE_XN)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int qi = (int)sat127(roundf(__fmul_rn(t[e], is)));
-            packed |= (uint)(qi & 0xFF) << (8 * e);
-            if (WRITE_XN && i0 + e < K) xn[(size_t)m * K + i0 + e] = t[e];
-        }
+            for (int e = 0; e < 4; e++)
+                if (i0 + e < K) xn[(size_t)m * K + i0 + e] = t[e];
         *(uint*)(q + ((size_t)m * nsb + seg) * 256u + lane * 4u) = packed;
         if (lane == 0) scales[(size_t)m * nsb + seg] = scale;
     }
@@ -506,15 +502,10 @@ __device__ __forceinline__ void gemv_fq8k_q4k_body(const float* __restrict__ x, 
     // quantize x: wave `wave` owns segments wave, wave+4, ...; a lane holds 4 consecutive values
     for (uint seg = wave; seg < nsb; seg += 4u) {
         float4 v = *(const float4*)(x + (size_t)seg * 256u + lane * 4u);
-        float a = wave_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        float a = wave_amax(amax4(v));
         float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
         float inv = __fdiv_rn(1.0f, scale);
-        int q0 = (int)sat127(roundf(__fmul_rn(v.x, inv)));
-        int q1 = (int)sat127(roundf(__fmul_rn(v.y, inv)));
-        int q2 = (int)sat127(roundf(__fmul_rn(v.z, inv)));
-        int q3 = (int)sat127(roundf(__fmul_rn(v.w, inv)));
-        *(uint*)(sx + seg * FQ_SEG + lane * 4u) =
-            (uint)(q0 & 0xFF) | ((uint)(q1 & 0xFF) << 8) | ((uint)(q2 & 0xFF) << 16) | ((uint)(q3 & 0xFF) << 24);
+        *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(v, inv);
         if (lane == 0) ss[seg] = scale;
     }
     __syncthreads();
@@ -637,15 +628,10 @@ __device__ __forceinline__ void gemv_fq8k_q4k_x4_body(const float* __restrict__ 
             const uint nseg = seg + nw * NB;
             if (s0 + nw * NB < nsb) v[i] = *(const float4*)(x + (size_t)min(nseg, nsb - 1u) * 256u + lane * 4u);
             if (seg < nsb) {
-                float a = wave_max(fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w))));
+                float a = wave_amax(amax4(t));
                 float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
                 float inv = __fdiv_rn(1.0f, scale);
-                int q0 = (int)sat127(roundf(__fmul_rn(t.x, inv)));
-                int q1 = (int)sat127(roundf(__fmul_rn(t.y, inv)));
-                int q2 = (int)sat127(roundf(__fmul_rn(t.z, inv)));
-                int q3 = (int)sat127(roundf(__fmul_rn(t.w, inv)));
-                *(uint*)(sx + seg * FQ_SEG + lane * 4u) =
-                    (uint)(q0 & 0xFF) | ((uint)(q1 & 0xFF) << 8) | ((uint)(q2 & 0xFF) << 16) | ((uint)(q3 & 0xFF) << 24);
+                *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(t, inv);
                 if (lane == 0) ss[seg] = scale;
             }
         }

@@ -452,12 +452,15 @@ moe_down_q6k_m(const signed char* aq, const float* as_, const uchar* wd, float* 
 // 256 values) with quant_q8k's rule (crates/ojas-cpu/src/cpu_math.rs:539-563), the operations of
 // the quantize_q8k kernel.  A thread owns 8 consecutive values, 32 lanes side by side a segment.
 __device__ __forceinline__ uint2 oct_quant_q8k(float4 a, float4 b, float& scale) {
-    float m = fmaxf(amax4(a), amax4(b));
-    m = fmaxf(m, dpp_f32<OJK_DPP_QUAD_XOR1>(m));
-    m = fmaxf(m, dpp_f32<OJK_DPP_QUAD_XOR2>(m));
-    m = fmaxf(m, dpp_f32<OJK_DPP_ROW_HALF_MIRROR>(m));
-    m = fmaxf(m, dpp_f32<OJK_DPP_ROW_MIRROR>(m));
-    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    // (not negative and no NaN, so integer maxima; a segment is a half of the wave, the other may be idle)
+    int mi = __float_as_int(fmaxf(fmaxf(amax4(a), amax4(b)), 0.0f));
+    mi = max(mi, dpp_i32<OJK_DPP_QUAD_XOR1>(mi));
+    mi = max(mi, dpp_i32<OJK_DPP_QUAD_XOR2>(mi));
+    mi = max(mi, dpp_i32<OJK_DPP_ROW_HALF_MIRROR>(mi));
+    mi = max(mi, dpp_i32<OJK_DPP_ROW_MIRROR>(mi));
+    const int first = max(__builtin_amdgcn_readlane(mi, 0), __builtin_amdgcn_readlane(mi, 16));
+    const int second = max(__builtin_amdgcn_readlane(mi, 32), __builtin_amdgcn_readlane(mi, 48));
+    const float m = __int_as_float((threadIdx.x & 32u) ? second : first);
     scale = m > 0.0f ? __fdiv_rn(m, 127.0f) : 1.0f;
     const float inv = __fdiv_rn(1.0f, scale);
     return make_uint2(q8k_pack4(a, inv), q8k_pack4(b, inv));

@@ -192,6 +192,32 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
                max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
+// A quantizer's amax: wave_max of values that are not negative or NaN (which is passed over; all NaN: 0).  Such values order
+// like their bits.
+__device__ __forceinline__ float wave_amax(float v) {
+    return __int_as_float(wave_max_i32(__float_as_int(fmaxf(v, 0.0f))));
+}
+// The int8 code of a scaled activation as the reference's quantizers round it, half away from zero, with sat127's
+// saturation.  (int)trunc(v + copysign(0.5 - 2^-25, v)) is round() for every float below 2^22, the conversion truncates,
+// saturates and makes a NaN 0: five instructions a value for fourteen (compared over all 2^32 values).  The empty asm in
+// `rounded` keeps the product before it from being contracted into the sum.
+__device__ __forceinline__ int code_i8(float v) {
+    v = rounded(v);
+    const float h = v + copysignf(0x1.fffffep-2f, v);
+    int c;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(c) : "v"(h));
+    return min(max(c, -127), 127);
+}
+// Four codes as the bytes of a dword.
+__device__ __forceinline__ uint pack_i8(int a, int b, int c, int d) {
+    const uint lo = __builtin_amdgcn_perm((uint)b, (uint)a, 0x0C0C0400u), hi = __builtin_amdgcn_perm((uint)d, (uint)c, 0x0C0C0400u);
+    return lo | (hi << 16);
+}
+// Four values times 1 / scale as codes; their amax.
+__device__ __forceinline__ uint q8k_pack4(float4 v, float inv) {
+    return pack_i8(code_i8(__fmul_rn(v.x, inv)), code_i8(__fmul_rn(v.y, inv)), code_i8(__fmul_rn(v.z, inv)), code_i8(__fmul_rn(v.w, inv)));
+}
+__device__ __forceinline__ float amax4(float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
 __device__ __forceinline__ int wave_sum_i32(int v) {
     v += dpp_i32<OJK_DPP_QUAD_XOR1>(v);
     v += dpp_i32<OJK_DPP_QUAD_XOR2>(v);

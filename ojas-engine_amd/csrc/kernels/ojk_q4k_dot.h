@@ -38,16 +38,6 @@ __device__ __forceinline__ Q4kFrag q4k_load_frag(const signed char* xq, const fl
 // q = clamp(round_half_away(v * (1/scale))), crates/ojas-cpu/src/cpu_math.rs:539-563) needs one
 // maximum over the group and nothing outside registers.  Same operations as the quantize_q8k
 // kernel, hence the same bytes.
-__device__ __forceinline__ uint q8k_pack4(float4 v, float inv) {
-    float a = sat127(roundf(__fmul_rn(v.x, inv)));
-    float b = sat127(roundf(__fmul_rn(v.y, inv)));
-    float c = sat127(roundf(__fmul_rn(v.z, inv)));
-    float d = sat127(roundf(__fmul_rn(v.w, inv)));
-    return ((uint)(int)a & 0xFFu) | (((uint)(int)b & 0xFFu) << 8) | (((uint)(int)c & 0xFFu) << 16) | ((uint)(int)d << 24);
-}
-
-__device__ __forceinline__ float amax4(float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
-
 __device__ __forceinline__ Q4kFrag q4k_quant_frag(const float* x, uint sb, uint l) {
     const float4* p = (const float4*)(x + (size_t)sb * 256u + (l >> 1) * 64u + (l & 1u) * 16u);
     float4 lo[4], hi[4];

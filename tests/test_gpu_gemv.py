@@ -45,6 +45,43 @@ def test_quantize_q8k_is_bit_exact(gpu, orc, pkg):
             assert np.array_equal(gq[t], wq), (k, t)
 
 
+@pytest.mark.parametrize("through", ["quant_q8k", "rmsnorm", "sides"])
+def test_quantizers_round_halves_away_from_zero(gpu, orc, pkg, through):
+    """Every n + 1/2 up to 127 and the floats beside it, both signs, at a scale of exactly 1 (each segment holds a 127): the
+    codes the oracle gives, bit for bit, out of each quantizer that shares the rounding."""
+    h = np.arange(0, 127, dtype=np.float32) + np.float32(0.5)
+    v = np.concatenate([h, np.nextafter(h, np.float32(0)), np.nextafter(h, np.float32(200)), [1e-30, 0.0]])
+    v = v[v < 127]
+    v = np.concatenate([v, -v]).astype(np.float32)
+    seg = np.full((-(-len(v) // 255), 256), 127.0, np.float32)
+    seg[:, :255] = np.resize(v, (seg.shape[0], 255))
+    k = seg.size
+    if through == "sides":      # the batch's quantizer, through a product that has to be the one of the codes themselves
+        m = 40
+        w = pkg.synth.weights(12, 256, k, "halves", k)
+        lin, yd, y2 = gpu.lin(12, 256, k, w), gpu.alloc(m * 256), gpu.alloc(m * 256)
+        x = np.tile(seg.ravel(), (m, 1))
+        gpu.mm(gpu.upload(x), lin, yd, m, act_mode=pkg.ACT_Q8K)
+        codes = orc.quant_q8k(x[0])[1].astype(np.float32)      # at scale 1 the codes are values with the same codes
+        gpu.mm(gpu.upload(np.tile(codes, (m, 1))), lin, y2, m, act_mode=pkg.ACT_Q8K)
+        assert np.array_equal(gpu.read(yd, m * 256).view(np.uint32), gpu.read(y2, m * 256).view(np.uint32))
+        return
+    xd, q, s = gpu.upload(seg), gpu.alloc_bytes(k), gpu.alloc(k // 256)
+    if through == "rmsnorm":    # against the quantizer on the normalised values it writes beside the codes' scales
+        g = np.ones(k, np.float32)
+        gpu.rmsnorm_quant_q8k(xd, gpu.upload(g), 1e-5, 1, k, q, s)
+        inv = np.float32(1) / np.sqrt(np.float32(np.mean(seg.astype(np.float64) ** 2)) + np.float32(1e-5))
+        _, wq, _ = orc.quant_q8k((seg.ravel() * inv).astype(np.float32))
+        # the norm moves a half by an ulp either way: codes agree except there, by one
+        d = np.abs(gpu.read(q, k, np.int8).astype(int) - wq.ravel().astype(int))
+        assert d.max() <= 1 and not d[np.abs(seg.ravel() * 2 % 2 - 1) > 0.01].any()
+        return
+    gpu.quant_q8k(xd, 1, k, q, s)
+    ws, wq, _ = orc.quant_q8k(seg.ravel())
+    assert np.all(ws == 1.0) and np.array_equal(gpu.read(s, k // 256), ws)
+    assert np.array_equal(gpu.read(q, k, np.int8), wq.ravel())
+
+
 @pytest.mark.parametrize("k,m,off,dt", [(768, 400, 0, "f32"), (300, 700, 0, "f32"), (4096, 70, 1, "f32"), (1024, 300, 0, "bf16"),
                                         (300, 600, 1, "bf16")])
 def test_quantize_q8k_batches_a_segment_per_wave(gpu, orc, pkg, k, m, off, dt):
