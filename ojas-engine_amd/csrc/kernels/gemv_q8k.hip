@@ -556,148 +556,6 @@ gemv_fq8k_q4k_wide(const float* x, const uchar* w, float* y, uint K, uint N, uin
     gemv_fq8k_q4k_body<2>(x, w, y, K, N, NRB);
 }
 
-// ---- the folded quantizer over up to four tensors ----------------------------------------------
-//   gemv_fq8k_q4k_x4_{r1,r2}(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC)     x: f32[K], K <= 16384
-// One launch per stage of a decode layer: the stage's f32 activations are quantized by every workgroup into LDS (the
-// arithmetic of quantize_q8k: results are bit-identical to quantizer + matvec launches) and multiplied with up to four
-// weight tensors that share them (q/k/v, gate/up; a single tensor passes E0 = E1 = E2 = E3).  ACC adds onto y (the
-// residual).  Vector memory operations return in order, so the activations are requested FIRST and the workgroup's
-// first weights second: the quantization then runs while those weights are still on their way instead of queueing
-// behind them.  A workgroup (256, 512 or 1024 threads) walks NRB rows, its waves R at a time.  The quantization is
-// about 110 vector instructions per segment and wave — as much as the dot products of twenty rows for K = 4096 — and
-// every workgroup repeats it, so the launch wants few, large workgroups: one or two per CU.
-template <int R>
-__device__ __forceinline__ void gemv_fq8k_q4k_x4_body(const float* __restrict__ x, const uchar* w0, const uchar* w1,
-                                                      const uchar* w2, const uchar* w3, float* y0, float* y1, float* y2,
-                                                      float* y3, uint K, uint E0, uint E1, uint E2, uint E3, uint NRB,
-                                                      uint ACC) {
-    __shared__ __attribute__((aligned(16))) signed char sx[(FQ_MAX_K / 256u) * FQ_SEG];
-    __shared__ float ss[FQ_MAX_K / 256u];
-    const uint tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, nw = blockDim.x >> 6;
-    const uint nsb = K >> 8, g = lane >> 3, l = lane & 7u, c = l >> 1;
-    const uint row_end = min((blockIdx.x + 1u) * NRB, E3);
-    uint row0 = blockIdx.x * NRB + wave * R;
-    // row r0 + r of the stacked tensors -> its block bytes and its output
-    auto locate = [&](uint r0, X4Row (&rw)[R]) {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const uint gr = min(r0 + r, E3 - 1u);
-            const uchar* w;
-            float* y;
-            uint lr;
-            if (gr < E0) { w = w0; y = y0; lr = gr; }
-            else if (gr < E1) { w = w1; y = y1; lr = gr - E0; }
-            else if (gr < E2) { w = w2; y = y2; lr = gr - E1; }
-            else { w = w3; y = y3; lr = gr - E2; }
-            rw[r].w = w + (size_t)lr * nsb * Q4K_BYTES;
-            rw[r].y = y + lr;
-        }
-    };
-    auto fetch = [&](const X4Row (&rw)[R], uint sb, uint4 (&hdr)[R], uint4 (&qs)[R]) {
-        const uint sbc = min(sb, nsb - 1u);
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const uchar* blk = rw[r].w + (size_t)sbc * Q4K_BYTES;
-            hdr[r] = *(const uint4*)blk;
-            qs[r] = *(const uint4*)(blk + 16u + l * 16u);
-        }
-    };
-    // 1. the activations, four segments per wave at a time (wave `wave` owns segments wave, wave + nw, ...; a lane
-    //    holds 4 consecutive values), the first batch requested before anything else
-    constexpr int NB = 4;
-    float4 v[NB];
-#pragma unroll
-    for (int i = 0; i < NB; i++) {
-        const uint seg = wave + nw * (uint)i;
-        v[i] = *(const float4*)(x + (size_t)min(seg, nsb - 1u) * 256u + lane * 4u);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // 2. the first step's weights
-    X4Row rwc[R], rwn[R];
-    uint4 hc[R], qc[R], hn[R], qn[R];
-    locate(row0, rwc);
-    fetch(rwc, g, hc, qc);
-    __builtin_amdgcn_sched_barrier(0);
-    // 3. quantize into LDS
-    for (uint s0 = 0; s0 < nsb; s0 += nw * NB) {
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const uint seg = s0 + wave + nw * (uint)i;
-            const float4 t = v[i];
-            // the next batch's request goes out as soon as the register is free
-            const uint nseg = seg + nw * NB;
-            if (s0 + nw * NB < nsb) v[i] = *(const float4*)(x + (size_t)min(nseg, nsb - 1u) * 256u + lane * 4u);
-            if (seg < nsb) {
-                float a = wave_amax(amax4(t));
-                float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
-                float inv = __fdiv_rn(1.0f, scale);
-                *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(t, inv);
-                if (lane == 0) ss[seg] = scale;
-            }
-        }
-    }
-    __syncthreads();
-    // 4. the rows: one stream of (row group, super-block step) units, the next unit's weights requested before the
-    //    current one is multiplied
-    float acc[R], add[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        acc[r] = 0.0f;
-        add[r] = (ACC && row0 < row_end) ? *rwc[r].y : 0.0f;
-    }
-    uint sb = g;
-    while (row0 < row_end) {
-        uint nsb_next = sb + 8u, nrow = row0;
-        const bool last = nsb_next >= nsb + g;    // (sb - g) + 8 >= nsb: this was the group's last step
-        if (last) { nsb_next = g; nrow = row0 + nw * R; }
-        if (last) locate(nrow, rwn);
-        else {
-#pragma unroll
-            for (int r = 0; r < R; r++) rwn[r] = rwc[r];
-        }
-        if (nrow < row_end) fetch(rwn, nsb_next, hn, qn);
-        if (sb < nsb) {
-            Q4kFrag f;
-            const signed char* p = sx + sb * FQ_SEG + c * 64u + (l & 1u) * 16u;
-            f.xl = *(const uint4*)p;
-            f.xh = *(const uint4*)(p + 32);
-            f.bl = bytesum4(f.xl);
-            f.bh = bytesum4(f.xh);
-            f.sx = ss[sb];
-#pragma unroll
-            for (int r = 0; r < R; r++) acc[r] += q4k_lane_dot(hc[r], qc[r], c, f);
-        }
-        if (last) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                float t = R == 2 ? 0.0f : wave_sum(acc[r]);
-                if (R == 2 && r == 0) {     // both sums in one pass; lane r holds row r's
-                    const float t2 = wave_sum2(acc[0], acc[R - 1], lane);
-                    if (lane < 2u && row0 + lane < row_end) *(lane ? rwc[R - 1].y : rwc[0].y) = ACC ? (lane ? add[R - 1] : add[0]) + t2 : t2;
-                }
-                if (R != 2 && lane == 0 && row0 + r < row_end) *rwc[r].y = ACC ? add[r] + t : t;
-                acc[r] = 0.0f;
-                add[r] = (ACC && nrow < row_end) ? *rwn[r].y : 0.0f;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < R; r++) { rwc[r] = rwn[r]; hc[r] = hn[r]; qc[r] = qn[r]; }
-        sb = nsb_next;
-        row0 = nrow;
-    }
-}
-
-extern "C" __global__ void __launch_bounds__(1024)
-gemv_fq8k_q4k_x4_r1(const float* x, const uchar* w0, const uchar* w1, const uchar* w2, const uchar* w3, float* y0, float* y1,
-                    float* y2, float* y3, uint K, uint E0, uint E1, uint E2, uint E3, uint NRB, uint ACC) {
-    gemv_fq8k_q4k_x4_body<1>(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC);
-}
-extern "C" __global__ void __launch_bounds__(1024)
-gemv_fq8k_q4k_x4_r2(const float* x, const uchar* w0, const uchar* w1, const uchar* w2, const uchar* w3, float* y0, float* y1,
-                    float* y2, float* y3, uint K, uint E0, uint E1, uint E2, uint E3, uint NRB, uint ACC) {
-    gemv_fq8k_q4k_x4_body<2>(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC);
-}
-
 // Batched form: y[M][N] (+)= quantized x[M][K] . W^T.  One wave per row; the row's weights are
 // read and unpacked once per tile of MT tokens.
 template <int MT>
@@ -869,6 +727,7 @@ struct One8 {                             // eight lanes a super-block: Q4_K, Q5
     B b;
     typedef Q4kFrag X;
     __device__ __forceinline__ void load(const uchar* blk, uint u) { b.load(blk, u); }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint at, uint u) { b.load_buf(rs, at, u); }
     static __device__ __forceinline__ X frag(const signed char* sx, const float* ss, uint sb, uint u) {
         X f;
         const signed char* p = sx + sb * FQ_SEG + (u >> 1) * 64u + (u & 1u) * 16u;
@@ -891,11 +750,38 @@ struct One6 {                             // four: Q6_K
     }
     __device__ __forceinline__ float dot(const X& f, uint) const { return q6k_lane_dot(b, f); }
 };
-template <int R, class W, bool BF16>
-__device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, const uchar* __restrict__ w, float* __restrict__ y,
-                                                   uint K, uint N, uint NRB, uint ACC) {
-    __shared__ __attribute__((aligned(16))) signed char sx[(FQ_MAX_K / 256u) * FQ_SEG];
-    __shared__ float ss[FQ_MAX_K / 256u];
+struct One6R {                            // the same through a descriptor, unpacked when it is multiplied
+    static constexpr uint LANES = 4u, BYTES = Q6K_BYTES;
+    uint4 qa, qb, qh;
+    uint2 s;
+    uint d16;
+    typedef Q6kX X;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint at, uint u) {
+        const uint hf = u >> 1, l0 = (u & 1u) * 16u;
+        qa = buf_load16(rs, at + hf * 64u + l0);
+        qb = buf_load16(rs, at + hf * 64u + l0 + 32u);
+        qh = buf_load16(rs, at + 128u + hf * 32u + l0);
+        s = buf_load8(rs, at + 192u + hf * 8u);
+        d16 = buf_load2(rs, at + 208u);
+    }
+    static __device__ __forceinline__ X frag(const signed char* sx, const float* ss, uint sb, uint u) { return One6::frag(sx, ss, sb, u); }
+    __device__ __forceinline__ float dot(const X& f, uint u) const {
+        Q6kW r;
+        r.qa = {qa.x, qa.y, qa.z, qa.w};
+        r.qb = {qb.x, qb.y, qb.z, qb.w};
+        r.qh = {qh.x, qh.y, qh.z, qh.w};
+        uint s0 = s.x, s1 = s.y;
+        asm volatile("" : "+v"(s0), "+v"(s1));      // (not unpacked as soon as they are loaded: that would wait for them)
+        const uint is = u & 1u, a = s0 >> (8u * is), b = s1 >> (8u * is);       // bytes is, is + 2, is + 4, is + 6 of the half's scales
+        r.sc4 = (a & 0xFFu) | ((a >> 8) & 0xFF00u) | ((b & 0xFFu) << 16) | ((b << 8) & 0xFF000000u);
+        r.d16 = d16;
+        return q6k_lane_dot(r, f);
+    }
+};
+// LOC gives a row's block bytes and its output.
+struct FqRow { const uchar* w; float* y; };
+template <int R, class W, bool BF16, class LOC>
+__device__ __forceinline__ void gemv_fq8k_loop(const void* __restrict__ xv, const LOC loc, uint K, uint N, uint NRB, uint ACC, signed char* sx, float* ss) {
     const uint tid = threadIdx.x, lane = tid & 63u, wave = (uint)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), nw = blockDim.x >> 6;
     constexpr uint STEP = 64u / W::LANES;
     const uint nsb = K >> 8, g = lane / W::LANES, l = lane % W::LANES;
@@ -903,7 +789,7 @@ __device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, 
     uint row0 = blockIdx.x * NRB + wave * R;
     auto fetch = [&](uint r0, uint sb, W (&o)[R]) {
 #pragma unroll
-        for (int r = 0; r < R; r++) o[r].load(w + ((size_t)min(r0 + r, N - 1u) * nsb + min(sb, nsb - 1u)) * W::BYTES, l);
+        for (int r = 0; r < R; r++) o[r].load(loc(min(r0 + r, N - 1u)).w + min(sb, nsb - 1u) * W::BYTES, l);
     };
     typedef typename std::conditional<BF16, uint2, float4>::type X4;
     constexpr int NB = 4;
@@ -924,7 +810,7 @@ __device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, 
             else t = v[i];
             if (s0 + nw * NB < nsb) v[i] = ((const X4*)xv)[min(seg + nw * NB, nsb - 1u) * 64u + lane];
             if (seg < nsb) {
-                const float a = wave_max(amax4(t));
+                const float a = wave_amax(amax4(t));
                 const float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
                 *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(t, __fdiv_rn(1.0f, scale));
                 if (lane == 0) ss[seg] = scale;
@@ -949,7 +835,7 @@ __device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, 
         if (last) {
             float t = R == 2 ? wave_sum2(acc[0], acc[R - 1], lane) : wave_sum(acc[0]);
             if (lane < (uint)R && row0 + lane < row_end) {
-                float* o = y + row0 + lane;
+                float* o = loc(row0 + lane).y;
                 *o = ACC ? *o + t : t;
             }
 #pragma unroll
@@ -961,15 +847,156 @@ __device__ __forceinline__ void gemv_fq8k_one_body(const void* __restrict__ xv, 
         row0 = nrow;
     }
 }
+// The same for four units a wave and more, a unit being R rows times the super-blocks of one step.  D units are in flight in
+// registers of their own, and a unit's registers are asked for again as soon as it is multiplied: no load has a branch around it
+// and no loaded register is copied, for either makes the compiler wait for loads that it need not wait for (as the loop above
+// does: there a step is hidden behind nothing but the step before it).  Loads go through a descriptor of the row's length, so lanes
+// past the row's end and units past the wave's last read zeros and no memory.  The address unit still takes its time over them,
+// which is why few units stay with the loop, or for Q4_K, two and three of them, with straight code (the other formats have no
+// registers for it).  Loop / ring, whole call, us: Q4_K 9000 x 5120 10.6 / 9.6, 5300 x 11008 12.1 / 10.7, 30000 x 1792 11.2 / 9.0, Q5_K 30000 x
+// 2560 18.0 / 16.0, Q6_K 12000 x 5120 17.7 / 16.1, 30000 x 11008 61.1 / 57.3; one to three units: Q5_K 7500 x 4096 8.7 / 9.3, Q6_K 7500 x
+// 11008 19.0 / 20.0; Q4_K straight, a stage: 4096 x 3072 5.3 / 4.8, 6144 x 4096 6.5 / 6.2, 22016 x 2048 8.2 / 7.9.
+template <class W> constexpr uint FQ_FROM = W::BYTES == Q4K_BYTES ? 2u : 4u;
+template <int R, class W, bool BF16, bool ACC, class LOC>
+__device__ __forceinline__ void gemv_fq8k_ring(const void* __restrict__ xv, const LOC loc, uint K, uint N, uint NRB, uint units, signed char* sx, float* ss) {
+    constexpr int D = 2;
+    const uint tid = threadIdx.x, lane = tid & 63u, wave = (uint)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), nw = blockDim.x >> 6;
+    constexpr uint STEP = 64u / W::LANES;
+    const uint nsb = K >> 8, g = lane / W::LANES, l = lane % W::LANES, steps = (nsb + STEP - 1u) / STEP, rb = nsb * W::BYTES;
+    const uint row_end = min((blockIdx.x + 1u) * NRB, N);
+    const uint row0 = blockIdx.x * NRB + wave * R;
+    typedef typename std::conditional<BF16, uint2, float4>::type X4;
+    // 1. the activations, four segments per wave at a time (wave `wave` owns segments wave, wave + nw, ...; a lane holds 4
+    //    consecutive values), the first batch requested before anything else
+    constexpr int NB = 4;
+    X4 v[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) v[i] = ((const X4*)xv)[min(wave + nw * (uint)i, nsb - 1u) * 64u + lane];
+    __builtin_amdgcn_sched_barrier(0);
+    // 2. the first units' weights
+    uint frow = row0, fstep = 0;
+    W buf[D][R];
+    float add[D];
+    const auto fetch = [&](W (&o)[R], float& ad) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const bool on = frow + r < row_end;
+            const uchar* base = loc(on ? frow + r : N - 1u).w;
+            const uint odd = (uint)(size_t)base & 3u;       // (a descriptor starts on a dword)
+            const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(base - odd), 0, on ? (int)(rb + odd) : 0, 0x00020000);
+            o[r].load(rs, odd + (fstep * STEP + g) * W::BYTES, l);
+        }
+        if (ACC) ad = lane < (uint)R && frow + lane < row_end ? *loc(frow + lane).y : 0.0f;
+        const bool wrap = fstep + 1u == steps;
+        fstep = wrap ? 0u : fstep + 1u;
+        frow = wrap ? frow + nw * R : frow;
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) fetch(buf[d], add[d]);
+    __builtin_amdgcn_sched_barrier(0);
+    // 3. quantize into LDS
+    const auto quantize = [&](const X4 raw, uint seg) {
+        float4 t;
+        if constexpr (BF16) t = make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u),
+                                            __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xFFFF0000u));
+        else t = raw;
+        const float a = wave_amax(amax4(t));
+        const float scale = a > 0.0f ? __fdiv_rn(a, 127.0f) : 1.0f;
+        *(uint*)(sx + seg * FQ_SEG + lane * 4u) = q8k_pack4(t, __fdiv_rn(1.0f, scale));
+        if (lane == 0) ss[seg] = scale;
+    };
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+        if (wave + nw * (uint)i < nsb) quantize(v[i], wave + nw * (uint)i);
+    for (uint seg = wave + nw * NB; seg < nsb; seg += nw) quantize(((const X4*)xv)[seg * 64u + lane], seg);   // (K > 1024 nw)
+    __syncthreads();
+    // 4. the units
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.0f;
+    uint row = row0, step = 0;
+    const auto multiply = [&](const W (&u)[R], float ad) {
+        if (row >= row_end) return;
+        const typename W::X f = W::frag(sx, ss, min(step * STEP + g, nsb - 1u), l);     // (lanes past the row hold zeros)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] += u[r].dot(f, l);
+        if (++step == steps) {
+            const float t = R == 2 ? wave_sum2(acc[0], acc[R - 1], lane) : wave_sum(acc[0]);
+            if (lane < (uint)R && row + lane < row_end) *loc(row + lane).y = ACC ? ad + t : t;
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] = 0.0f;
+            step = 0;
+            row += nw * R;
+        }
+    };
+    if (FQ_FROM<W> == 2u && units <= 3u) {      // straight: two in flight, the third behind the first
+        multiply(buf[0], add[0]);
+        if (units == 3u) {
+            fetch(buf[0], add[0]);
+            multiply(buf[1], add[1]);
+            multiply(buf[0], add[0]);
+        } else {
+            multiply(buf[1], add[1]);
+        }
+        return;
+    }
+    while (row < row_end) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            multiply(buf[d], add[d]);
+            fetch(buf[d], add[d]);
+        }
+    }
+}
+template <int R, class W, class WR, bool BF16, class LOC>
+__device__ __forceinline__ void gemv_fq8k_rows(const void* xv, const LOC loc, uint K, uint N, uint NRB, uint ACC) {
+    __shared__ __attribute__((aligned(16))) signed char sx[(FQ_MAX_K / 256u) * FQ_SEG];
+    __shared__ float ss[FQ_MAX_K / 256u];
+    const uint per = (blockDim.x >> 6) * R, units = (NRB + per - 1u) / per * (((K >> 8) * W::LANES + 63u) / 64u);
+    if (R == 1 || units < FQ_FROM<W>) gemv_fq8k_loop<R, W, BF16>(xv, loc, K, N, NRB, ACC, sx, ss);
+    else if (ACC) gemv_fq8k_ring<R, WR, BF16, true>(xv, loc, K, N, NRB, units, sx, ss);
+    else gemv_fq8k_ring<R, WR, BF16, false>(xv, loc, K, N, NRB, units, sx, ss);
+}
 #define FQ8K_ONE(FMT, W, SUF, BF16, R)                                                                            \
     extern "C" __global__ void __launch_bounds__(1024) gemv_fq8k_##FMT##_one##SUF##_r##R(                         \
         const void* x, const uchar* w, float* y, uint K, uint N, uint NRB, uint ACC) {                            \
-        gemv_fq8k_one_body<R, W, BF16>(x, w, y, K, N, NRB, ACC);                                                  \
+        const size_t rb = (size_t)(K >> 8) * W::BYTES;                                                            \
+        gemv_fq8k_rows<R, W, typename std::conditional<W::LANES == 4u, One6R, W>::type, BF16>(                    \
+            x, [=](uint r) { return FqRow{w + r * rb, y + r}; }, K, N, NRB, ACC);                                 \
     }
 #define FQ8K_ONES(FMT, W) FQ8K_ONE(FMT, W, , false, 1) FQ8K_ONE(FMT, W, , false, 2) FQ8K_ONE(FMT, W, _bf16, true, 1) FQ8K_ONE(FMT, W, _bf16, true, 2)
 FQ8K_ONES(q4k, One8<W4k>)
 FQ8K_ONES(q5k, One8<W5k>)
 FQ8K_ONES(q6k, One6)
+
+// ---- and over up to four tensors ------------------------------------------------------------------
+//   gemv_fq8k_q4k_x4_{r1,r2}(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC)     x: f32[K], K <= 16384
+// One launch per stage of a decode layer: up to four Q4_K tensors share the stage's f32 activations (q/k/v, gate/up; a single
+// tensor passes E0 = E1 = E2 = E3).  ACC adds onto y (the residual).  The launch wants few, large workgroups (256, 512 or 1024
+// threads), one per CU: every workgroup repeats the quantization.
+template <int R>
+__device__ __forceinline__ void gemv_fq8k_q4k_x4_body(const float* x, const uchar* w0, const uchar* w1, const uchar* w2, const uchar* w3,
+                                                      float* y0, float* y1, float* y2, float* y3, uint K, uint E0, uint E1, uint E2,
+                                                      uint E3, uint NRB, uint ACC) {
+    const size_t rb = (size_t)(K >> 8) * Q4K_BYTES;
+    // row r of the stacked tensors
+    gemv_fq8k_rows<R, One8<W4k>, One8<W4k>, false>(x, [=](uint r) {
+        if (r < E0) return FqRow{w0 + r * rb, y0 + r};
+        if (r < E1) return FqRow{w1 + (r - E0) * rb, y1 + (r - E0)};
+        if (r < E2) return FqRow{w2 + (r - E1) * rb, y2 + (r - E1)};
+        return FqRow{w3 + (r - E2) * rb, y3 + (r - E2)};
+    }, K, E3, NRB, ACC);
+}
+extern "C" __global__ void __launch_bounds__(1024)
+gemv_fq8k_q4k_x4_r1(const float* x, const uchar* w0, const uchar* w1, const uchar* w2, const uchar* w3, float* y0, float* y1,
+                    float* y2, float* y3, uint K, uint E0, uint E1, uint E2, uint E3, uint NRB, uint ACC) {
+    gemv_fq8k_q4k_x4_body<1>(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC);
+}
+extern "C" __global__ void __launch_bounds__(1024)
+gemv_fq8k_q4k_x4_r2(const float* x, const uchar* w0, const uchar* w1, const uchar* w2, const uchar* w3, float* y0, float* y1,
+                    float* y2, float* y3, uint K, uint E0, uint E1, uint E2, uint E3, uint NRB, uint ACC) {
+    gemv_fq8k_q4k_x4_body<2>(x, w0, w1, w2, w3, y0, y1, y2, y3, K, E0, E1, E2, E3, NRB, ACC);
+}
 
 // ---- the fused launches for the other K-quants ---------------------------------------------------
 // A Q4_K_M file keeps some tensors of a stage in Q6_K or Q5_K (attention v, the feed-forward down) beside Q4_K ones;

@@ -289,6 +289,20 @@ __device__ __forceinline__ uint iq4_levels_of(uint q) {
     return (hi & mask) | (lo & ~mask);
 }
 
+// ---- loads through a buffer descriptor ----------------------------------------------------------
+// Bytes at `at` from the descriptor's base; past its length: zeros, and no memory is touched.
+__device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t rs, uint at) {
+    typedef uint u4 __attribute__((ext_vector_type(4)));
+    const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)at, 0, 0);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint2 buf_load8(__amdgpu_buffer_rsrc_t rs, uint at) {
+    typedef uint u2 __attribute__((ext_vector_type(2)));
+    const u2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)at, 0, 0);
+    return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint buf_load2(__amdgpu_buffer_rsrc_t rs, uint at) { return (ushort)__builtin_amdgcn_raw_buffer_load_b16(rs, (int)at, 0, 0); }
+
 // ---- global -> LDS copies by the memory system ------------------------------------------------
 // One instruction moves 16 bytes per lane from base + voff to LDS bytes lds_addr + 16 lane .. (1 KB
 // per wave, contiguous in LDS whatever the global addresses; lds_addr is the same in every lane).

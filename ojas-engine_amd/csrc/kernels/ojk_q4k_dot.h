@@ -118,6 +118,10 @@ struct W4k {
         h = *(const uint4*)blk;
         q = *(const uint4*)(blk + 16u + l * 16u);
     }
+    __device__ __forceinline__ void load_buf(__amdgpu_buffer_rsrc_t rs, uint at, uint l) {
+        h = buf_load16(rs, at);
+        q = buf_load16(rs, at + 16u + l * 16u);
+    }
     __device__ __forceinline__ float dot(uint c, const Q4kFrag& f) const { return q4k_lane_dot(h, q, c, f); }
 };
 struct W5k {
@@ -127,6 +131,11 @@ struct W5k {
         h = *(const uint4*)blk;
         qh = *(const uint4*)(blk + 16u + (l & 1u) * 16u);
         q = *(const uint4*)(blk + 48u + l * 16u);
+    }
+    __device__ __forceinline__ void load_buf(__amdgpu_buffer_rsrc_t rs, uint at, uint l) {
+        h = buf_load16(rs, at);
+        qh = buf_load16(rs, at + 16u + (l & 1u) * 16u);
+        q = buf_load16(rs, at + 48u + l * 16u);
     }
     __device__ __forceinline__ float dot(uint c, const Q4kFrag& f) const { return q5k_lane_dot(h, q, qh, c, f); }
 };

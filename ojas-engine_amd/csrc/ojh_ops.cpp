@@ -562,6 +562,19 @@ extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_bu
 
 static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y);
 static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum);
+static bool fq_one_alone(const ojh_device *dev, const ojh_lin *w);
+// The token's codes and scales, as the two launches ask for them.
+static int fq_scratch(ojh_device *dev, uint32_t K) {
+    ojh_buf *b;
+    int rc = ojh_scratch_get(dev, "xq", K, &b);
+    return rc ? rc : ojh_scratch_get(dev, "xs", K / 64, &b);
+}
+// A recorded call of the two launches (more rows, or a bias) can ask for nothing: what they need is left behind by a call
+// that takes one launch, some KB.
+static void fq_leave_scratch(ojh_device *dev, uint32_t K) {
+    ojh_buf *b;
+    if (!dev->capturing && !ojh_scratch_spare(dev, "xq", K, &b, true)) (void)ojh_scratch_spare(dev, "xs", K / 64, &b, true);
+}
 
 // One stage of a decode layer in ONE launch: 1 to 4 projections of one f32 vector, the vector quantized inside the launch.
 extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int count, const ojh_lin *const *ws,
@@ -587,13 +600,20 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     if ((rc = ensure(dev, "gemv_q8k"))) return rc;
     for (int i = 0; i < count; i++)
         if (ojh_grid_type(ws[i]->type) && (rc = ensure(dev, "iq_grid"))) return rc;
-    // Measured on MI355X (weights streamed from HBM): the single launch wins on a small stage (q/k/v of an 8B model:
-    // 6.6 against 7.7 us), ties on 4096 x 4096 and loses from there on — few large workgroups cannot keep as many bytes
-    // in flight as the plain matvec's thousands of small ones, and many small ones repeat the quantization too often.
-    // OJAS_HIP_FQ_MULTI = 0 never takes it, 2 takes it at every size.
-    const bool small_stage = total * K <= 32u * 1024u * 1024u && K <= 4096u;
+    // The single launch against two (quantizer, matvec), us a stage in a recorded chain, weights from HBM: 6144 x 1024 5.7 / 4.5, 28672 x
+    // 4096 15.7 / 14.8, 6144 x 8192 10.8 / 8.8, 4096 x 14336 11.2 / 10.1, 36000 x 5120 23.8 / 22.2, 65536 x 2048 17.4 / 16.7.  Beyond, the plain
+    // matvec's thousands of small workgroups keep more bytes in flight: 49152 x 4096 23.0 / 23.1, x 8192 41.6 / 43.2, 65536 x
+    // 4096 29.0 / 29.9; a long token for few rows is quantized too often: 600 x 14336 6.9 / 7.1.  Not where an output lies
+    // over x: a workgroup may store its rows before another has read the token.  OJAS_HIP_FQ_MULTI = 0 never takes it, 2 at every size.
+    const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
+    const bool small_stage = total <= (uint64_t)(K <= 2048u ? 256u : 144u) * cus && (K <= 12288u || total >= 6ull * cus);
+    // (the larger of these have two launches' scratch behind them all the same: a limit or a recording that has none refuses
+    // them, and a recorded call that takes two launches finds it)
+    const bool alone = total * K <= 32u * 1024u * 1024u && K <= 4096u;
+    for (int i = 0; i < count; i++)
+        if (overlap(at(x, x_off), (size_t)K * 4, at(ys[i], y_offs ? y_offs[i] : 0), (size_t)ws[i]->n * 4)) fused = false;
     if (count == 1 && !fused && dev->fq_multi && fq_one_taken(dev, ws[0], at(x, x_off), (size_t)K * 4, at(ys[0], y_offs ? y_offs[0] : 0)))
-        return fq_one_launch(dev, at(x, x_off), OJH_X_F32, ws[0], ojh_format(ws[0]->type), at(ys[0], y_offs ? y_offs[0] : 0), accum);
+        return !fq_one_alone(dev, ws[0]) && (rc = fq_scratch(dev, K)) ? rc : fq_one_launch(dev, at(x, x_off), OJH_X_F32, ws[0], ojh_format(ws[0]->type), at(ys[0], y_offs ? y_offs[0] : 0), accum);
     if (!fused || K > 16384 || dev->fq_multi == 0 || (dev->fq_multi == 1 && !small_stage)) {   // quantize once, then the per-format launches
         size_t nsb = K / 256;
         ojh_buf *xq, *xs;
@@ -622,7 +642,8 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     // Every workgroup repeats the quantization (as many vector instructions as the dots of some twenty rows), so the
     // launch takes few, large workgroups — `fq_blocks_per_cu` per CU, `fq_threads` threads each — and deals the rows
     // evenly between them.
-    const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
+    if (alone || dev->fq_multi == 2) fq_leave_scratch(dev, K);
+    else if ((rc = fq_scratch(dev, K))) return rc;
     int r = dev->fq_rows ? dev->fq_rows : 2;
     uint32_t want = cus * dev->fq_multi_blocks;
     uint32_t nrb = (run + want - 1) / want;
@@ -813,36 +834,49 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
     return ojh_launch(dev, name, {xh->ptr, wdeq->ptr, yp}, {K, N, (uint32_t)(accum != 0), m}, sg, sb);
 }
 
-// One small K-quant projection of one token: quantizer and matvec in one launch.  It repeats the quantization in every
-// workgroup and keeps fewer bytes in flight than the plain matvec, so it stays with matrices whose second launch costs more.
-// Two launches / one, call to call, us: 1024 x 4096 Q4_K 8.0 / 4.4; 4096^2 Q4_K 7.8 / 4.6, Q5_K 7.9 / 5.1, Q6_K 7.8 / 6.0; 14336
-// x 4096 Q4_K 9.1 / 8.5, Q5_K 11.8 / 9.9; where the host issues a launch in 3 us instead of 4: 1024 x 4096 Q4_K 6.1 / 3.7, 30000 x
-// 1792 8.5 / 8.8, 12000 x 4096 Q5_K 10.6 / 8.9, 2000 x 6144 6.6 / 5.9.
-// Beyond sixteen rows a CU, one a wave, the waves take a second pair of rows while others idle: that pays for a short walk over K only
-// (K > 4096: 4468 x 5632 Q5_K 7.2 / 8.3, 4311 x 4864 Q4_K 6.6 / 6.9), and for Q6_K, four lanes a super-block, not at all (9216 x 1024
-// 6.8 / 7.8, 6144 x 2048 6.7 / 7.2, 4369 x 3840 6.7 / 7.7).  A longer K costs steps: 2800 x 8192 Q4_K 6.6 / 6.8, 2304 x 8192 Q5_K
-// 6.7 / 7.3, 1500 x 8192 6.6 / 6.9, 1024 x 14336 Q4_K 8.0 / 8.2, Q6_K 8.0 / 9.5.
+// One K-quant projection of one token: quantizer and matvec in one launch.  Two launches / one, call to call, us:
+//   Q5_K   600 x 4096 5.7 / 4.8, 4096^2 6.8 / 6.0, 9000 x 4096 11.4 / 10.1, 30000 x 8192 42.1 / 34.5, 128256 x 2560 66.9 / 58.0: everywhere
+//   Q4_K   1024 x 4096 5.8 / 4.3, 9000 x 5120 10.8 / 9.6, 5300 x 14336 15.0 / 12.3, 30000 x 4096 16.3 / 16.0; output heads have a form of their
+//          own that keeps more bytes in flight, so from 32768 rows only a short K: 65536 x 1792 16.8 / 15.8, x 4096 29.1 / 30.9
+//   Q6_K   four lanes take a super-block, sixteen super-blocks a step.  Up to sixteen rows a CU, one a wave: 4096^2 7.9 / 6.4, 4096 x 11008
+//          13.9 / 11.6, 1500 x 14336 10.7 / 9.7, but 1024 x 14336 8.4 / 8.5.  Beyond, the waves take further pairs of rows: four units a wave
+//          (gemv_fq8k_ring) are ahead, 12000 x 5120 16.8 / 16.1, 30000 x 14336 88 / 74, 65536 x 1024 38.0 / 23.0 (output heads have a form of
+//          their own, a step of which is mostly idle at a short K), but not where one step is full, 30000 x 4096 23.9 / 25.2; fewer only
+//          where the last step is mostly full, 7500 x 4096 10.4 / 9.6, 5300 x 8192 13.7 / 12.7, not 9216 x 1024 7.5 / 7.7, 7500 x 5120 13.6 / 13.0.
 // Not where y lies over x: a workgroup may store its rows before another has read the token.
 static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y) {
+    const uint32_t K = w->k, N = w->n, cus = (uint32_t)dev->prop.multiProcessorCount;
+    if ((w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) || overlap(x, x_bytes, y, (size_t)N * 4) || K > 16384u) return false;
+    if (dev->fq_one != 1) return dev->fq_one == 2;
+    if (w->type == OJH_Q4_K) return (N < 32768u || K <= 2048u) && (K <= 12288u || N >= 5u * cus);
+    if (w->type == OJH_Q5_K) return K <= 8192u || N >= (K <= 12288u ? 5u : 16u) * cus;
+    const uint32_t nsb = K / 256, steps = (nsb + 15) / 16, nrb = (N + cus - 1) / cus;
+    if (nrb <= 16u) return K <= 8192u || nrb >= 5u;
+    if ((nrb + 31) / 32 * steps >= 4u) return steps > 1 || nsb <= 12;
+    return nrb >= 20u && nsb >= 15 && 5 * nsb >= 64 * steps;
+}
+// Those that need nothing but themselves; the others ask for the two launches' scratch although they do without, so what a limit on
+// scratch or a recording refuses does not depend on the route, and a recorded call that takes two launches finds it.
+static bool fq_one_alone(const ojh_device *dev, const ojh_lin *w) {
     const uint32_t K = w->k, mi = (uint32_t)(((uint64_t)w->n * K + (1u << 20) - 1) >> 20);
-    if ((w->type != OJH_Q4_K && w->type != OJH_Q5_K && w->type != OJH_Q6_K) || overlap(x, x_bytes, y, (size_t)w->n * 4)) return false;
-    if (dev->fq_one != 1) return dev->fq_one == 2 && K <= 16384u;
-    if (w->n >= 32768u || K > 8192u) return false; // (heads have forms of their own)
+    if (dev->fq_one == 2) return true;
+    if (w->n >= 32768u || K > 8192u) return false;
     if (w->type != OJH_Q6_K && K <= 4096u) return mi <= (w->type == OJH_Q5_K ? 56u : 32u);
     if (w->n > 16u * (uint32_t)dev->prop.multiProcessorCount) return false;
     return mi <= (w->type == OJH_Q6_K ? (K <= 4096u ? 16u : 8u) : w->type == OJH_Q4_K ? 18u : K <= 6144u ? 14u : 8u);
 }
 static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w, const ojh_block_format *f, void *yp, int accum) {
     const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
-    uint32_t nrb = (w->n + cus - 1) / cus;         // a workgroup of sixteen waves per CU; two rows a wave where it has more than one
-    const uint32_t r = nrb > 16 ? 2 : 1;
+    // A workgroup of sixteen waves per CU; two rows a wave where it has more than one, and where a row alone is several steps (us,
+    // one row a wave / two: Q4_K 1024 x 2560 4.5 / 4.8, x 8192 5.9 / 5.6, x 14336 7.9 / 7.3, Q5_K 1500 x 8192 6.2 / 6.9, x 14336 10.2 / 9.2)
+    uint32_t nrb = (w->n + cus - 1) / cus;
+    const bool steps = w->type == OJH_Q4_K ? w->k >= 8192u : w->type == OJH_Q5_K && w->k > 8192u && w->n >= 5u * cus;
+    const uint32_t r = dev->fq_rows ? (uint32_t)dev->fq_rows : nrb > 16 || steps ? 2 : 1;
     nrb = (nrb + r - 1) / r * r;
     const uint32_t grid[3] = {(w->n + nrb - 1) / nrb, 1, 1}, block[3] = {1024, 1, 1};
     const std::string name = std::string("gemv_fq8k_") + f->tag + (x_dtype == OJH_X_BF16 ? "_one_bf16_r" : "_one_r") + (r == 2 ? "2" : "1");
     int rc = ensure(dev, "gemv_q8k");
-    // (a recorded call of the two launches — more rows, or a bias — can ask for nothing: what they need is left behind, some KB)
-    ojh_buf *b;
-    if (!dev->capturing && !ojh_scratch_spare(dev, "xq", w->k, &b, true)) (void)ojh_scratch_spare(dev, "xs", w->k / 64, &b, true);
+    fq_leave_scratch(dev, w->k);
     return rc ? rc : ojh_launch(dev, name.c_str(), {xp, at(w->raw, w->off), yp}, {w->k, w->n, nrb, (uint32_t)(accum != 0)}, grid, block);
 }
 
@@ -1104,7 +1138,8 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         grid[0] = (N + nrb - 1) / nrb;
         return ojh_launch(dev, name, {at(x, x_off), wp, yp}, {K, N, nrb}, grid, block);
     }
-    if (q8k && m == 1 && !bias && fq_one_taken(dev, w, at(x, x_off), K * esz, yp)) return fq_one_launch(dev, at(x, x_off), x_dtype, w, f, yp, accum);
+    if (q8k && m == 1 && !bias && fq_one_taken(dev, w, at(x, x_off), K * esz, yp))
+        return !fq_one_alone(dev, w) && (rc = fq_scratch(dev, K)) ? rc : fq_one_launch(dev, at(x, x_off), x_dtype, w, f, yp, accum);
     if (q8k) {
         if ((rc = ensure(dev, "gemv_q8k"))) return rc;
         size_t nsb = K / 256;

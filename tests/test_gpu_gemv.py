@@ -791,3 +791,50 @@ def test_one_launch_where_it_is_ahead(pkg, monkeypatch, ty, n, k, one):
                 g.mm(xd, lin, y, 1, act_mode=pkg.ACT_Q8K)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("ty,n,k,multi", [(Q4_K, 4097, 4352, False), (Q4_K, 36863, 2304, True), (Q4_K, 32767, 2304, False), (Q4_K, 300, 8448, False),
+                                          (Q4_K, 33001, 768, False), (Q4_K, 1537, 12544, True), (Q4_K, 5121, 16384, True),
+                                          (Q5_K, 4097, 8448, False), (Q5_K, 1281, 11008, True), (Q5_K, 33003, 1280, False),
+                                          (Q6_K, 5121, 3840, False), (Q6_K, 5123, 8448 + 256 * 10, True), (Q6_K, 32769, 1024, False),
+                                          (Q6_K, 1281, 14336, False), (Q6_K, 33001, 2560, True)])
+def test_larger_projections_in_one_launch(gpu, orc, pkg, ty, n, k, multi):
+    """Both sides of the rows and steps where a wave's ring of units starts, ends within a step or a row pair, or stays empty: the
+    bits of the two launches, plain and accumulating, f32 and bf16, nothing written past the rows."""
+    some, x = _inputs(pkg, ty, 64, k, "ring")
+    raw = np.tile(np.asarray(some).reshape(64, -1), (n // 64 + 1, 1))[:n].ravel()
+    xb = pkg.synth.to_bf16_bits(x)
+    lin = gpu.lin(ty, n, k, raw)
+    for bf, acc in ((False, False), (False, True), (True, False)):
+        if multi and bf:
+            continue
+        xf = pkg.synth.bf16_bits_to_f32(xb) if bf else x
+        xd = gpu.upload_bytes(xb.view(np.uint8)) if bf else gpu.upload(xf)
+        xq, xs = gpu.alloc_bytes(k), gpu.alloc(k // 256)
+        y0 = pkg.synth.normal_f32(n, "ring", "y0") if acc else np.zeros(n, np.float32)
+        y1, y2 = gpu.upload(y0), gpu.upload(np.concatenate([y0, np.full(4, -7.25, np.float32)]))
+        gpu.quant_q8k(gpu.upload(xf), 1, k, xq, xs)
+        gpu.mm_q8k(xq, xs, lin, y1, accum=acc)
+        if multi:
+            gpu.mm_multi(xd, [lin], [y2], accum=acc)
+        else:
+            gpu.mm(xd, lin, y2, 1, accum=acc, x_dtype=pkg.X_BF16 if bf else pkg.X_F32)
+        got = gpu.read(y2, n + 4)
+        assert np.all(got[n:] == -7.25)
+        assert np.array_equal(got[:n].view(np.uint32), gpu.read(y1, n).view(np.uint32))
+        if not acc:
+            assert peak_err(got[:64], orc.matvec_kq(some, ty, 64, k, xf)) <= TOL_Q8K_SEEN
+
+
+@pytest.mark.parametrize("rows", [(1024,), (1024, 512)])
+def test_a_stage_written_over_its_vector(gpu, pkg, rows):
+    """An output over x: quantized ahead of the rows, the bits of outputs of their own."""
+    k = 1024
+    x = pkg.synth.normal_f32(k, "stage-over", "x")
+    lins = [gpu.lin(Q4_K, n, k, pkg.synth.q4k_weights(n, k, "stage-over", n)) for n in rows]
+    xd, own, both = gpu.upload(x), [gpu.alloc(n) for n in rows], gpu.upload(x)
+    gpu.mm_multi(xd, lins, own)
+    ys = [both] + [gpu.alloc(n) for n in rows[1:]]
+    gpu.mm_multi(both, lins, ys)
+    for n, a, b in zip(rows, own, ys):
+        assert np.array_equal(gpu.read(a, n).view(np.uint32), gpu.read(b, n).view(np.uint32))
