@@ -418,6 +418,22 @@ __device__ __forceinline__ void gemv_nat_q80_m_body(const float* __restrict__ x,
     }
 }
 
+// Q8_0 as a row trait (ojk_rows.h): four lanes a block
+struct Q80W {
+    static constexpr uint XGAP = 4u, STEP = 16u, BYTES = Q80_BYTES;
+    static __device__ __forceinline__ uint units(uint K) { return K >> 5; }
+    static __device__ __forceinline__ uint unit_of(uint lane) { return lane >> 2; }
+    static __device__ __forceinline__ uint x_off(uint lane) { return (lane & 3u) * 8u; }
+    static __device__ __forceinline__ uint x_unit(uint) { return 32u; }
+    struct Frag { uint d16; u32x2_a2 q; };
+    static __device__ __forceinline__ Frag load(const uchar* row, uint u, uint lane) {
+        const uchar* blk = row + (size_t)u * Q80_BYTES;
+        return {*(const ushort*)blk, *(const u32x2_a2*)(blk + 2u + (lane & 3u) * 8u)};
+    }
+    static __device__ __forceinline__ float dot(const Frag& f, uint, float4 x0, float4 x1, float) { return q80_lane_dot(f.d16, f.q, x0, x1); }
+};
+GEMV_NAT_MS(q80, Q80W)
+
 // ------------------------------------------------------------------ IQ4_NL, IQ4_XS and the legacy 32-weight blocks
 // (row traits Iq4nlW, Iq4xsW, Q40W, Q41W, Q50W, Q51W, Mxfp4W: ojk_rows.h)
 GEMV_NAT_SUB32_PX(iq4nl, Iq4nlS32)
@@ -432,6 +448,13 @@ GEMV_NAT_SUB32_PX(q50, Q50S32)
 GEMV_NAT_SUB32_PX(q51, Q51S32)
 GEMV_NAT_IQ4_PX(mxfp4, Mxfp4W)
 GEMV_NAT_IQ4_PX(q5k, Q5kW)
+GEMV_NAT_MS(iq4nl, Iq4nlW)
+GEMV_NAT_MS(iq4xs, Iq4xsW)
+GEMV_NAT_MS(q40, Q40W)
+GEMV_NAT_MS(q41, Q41W)
+GEMV_NAT_MS(q50, Q50W)
+GEMV_NAT_MS(q51, Q51W)
+GEMV_NAT_MS(mxfp4, Mxfp4W)
 
 template <int R, int MODE>
 __device__ __forceinline__ void gemv_nat_q5k_body(const float* x, const uchar* w, float* y, const float* bs, uint K, uint N) {

@@ -75,6 +75,64 @@ __device__ __forceinline__ void gemv_nat_iq4_m_body(const float* __restrict__ x,
     }
 }
 
+// A few tokens against many steps of K: gemv_nat_<fmt>_ms(x, w, y, K, N, M, ACC), the _m entry's arguments and grid.  A workgroup of
+// n waves owns n rows, four at a time; its waves take a step of K each in turn for all four rows, and their sums meet in LDS
+// in wave order.  A lane's f32 activations, 8 bytes a weight at two tokens, are what such a call asks the address unit for: a wave
+// that walks a row by itself fetches them again for every row.  Whole call, _m / _ms, us: IQ4_XS 14336 x 4096 at 3 tokens 37.4 / 17.7,
+// 4096 x 14336 at 2 19.8 / 15.0, 27347 x 13312 at 3 259 / 94.6; Q8_0 14336 x 4096 at 2 22.5 / 15.2, at 3 35.5 / 17.2.  With few steps of K
+// some waves have none: 30000 x 1280 IQ4_XS at 2 16.2 / 18.1, at 3 28.8 / 20.4, 1599 x 1024 at 4 4.4 / 4.7 (two waves on two rows there: 21.9 and 24.6).
+template <class W, int MT>
+__device__ __forceinline__ void gemv_nat_ms_body(const float* __restrict__ x, const uchar* __restrict__ w,
+                                                 float* __restrict__ y, uint K, uint N, uint M, uint ACC) {
+    constexpr uint R = 4u;
+    __shared__ float red[16][MT][R];
+    const uint lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const uint nu = W::units(K), first = blockIdx.x * nw, end = min(first + nw, N);
+    const size_t rb = (size_t)nu * W::BYTES;
+    for (uint row0 = first; row0 < end; row0 += R) {
+        for (uint m0 = 0; m0 < M; m0 += MT) {
+            float acc[MT][R];
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (uint r = 0; r < R; r++) acc[i][r] = 0.0f;
+            for (uint u = W::unit_of(lane) + wave * W::STEP; u < nu; u += nw * W::STEP) {
+                typename W::Frag f[R];
+#pragma unroll
+                for (uint r = 0; r < R; r++) f[r] = W::load(w + (size_t)min(row0 + r, end - 1u) * rb, u, lane);
+#pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    const float* xp = x + (size_t)min(m0 + i, M - 1u) * K + (size_t)u * W::x_unit(0) + W::x_off(lane);
+                    const float4 x0 = *(const float4*)xp, x1 = *(const float4*)(xp + W::XGAP);
+                    const float xsum = sum4(x0) + sum4(x1);
+#pragma unroll
+                    for (uint r = 0; r < R; r++) acc[i][r] += W::dot(f[r], lane, x0, x1, xsum);
+                }
+            }
+            if (row0 > first || m0 > 0u) __syncthreads();       // the sums before have been read
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const float t = wave_sum4(acc[i][0], acc[i][1], acc[i][2], acc[i][3], lane);
+                if (lane < R) red[wave][i][lane] = t;
+            }
+            __syncthreads();
+            const uint i = threadIdx.x / R, r = threadIdx.x % R;
+            if (i < (uint)MT && m0 + i < M && row0 + r < end) {
+                float t = red[0][i][r];
+                for (uint v = 1; v < nw; v++) t += red[v][i][r];
+                float* o = y + (size_t)(m0 + i) * N + row0 + r;
+                *o = ACC ? *o + t : t;
+            }
+        }
+    }
+}
+#define GEMV_NAT_MS(FMT, W)                                                                                \
+    extern "C" __global__ void __launch_bounds__(256) gemv_nat_##FMT##_ms(                                 \
+        const float* x, const uchar* w, float* y, uint K, uint N, uint M, uint ACC) {                      \
+        if (M <= 2) gemv_nat_ms_body<W, 2>(x, w, y, K, N, M, ACC);                                         \
+        else if (M == 3) gemv_nat_ms_body<W, 3>(x, w, y, K, N, M, ACC);                                    \
+        else gemv_nat_ms_body<W, 4>(x, w, y, K, N, M, ACC); }
+
 // Many rows (an output head): a 4-bit row is an eighth of the bytes of the f32 activations it meets, so
 // a wave that fetches its activation fragments again for every few rows is bound by those loads, not
 // by HBM (2.7 TB/s at 128256 x 4096).  Here rows are grid-stride and the wave keeps its share of x —

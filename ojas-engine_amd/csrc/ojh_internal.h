@@ -146,6 +146,7 @@ struct ojh_block_format {
 };
 const ojh_block_format *ojh_format(uint32_t ggml_type);
 bool ojh_float_rows(uint32_t ggml_type);   // the CPU path reads f32 activations for this format
+bool ojh_shares_rows(uint32_t ggml_type);  // has a few-token matvec whose waves share rows (gemv_nat_<fmt>_ms)
 size_t ojh_block_align(const ojh_block_format *f);
 uint32_t ojh_matmul_q8row_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M);  // K slices of the row-int8 tile (1: whole)
 uint32_t ojh_gemm_q8k_gs_slices(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M);   // K slices of the Q6_K / Q5_K int8 tile (1: whole)

@@ -37,6 +37,9 @@ static const ojh_block_format kFormats[] = {
 // Formats whose CPU path multiplies the raw row with f32 activations (dot_q80, dot_iq4nl, dot_iq4xs:
 // crates/ojas-cpu/src/cpu_math.rs:1131-1141, :1179) instead of quantizing them per 256.
 bool ojh_float_rows(uint32_t t) { return t == OJH_Q8_0 || ojh_float_only(t); }
+bool ojh_shares_rows(uint32_t t) {
+    return t == OJH_Q8_0 || t == OJH_IQ4_NL || t == OJH_IQ4_XS || t == OJH_Q4_0 || t == OJH_Q4_1 || t == OJH_Q5_0 || t == OJH_Q5_1 || t == OJH_MXFP4;
+}
 // ... and for which this library has the f32-activation matvecs only: no int8-activation form, no MFMA tile
 // (the IQ4 types, and the legacy 32-weight blocks and Q2_K / Q3_K, which the reference runs on its GPU path alone)
 // (of the grid-codebook formats the CPU path multiplies IQ3_S and IQ2_S with f32 activations, dot_iq3s / dot_iq2s, and
@@ -2160,6 +2163,7 @@ static std::vector<ojh_kernel_spec> build_manifest() {
         add(g + "_accum", fam_nat, 3, 2, f.type, 4, check_gemv_nat, shape_rows);
         add(g + "_bias", fam_nat, 4, 2, f.type, 4, check_gemv_nat, shape_rows);
         add(g + "_m", fam_nat, 3, 4, f.type, 1, check_gemv_nat_m, shape_rows);
+        if (ojh_shares_rows(f.type)) add(g + "_ms", fam_nat, 3, 4, f.type, 1, check_gemv_nat_m, shape_rows);
         if (f.type != OJH_Q8_0) add(g + "_px", fam_nat, 3, 2, f.type, 2, check_gemv_nat_px, shape_px);
         if (ojh_float_only(f.type)) continue;   // f32 activations only, no MFMA tile
         if (f.type == OJH_Q8_0) {

@@ -838,3 +838,30 @@ def test_a_stage_written_over_its_vector(gpu, pkg, rows):
     gpu.mm_multi(both, lins, ys)
     for n, a, b in zip(rows, own, ys):
         assert np.array_equal(gpu.read(a, n).view(np.uint32), gpu.read(b, n).view(np.uint32))
+
+
+@pytest.mark.parametrize("ty", [8, 20, 23, 2, 3, 6, 7, 139])
+@pytest.mark.parametrize("n,k,m,waves", [(1, 512, 1, 4), (7, 2304, 2, 4), (130, 1280, 3, 4), (1001, 4096, 4, 4), (35, 2816, 5, 3), (18, 13312, 9, 1), (9, 256, 2, 2)])
+def test_few_tokens_with_shared_rows(gpu, orc, pkg, ty, n, k, m, waves):
+    """`gemv_nat_<fmt>_ms`: fewer rows than waves, waves without a step, tokens past a pass of four, every count of waves; set and
+    accumulate against the exact block values in double, nothing past the rows; the f32 sums associate differently from _m's."""
+    raw = pkg.synth.weights(ty, n, k, "shared", ty, n, k)
+    x = pkg.synth.normal_f32(m * k, "shared", "x", k, m).reshape(m, k)
+    gpu.ensure_family("gemv")
+    name = "gemv_nat_%s" % {8: "q80", 20: "iq4nl", 23: "iq4xs", 2: "q40", 3: "q41", 6: "q50", 7: "q51", 139: "mxfp4"}[ty]
+    y0 = pkg.synth.normal_f32(m * n, "shared", "y0")
+    xd, wd = gpu.upload(x), gpu.upload_bytes(raw)
+    out = {}
+    for entry in ("_m", "_ms"):
+        for acc in (0, 1):
+            yd = gpu.upload(np.concatenate([y0, np.full(4, -7.25, np.float32)]))
+            gpu.dispatch(gpu.begin(), name + entry, [(xd, 0), (wd, 0), (yd, 0)], [k, n, m, acc], [(n + waves - 1) // waves, 1, 1], [64 * waves, 1, 1])
+            got = gpu.read(yd, m * n + 4)
+            assert np.all(got[m * n:] == -7.25)
+            out[entry, acc] = got[:m * n].reshape(m, n) - (y0.reshape(m, n) if acc else 0)
+    for t in range(m):
+        want = orc.matmul_ref(raw, ty, n, k, x[t])[0]
+        # 4e-6: two orders of the same f32 sums, (k / 64 + 8) 2^-24 of the partial sums; accumulating rounds at y0's magnitude
+        assert peak_err(out["_ms", 0][t], want) <= TOL_FLOAT
+        assert peak_err(out["_ms", 0][t], out["_m", 0][t]) <= 4e-6
+        assert peak_err(out["_ms", 1][t], out["_ms", 0][t]) <= 4e-6 * max(1.0, 8.0 / max(1e-30, float(np.max(np.abs(want)))))
