@@ -217,21 +217,28 @@ static uint32_t q4k_xt_min_tokens(const ojh_device *dev, uint32_t K, uint32_t N)
 // 16.7 / 12.4, 1024 x 4096 15.3 / 11.4, 4096 x 14336 35.2 / 22.3; at 12 tokens 17.7 / 20.4, 8.9 / 12.3, 8.5 / 11.4).  Not for
 // short rows, where its fixed part shows (6000 x 1024 8.9 / 9.8, 4000 x 1792 10.0 / 10.4, 3500 x 2048 level, 2000 x 2048 10.9 / 9.9),
 // unless more 64-row tiles than half the CUs make the few-token kernel walk two tiles a wave (8400 x 1024 11.1 / 8.6, x 2048
-// 18.9 / 12.3).
+// 18.9 / 12.3).  Matrices of fewer rows than its slices fill half the CUs with (960 on 256) take it too, from 33 tokens also short
+// ones, where the few-token kernel's row tiles leave more of them idle: 730 x 5632 at 22 tokens 20.8 / 12.4, at 64 43.9 / 12.9, 256 x 2048
+// at 64 19.8 / 10.2, x 14336 at 64 105 / 17.3.  Up to 64 tokens, half a tile: more keep the sums' order of ojh_mm_noalloc, which has no
+// scratch for slices.
 static bool q4k_xk_early(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
     const bool ahead = K > 2048 || (K == 2048 && N <= 2560) || (N + 63) / 64 * 2 > (uint32_t)dev->prop.multiProcessorCount;
-    return ahead && m >= 17 && dev->q4k_xt_min_m == 1 && q4k_xk_slices(dev, K, N, m);
+    if (m > 64 && !q4k_xt_slices(dev, K, N, m)) return false;
+    return (ahead || (m > 32 && K >= 1024)) && m >= 17 && dev->q4k_xt_min_m == 1 && q4k_xk_slices(dev, K, N, m);
 }
-// What a Q4_K product of m tokens does about that tile.  From q4k_xt_min_tokens it takes it.  The few-token kernels need none of
-// its scratch, so a product of fewer tokens takes it only where all of that is to be had (and takes none where some is not),
-// which is asked for here, once a product.
+// What a Q4_K product of m tokens does about that tile.  From q4k_xt_min_tokens it takes it (q4k_xt_must).  The few-token kernels need
+// none of its scratch, so a product of fewer tokens, or of too few rows for that, takes it only where all of that is to be had (and
+// takes none where some is not), which is asked for here, once a product.
 enum { XT_ASK = -1, XT_NO, XT_TAKE, XT_SIDES };    // XT_SIDES: taken, its side arrays written by the quantizer
+static bool q4k_xt_must(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t m) {
+    return m >= q4k_xt_min_tokens(dev, K, N) && q4k_xt_slices(dev, K, N, m);
+}
 static int q4k_xt_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, const void *wp) {
     const uint32_t K = w->k, N = w->n;
-    if (w->type != OJH_Q4_K || !dev->q4k_xt_min_m || dev->no_scratch || !q4k_xt_slices(dev, K, N, m) || (uint64_t)m * K > 0xFFFFFFFFull ||
+    if (w->type != OJH_Q4_K || !dev->q4k_xt_min_m || dev->no_scratch || (uint64_t)m * K > 0xFFFFFFFFull ||
         (uint64_t)w->row_bytes * N > 0xFFFFFFFFull || (uintptr_t)wp % 16)
         return XT_NO;
-    if (m >= q4k_xt_min_tokens(dev, K, N)) return XT_TAKE;
+    if (q4k_xt_must(dev, K, N, m)) return XT_TAKE;
     if (!q4k_xk_early(dev, K, N, m) || ensure(dev, "gemm_q8k")) return XT_NO;
     const size_t z = q4k_xk_slices(dev, K, N, m), mp = (m + 127) / 128 * 128, nsb = K / 256, tiles = (size_t)((N + 63) / 64) * (mp / 128);
     const size_t xst = nsb * mp * 4, sums = nsb * mp * 32, part = tiles * z * 32768, cnt = tiles * 4;
@@ -244,7 +251,7 @@ static int q4k_xt_ready(ojh_device *dev, const ojh_lin *w, uint32_t m, const voi
 }
 
 static int xt_scratch(ojh_device *dev, const ojh_lin *w, uint32_t m, const char *name, size_t bytes, ojh_buf **out) {
-    return m >= q4k_xt_min_tokens(dev, w->k, w->n) ? ojh_scratch_get(dev, name, bytes, out) : ojh_scratch_spare(dev, name, bytes, out);
+    return q4k_xt_must(dev, w->k, w->n, m) ? ojh_scratch_get(dev, name, bytes, out) : ojh_scratch_spare(dev, name, bytes, out);
 }
 
 int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, const ojh_block_format *f, void *yp,

@@ -385,3 +385,31 @@ def test_three_slices_of_whole_tiles_stay_with_two_workgroups_a_cu(pkg, monkeypa
     """130 tiles of more than 64 tokens over three slices of K keep the form that shares a CU; 64 tokens, and two slices, do not."""
     old, new = _bits_of_both_forms(pkg, monkeypatch, m, n, k)
     assert np.array_equal(old, new) != taken
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 1, 2304), (33, 65, 1024), (32, 64, 5632), (64, 730, 2560), (129, 63, 4096), (300, 130, 3072), (100, 959, 1280)])
+@pytest.mark.parametrize("accum", [False, True])
+def test_few_rows_take_the_tile_in_slices(gpu, orc, pkg, monkeypatch, m, n, k, accum):
+    """Fewer rows than the slices fill half the CUs with: against matvec_kq, one row, rows past a tile, tokens past one; and where
+    there is no room for the tile's scratch the few-token kernel still takes the call."""
+    w, x = _case(pkg, m, n, k, "few-rows")
+    y0 = pkg.synth.normal_f32(m * n, "gq", "y0", m, n).reshape(m, n) if accum else np.zeros((m, n), np.float32)
+    got = []
+    for room in (None, str(m * k * 2)):         # (the codes and scales, and half as much again)
+        if room:
+            monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", room)
+        g = pkg.HipGpu(0) if room else gpu
+        try:
+            yd = g.upload(np.concatenate([y0.ravel(), np.full(16, 4242.5, np.float32)]))
+            g.mm(g.upload(x), g.lin(Q4_K, n, k, w), yd, m, accum=accum, act_mode=pkg.ACT_Q8K)
+            out = g.read(yd, m * n + 16)
+            assert np.all(out[m * n:] == 4242.5)
+            got.append(out[:m * n].reshape(m, n) - y0)
+        finally:
+            if room:
+                g.close()
+    for t in sorted({0, m // 2, m - 1}):
+        want = orc.matvec_kq(w, Q4_K, n, k, x[t])
+        tol = TOL_SEEN * max(1.0, 4.0 * float(np.max(np.abs(y0))) / max(1e-30, float(np.max(np.abs(want)))))
+        for out in got:
+            assert peak_err(out[t], want) <= tol, t
