@@ -494,6 +494,14 @@ extern "C" int ojh_mm_q8k(ojh_device *dev, const ojh_buf *xq, const ojh_buf *xsc
     return ojh_mm_q8k_launch(dev, xq->ptr, xscales->ptr, w, f, at(y, y_off), bias, m, accum);
 }
 
+// Whether no two of a stage's outputs share a byte: otherwise its projections run one behind the other, as separate calls do.
+static bool ys_apart(int count, const ojh_lin *const *ws, ojh_buf *const *ys, const size_t *y_offs) {
+    for (int i = 1; i < count; i++)
+        for (int j = 0; j < i; j++)
+            if (overlap(at(ys[i], y_offs ? y_offs[i] : 0), (size_t)ws[i]->n * 4, at(ys[j], y_offs ? y_offs[j] : 0), (size_t)ws[j]->n * 4)) return false;
+    return true;
+}
+
 extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_buf *xscales, int count,
                                 const ojh_lin *const *ws, ojh_buf *const *ys, const size_t *y_offs) {
     if (!dev || !ws || !ys) return ojh_fail(OJH_ERR_ARG, "ojh_mm_q8k_multi: NULL argument");
@@ -520,7 +528,8 @@ extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_bu
         if (ojh_grid_type(ws[i]->type) && (rc = ensure(dev, "iq_grid"))) return rc;
     // a stage that mixes Q4_K, Q5_K and Q6_K tensors (a Q4_K_M file does): still one launch, every row in its own
     // format's arithmetic
-    bool kquants = count > 1;
+    const bool apart = ys_apart(count, ws, ys, y_offs);
+    bool kquants = count > 1 && apart;
     for (int i = 0; i < count; i++)
         if (ws[i]->type != OJH_Q4_K && ws[i]->type != OJH_Q5_K && ws[i]->type != OJH_Q6_K) kquants = false;
     if (!grouped && kquants) {
@@ -540,7 +549,7 @@ extern "C" int ojh_mm_q8k_multi(ojh_device *dev, const ojh_buf *xq, const ojh_bu
         uint32_t grid[3] = {(run + 3) / 4, 1, 1}, block[3] = {256, 1, 1};
         return ojh_launch(dev, "gemv_q8k_kq_x4", p, {ws[0]->k, ends[0], ends[1], ends[2], ends[3], types}, grid, block);
     }
-    if (!grouped || count == 1) {   // formats without a grouped entry: one launch per projection
+    if (!grouped || count == 1 || !apart) {   // formats without a grouped entry, outputs over each other: one launch per projection
         for (int i = 0; i < count; i++) {
             const ojh_block_format *fi = ojh_format(ws[i]->type);
             if ((rc = ojh_mm_q8k_launch(dev, xq->ptr, xscales->ptr, ws[i], fi, at(ys[i], y_offs ? y_offs[i] : 0), nullptr, 1, 0)))
@@ -611,12 +620,14 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     // 4096 15.7 / 14.8, 6144 x 8192 10.8 / 8.8, 4096 x 14336 11.2 / 10.1, 36000 x 5120 23.8 / 22.2, 65536 x 2048 17.4 / 16.7.  Beyond, the plain
     // matvec's thousands of small workgroups keep more bytes in flight: 49152 x 4096 23.0 / 23.1, x 8192 41.6 / 43.2, 65536 x
     // 4096 29.0 / 29.9; a long token for few rows is quantized too often: 600 x 14336 6.9 / 7.1.  Not where an output lies
-    // over x: a workgroup may store its rows before another has read the token.  OJAS_HIP_FQ_MULTI = 0 never takes it, 2 at every size.
+    // over x: a workgroup may store its rows before another has read the token; nor where two lie over each other: they are
+    // added to, or set, in order.  OJAS_HIP_FQ_MULTI = 0 never takes it, 2 at every size.
     const uint32_t cus = (uint32_t)dev->prop.multiProcessorCount;
     const bool small_stage = total <= (uint64_t)(K <= 2048u ? 256u : 144u) * cus && (K <= 12288u || total >= 6ull * cus);
     // (the larger of these have two launches' scratch behind them all the same: a limit or a recording that has none refuses
     // them, and a recorded call that takes two launches finds it)
     const bool alone = total * K <= 32u * 1024u * 1024u && K <= 4096u;
+    if (!ys_apart(count, ws, ys, y_offs)) fused = false;
     for (int i = 0; i < count; i++)
         if (overlap(at(x, x_off), (size_t)K * 4, at(ys[i], y_offs ? y_offs[i] : 0), (size_t)ws[i]->n * 4)) fused = false;
     if (count == 1 && !fused && dev->fq_multi && fq_one_taken(dev, ws[0], at(x, x_off), (size_t)K * 4, at(ys[0], y_offs ? y_offs[0] : 0)))

@@ -865,3 +865,28 @@ def test_few_tokens_with_shared_rows(gpu, orc, pkg, ty, n, k, m, waves):
         assert peak_err(out["_ms", 0][t], want) <= TOL_FLOAT
         assert peak_err(out["_ms", 0][t], out["_m", 0][t]) <= 4e-6
         assert peak_err(out["_ms", 1][t], out["_ms", 0][t]) <= 4e-6 * max(1.0, 8.0 / max(1e-30, float(np.max(np.abs(want)))))
+
+
+@pytest.mark.parametrize("k,ns,tys", [(4352, (600, 600), (Q4_K, Q4_K)), (1024, (700, 500, 700), (Q4_K, Q4_K, Q4_K)), (2048, (300, 300), (Q4_K, Q6_K)),
+                                      (4096, (4096, 4608), (Q4_K, Q4_K))])
+def test_projections_onto_the_same_output(gpu, pkg, k, ns, tys):
+    """Outputs over each other, wholly or in part: every projection is added, or the last set, as calls of one projection each
+    in order do."""
+    x = pkg.synth.normal_f32(k, "same-y", "x", k)
+    lins = [gpu.lin(ty, n, k, pkg.synth.weights(ty, n, k, "same-y", i, n, k)) for i, (n, ty) in enumerate(zip(ns, tys))]
+    xd, xq, xs = gpu.upload(x), gpu.alloc_bytes(k), gpu.alloc(k // 256)
+    gpu.quant_q8k(xd, 1, k, xq, xs)
+    offs = [64 * 4 * i for i in range(len(ns))]
+    room = max(o // 4 + n for o, n in zip(offs, ns))
+    y0 = pkg.synth.normal_f32(room, "same-y", "y0", room)
+    for acc in (True, False):
+        for at in (None, offs):
+            ya, yb = gpu.upload(y0), gpu.upload(y0)
+            gpu.mm_multi(xd, lins, [ya] * len(ns), at, accum=acc)
+            for i, lin in enumerate(lins):
+                gpu.mm_q8k(xq, xs, lin, yb, 1, acc, y_off=at[i] if at else 0)
+            assert np.array_equal(gpu.read(ya, room).view(np.uint32), gpu.read(yb, room).view(np.uint32)), (acc, at)
+            if not acc:
+                yc = gpu.upload(y0)
+                gpu.mm_q8k_multi(xq, xs, lins, [yc] * len(ns), at)
+                assert np.array_equal(gpu.read(yc, room).view(np.uint32), gpu.read(yb, room).view(np.uint32)), at
