@@ -376,7 +376,8 @@ int ojh_moe_route(ojh_device *dev, const ojh_buf *logits, uint32_t n_tokens, uin
  * reference's GPU expert kernels for those formats, crates/ojas-core/src/quant_src.rs:174-179);
  * OJH_ACT_AUTO and OJH_ACT_Q8K keep the CPU path's int8-activation arithmetic for them.
  * Expert indices must be below n_expert (one that is not never reads outside the tensors; what
- * it contributes is unspecified). Up to 2 tokens run as two launches addressed
+ * it contributes is unspecified, but comes of this call alone: the router's ~0 for a token with a NaN or infinite logit
+ * counts as the last expert for K-quant and grouped experts, as nothing for the per-assignment f32 kernels). Up to 2 tokens run as two launches addressed
  * by assignment (bit-identical to the grouped integer-dot pipeline) when d <= 8192, n_ff <= 2048,
  * ksel <= 64 and ksel * n_ff <= 32768 (beyond that the grouped pipeline serves them; forcing the
  * two-launch form with OJAS_HIP_MOE=3 then returns OJH_ERR_UNSUPPORTED); larger batches are grouped

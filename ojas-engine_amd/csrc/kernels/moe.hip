@@ -217,7 +217,9 @@ moe_topk_v3(const float* lg, const float* bias, uint* idx, float* wgt, uint E, u
 // ------------------------------------------------------------------ grouping
 // Counting sort of the NA assignments by expert: counts[E], offsets[E+1], list[NA] (assignment
 // ids, expert-major; the order inside an expert's group is arbitrary and has no effect on the
-// results, which are stored per assignment).  One workgroup; E <= 1024.
+// results, which are stored per assignment).  One workgroup; E <= 1024.  An index past the last expert counts as the last
+// one, as in the decode form: the router writes ~0 where it chose nothing, and what is added up behind the products has to be
+// this call's.
 __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uint* __restrict__ counts, uint* __restrict__ offsets,
                                                uint* __restrict__ list, uint NA, uint E, uint* cnt, uint* off) {
     const uint tid = threadIdx.x;
@@ -228,7 +230,7 @@ __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uin
     for (uint a0 = tid; a0 < NA; a0 += 8u * 256u) {
         uint e[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? idx[a0 + (uint)u * 256u] : 0xFFFFFFFFu;
+        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(idx[a0 + (uint)u * 256u], E - 1u) : 0xFFFFFFFFu;
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (e[u] < E) atomicAdd(&cnt[e[u]], 1u);
@@ -273,7 +275,7 @@ __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uin
     for (uint a0 = tid; a0 < NA; a0 += 8u * 256u) {
         uint e[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? idx[a0 + (uint)u * 256u] : 0xFFFFFFFFu;
+        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(idx[a0 + (uint)u * 256u], E - 1u) : 0xFFFFFFFFu;
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (e[u] < E) list[off[e[u]] + atomicAdd(&cnt[e[u]], 1u)] = a0 + (uint)u * 256u;
@@ -812,16 +814,16 @@ __device__ __forceinline__ MiFound<NQ> mi_find(const uint* __restrict__ idx, uin
     const bool by_a = NA < E;
     uint v[NQ];
 #pragma unroll
-    for (uint q = 0; q < NQ; q++) v[q] = 64u * q < NA && lane + 64u * q < NA ? idx[lane + 64u * q] : 0xFFFFFFFFu;
+    for (uint q = 0; q < NQ; q++) v[q] = 64u * q < NA && lane + 64u * q < NA ? min(idx[lane + 64u * q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
     MiFound<NQ> f;
-    f.e = by_a ? (uint)__builtin_amdgcn_readfirstlane((int)idx[y]) : y;
+    f.e = by_a ? min((uint)__builtin_amdgcn_readfirstlane((int)idx[y]), E - 1u) : y;
     bool first = true;
 #pragma unroll
     for (uint q = 0; q < NQ; q++) {
         f.m[q] = __ballot(v[q] == f.e);
         if (by_a && 64u * q <= y && (f.m[q] & (y - 64u * q < 64u ? (1ull << (y - 64u * q)) - 1ull : ~0ull))) first = false;
     }
-    if (f.e >= E || !first) {
+    if (!first) {
 #pragma unroll
         for (uint q = 0; q < NQ; q++) f.m[q] = 0ull;
     }
@@ -1468,8 +1470,8 @@ __device__ __forceinline__ MtFound mt_find(const uint* __restrict__ idx, uint NA
     const bool by_a = NA < E;
     uint v[8], mine = 0u, ahead = 0u;
 #pragma unroll
-    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? idx[first + 64u * q] : 0xFFFFFFFFu;
-    const uint e = by_a ? (uint)__builtin_amdgcn_readfirstlane((int)idx[y]) : y;
+    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? min(idx[first + 64u * q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
+    const uint e = by_a ? min((uint)__builtin_amdgcn_readfirstlane((int)idx[y]), E - 1u) : y;
 #pragma unroll
     for (uint q = 0; q < 8u; q++) {
         mine += (uint)__popcll(__ballot(v[q] == e));
@@ -1485,7 +1487,7 @@ __device__ __forceinline__ MtFound mt_find(const uint* __restrict__ idx, uint NA
         n += c;
         ahead += wt[16u + w];
     }
-    if (ahead || e >= E) n = 0u;
+    if (ahead) n = 0u;
     n = (uint)__builtin_amdgcn_readfirstlane((int)n);
     if (n) {
         ushort* const lst = (ushort*)(lds + MT_LDS - MT_LIST(n));

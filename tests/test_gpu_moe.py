@@ -912,3 +912,48 @@ def test_products_that_find_their_assignments_against_lists(gpu, orc, pkg, monke
         want = orc.moe_ffn(x[t:t + 1], gi[t * ksel:(t + 1) * ksel].reshape(1, -1), gw[t * ksel:(t + 1) * ksel].reshape(1, -1), gate, up, Q4_K, down, dty, E, nff,
                            mode=0)
         assert peak_err(got[t * d:(t + 1) * d] - y0[t], want[0]) <= TOL, t
+
+
+@pytest.mark.parametrize("ty,T,E,ksel,env", [(Q4_K, 3, 12, 4, {"OJAS_HIP_MOE": "3"}), (Q4_K, 2, 12, 4, {"OJAS_HIP_MOE_DEC_TOKENS": "0"}),
+                                             (14, 9, 12, 4, {"OJAS_HIP_MOE": "2"}), (Q4_K, 9, 12, 4, {"OJAS_HIP_MOE": "1"}),
+                                             (13, 9, 12, 4, {"OJAS_HIP_MOE": "1", "OJAS_HIP_MOE_FUSE": "0"}), (Q4_K, 2, 12, 4, {"OJAS_HIP_MOE": "1"}),
+                                             (Q4_K, 9, 12, 4, {"OJAS_HIP_MOE": "2", "OJAS_HIP_MOE_FUSE": "0"}), (Q4_K, 9, 12, 4, {"OJAS_HIP_MOE": "4"}),
+                                             (14, 60, 12, 4, {}), (Q8_0, 40, 4, 2, {})])
+def test_a_token_that_no_expert_was_chosen_for(pkg, monkeypatch, ty, T, E, ksel, env):
+    """The router leaves ~0 where a logit is NaN or infinite.  In every form of the layer but the per-assignment f32 kernels such a
+    token gets the last expert's output, whatever ran before it, and the tokens beside it keep their bits."""
+    d, nff = 512, 256
+    gu = Q8_0 if ty == Q8_0 else Q4_K
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    g = pkg.HipGpu(0)
+    try:
+        lins = [g.lin(t, n, k, pkg.synth.weights(t, n, k, "nochoice", i, ty)) for i, (t, n, k) in enumerate([(gu, E * nff, d), (gu, E * nff, d), (ty, E * d, nff)])]
+        x = pkg.synth.normal_f32(T * d, "nochoice", "x", T).reshape(T, d)
+        lg = pkg.synth.normal_f32(T * E, "nochoice", "lg", T, E).reshape(T, E)
+        bad = lg.copy()
+        lost = [0, T // 2] if T > 3 else [T - 1]
+        bad[lost[0], 1] = np.nan
+        bad[lost[-1], E - 1] = np.inf
+        idx, wgt, yd = g.alloc_bytes(T * ksel * 4), g.alloc(T * ksel), g.alloc(T * d)
+
+        def layer(xs, logits):
+            g.memset0(yd)
+            g.moe_ffn_routed(g.upload(xs), T, d, nff, E, ksel, g.upload(logits), idx, wgt, *lins, yd)
+            return g.read(yd, T * d).reshape(T, d)
+
+        fine = layer(x, lg)
+        got = []
+        for before in (100.0 * x, -x):
+            layer(before[::-1], lg[::-1])
+            got.append(layer(x, bad))
+        gi, gw = g.read(idx, T * ksel, np.uint32).reshape(T, ksel), g.read(wgt, T * ksel)
+        assert np.all(gi[lost] == 0xFFFFFFFF)
+        g.moe_ffn(g.upload(x), T, d, nff, E, ksel, g.upload_bytes(np.minimum(gi, E - 1).ravel().view(np.uint8)), g.upload(gw), *lins, yd)
+        want = g.read(yd, T * d).reshape(T, d)
+        others = [t for t in range(T) if t not in lost]
+        for y in got:
+            assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+            assert np.array_equal(y[others].view(np.uint32), fine[others].view(np.uint32))
+    finally:
+        g.close()
