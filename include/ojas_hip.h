@@ -216,8 +216,9 @@ int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dtype, const o
  * The int8 activations and their per-256 scales are staged in a static device array of
  * `ojh_noalloc_scratch_bytes()` bytes (1 MiB of activations + their scales) that each GPU holds
  * until the process ends, so the call allocates and frees nothing; the results are
- * those of `ojh_mm(..., OJH_ACT_Q8K)` bit for bit below 17 tokens (of one token, `ojh_mm` may quantize
- * inside the product's launch, this entry in one of its own); from there `ojh_mm` may take a
+ * those of `ojh_mm(..., OJH_ACT_Q8K)` bit for bit below 17 tokens (Q5_K: below 9, and below 5 from 8192
+ * rows or a K beyond 8192; of one token, `ojh_mm` may quantize inside the product's launch, this entry
+ * in one of its own); from there `ojh_mm` may take a
  * prefill tile or K slices that stage more in library scratch, which this entry never does (Q4_K stays
  * on the few-token kernels, Q6_K / Q5_K take their 128-token tile unsliced: the same integer sums, the
  * f32 terms equal to rounding).  K-quant weights (Q4_K, Q5_K, Q6_K), f32 or bf16

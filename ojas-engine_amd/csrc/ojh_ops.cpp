@@ -368,18 +368,18 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
     // (from where it was measured ahead of what it replaces, rows streamed from HBM.  Q6_K: from 17 tokens on matrices of
     // more than 4096 rows or a longer K than that — 7168 x 2048 at 24 tokens 14.6 against 20.4 us for two launches of 16,
     // 730 x 5632 17.7 against 21.2, 14336 x 4096 24.2 against 39 — from 33 on the others, where two launches are level or
-    // ahead (4096 x 4096: 18.2 against 17.8, 2048 x 1536 13.2 against 12.9), and from 9 where 16 tokens no longer fit the
-    // few-row kernel (4096 x 14336 at 12 tokens 26.3 against 33.4 for two launches of 8).  Q5_K, whose few-token form is
+    // ahead (4096 x 4096: 18.2 against 17.8, 2048 x 1536 13.2 against 12.9).  Below 17 tokens Q6_K keeps the bits of
+    // ojh_mm_noalloc, which has no scratch for K slices, also where 16 tokens no longer fit the few-row kernel (4096 x 14336
+    // at 12 tokens: two launches of 8 take 33.4, the slices took 26.3).  Q5_K, whose few-token form is
     // the integer-dot kernel: from 5 tokens on large matrices (14336 x 4096 at 5 tokens 22.6, at 3 22.6 against 17.7 there),
     // from 9 on small ones (4096 x 4096 at 8 tokens 17.4 against 12.4, 730 x 5632 17.7 against 13.5).)
     // Below the second threshold a call takes the tile only where all it needs is to be had (a recorded call may ask for
     // nothing), and leaves its scratch to calls that cannot do without.
     const bool gs_large = N >= 8192 || K > 8192;
-    const bool q6k_few = (N + 15) / 16 <= 2u * (uint32_t)dev->prop.multiProcessorCount && ojh_q6k_mk_lds(K, 16) > 163840;
     const uint32_t gs_min = dev->kq_gs_min_m != 1 ? dev->kq_gs_min_m
                             : w->type == OJH_Q6_K ? (gs_large ? 17u : 33u) : (gs_large ? 5u : 9u);
     const uint32_t gs_early = dev->kq_gs_min_m != 1 || w->type != OJH_Q6_K || dev->no_scratch ? gs_min
-                              : q6k_few ? 9u : N > 4096 || K > 4096 ? 17u : 33u;
+                              : N > 4096 || K > 4096 ? 17u : 33u;
     if ((w->type == OJH_Q6_K || w->type == OJH_Q5_K) && gs_min && m >= gs_early && K % 256 == 0 &&
         (uintptr_t)xq % 16 == 0 && (w->type == OJH_Q6_K ? dwords_ok : (uintptr_t)wp % 16 == 0)) {
         int rc;

@@ -53,6 +53,29 @@ def test_no_alloc_matches_mm_on_consecutive_calls(gpu, pkg, orc):
     _both(gpu, pkg, orc, Q6_K, 130, 256, 1, "e", accum=True)
 
 
+@pytest.mark.parametrize("ty,n,k,ms", [(Q6_K, 300, 14336, (9, 12, 16)), (Q6_K, 4100, 9984, (9, 16)), (Q6_K, 130, 4352, (2, 16)),
+                                       (Q6_K, 8448, 1024, (16,)), (Q4_K, 300, 14336, (5, 16)), (Q4_K, 960, 1024, (16,))])
+def test_no_alloc_matches_mm_up_to_sixteen_tokens(gpu, pkg, orc, ty, n, k, ms):
+    """... over the whole range that the header promises: long rows whose 16 tokens do not fit the few-row kernel among them."""
+    gpu.ensure_family("gemv_q8k")
+    gpu.ensure_family("gemm_q8k")
+    for m in ms:
+        _both(gpu, pkg, orc, ty, n, k, m, "up-to-16 %d" % m)
+
+
+def test_no_alloc_matches_mm_on_q5k_rows(gpu, pkg):
+    """... for Q5_K up to where `ojh_mm` takes K slices of the matrix tile."""
+    gpu.ensure_family("gemv_q8k")
+    gpu.ensure_family("gemm_q8k")
+    for n, k, m in ((300, 2048, 8), (8192, 512, 4), (96, 8448, 4)):
+        lin = gpu.lin(Q5_K, n, k, pkg.synth.weights(Q5_K, n, k, "noalloc", "q5"))
+        xd, ya, yb = gpu.upload(pkg.synth.normal_f32(m * k, "noalloc", "q5x")), gpu.alloc(m * n), gpu.alloc(m * n)
+        gpu.mm(xd, lin, ya, m, act_mode=pkg.ACT_Q8K)
+        gpu.mm_noalloc(xd, lin, yb, m)
+        assert np.array_equal(gpu.read(yb, m * n).view(np.uint32), gpu.read(ya, m * n).view(np.uint32)), (n, k, m)
+        lin.free()
+
+
 def test_no_alloc_takes_the_unsliced_prefill_tile(gpu, pkg, orc):
     """Q6_K rows against 40 tokens: `ojh_mm` runs the 128-token tile over K slices that meet in library scratch, the entry
     that allocates nothing runs the same tile whole — the same integer sums, the super-blocks' f32 terms added in one
