@@ -49,16 +49,51 @@ static double moe_expert_bytes(uint32_t d, uint32_t n_ff, uint32_t down_type) {
 static bool moe_tiles(const ojh_device *dev, uint64_t NA, uint32_t E) {
     return dev->moe_mode == 1 || dev->moe_mode == 4 || (dev->moe_mode == 0 && NA >= (uint64_t)4 * E);
 }
+// Scratch of the grouped launches.  Every call of three tokens and more asks for all of it, also where its own launches need
+// less: the routes alternate with the batch (128 experts of 2048 x 768: lists at 16 tokens, none at 8 or 64), and a recorded
+// call, which can ask for nothing, finds what an eager one of as many tokens has left, whichever way the two run.
+struct MoeScratch {
+    ojh_buf *xq, *xs, *act, *aq, *as, *dv, *grp;
+};
+static int moe_scratch(ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, MoeScratch *s) {
+    const size_t NA = (size_t)T * ksel;
+    int rc;
+    if ((rc = ojh_scratch_get(dev, "moe_xq", (size_t)T * d, &s->xq))) return rc;
+    if ((rc = ojh_scratch_get(dev, "moe_xs", (size_t)T * (d / 256) * 4, &s->xs))) return rc;
+    if ((rc = ojh_scratch_get(dev, "moe_act", NA * n_ff * 4, &s->act))) return rc;
+    if ((rc = ojh_scratch_get(dev, "moe_aq", NA * n_ff, &s->aq))) return rc;
+    if ((rc = ojh_scratch_get(dev, "moe_as", NA * (n_ff / 256) * 4, &s->as))) return rc;
+    if ((rc = ojh_scratch_get(dev, "moe_dv", NA * d * 4, &s->dv))) return rc;
+    return ojh_scratch_get(dev, "moe_grp", ((size_t)2 * E + 1 + NA) * 4, &s->grp);   // counts[E] | offsets[E+1] | list[NA]
+}
+// ... and whether it is to be had, for two tokens, which can do without
+static bool moe_scratch_fits(const ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel) {
+    const size_t NA = (size_t)T * ksel;
+    return (dev->modules.count("gemv_q8k") || !dev->capturing) &&
+           ojh_scratch_fits(dev, {{"moe_xq", (size_t)T * d}, {"moe_xs", (size_t)T * (d / 256) * 4}, {"moe_act", NA * n_ff * 4}, {"moe_aq", NA * n_ff},
+                                  {"moe_as", NA * (n_ff / 256) * 4}, {"moe_dv", NA * d * 4}, {"moe_grp", ((size_t)2 * E + 1 + NA) * 4}});
+}
 // Whether a few tokens run in the decode form, two launches addressed by assignment: one token always, more while an expert's
 // bytes for each of their assignments are few — each is read by itself, and every workgroup quantizes its token (whole layer,
 // decode form against the grouped launches: 2 tokens, 24 MB 16.7 against 17.4 us, 42 MB 21.5 against 18.2; 3 - 6 tokens, 11
-// MB 11.4 against 14.2, 15 MB 12.3 against 14.2, 21 MB 17.9 against 14.9).
-static bool moe_decodes(const ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t ksel, uint32_t down_type) {
+// MB 11.4 against 14.2, 15 MB 12.3 against 14.2, 21 MB 17.9 against 14.9).  Two tokens also where the grouped launches' scratch is
+// not to be had: the decode form needs `moe_act` alone.
+static bool moe_decodes(const ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, uint32_t down_type) {
     // what the two launches stage in LDS; the down launch keeps one partial sum per slot and lane group for up to 64 slots
     if (!(d <= 8192 && n_ff <= 2048 && ksel <= 64 && (uint64_t)ksel * n_ff <= 32768)) return false;
     if (dev->moe_mode) return dev->moe_mode == 3;
     if (dev->moe_dec_tokens >= 0) return T <= (uint32_t)dev->moe_dec_tokens;
-    return T == 1 || (double)T * ksel * moe_expert_bytes(d, n_ff, down_type) <= (T == 2 ? 32e6 : 16e6);
+    return T == 1 || (double)T * ksel * moe_expert_bytes(d, n_ff, down_type) <= (T == 2 ? 32e6 : 16e6) ||
+           (T == 2 && !moe_scratch_fits(dev, T, d, n_ff, E, ksel));
+}
+// What the decode form asks for: `moe_act`, and for tokens that would be grouped but for their experts' bytes all that a grouped
+// call does.
+static int moe_decode_scratch(ojh_device *dev, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E, uint32_t ksel, ojh_buf **act) {
+    if (T <= 2 || dev->moe_mode || dev->moe_dec_tokens >= 0) return ojh_scratch_get(dev, "moe_act", (size_t)T * ksel * n_ff * 4, act);
+    MoeScratch s;
+    int rc = ensure(dev, "gemv_q8k");
+    if (!rc && !(rc = moe_scratch(dev, T, d, n_ff, E, ksel, &s))) *act = s.act;
+    return rc;
 }
 // How the grouped products of K-quant experts that find their assignments in idx themselves run, four launches instead of six:
 // on the wave tiles from 3.4 - 0.75 d / 1024 assignments per expert, from 1.1 where a row of gate and up is longer than the dots'
@@ -95,12 +130,11 @@ extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T,
         return ojh_fail(OJH_ERR_ARG, "moe_ffn_routed: tokens=%u experts=%u (<= 1024) ksel=%u (<= 64, <= experts) out of range", T, E, ksel);
     const bool kq = gate->type == OJH_Q4_K && up->type == OJH_Q4_K &&
                     (down->type == OJH_Q4_K || down->type == OJH_Q5_K || down->type == OJH_Q6_K);
-    const bool fused = kq && act_mode != OJH_ACT_FLOAT && act_mode != OJH_ACT_FLOAT_EXACT && d && n_ff && d % 256 == 0 && n_ff % 256 == 0 &&
-                       moe_decodes(dev, T, d, n_ff, ksel, down->type) && dev->moe_route_fuse;
+    const bool whole = kq && act_mode != OJH_ACT_FLOAT && d && n_ff && d % 256 == 0 && n_ff % 256 == 0;
+    const bool decodes = whole && moe_decodes(dev, T, d, n_ff, E, ksel, down->type);
     int rc;
-    if (!fused) {
-        if (kq && act_mode != OJH_ACT_FLOAT && d && n_ff && !moe_decodes(dev, T, d, n_ff, ksel, down->type) &&
-            moe_finds(dev, T, d, n_ff, E, ksel, down->type) != MOE_LISTS) {
+    if (!decodes || act_mode == OJH_ACT_FLOAT_EXACT || !dev->moe_route_fuse) {
+        if (whole && !decodes && moe_finds(dev, T, d, n_ff, E, ksel, down->type) != MOE_LISTS) {
             if ((rc = span("moe_route: logits", logits, (size_t)T * E * 4, 4))) return rc;
             return ffn(dev, x, T, d, n_ff, E, ksel, idx, wgt, gate, up, down, y, accum, act_mode, logits);
         }
@@ -118,7 +152,7 @@ extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T,
     if ((rc = span("moe_ffn_routed: y", y, (size_t)T * d * 4, 4))) return rc;
     if ((rc = ensure(dev, "moe"))) return rc;
     ojh_buf *act;
-    if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
+    if ((rc = moe_decode_scratch(dev, T, d, n_ff, E, ksel, &act))) return rc;
     uint32_t b256[3] = {256, 1, 1}, g1[3] = {(n_ff + 7) / 8, NA, 1}, g2[3] = {(d + 7) / 8, T, 1};
     if ((rc = ojh_launch(dev, "moe_gu_q4k_decr",
                          {x->ptr, (char *)gate->raw->ptr + gate->off, (char *)up->raw->ptr + up->off, act->ptr, logits->ptr,
@@ -287,16 +321,16 @@ static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32
     if ((rc = span("moe_ffn: y", y, (size_t)T * d * 4, 4))) return rc;
     if ((rc = ensure(dev, "moe")) || (rc = ensure(dev, "gemv_q8k"))) return rc;
 
-    const uint32_t nsb_d = d / 256, nsb_f = n_ff / 256;
     uint32_t b256[3] = {256, 1, 1};
     // A few tokens: two launches addressed by assignment, activations quantized in registers,
     // weighted sum inside the down launch (bit-identical to the grouped integer-dot pipeline).
     // Measured on MI355X the grouped pipeline takes over once tokens start sharing experts.
-    if (dev->moe_mode == 3 && !moe_decodes(dev, T, d, n_ff, ksel, down->type))
+    const bool decodes = !logits && moe_decodes(dev, T, d, n_ff, E, ksel, down->type);
+    if (dev->moe_mode == 3 && !decodes)
         return ojh_fail(OJH_ERR_UNSUPPORTED, "moe_ffn: the decode form serves d <= 8192, n_ff <= 2048, ksel <= 64 and ksel * n_ff <= 32768");
-    if (moe_decodes(dev, T, d, n_ff, ksel, down->type)) {
+    if (decodes) {
         ojh_buf *act;
-        if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
+        if ((rc = moe_decode_scratch(dev, T, d, n_ff, E, ksel, &act))) return rc;
         uint32_t g1[3] = {(n_ff + 7) / 8, NA, 1};
         if ((rc = ojh_launch(dev, "moe_gu_q4k_dec",
                              {x->ptr, (char *)gate->raw->ptr + gate->off, (char *)up->raw->ptr + up->off, act->ptr, idx->ptr},
@@ -306,17 +340,15 @@ static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32
         return ojh_launch(dev, down_dec.c_str(), {act->ptr, (char *)down->raw->ptr + down->off, idx->ptr, wgt->ptr, y->ptr},
                           {n_ff, d, ksel, E, (uint32_t)(accum != 0)}, g2, b256);
     }
+    MoeScratch buf;
+    if ((rc = moe_scratch(dev, T, d, n_ff, E, ksel, &buf))) return rc;
+    ojh_buf *const xq = buf.xq, *const xs = buf.xs, *const act = buf.act, *const dv = buf.dv;
     if (const int found = moe_finds(dev, T, d, n_ff, E, ksel, down->type); found != MOE_LISTS) {
         // 1. the tokens quantized (and routed), 2. gate / up with SiLU * mul, 3. down over activations it quantizes itself
         // (the CPU path quantizes `act` inside matvec_kq), 4. the router-weighted sum over slots, in slot order
         const bool tiles = found == MOE_FIND_TILES;
         const uint32_t ny = std::min(E, NA);
         const void *wg = (char *)gate->raw->ptr + gate->off, *wu = (char *)up->raw->ptr + up->off, *wd = (char *)down->raw->ptr + down->off;
-        ojh_buf *xq, *xs, *act, *dv;
-        if ((rc = ojh_scratch_get(dev, "moe_xq", (size_t)T * d, &xq))) return rc;
-        if ((rc = ojh_scratch_get(dev, "moe_xs", (size_t)T * nsb_d * 4, &xs))) return rc;
-        if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
-        if ((rc = ojh_scratch_get(dev, "moe_dv", (size_t)NA * d * 4, &dv))) return rc;
         if (logits) {
             uint32_t g[3] = {T, 1, 1}, b[3] = {512, 1, 1};
             rc = ojh_launch(dev, "moe_topk_quant", {logits->ptr, idx->ptr, wgt->ptr, x->ptr, xq->ptr, xs->ptr}, {E, ksel, d}, g, b);
@@ -340,16 +372,8 @@ static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32
         uint32_t gs[3] = {(uint32_t)(((uint64_t)T * d + 255) / 256), 1, 1};
         return ojh_launch(dev, "moe_combine", {dv->ptr, wgt->ptr, y->ptr}, {T, ksel, d, (uint32_t)(accum != 0)}, gs, b256);
     }
-    ojh_buf *xq, *xs, *act, *aq, *as_, *dv, *grp;
-    if ((rc = ojh_scratch_get(dev, "moe_xq", (size_t)T * d, &xq))) return rc;
-    if ((rc = ojh_scratch_get(dev, "moe_xs", (size_t)T * nsb_d * 4, &xs))) return rc;
-    if ((rc = ojh_scratch_get(dev, "moe_act", (size_t)NA * n_ff * 4, &act))) return rc;
-    if ((rc = ojh_scratch_get(dev, "moe_aq", (size_t)NA * n_ff, &aq))) return rc;
-    if ((rc = ojh_scratch_get(dev, "moe_as", (size_t)NA * nsb_f * 4, &as_))) return rc;
-    if ((rc = ojh_scratch_get(dev, "moe_dv", (size_t)NA * d * 4, &dv))) return rc;
-    // counts[E] | offsets[E+1] | list[NA]
-    if ((rc = ojh_scratch_get(dev, "moe_grp", ((size_t)2 * E + 1 + NA) * 4, &grp))) return rc;
-    uint32_t *counts = (uint32_t *)grp->ptr, *offsets = counts + E, *list = offsets + E + 1;
+    ojh_buf *const aq = buf.aq, *const as_ = buf.as;
+    uint32_t *counts = (uint32_t *)buf.grp->ptr, *offsets = counts + E, *list = offsets + E + 1;
 
     // Expert products: on the matrix cores once experts see a few tokens each (measured crossover on
     // MI355X, 128 experts of 2048 x 768: 4 assignments per expert — 48 tokens of top-8 take 105 us on dots and 115 on

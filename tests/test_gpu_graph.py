@@ -254,3 +254,114 @@ def test_a_batch_of_a_few_more_tokens_is_recorded_after_an_eager_one(orc, pkg):
         graph.free()
     finally:
         g.close()
+
+
+def _layer(g, pkg, E, d, nff, dty, tag):
+    """Expert tensors of one layer, a few experts' rows repeated, as what `moe_ffn_routed` takes."""
+    lins = []
+    for ty, n, k in ((Q4_K, nff, d), (Q4_K, nff, d), (dty, d, nff)):
+        few = min(E, 4)
+        rows = pkg.synth.weights(ty, few * n, k, "graph-moe", tag, ty, n, k, len(lins))
+        lins.append(g.lin(ty, E * n, k, np.tile(rows, -(-E // few))[:len(rows) // few * E]))
+    return lins
+
+
+def _expert_call(g, pkg, lins, T, E, ksel, d, nff):
+    x = pkg.synth.normal_f32(T * d, "graph-moe", "x", T, d)
+    lg = pkg.synth.normal_f32(T * E, "graph-moe", "lg", T, E)
+    bufs = [g.upload(x), g.upload(lg), g.alloc_bytes(T * ksel * 4), g.alloc(T * ksel), g.alloc(T * d)]
+
+    def call():
+        g.moe_ffn_routed(bufs[0], T, d, nff, E, ksel, bufs[1], bufs[2], bufs[3], *lins, bufs[4])
+
+    return call, bufs[4], T * d
+
+
+def _replays(g, calls):
+    """The calls recorded one after the other: three replays against the eager results of another time."""
+    g.capture_begin()
+    try:
+        for call, _, _ in calls:
+            call()
+    finally:
+        graph = g.capture_end()
+    outs = []
+    for _ in range(3):
+        for _, y, _ in calls:
+            g.memset0(y)
+        graph.launch()
+        outs.append([g.read(y, n) for _, y, n in calls])
+        for call, y, n in calls:
+            g.memset0(y)
+            call()
+            outs[-1].append(g.read(y, n))
+    graph.free()
+    return outs
+
+
+def test_expert_layers_are_recorded_after_an_eager_one_of_more_tokens(pkg):
+    """300 experts, top 8: 200 tokens find their assignments on the wave tiles, 70 take lists, 40 find theirs on integer dots, 4 take
+    the decode form.  What the first leaves behind is enough for the others, whichever way each runs."""
+    E, ksel, d, nff = 300, 8, 256, 256
+    g = pkg.HipGpu(0)
+    try:
+        lins = _layer(g, pkg, E, d, nff, Q4_K, "many")
+        first, y, n = _expert_call(g, pkg, lins, 200, E, ksel, d, nff)
+        first()
+        assert np.isfinite(g.read(y, n)).all()
+        calls = [_expert_call(g, pkg, lins, T, E, ksel, d, nff) for T in (70, 40, 4)]
+        for out in _replays(g, calls):
+            for a, b in zip(out[:3], out[3:]):
+                assert a.any() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        g.close()
+
+
+def test_an_expert_layer_of_larger_experts_is_recorded_after_one_in_the_decode_form(pkg):
+    """4 tokens of a layer whose experts are small enough for the decode form leave behind what the next layer's, with a finer down
+    tensor, need grouped."""
+    T, E, ksel, d, nff = 4, 8, 4, 1024, 512
+    g = pkg.HipGpu(0)
+    try:
+        small, large = (_layer(g, pkg, E, d, nff, ty, "mixed") for ty in (Q4_K, 14))
+        eager = _expert_call(g, pkg, small, T, E, ksel, d, nff)
+        eager[0]()
+        calls = [_expert_call(g, pkg, large, T, E, ksel, d, nff), eager]
+        for out in _replays(g, calls):
+            for a, b in zip(out[:2], out[2:]):
+                assert a.any() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("limit", [None, 65536])
+def test_two_tokens_of_large_experts_without_the_grouped_scratch(pkg, monkeypatch, limit):
+    """Two tokens over experts of more than 32 MB in all are grouped where the scratch is to be had.  Recorded after one token of
+    another layer, or under a limit that holds the activations alone, they run in the decode form, which needs no more than that."""
+    T, E, ksel, d, nff = 2, 16, 8, 2048, 768
+    if limit:
+        monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", str(limit))
+    g = pkg.HipGpu(0)
+    try:
+        lins, other = _layer(g, pkg, E, d, nff, Q4_K, "two"), _layer(g, pkg, 8, 256, 2048, Q4_K, "one")
+        call, y, n = _expert_call(g, pkg, lins, T, E, ksel, d, nff)
+        if limit:
+            call()
+            got = [g.read(y, n)]
+        else:
+            _expert_call(g, pkg, other, 1, 8, 8, 256, 2048)[0]()
+            got = [out[0] for out in _replays(g, [(call, y, n)])]
+    finally:
+        g.close()
+    monkeypatch.setenv("OJAS_HIP_MOE", "3")
+    monkeypatch.setenv("OJAS_HIP_SCRATCH_MAX", "0")
+    g = pkg.HipGpu(0)
+    try:
+        call, y, n = _expert_call(g, pkg, _layer(g, pkg, E, d, nff, Q4_K, "two"), T, E, ksel, d, nff)
+        call()
+        want = g.read(y, n)
+    finally:
+        g.close()
+    assert want.any()
+    for out in got:
+        assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
