@@ -134,7 +134,7 @@ extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T,
     const bool decodes = whole && moe_decodes(dev, T, d, n_ff, E, ksel, down->type);
     int rc;
     if (!decodes || act_mode == OJH_ACT_FLOAT_EXACT || !dev->moe_route_fuse) {
-        if (whole && !decodes && moe_finds(dev, T, d, n_ff, E, ksel, down->type) != MOE_LISTS) {
+        if (whole && !decodes && dev->moe_route_fuse && moe_finds(dev, T, d, n_ff, E, ksel, down->type) != MOE_LISTS) {
             if ((rc = span("moe_route: logits", logits, (size_t)T * E * 4, 4))) return rc;
             return ffn(dev, x, T, d, n_ff, E, ksel, idx, wgt, gate, up, down, y, accum, act_mode, logits);
         }
