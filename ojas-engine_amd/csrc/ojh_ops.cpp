@@ -856,11 +856,13 @@ static int f16d_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *w,
 //   Q5_K   600 x 4096 5.7 / 4.8, 4096^2 6.8 / 6.0, 9000 x 4096 11.4 / 10.1, 30000 x 8192 42.1 / 34.5, 128256 x 2560 66.9 / 58.0: everywhere
 //   Q4_K   1024 x 4096 5.8 / 4.3, 9000 x 5120 10.8 / 9.6, 5300 x 14336 15.0 / 12.3, 30000 x 4096 16.3 / 16.0; output heads have a form of their
 //          own that keeps more bytes in flight, so from 32768 rows only a short K: 65536 x 1792 16.8 / 15.8, x 4096 29.1 / 30.9
-//   Q6_K   four lanes take a super-block, sixteen super-blocks a step.  Up to sixteen rows a CU, one a wave: 4096^2 7.9 / 6.4, 4096 x 11008
-//          13.9 / 11.6, 1500 x 14336 10.7 / 9.7, but 1024 x 14336 8.4 / 8.5.  Beyond, the waves take further pairs of rows: four units a wave
-//          (gemv_fq8k_ring) are ahead, 12000 x 5120 16.8 / 16.1, 30000 x 14336 88 / 74, 65536 x 1024 38.0 / 23.0 (output heads have a form of
-//          their own, a step of which is mostly idle at a short K), but not where one step is full, 30000 x 4096 23.9 / 25.2; fewer only
-//          where the last step is mostly full, 7500 x 4096 10.4 / 9.6, 5300 x 8192 13.7 / 12.7, not 9216 x 1024 7.5 / 7.7, 7500 x 5120 13.6 / 13.0.
+//   Q6_K   four lanes take a super-block, sixteen super-blocks a step.  Up to sixteen rows a CU, one a wave: 4096^2 7.7 / 6.4, 4096 x 11008
+//          14.2 / 12.2, 2500 x 14336 13.5 / 11.5, but 1024 x 14336 8.4 / 8.9.  Beyond, the waves take pairs of rows.  Four units a wave
+//          (gemv_fq8k_ring) are ahead, 12000 x 5120 17.4 / 16.6, 30000 x 9984 62.5 / 56.7, 50000 x 1024 31.3 / 19.2 (output heads have a form
+//          of their own, a step of which is mostly idle at a short K), but not where one step is full, 30000 x 4096 25.6 / 25.8, 50000 x
+//          4096 36.5 / 39.0.  Fewer: from 28 rows a CU, where fewer would leave waves without a pair, and rows of fifteen super-blocks,
+//          7500 x 3840 9.7 / 9.5, x 5120 13.7 / 13.4, not 7500 x 3072 9.2 / 9.3; from 500 super-blocks a CU with less, 5300 x 6144 12.1 / 11.7,
+//          4608 x 9984 15.5 / 15.1, not 6144 x 5120 11.6 / 11.9; one step up to 64, 16000 x 4096 level, 24000 x 4096 21.2 / 21.5.
 // Not where y lies over x: a workgroup may store its rows before another has read the token.
 static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x, size_t x_bytes, const void *y) {
     const uint32_t K = w->k, N = w->n, cus = (uint32_t)dev->prop.multiProcessorCount;
@@ -871,7 +873,7 @@ static bool fq_one_taken(const ojh_device *dev, const ojh_lin *w, const void *x,
     const uint32_t nsb = K / 256, steps = (nsb + 15) / 16, nrb = (N + cus - 1) / cus;
     if (nrb <= 16u) return K <= 8192u || nrb >= 5u;
     if ((nrb + 31) / 32 * steps >= 4u) return steps > 1 || nsb <= 12;
-    return nrb >= 20u && nsb >= 15 && 5 * nsb >= 64 * steps;
+    return nsb >= 15 && (nrb >= 28u ? steps > 1 || nrb <= 64u : nrb * nsb >= 500u);
 }
 // Those that need nothing but themselves; the others ask for the two launches' scratch although they do without, so what a limit on
 // scratch or a recording refuses does not depend on the route, and a recorded call that takes two launches finds it.

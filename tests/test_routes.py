@@ -52,7 +52,8 @@ int ojh_launch(ojh_device *dev, const char *name, const std::vector<void *> &ptr
     if (!dev->modules.count(s->family)) return ojh_fail(OJH_ERR_NOT_LOADED, "%s: family %s", name, s->family);
     size_t need[16] = {}, align[16];
     for (size_t &a : align) a = 4;
-    if (int rc = s->check(s, consts.data(), grid, block, need, align)) return rc;
+    const uint32_t b[3] = {strstr(name, "fq8k_q4k_x4") ? 256 : block[0], block[1], block[2]};     // (a caller's own dispatch of that one: 256 threads)
+    if (int rc = s->check(s, consts.data(), grid, b, need, align)) return rc;
     for (size_t i = 0; i < ptrs.size(); i++)
         if (ptrs[i] && (uintptr_t)ptrs[i] % align[i]) return ojh_fail(-98, "%s: buffer %zu not aligned", name, i);
     g_log += std::string(name) + " ";
@@ -193,3 +194,13 @@ def test_the_router_is_a_launch_of_its_own_where_that_is_asked_for(lib, form):
         assert fused == ["moe_gu_q4k_decr"] + apart[2:]
     else:
         assert fused == ["moe_topk_quant"] + apart[2:]
+
+
+@pytest.mark.parametrize("n,k,one", [(4096, 4096, True), (2500, 14336, True), (1024, 14336, False), (7500, 5120, True), (7500, 3840, True), (7500, 3072, False),
+                                     (5300, 6144, True), (4608, 9984, True), (6144, 5120, False), (6144, 4096, False), (16000, 4096, True), (24000, 4096, False),
+                                     (12000, 5120, True), (30000, 9984, True), (30000, 4096, False), (30000, 3072, True), (50000, 1024, True), (50000, 4096, False)])
+def test_one_token_of_q6k_rows_on_either_side_of_the_line(lib, n, k, one):
+    """The sizes whose times stand beside the rule take the form that is ahead there."""
+    got = Dev(lib).mm(Q6_K, n, k, 1)
+    assert (got[0].startswith("gemv_fq8k_q6k_one") and len(got) == 1) == one, got
+    assert one or got[0] == "quantize_q8k"
