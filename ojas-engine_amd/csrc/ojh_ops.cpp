@@ -3,6 +3,7 @@
 // reference (crates/ojas-cuda/src/qwen35.rs:174-201, :644-702; Metal twin
 // crates/ojas-models/src/decoder/dispatch.rs:288-626).
 #include <cstdlib>
+#include <cmath>
 #include <cstring>
 
 #include "ojh_internal.h"
@@ -592,6 +593,19 @@ static void fq_leave_scratch(ojh_device *dev, uint32_t K) {
     if (!dev->capturing && !ojh_scratch_spare(dev, "xq", K, &b, true)) (void)ojh_scratch_spare(dev, "xs", K / 64, &b, true);
 }
 
+// A workgroup's rows are one run of bytes, so workgroups lie `nrb` rows apart, and where that is close to a 128th above or below 512 KB
+// or 1 MB their streams meet in the same channels: two rows more a workgroup then (us, as dealt / two more: Q4_K 26000 x 9216
+// 33.3 / 27.9, 24000 x 9984 32.1 / 27.7, 52000 x 9216 56.0 / 51.3, Q5_K 38400 x 5120 34.3 / 30.4, Q6_K 23040 x 7168 35.1 / 33.2).  No
+// such distance below 400 KB.
+static uint32_t fq_rows_dealt(uint32_t nrb, uint32_t r, size_t row_bytes) {
+    for (;; nrb += r) {
+        const double apart = (double)nrb * (double)row_bytes;
+        if (apart < 400e3) return nrb;
+        const double off = std::fabs(apart / std::exp2(std::round(std::log2(apart))) - 1.0);
+        if (std::fabs(off - 1.0 / 128) > 1.0 / 400) return nrb;
+    }
+}
+
 // One stage of a decode layer in ONE launch: 1 to 4 projections of one f32 vector, the vector quantized inside the launch.
 extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int count, const ojh_lin *const *ws,
                             ojh_buf *const *ys, const size_t *y_offs, int accum) {
@@ -665,7 +679,7 @@ extern "C" int ojh_mm_multi(ojh_device *dev, const ojh_buf *x, size_t x_off, int
     int r = dev->fq_rows ? dev->fq_rows : 2;
     uint32_t want = cus * dev->fq_multi_blocks;
     uint32_t nrb = (run + want - 1) / want;
-    nrb = (nrb + (uint32_t)r - 1) / (uint32_t)r * (uint32_t)r;
+    nrb = fq_rows_dealt((nrb + (uint32_t)r - 1) / (uint32_t)r * (uint32_t)r, (uint32_t)r, ws[0]->row_bytes);
     uint32_t grid[3] = {(run + nrb - 1) / nrb, 1, 1}, block[3] = {dev->fq_threads, 1, 1};
     return ojh_launch(dev, r == 2 ? "gemv_fq8k_q4k_x4_r2" : "gemv_fq8k_q4k_x4_r1", p,
                       {K, ends[0], ends[1], ends[2], ends[3], nrb, (uint32_t)(accum != 0)}, grid, block);
@@ -892,7 +906,7 @@ static int fq_one_launch(ojh_device *dev, void *xp, int x_dtype, const ojh_lin *
     uint32_t nrb = (w->n + cus - 1) / cus;
     const bool steps = w->type == OJH_Q4_K ? w->k >= 8192u : w->type == OJH_Q5_K && w->k > 8192u && w->n >= 5u * cus;
     const uint32_t r = dev->fq_rows ? (uint32_t)dev->fq_rows : nrb > 16 || steps ? 2 : 1;
-    nrb = (nrb + r - 1) / r * r;
+    nrb = fq_rows_dealt((nrb + r - 1) / r * r, r, w->row_bytes);
     const uint32_t grid[3] = {(w->n + nrb - 1) / nrb, 1, 1}, block[3] = {1024, 1, 1};
     const std::string name = std::string("gemv_fq8k_") + f->tag + (x_dtype == OJH_X_BF16 ? "_one_bf16_r" : "_one_r") + (r == 2 ? "2" : "1");
     int rc = ensure(dev, "gemv_q8k");

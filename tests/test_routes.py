@@ -15,6 +15,7 @@ RUNTIME = r"""
 #include <algorithm>
 #include <cstring>
 static std::string g_log, g_error;
+static std::vector<uint32_t> g_consts;
 static uintptr_t g_next = 1ull << 40;
 static ojh_buf *fake(size_t bytes) {
     ojh_buf *b = new ojh_buf;
@@ -57,6 +58,7 @@ int ojh_launch(ojh_device *dev, const char *name, const std::vector<void *> &ptr
     for (size_t i = 0; i < ptrs.size(); i++)
         if (ptrs[i] && (uintptr_t)ptrs[i] % align[i]) return ojh_fail(-98, "%s: buffer %zu not aligned", name, i);
     g_log += std::string(name) + " ";
+    g_consts = consts;
     return OJH_OK;
 }
 static size_t held(const ojh_device *dev) {
@@ -109,6 +111,7 @@ extern "C" void dev_set(ojh_device *d, const char *key, long v) {
     else if (!strcmp(key, "scratch_max")) d->scratch_max = (uint64_t)v;
     else abort();
 }
+extern "C" uint32_t last_const(int i) { return g_consts[i]; }      // of the last launch
 static int out(int rc, char *log, size_t room) {
     snprintf(log, room, "%s", rc ? g_error.c_str() : g_log.c_str());
     return rc;
@@ -204,3 +207,13 @@ def test_one_token_of_q6k_rows_on_either_side_of_the_line(lib, n, k, one):
     got = Dev(lib).mm(Q6_K, n, k, 1)
     assert (got[0].startswith("gemv_fq8k_q6k_one") and len(got) == 1) == one, got
     assert one or got[0] == "quantize_q8k"
+
+
+@pytest.mark.parametrize("ty,n,k,want", [(Q4_K, 26000, 9216, 104), (Q4_K, 24000, 9984, 96), (Q4_K, 22000, 10752, 88), (Q4_K, 25500, 9216, 100), (Q4_K, 27000, 9216, 106),
+                                         (Q5_K, 38400, 5120, 152), (Q5_K, 42496, 9216, 166), (Q6_K, 23040, 7168, 92), (Q4_K, 4096, 4096, 16), (Q5_K, 128256, 2560, 502)])
+def test_workgroups_do_not_lie_where_their_streams_meet(lib, ty, n, k, want):
+    """A row count a workgroup that puts them a 128th off 512 KB or 1 MB apart is raised by two; others are dealt evenly over 256 CUs."""
+    dev = Dev(lib)
+    assert "_one_r" in dev.mm(ty, n, k, 1)[-1] and lib.last_const(2) == want
+    if ty == Q4_K and k > 4096:
+        assert dev.multi(ty, n, k, 1, 0, False) == ["gemv_fq8k_q4k_x4_r2"] and lib.last_const(5) == want
