@@ -75,12 +75,15 @@ __device__ __forceinline__ void gemv_nat_iq4_m_body(const float* __restrict__ x,
     }
 }
 
-// A few tokens against many steps of K: gemv_nat_<fmt>_ms(x, w, y, K, N, M, ACC), the _m entry's arguments and grid.  A workgroup of
+// Two tokens and more against many steps of K: gemv_nat_<fmt>_ms(x, w, y, K, N, M, ACC), the _m entry's arguments and grid.  A workgroup of
 // n waves owns n rows, four at a time; its waves take a step of K each in turn for all four rows, and their sums meet in LDS
 // in wave order.  A lane's f32 activations, 8 bytes a weight at two tokens, are what such a call asks the address unit for: a wave
 // that walks a row by itself fetches them again for every row.  Whole call, _m / _ms, us: IQ4_XS 14336 x 4096 at 3 tokens 37.4 / 17.7,
 // 4096 x 14336 at 2 19.8 / 15.0, 27347 x 13312 at 3 259 / 94.6; Q8_0 14336 x 4096 at 2 22.5 / 15.2, at 3 35.5 / 17.2.  With few steps of K
 // some waves have none: 30000 x 1280 IQ4_XS at 2 16.2 / 18.1, at 3 28.8 / 20.4, 1599 x 1024 at 4 4.4 / 4.7 (two waves on two rows there: 21.9 and 24.6).
+// More than four tokens (f32 activations asked for, a K without a tile) are further passes of four over the rows, as in the _m entry:
+// Q8_0 4096 x 4096 at 5 24.0 / 16.4, at 16 41.5 / 27.8, at 31 76.5 / 48.8, 14336 x 1280 at 9 42.2 / 30.7, 4096 x 14336 at 31 268 / 176; Q5_0
+// 1001 x 2304 at 8 13.0 / 8.9, IQ4_XS 2000 x 1280 at 64 42.2 / 38.5, 4096 x 4096 at 300 801 / 398: ahead at each of 8 shapes.
 template <class W, int MT>
 __device__ __forceinline__ void gemv_nat_ms_body(const float* __restrict__ x, const uchar* __restrict__ w,
                                                  float* __restrict__ y, uint K, uint N, uint M, uint ACC) {

@@ -1248,8 +1248,8 @@ extern "C" int ojh_mm(ojh_device *dev, const ojh_buf *x, size_t x_off, int x_dty
         if (bias) p.push_back(bias->ptr);
         return ojh_launch(dev, name.c_str(), p, {K, N}, grid, block);
     }
-    // (waves that share rows where a row is many steps of 512 weights: two tokens from the fifth, more from the third; both sides
-    // at gemv_nat_ms_body)
+    // (waves that share rows where a row is many steps of 512 weights: two tokens from the fifth, more, also beyond four, from the
+    // third; both sides at gemv_nat_ms_body)
     const bool shared = ojh_shares_rows(w->type) && K > (m == 2 ? 2048u : 1024u);
     grid[0] = (N + 3) / 4;
     return ojh_launch(dev, (base + (shared ? "_ms" : "_m")).c_str(), {xp, wp, yp}, {K, N, m, (uint32_t)(accum != 0)}, grid, block);

@@ -217,3 +217,11 @@ def test_workgroups_do_not_lie_where_their_streams_meet(lib, ty, n, k, want):
     assert "_one_r" in dev.mm(ty, n, k, 1)[-1] and lib.last_const(2) == want
     if ty == Q4_K and k > 4096:
         assert dev.multi(ty, n, k, 1, 0, False) == ["gemv_fq8k_q4k_x4_r2"] and lib.last_const(5) == want
+
+
+@pytest.mark.parametrize("ty,tag,k,m,shared", [(Q8_0, "q80", 2080, 2, True), (Q8_0, "q80", 2048, 2, False), (IQ4_XS, "iq4xs", 1280, 3, True),
+                                               (IQ4_XS, "iq4xs", 1024, 3, False), (Q8_0, "q80", 4096, 31, True), (Q8_0, "q80", 2080, 300, True),
+                                               (Q8_0, "q80", 992, 300, False)])
+def test_tokens_from_which_waves_share_rows(lib, ty, tag, k, m, shared):
+    """f32 activations: both sides of the row length, two tokens, three, and batches that no tile takes."""
+    assert Dev(lib).mm(ty, 2000, k, m, FLOAT) == ["gemv_nat_%s_%s" % (tag, "ms" if shared else "m")]
