@@ -391,7 +391,7 @@ def test_three_slices_of_whole_tiles_stay_with_two_workgroups_a_cu(pkg, monkeypa
 @pytest.mark.parametrize("accum", [False, True])
 def test_few_rows_take_the_tile_in_slices(gpu, orc, pkg, monkeypatch, m, n, k, accum):
     """Fewer rows than the slices fill half the CUs with: against matvec_kq, one row, rows past a tile, tokens past one; and where
-    there is no room for the tile's scratch the few-token kernel still takes the call."""
+    there is no room for the tile's scratch the few-token kernel still takes the call (which calls take the tile: test_routes.py)."""
     w, x = _case(pkg, m, n, k, "few-rows")
     y0 = pkg.synth.normal_f32(m * n, "gq", "y0", m, n).reshape(m, n) if accum else np.zeros((m, n), np.float32)
     got = []

@@ -102,7 +102,8 @@ def test_router_path_matches_the_cpu_reference(gpu, orc, pkg, ty, m, n, k, accum
 
 @pytest.mark.parametrize("ty,m,n,k", [(Q6_K, 17, 4100, 512), (Q6_K, 32, 130, 4352), (Q6_K, 9, 300, 14336), (Q6_K, 16, 4096, 14336)])
 def test_few_tokens_from_which_the_tile_is_ahead(gpu, orc, pkg, ty, m, n, k):
-    """Both sides of the row and K bounds of the early crossover, through `ojh_mm`; 9 and 16 tokens of a long K stay before it."""
+    """Both sides of the row and K bounds of the early crossover, through `ojh_mm`; 9 and 16 tokens of a long K stay before it
+    (which calls take the tile: test_routes.py)."""
     w, x = _case(pkg, ty, m, n, k, "early")
     lin = gpu.lin(ty, n, k, w)
     yd = gpu.upload(np.full(m * n + n, 4242.5, np.float32))

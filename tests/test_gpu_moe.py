@@ -875,7 +875,7 @@ def test_expert_ffn_in_both_forms_of_the_wave_tiles(gpu, orc, pkg, T, E, ksel, d
                                                 (9, 1000, 3, 512, 768, Q4_K), (4, 2, 2, 4096, 512, 14), (70, 12, 5, 1536, 512, Q4_K)])
 def test_products_that_find_their_assignments_against_lists(gpu, orc, pkg, monkeypatch, mode, T, E, ksel, d, nff, dty):
     """The four-launch forms (integer dots `_mi` / `_mil`, wave tiles `_ti`) against the grouping's lists, bit for bit: fewer and more
-    assignments than experts, 128 and 512 of them and one more, rows of half, one and two steps of the dots, an expert with
+    assignments than experts, 128 and 512 of them, rows of half, one and two steps of the dots, an expert with
     more than 64, one with none; idx and wgt as the router alone writes them, y accumulated onto."""
     gate = pkg.synth.q4k_weights(E * nff, d, "moefind", "g", E, d, nff)
     up = pkg.synth.q4k_weights(E * nff, d, "moefind", "u", E, d, nff)
@@ -912,6 +912,17 @@ def test_products_that_find_their_assignments_against_lists(gpu, orc, pkg, monke
         want = orc.moe_ffn(x[t:t + 1], gi[t * ksel:(t + 1) * ksel].reshape(1, -1), gw[t * ksel:(t + 1) * ksel].reshape(1, -1), gate, up, Q4_K, down, dty, E, nff,
                            mode=0)
         assert peak_err(got[t * d:(t + 1) * d] - y0[t], want[0]) <= TOL, t
+
+
+@pytest.mark.parametrize("mode,T,E,ksel,d,nff,dty", [("2", 43, 60, 3, 512, 256, Q4_K), ("2", 171, 100, 3, 256, 256, 13), ("1", 171, 100, 3, 256, 256, 13),
+                                                     ("1", 205, 8, 5, 256, 512, Q4_K), ("1", 256, 100, 8, 256, 256, 14), ("1", 512, 16, 8, 512, 256, 13),
+                                                     ("1", 512, 128, 8, 256, 512, Q4_K), ("1", 241, 128, 17, 256, 256, 14), ("1", 512, 16, 8, 4096, 256, Q4_K),
+                                                     ("1", 512, 16, 8, 4352, 256, Q4_K)])
+def test_many_assignments_found_against_lists(gpu, orc, pkg, monkeypatch, mode, T, E, ksel, d, nff, dty):
+    """The same for 129 and 513 assignments on the dots (two words a lane and eight; lists beyond 512), for 513 to 4096 on the tiles,
+    where a wave scans them in more than one step, an expert with nearly all of a slot's among them, eight waves and sixteen; and the
+    last that are found: one more than 4096, a list that no longer fits beside sixteen tokens."""
+    test_products_that_find_their_assignments_against_lists(gpu, orc, pkg, monkeypatch, mode, T, E, ksel, d, nff, dty)
 
 
 @pytest.mark.parametrize("ty,T,E,ksel,env", [(Q4_K, 3, 12, 4, {"OJAS_HIP_MOE": "3"}), (Q4_K, 2, 12, 4, {"OJAS_HIP_MOE_DEC_TOKENS": "0"}),

@@ -179,6 +179,13 @@ class Dev:
         return self._log(self.lib.route_multi, ty, n, k, count, ctypes.c_size_t(step), int(accum))
 
 
+def _form(launches):
+    """Which form of the expert layer these launches are."""
+    names = " ".join(launches)
+    return "decode" if "_dec" in names else "tiles" if "_ti" in names else "dots" if "q4k_mi" in names else \
+        "lists dense" if "_gs" in names else "lists tiles" if "_mt" in names else "lists"
+
+
 # (T, E, ksel, d, n_ff, down) of one layer for each form
 FORMS = {"decode": (1, 128, 8, 2048, 768, Q4_K), "dots": (4, 128, 8, 2048, 768, Q4_K), "tiles": (64, 128, 8, 2048, 768, Q4_K),
          "lists": (16, 128, 8, 2048, 768, Q4_K)}
@@ -225,3 +232,74 @@ def test_workgroups_do_not_lie_where_their_streams_meet(lib, ty, n, k, want):
 def test_tokens_from_which_waves_share_rows(lib, ty, tag, k, m, shared):
     """f32 activations: both sides of the row length, two tokens, three, and batches that no tile takes."""
     assert Dev(lib).mm(ty, 2000, k, m, FLOAT) == ["gemv_nat_%s_%s" % (tag, "ms" if shared else "m")]
+
+
+@pytest.mark.parametrize("T,E,ksel,d,nff,down,form", [
+    # the decode form: one token always, two up to 32 MB of experts for their assignments, up to 16 MB more
+    (1, 128, 8, 4096, 2048, Q4_K, "decode"), (2, 128, 8, 2048, 512, Q4_K, "decode"), (2, 128, 8, 2048, 768, Q4_K, "dots"),
+    (6, 96, 4, 512, 768, Q4_K, "decode"), (4, 8, 4, 1024, 512, Q4_K, "decode"), (4, 8, 4, 1024, 512, Q6_K, "dots"), (3, 96, 8, 1536, 768, Q6_K, "dots"),
+    # dots below 3.4 - 0.75 d / 1024 assignments an expert, tiles from there; from 1.1 where a row is more than one step
+    (42, 128, 8, 1024, 512, Q4_K, "dots"), (43, 128, 8, 1024, 512, Q4_K, "tiles"), (14, 64, 8, 2048, 768, Q4_K, "dots"), (16, 64, 8, 2048, 768, Q4_K, "tiles"),
+    (8, 64, 8, 2304, 768, Q4_K, "dots"), (9, 64, 8, 2304, 768, Q4_K, "tiles"),
+    # lists where one-step rows have more than 150 MB, beyond what the kernels find, where the dense tile is ahead
+    (8, 128, 8, 2048, 768, Q4_K, "dots"), (16, 128, 8, 2048, 768, Q4_K, "lists"), (64, 300, 8, 256, 256, Q4_K, "dots"), (65, 300, 8, 256, 256, Q4_K, "lists"),
+    (512, 128, 8, 1024, 512, Q4_K, "tiles"), (513, 128, 8, 1024, 512, Q4_K, "lists tiles"), (512, 64, 8, 4096, 512, Q4_K, "tiles"),
+    (512, 64, 8, 4352, 512, Q4_K, "lists tiles"),
+    (30, 12, 4, 1024, 512, Q6_K, "lists dense"), (29, 12, 4, 1024, 512, Q6_K, "tiles"), (33, 13, 4, 1024, 512, Q6_K, "tiles"),
+    (512, 16, 6, 1024, 512, Q5_K, "lists dense"), (511, 16, 6, 1024, 512, Q5_K, "tiles"), (512, 16, 6, 1024, 512, Q4_K, "tiles"),
+    (8, 128, 8, 2048, 2304, Q4_K, "lists")])
+def test_forms_of_the_expert_layer_on_either_side_of_their_lines(lib, T, E, ksel, d, nff, down, form):
+    for routed in (True, False):
+        assert _form(Dev(lib).moe(T, E, ksel, d, nff, down, routed=routed)) == form
+
+
+def test_two_tokens_without_the_grouped_scratch_keep_the_decode_form(lib):
+    """... while the calls of three tokens that are grouped are refused where it is not to be had."""
+    shape = (128, 8, 2048, 768)
+    assert _form(Dev(lib, scratch_max=2 * 8 * 768 * 4).moe(2, *shape)) == "decode"
+    dev = Dev(lib)
+    dev.moe(1, 128, 16, 2048, 768)
+    dev.set(capturing=1)
+    assert _form(dev.moe(2, *shape)) == "decode"
+    with pytest.raises(AssertionError, match="gemv_q8k"):
+        dev.moe(3, *shape)
+    with pytest.raises(AssertionError, match="limit"):
+        Dev(lib, scratch_max=3 * 8 * 768 * 4).moe(3, *shape)
+
+
+@pytest.mark.parametrize("T,then", [(64, 16), (64, 8), (64, 2), (8, 4), (9, 3)])
+def test_an_expert_layer_is_recorded_after_any_of_more_tokens(lib, T, then):
+    dev = Dev(lib)
+    dev.moe(T, 128, 8, 2048, 768)
+    dev.set(capturing=1)
+    assert dev.moe(then, 128, 8, 2048, 768) == Dev(lib).moe(then, 128, 8, 2048, 768)
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(17, 1, 2304, True), (33, 65, 1024, True), (32, 64, 5632, True), (64, 730, 2560, True), (16, 64, 5632, False),
+                                        (32, 65, 1024, False), (65, 63, 4096, False), (129, 63, 4096, False), (100, 959, 1280, False)])
+def test_few_rows_of_q4k_take_the_tile_up_to_half_a_tile_of_tokens(lib, m, n, k, tile):
+    """Matrices of fewer rows than the slices fill half the CUs with: eight slices of the tile from 17 tokens (33 on short rows) to 64,
+    and the few-token kernel without room for them."""
+    for room, taken in ((0, tile), (m * k + m * k // 64 * 2, False)):
+        got = Dev(lib, scratch_max=room).mm(Q4_K, n, k, m, Q8K)
+        assert ("gemm_q8k_q4k_xk64_sr" in got) == taken, got
+
+
+@pytest.mark.parametrize("ty,m,n,k,tile", [(Q6_K, 17, 4100, 512, True), (Q6_K, 17, 4096, 512, False), (Q6_K, 32, 130, 4352, True), (Q6_K, 32, 130, 4096, False),
+                                           (Q6_K, 16, 4100, 512, False), (Q6_K, 9, 300, 14336, False), (Q6_K, 16, 4096, 14336, False), (Q6_K, 33, 130, 4096, True),
+                                           (Q5_K, 5, 8192, 512, True), (Q5_K, 4, 8192, 512, False), (Q5_K, 9, 300, 512, True), (Q5_K, 8, 300, 512, False)])
+def test_tokens_from_which_q6k_and_q5k_rows_take_the_int8_tile(lib, ty, m, n, k, tile):
+    got = Dev(lib).mm(ty, n, k, m, Q8K)
+    assert any("_gs" in name for name in got) == tile, got
+    if tile and ty == Q6_K and m < 33:      # the early tile: not where its slices have no room
+        assert not any("_gs_sr" in name for name in Dev(lib, scratch_max=m * k + m * k // 64 * 2).mm(ty, n, k, m, Q8K))
+
+
+@pytest.mark.parametrize("ty", [Q4_K, Q5_K])
+@pytest.mark.parametrize("accum", [False, True])
+def test_outputs_over_each_other_take_a_launch_each(lib, ty, accum):
+    n, k = 600, 4352
+    apart, over = (Dev(lib).multi(ty, n, k, 3, step, accum) for step in (n * 4, n * 4 - 4))
+    assert over[0] == "quantize_q8k" and len(over) == 4 and len(set(over[1:])) == 1
+    if ty == Q4_K:
+        assert apart == ["gemv_fq8k_q4k_x4_r2"]
