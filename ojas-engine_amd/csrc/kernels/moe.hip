@@ -219,7 +219,7 @@ moe_topk_v3(const float* lg, const float* bias, uint* idx, float* wgt, uint E, u
 // ids, expert-major; the order inside an expert's group is arbitrary and has no effect on the
 // results, which are stored per assignment).  One workgroup; E <= 1024.  An index past the last expert counts as the last
 // one, as in the decode form: the router writes ~0 where it chose nothing, and what is added up behind the products has to be
-// this call's.
+// this call's.  (Clamped once all are loaded: inside the condition of its load each would be waited for by itself.)
 __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uint* __restrict__ counts, uint* __restrict__ offsets,
                                                uint* __restrict__ list, uint NA, uint E, uint* cnt, uint* off) {
     const uint tid = threadIdx.x;
@@ -230,7 +230,9 @@ __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uin
     for (uint a0 = tid; a0 < NA; a0 += 8u * 256u) {
         uint e[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(idx[a0 + (uint)u * 256u], E - 1u) : 0xFFFFFFFFu;
+        for (int u = 0; u < 8; u++) e[u] = idx[min(a0 + (uint)u * 256u, NA - 1u)];
+#pragma unroll
+        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(e[u], E - 1u) : 0xFFFFFFFFu;
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (e[u] < E) atomicAdd(&cnt[e[u]], 1u);
@@ -275,7 +277,9 @@ __device__ __forceinline__ void moe_group_body(const uint* __restrict__ idx, uin
     for (uint a0 = tid; a0 < NA; a0 += 8u * 256u) {
         uint e[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(idx[a0 + (uint)u * 256u], E - 1u) : 0xFFFFFFFFu;
+        for (int u = 0; u < 8; u++) e[u] = idx[min(a0 + (uint)u * 256u, NA - 1u)];
+#pragma unroll
+        for (int u = 0; u < 8; u++) e[u] = a0 + (uint)u * 256u < NA ? min(e[u], E - 1u) : 0xFFFFFFFFu;
 #pragma unroll
         for (int u = 0; u < 8; u++)
             if (e[u] < E) list[off[e[u]] + atomicAdd(&cnt[e[u]], 1u)] = a0 + (uint)u * 256u;
@@ -774,10 +778,10 @@ moe_topk_quant(const float* __restrict__ lg, uint* __restrict__ idx, float* __re
 //   moe_gu_q4k_mil(the same)                                          K <= 2048, beyond that _mil
 //   moe_down_{q4k,q5k,q6k}_mi(act, wd, dv, idx, K, N, NA, E)          grid [ceil(N / R), min(E, NA), 1] x 256, K <= 2048;
 //                                                                     R = 64 for K <= 512, 32 for K <= 1024, else 16
-// The _m entries' products and sums, bit for bit, over at most 4096 assignments as the router leaves them.  Workgroup y serves
+// The _m entries' products and sums, bit for bit, over at most MI_MOST assignments as the router leaves them.  Workgroup y serves
 // expert y, or with fewer assignments than experts the expert of assignment y if no earlier one has it: what finds its
 // expert's assignments is one load or a few of idx, no launch, and at 4 tokens a quarter of 128 experts' workgroups is
-// launched.  The down entries quantize the f32 activations they need into LDS (quantize_q8k's operations), 16 KB at a time.
+// launched.  The down entries quantize the f32 activations they need into LDS (quantize_q8k's operations), MI_STAGE codes at a time.
 // A row of up to 1024 (512) weights takes half (a quarter of) the lanes, so the wave holds two (four) rows side by side; a
 // longer one than 2048 is walked with four assignments' sums beside it, so that their expert's rows are read once and not
 // once each.  Whole layer: 96 experts of 768 x 2816 at 16 tokens 92.9 -> 85.6 us, of 512 x 1536 (Q6_K down) at 8 26.6 -> 19.6,
@@ -814,7 +818,9 @@ __device__ __forceinline__ MiFound<NQ> mi_find(const uint* __restrict__ idx, uin
     const bool by_a = NA < E;
     uint v[NQ];
 #pragma unroll
-    for (uint q = 0; q < NQ; q++) v[q] = 64u * q < NA && lane + 64u * q < NA ? min(idx[lane + 64u * q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
+    for (uint q = 0; q < NQ; q++) v[q] = 64u * q < NA ? idx[min(lane + 64u * q, NA - 1u)] : 0u;
+#pragma unroll
+    for (uint q = 0; q < NQ; q++) v[q] = lane + 64u * q < NA ? min(v[q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
     MiFound<NQ> f;
     f.e = by_a ? min((uint)__builtin_amdgcn_readfirstlane((int)idx[y]), E - 1u) : y;
     bool first = true;
@@ -904,7 +910,7 @@ moe_gu_q4k_mi(const signed char* __restrict__ xq, const float* __restrict__ xs, 
         if (K <= 1024u) moe_gu_mi_body<4, false>(xq, xs, wg, wu, act, K, N, KSEL, f);
         else moe_gu_mi_body<8, false>(xq, xs, wg, wu, act, K, N, KSEL, f);
     } else {
-        const MiFound<8> f = mi_find<8>(idx, NA, E);
+        const MiFound<MI_MOST / 64u> f = mi_find<MI_MOST / 64u>(idx, NA, E);
         if (K <= 1024u) moe_gu_mi_body<4, false>(xq, xs, wg, wu, act, K, N, KSEL, f);
         else moe_gu_mi_body<8, false>(xq, xs, wg, wu, act, K, N, KSEL, f);
     }
@@ -914,7 +920,7 @@ extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_pe
 moe_gu_q4k_mil(const signed char* __restrict__ xq, const float* __restrict__ xs, const uchar* __restrict__ wg,
                const uchar* __restrict__ wu, float* __restrict__ act, const uint* __restrict__ idx, uint K, uint N, uint KSEL, uint NA, uint E) {
     if (NA <= 128u) moe_gu_mi_body<8, true>(xq, xs, wg, wu, act, K, N, KSEL, mi_find<2>(idx, NA, E));
-    else moe_gu_mi_body<8, true>(xq, xs, wg, wu, act, K, N, KSEL, mi_find<8>(idx, NA, E));
+    else moe_gu_mi_body<8, true>(xq, xs, wg, wu, act, K, N, KSEL, mi_find<MI_MOST / 64u>(idx, NA, E));
 }
 
 #define MI_STAGE 8192u
@@ -974,7 +980,7 @@ __device__ __forceinline__ void moe_down_mi_pick(const float* __restrict__ act, 
         __shared__ __align__(16) signed char lq[MI_STAGE];                                                                   \
         __shared__ float ls[MI_STAGE / 256u];                                                                                \
         if (NA <= 128u) moe_down_mi_pick<W>(act, wd, dv, K, N, mi_find<2>(idx, NA, E), lq, ls);                              \
-        else moe_down_mi_pick<W>(act, wd, dv, K, N, mi_find<8>(idx, NA, E), lq, ls);                                         \
+        else moe_down_mi_pick<W>(act, wd, dv, K, N, mi_find<MI_MOST / 64u>(idx, NA, E), lq, ls);                                         \
     }
 MOE_DOWN_MI(q4k, W4k)
 MOE_DOWN_MI(q5k, W5k)
@@ -1470,7 +1476,9 @@ __device__ __forceinline__ MtFound mt_find(const uint* __restrict__ idx, uint NA
     const bool by_a = NA < E;
     uint v[8], mine = 0u, ahead = 0u;
 #pragma unroll
-    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? min(idx[first + 64u * q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
+    for (uint q = 0; q < 8u; q++) v[q] = q < steps ? idx[min(first + 64u * q, NA - 1u)] : 0u;
+#pragma unroll
+    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? min(v[q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
     const uint e = by_a ? min((uint)__builtin_amdgcn_readfirstlane((int)idx[y]), E - 1u) : y;
 #pragma unroll
     for (uint q = 0; q < 8u; q++) {

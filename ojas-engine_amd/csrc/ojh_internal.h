@@ -207,7 +207,7 @@ int ojh_mm_q8k_launch(ojh_device *dev, void *xq, void *xs, const ojh_lin *w, con
 int ojh_noalloc_setup(ojh_device *dev);   // resolves the static scratch array on the current GPU (ojh_noalloc.cpp)
 void ojh_gemm_q8k_tiles(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t M, uint32_t *rw, uint32_t *rt);   // row tiles per workgroup / per wave of gemm_q8k_q4k_mf
 uint32_t ojh_moe_mt_groups(const ojh_device *dev, uint32_t K, uint32_t N, uint32_t E, bool gu, uint32_t *threads);   // workgroups per expert of those entries, and their threads
-constexpr uint32_t OJH_MOE_FOUND = 4096, OJH_MOE_FOUND_BITS = 512;   // most assignments that the _ti (_mi, _mj) expert products look through themselves
+constexpr uint32_t OJH_MOE_FOUND = 4096, OJH_MOE_FOUND_BITS = 512;   // most assignments that the _ti (_mi) expert products look through themselves
 uint64_t ojh_moe_ti_lds(uint32_t K, uint32_t NA);   // LDS bytes of moe_{gu,down}_*_ti where one expert has every assignment
 uint64_t ojh_moe_mt_lds(uint32_t K);                // LDS bytes of moe_{gu,down}_q4k_mt (ojh_manifest.cpp)
 uint64_t ojh_gemm_q8k_mk_lds(uint32_t K, uint32_t M);   // LDS bytes of gemm_q8k_q4k_mk (ojh_manifest.cpp)
