@@ -1476,10 +1476,11 @@ __device__ __forceinline__ MtFound mt_find(const uint* __restrict__ idx, uint NA
     const bool by_a = NA < E;
     uint v[8], mine = 0u, ahead = 0u;
 #pragma unroll
-    for (uint q = 0; q < 8u; q++) v[q] = q < steps ? idx[min(first + 64u * q, NA - 1u)] : 0u;
-#pragma unroll
-    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? min(v[q], E - 1u) : 0xFFFFFFFFu;   // (as moe_group)
+    for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? idx[first + 64u * q] : 0xFFFFFFFFu;
     const uint e = by_a ? min((uint)__builtin_amdgcn_readfirstlane((int)idx[y]), E - 1u) : y;
+    if (e == E - 1u)        // (only its workgroups clamp what they have loaded, as moe_group does)
+#pragma unroll
+        for (uint q = 0; q < 8u; q++) v[q] = q < steps && first + 64u * q < NA ? min(v[q], E - 1u) : 0xFFFFFFFFu;
 #pragma unroll
     for (uint q = 0; q < 8u; q++) {
         mine += (uint)__popcll(__ballot(v[q] == e));
