@@ -275,9 +275,9 @@ def main() -> int:
                                "(q,k,v,o 4096; gate,up 14336x4096; down 4096x14336; head 128256x4096), "
                                "f32 activations N(0,1) quantized once per stage, weights in HBM",
                    "bytes_per_step": step_bytes, "weight_sets": args.copies,
-                   "launches_per_step": "one ojh_mm_multi call per stage: q/k/v in 1 launch with the quantizer folded in "
-                                        "(gemv_fq8k_q4k_x4_r2), the other four stages quantize_q8k + one gemv_q8k_q4k* launch "
-                                        "(gate/up grouped over separate tensors): 9 launches" if staged else
+                   "launches_per_step": "one ojh_mm_multi call per stage: q/k/v, o, gate/up and down in 1 launch each with the quantizer "
+                                        "folded in (gemv_fq8k_q4k_x4_r2), the head quantize_q8k + gemv_q8k_q4k_wide: "
+                                        "6 launches" if staged else
                                         "5 quantize_q8k + 5 gemv_q8k_q4k* (q/k/v and gate/up each one grouped "
                                         "launch over separate tensors)" if grouped else
                                         "5 quantize_q8k + 8 gemv_q8k_q4k*" if (not args.fused_quant) else
@@ -450,9 +450,9 @@ def extras(gpu, pkg, lin_q) -> dict:
                                        "int8_mfma_frac": round(2.0 * m * n * k / us / 1e6 / 5000.0, 4)}
                 del xf, y
             lin.free()
-        out[f"verify_prefill_{tag}_int8"] = {"arithmetic": "quant_q8k activations, integer dots per scale group on the int8 matrix cores "
-                                                           f"(v_mfma_i32_32x32x16_i8 per 16 weights of Q6_K, 32x32x32 per 32 of Q5_K), the scale "
-                                                           "a 24-bit multiply-add per result: dot_q6k / dot_q5k within 2e-5 of peak",
+        out[f"verify_prefill_{tag}_int8"] = {"arithmetic": "quant_q8k activations, scale x code as two int8 digits on the int8 matrix cores "
+                                                           "(v_mfma_i32_32x32x32_i8 twice per 32 weights), one f32 update per super-block: "
+                                                           "dot_q6k / dot_q5k within 2e-5 of peak",
                                              "peak_tops": 5000.0, "timed": f"quantize_q8k + gemm_q8k_{tag}_gs{{,_sr}}", **fam}
     # ---- speculative verify on the Q4_K output head of the decode step, bf16 activations
     head4 = lin_q[2]
@@ -591,10 +591,10 @@ def extras(gpu, pkg, lin_q) -> dict:
         fl = 2.0 * T * ksel * 3 * nff * d
         moe[f"T{T}"] = {"us": round(us, 1), "distinct_experts": distinct, "gbs": round(b / us / 1e3, 1),
                         "tflops": round(fl / us / 1e6, 2)}
-    out["moe_ffn_q4k_128x_top8"] = {"timed": "router + expert FFN, ojh_moe_ffn_routed (T <= 2: gate/up, the router inside it, and down launches addressed by assignment; above: router, quantize + group in one launch, gate/up, quantize, down, combine; T = 256 on int8 MFMA, moe_{gu,down}_q4k_mt, 32 assignments per staged pass)", **moe}
+    out["moe_ffn_q4k_128x_top8"] = {"timed": "router + expert FFN, ojh_moe_ffn_routed (T <= 2: gate/up, the router inside it, and down launches addressed by assignment; T = 16: router, quantize + group in one launch, gate/up, quantize, down, combine, integer dots moe_{gu,down}_q4k_m; T = 256: router + quantize in one launch, gate/up, down, combine, int8 MFMA moe_{gu,down}_q4k_ti)", **moe}
     del gate, up, down
-    # the same layer with finer expert tensors in a prefill batch: Q6_K down (int8 matrix tile per expert from 10
-    # assignments per expert) and all-Q8_0 experts (grouped f16 matrix tile from 4 per expert)
+    # the same layer with finer expert tensors in a prefill batch: Q6_K down (int8 MFMA, wave tiles
+    # moe_down_q6k_{ti,mt}) and all-Q8_0 experts (grouped f16 matrix tile from 4 per expert)
     mixed = {}
     gate = gpu.lin(pkg.Q4_K, E * nff, d, synth.q4k_weights(E * nff, d, "bench", "moe_gate"))
     up = gpu.lin(pkg.Q4_K, E * nff, d, synth.q4k_weights(E * nff, d, "bench", "moe_up"))
