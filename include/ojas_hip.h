@@ -378,22 +378,24 @@ int ojh_moe_route(ojh_device *dev, const ojh_buf *logits, uint32_t n_tokens, uin
  * OJH_ACT_AUTO and OJH_ACT_Q8K keep the CPU path's int8-activation arithmetic for them.
  * Expert indices must be below n_expert (one that is not never reads outside the tensors; what
  * it contributes is unspecified, but comes of this call alone: the router's ~0 for a token with a NaN or infinite logit
- * counts as the last expert for K-quant and grouped experts, as nothing for the per-assignment f32 kernels). Up to 2 tokens run as two launches addressed
+ * counts as the last expert for K-quant and grouped experts, as nothing for the per-assignment f32 kernels). One token, two while
+ * the experts of their assignments take up to 32 MB, more up to 16 MB, run as two launches addressed
  * by assignment (bit-identical to the grouped integer-dot pipeline) when d <= 8192, n_ff <= 2048,
  * ksel <= 64 and ksel * n_ff <= 32768 (beyond that the grouped pipeline serves them; forcing the
  * two-launch form with OJAS_HIP_MOE=3 then returns OJH_ERR_UNSUPPORTED); larger batches are grouped
- * by expert, on int8 MFMA from three to four assignments per expert (sums associate differently there:
- * last ulps). Environment: OJAS_HIP_MOE = 1 / 2 / 3 forces MFMA / grouped dots / the decode
- * form, OJAS_HIP_MOE_DEC_TOKENS moves the 8. */
+ * by expert, on int8 MFMA from one to four assignments per expert, by the layer's sizes (sums associate
+ * differently there: last ulps). Environment: OJAS_HIP_MOE = 1 / 2 / 3 forces MFMA / grouped dots / the
+ * decode form, OJAS_HIP_MOE_DEC_TOKENS gives the number of tokens up to which the decode form runs. */
 int ojh_moe_ffn(ojh_device *dev, const ojh_buf *x, uint32_t n_tokens, uint32_t d, uint32_t n_ff,
                 uint32_t n_expert, uint32_t ksel, const ojh_buf *idx, const ojh_buf *wgt,
                 const ojh_lin *gate, const ojh_lin *up, const ojh_lin *down, ojh_buf *y,
                 int accum, int act_mode);
 
 /* Router and expert FFN in one call: logits [n_tokens][n_expert] f32 -> idx, wgt [n_tokens][ksel] (written: softmax,
- * top ksel, renormalised — ojh_moe_route's arithmetic, the same bits) -> y as ojh_moe_ffn.  For up to 2 tokens over
- * Q4_K gate / up experts (the decode form of ojh_moe_ffn and its limits) the router runs inside the gate/up launch:
- * two launches per layer and token instead of three; every other case is ojh_moe_route followed by ojh_moe_ffn.
+ * top ksel, renormalised — ojh_moe_route's arithmetic, the same bits) -> y as ojh_moe_ffn.  For Q4_K gate / up
+ * experts in the decode form (one token, a few over small experts) the router runs inside the gate/up launch: two
+ * launches per layer instead of three; where the expert products find their assignments in idx themselves (up to 4096
+ * of them) it shares the quantizer's launch; every other case is ojh_moe_route followed by ojh_moe_ffn.
  * The op-level seam of the reference takes router logits or (idx, wgt) alike (ojas-cuda moe.rs:45-125 run back to
  * back by its decoders); OJAS_HIP_MOE_ROUTE_FUSE=0 keeps the router a launch of its own. */
 int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t n_tokens, uint32_t d, uint32_t n_ff,
