@@ -121,7 +121,8 @@ static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32
 
 // Router + expert FFN.  A few tokens over Q4_K gate / up experts: the router runs inside the gate/up launch of the
 // decode form (every workgroup routes its token itself; idx / wgt are written for the down launch and for the
-// caller) — two launches per layer instead of three; otherwise ojh_moe_route, then ojh_moe_ffn.
+// caller) — two launches per layer instead of three.  Products that find their assignments: the router shares the quantizer's
+// launch.  Otherwise ojh_moe_route, then ojh_moe_ffn.
 extern "C" int ojh_moe_ffn_routed(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32_t n_ff, uint32_t E,
                                   uint32_t ksel, const ojh_buf *logits, ojh_buf *idx, ojh_buf *wgt, const ojh_lin *gate,
                                   const ojh_lin *up, const ojh_lin *down, ojh_buf *y, int accum, int act_mode) {
@@ -305,7 +306,7 @@ static int ffn(ojh_device *dev, const ojh_buf *x, uint32_t T, uint32_t d, uint32
     if (gate->type != OJH_Q4_K || up->type != OJH_Q4_K || (down->type != OJH_Q4_K && down->type != OJH_Q5_K && down->type != OJH_Q6_K))
         return ojh_fail(OJH_ERR_UNSUPPORTED, "moe_ffn: gate and up must be Q4_K with down Q4_K, Q5_K or Q6_K, or gate/up among Q8_0, IQ4_XS, IQ4_NL, IQ3_S, IQ2_XXS, IQ2_S with down among Q8_0, IQ4_XS, IQ4_NL, IQ2_XXS, IQ3_XXS (gate %u, up %u, down %u)",
                         gate->type, up->type, down->type);
-    const bool down5 = down->type != OJH_Q4_K;   // Q5_K or Q6_K down tensors: integer dots at every batch size
+    const bool down5 = down->type != OJH_Q4_K;   // Q5_K or Q6_K down tensors have no workgroup-per-tile form: integer dots in its place
     const std::string down_dec = std::string("moe_down_") + ojh_format(down->type)->tag + "_dec";
     const std::string down_m = std::string("moe_down_") + ojh_format(down->type)->tag + "_m";
     const std::string down_mt = std::string("moe_down_") + ojh_format(down->type)->tag + "_mt";
